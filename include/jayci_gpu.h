@@ -160,8 +160,11 @@ typedef struct jci_ham jci_ham;
 #define JCI_SIGMA_PAIRS_SYM64 3
 #define JCI_SIGMA_DIRECT64 4
 #define JCI_SIGMA_DIRECT32 5
-#define JCI_SIGMA_FAST64 6  /* matrix-free, excitation tables, FP64 */
-#define JCI_SIGMA_FAST32 7  /* matrix-free, excitation tables, FP32 accumulation */
+#define JCI_SIGMA_FAST64 6  /* matrix-free, FP64: spaces of several blocks by dense products
+                               over their strings' replacements on MFMA, the others (and
+                               after jci_ham_fast_tiles / _split / _xcd set a shape) from
+                               excitation tables */
+#define JCI_SIGMA_FAST32 7  /* ... FP32 products and sums */
 #define JCI_SIGMA_FCI64 8   /* matrix-free, single-block (FCI) spaces, n <= 16, FP64 */
 #define JCI_SIGMA_FCI32 9   /* ... FP32 accumulation */
 #define JCI_SIGMA_GEMM64 10 /* dense-string full-CI sigma on MFMA (n <= 15, <= 65535 strings
@@ -248,7 +251,8 @@ int jci_sigma(jci_ham *h, int method, int nvec, const double *x, double *y);
  * needing more returns -1 with the sizes in jci_last_error() (the dense-string sigma then
  * runs its vectors in as many passes as the array allows, one vector of up to about
  * 128 MiB / (8 La) determinants in FP64).  All calls on one GPU share the array, so calls
- * that overlap on one GPU race; results equal jci_sigma_dev's bit for bit. */
+ * that overlap on one GPU race; results equal jci_sigma_dev's bit for bit.  (Truncated spaces
+ * that this size admits keep one vector's buffers with the Hamiltonian besides.) */
 int jci_sigma_dev_noalloc(jci_ham *h, int method, int nvec, const double *x_dev, double *y_dev);
 long long jci_sigma_noalloc_capacity(void);
 
@@ -332,13 +336,14 @@ int jci_bench_copy(jci_ctx *ctx, long long bytes, int reps, double *ms_per_launc
  * NULL) gets ms per launch indexed by JCI_SIGMA_* (0 where not available). */
 int jci_ham_autotune(jci_ham *h, int nvec, int reps, int *best64, int *best32, double *times);
 /* times[] above has JCI_SIGMA_GEMM32 + 1 entries */
-/* beta strings per tile of the matrix-free sigma (0 without excitation tables) */
+/* beta strings per tile of the table sigma (0 without excitation tables, or per block) */
 int jci_ham_fast_width(const jci_ham *h);
 /* tile shape of the matrix-free table sigma (the autotuner sets it): *width beta strings per
  * work-group (64, 128 or 256; 0 = per block, the smallest of 64 .. 512 that covers the
  * block's row, one launch per width) and *chunk alpha singles staged together (1, 2, 4 or 8;
  * 0 = the most that fit 64 KB of LDS, at most 4); values >= 0 set, -1 keeps; both are
- * returned */
+ * returned.  Setting any of the three shapes below makes the FAST methods of this Hamiltonian
+ * run the table kernels (their doubles tables are built then, if they were not needed so far) */
 int jci_ham_fast_tiles(jci_ham *h, int *width, int *chunk);
 /* *split 0: the table sigma runs as one fused kernel; 1..3: as two passes over the input
  * and a block-transposed copy of it (N * nvec more device elements): one spin's singles and

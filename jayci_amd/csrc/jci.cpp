@@ -4,6 +4,7 @@
 #include "slater.h"
 #include "sigma_fast.h"
 #include "sigma_gemm.h"
+#include "sigma_tx.h"
 #include "../../include/jayci_gpu.h"
 
 #include <math.h>
@@ -299,6 +300,17 @@ struct jci_ham {
     long long *d_tt_off, ntt;   // 16 x 16 transpose tiles per block
     void *d_xT;                 // block-transposed input
     size_t xT_bytes;
+    // contraction form of the truncated spaces' sigma (sigma_tx.h): the default of the FAST
+    // methods where it applies; a table-kernel shape chosen by the caller turns it off
+    TxPlan *tx;
+    TxDev txd;
+    int tx_off;
+    void *tx_mem[24];           // device arrays behind txd
+    int tx_nmem;
+    long long *d_ttx, nttx;     // 16 x 16 transpose tiles per block
+    void *d_txE, *d_txv, *d_txT, *d_txy;
+    size_t txE_bytes, txv_bytes, txT_bytes, txy_bytes;
+    int have_tables;            // doubles tables and launch maps of the table kernels built
     int have_fci;               // single-block space with n <= 16: FCI kernel usable
     FciArgs fci;
     int tuned64, tuned32;       // autotuned default methods (0 = not tuned)
@@ -517,43 +529,53 @@ static int set_orient(jci_ham *h)
     return 0;
 }
 
-static int build_fast(jci_ham *h, int W)
+// excitation tables of every string: the singles (kind 1), the doubles (2) or both (3)
+static int build_exc(jci_ham *h, int kind)
 {
     jci_space *s = h->sp;
     jci_ctx *c = s->ctx;
     const SpaceDesc &D = s->h;
-    bool same = s->na == s->nb;
+    const bool same = s->na == s->nb;
     for (int spin = 0; spin < (same ? 1 : 2); spin++) {
-        long long n = D.s[spin].gstart[D.s[spin].ngrp];
-        long long *c1, *c2;
-        int G = D.s[spin].ngrp;
-        JCI_CHECK(hipMallocAsync((void **)&c1, sizeof(long long) * (n + 1), c->stream));
-        JCI_CHECK(hipMallocAsync((void **)&c2, sizeof(long long) * (n + 1), c->stream));
-        JCI_CHECK(hipMalloc(&h->d_off1[spin], sizeof(long long) * (n + 1)));
-        JCI_CHECK(hipMalloc(&h->d_off2[spin], sizeof(long long) * (n + 1)));
-        JCI_CHECK(hipMalloc(&h->d_goff1[spin], sizeof(int) * n * (G + 1)));
-        JCI_CHECK(hipMalloc(&h->d_goff2[spin], sizeof(int) * n * (G + 1)));
-        RCHECK(jk_exc_count(s->d_desc, spin, n, s->d_mask[spin], c->d_binom, c1, c2,
+        const long long n = D.s[spin].gstart[D.s[spin].ngrp];
+        const int G = D.s[spin].ngrp;
+        long long *c1 = nullptr, *c2 = nullptr;
+        if (kind & 1) {
+            JCI_CHECK(hipMallocAsync((void **)&c1, sizeof(long long) * (n + 1), c->stream));
+            JCI_CHECK(hipMalloc(&h->d_off1[spin], sizeof(long long) * (n + 1)));
+            JCI_CHECK(hipMalloc(&h->d_goff1[spin], sizeof(int) * n * (G + 1)));
+        }
+        if (kind & 2) {
+            JCI_CHECK(hipMallocAsync((void **)&c2, sizeof(long long) * (n + 1), c->stream));
+            JCI_CHECK(hipMalloc(&h->d_off2[spin], sizeof(long long) * (n + 1)));
+            JCI_CHECK(hipMalloc(&h->d_goff2[spin], sizeof(int) * n * (G + 1)));
+        }
+        RCHECK(jk_exc_count(kind, s->d_desc, spin, n, s->d_mask[spin], c->d_binom, c1, c2,
                             h->d_goff1[spin], h->d_goff2[spin], c->stream));
-        RCHECK(jk_scan(c1, h->d_off1[spin], n, c->stream));
-        RCHECK(jk_scan(c2, h->d_off2[spin], n, c->stream));
-        JCI_CHECK(hipMemcpyAsync(&h->nexc1[spin], h->d_off1[spin] + n, sizeof(long long),
-                                 hipMemcpyDeviceToHost, c->stream));
-        JCI_CHECK(hipMemcpyAsync(&h->nexc2[spin], h->d_off2[spin] + n, sizeof(long long),
-                                 hipMemcpyDeviceToHost, c->stream));
+        if (kind & 1) {
+            RCHECK(jk_scan(c1, h->d_off1[spin], n, c->stream));
+            JCI_CHECK(hipMemcpyAsync(&h->nexc1[spin], h->d_off1[spin] + n, sizeof(long long),
+                                     hipMemcpyDeviceToHost, c->stream));
+        }
+        if (kind & 2) {
+            RCHECK(jk_scan(c2, h->d_off2[spin], n, c->stream));
+            JCI_CHECK(hipMemcpyAsync(&h->nexc2[spin], h->d_off2[spin] + n, sizeof(long long),
+                                     hipMemcpyDeviceToHost, c->stream));
+        }
         JCI_CHECK(hipStreamSynchronize(c->stream));
-        hipFreeAsync(c1, c->stream);
-        hipFreeAsync(c2, c->stream);
-        size_t a1 = h->nexc1[spin] > 0 ? h->nexc1[spin] : 1, a2 = h->nexc2[spin] > 0 ? h->nexc2[spin] : 1;
-        if (hipMalloc(&h->d_e1[spin], sizeof(int2) * a1) != hipSuccess ||
-            hipMalloc(&h->d_v1[spin], sizeof(double) * a1) != hipSuccess ||
-            hipMalloc(&h->d_e2[spin], sizeof(int2) * a2) != hipSuccess ||
-            hipMalloc(&h->d_v2[spin], sizeof(double) * a2) != hipSuccess) {
+        if (c1) hipFreeAsync(c1, c->stream);
+        if (c2) hipFreeAsync(c2, c->stream);
+        const size_t a1 = h->nexc1[spin] > 0 ? h->nexc1[spin] : 1, a2 = h->nexc2[spin] > 0 ? h->nexc2[spin] : 1;
+        if (((kind & 1) && (hipMalloc(&h->d_e1[spin], sizeof(int2) * a1) != hipSuccess ||
+                            hipMalloc(&h->d_v1[spin], sizeof(double) * a1) != hipSuccess)) ||
+            ((kind & 2) && (hipMalloc(&h->d_e2[spin], sizeof(int2) * a2) != hipSuccess ||
+                            hipMalloc(&h->d_v2[spin], sizeof(double) * a2) != hipSuccess))) {
+            (void)hipGetLastError();
             jci_set_error("excitation tables: out of device memory (%lld + %lld entries)",
                           h->nexc1[spin], h->nexc2[spin]);
             return -3;
         }
-        RCHECK(jk_exc_fill(s->d_desc, spin, n, s->d_mask[spin], c->d_binom, h->d_m1, h->d_m2,
+        RCHECK(jk_exc_fill(kind, s->d_desc, spin, n, s->d_mask[spin], c->d_binom, h->d_m1, h->d_m2,
                            h->d_off1[spin], h->d_off2[spin], h->d_goff1[spin], h->d_goff2[spin],
                            h->d_e1[spin], h->d_v1[spin], h->d_e2[spin], h->d_v2[spin], c->stream));
     }
@@ -564,9 +586,224 @@ static int build_fast(jci_ham *h, int W)
         h->d_v1[1] = h->d_v1[0]; h->d_v2[1] = h->d_v2[0];
         h->nexc1[1] = h->nexc1[0]; h->nexc2[1] = h->nexc2[0];
     }
-    int n = D.norbs, mp = n * (n + 1) / 2;
+    return 0;
+}
+
+static void free_doubles(jci_ham *h)
+{
+    for (int sp = 0; sp < 2; sp++) {
+        if (sp == 1 && h->d_off2[1] == h->d_off2[0]) break;
+        hipFree(h->d_off2[sp]); hipFree(h->d_goff2[sp]); hipFree(h->d_e2[sp]); hipFree(h->d_v2[sp]);
+    }
+    for (int sp = 0; sp < 2; sp++) {
+        h->d_off2[sp] = nullptr; h->d_goff2[sp] = nullptr; h->d_e2[sp] = nullptr; h->d_v2[sp] = nullptr;
+    }
+}
+
+// vectors up to this many determinants keep one vector's buffers of the contraction form from
+// the start, for the allocation-free entry point (its own staging bounds the larger ones out)
+#define TX_NOALLOC_DETS (16LL << 20)
+// elements of the intermediate per vector and round: 32M (256 MB in FP64)
+#define TX_ELEMS (32LL << 20)
+
+static int grow(void **p, size_t *have, size_t want, const char *what);
+
+// buffers of nvec vectors; copy: the input is converted or gathered into vector-major form
+static int tx_buffers(jci_ham *h, int nvec, bool copy)
+{
+    const size_t N = (size_t)h->sp->h.ndets;
+    RCHECK(grow(&h->d_txE, &h->txE_bytes, sizeof(double) * nvec * (size_t)h->tx->elems, "the intermediate"));
+    if (copy) RCHECK(grow(&h->d_txv, &h->txv_bytes, sizeof(double) * nvec * N, "the input vectors"));
+    RCHECK(grow(&h->d_txT, &h->txT_bytes, sizeof(double) * nvec * N, "the transposed input"));
+    return grow(&h->d_txy, &h->txy_bytes, sizeof(double) * nvec * N, "the transposed result");
+}
+
+static int tx_upload(jci_ham *h, const void *src, size_t bytes, void **out)
+{
+    jci_ctx *c = h->sp->ctx;
+    void *d = nullptr;
+    if (hipMalloc(&d, bytes ? bytes : 16) != hipSuccess) {
+        (void)hipGetLastError();
+        jci_set_error("contraction lists: out of device memory (%zu bytes)", bytes);
+        return -3;
+    }
+    h->tx_mem[h->tx_nmem++] = d;
+    *out = d;
+    if (src && bytes) {
+        JCI_CHECK(hipMemcpyAsync(d, src, bytes, hipMemcpyHostToDevice, c->stream));
+        JCI_CHECK(hipStreamSynchronize(c->stream));   // src is the caller's pageable memory
+    }
+    return 0;
+}
+
+// lists and tables of the contraction form; leaves h->tx null where it does not apply
+static int build_tx(jci_ham *h)
+{
+    jci_space *s = h->sp;
+    jci_ctx *c = s->ctx;
+    const SpaceDesc &D = s->h;
+    SpaceDesc T;
+    jci_transpose_desc(D, &T);
+    TxPlan *P = new TxPlan();
+    if (tx_plan(D, T, TX_ELEMS, P)) {
+        delete P;
+        return 0;
+    }
+    h->tx = P;
+    const bool same = s->na == s->nb;
+    const int n = D.norbs, mp = n * (n + 1) / 2, np = n * (n - 1) / 2;
+    TxDev &d = h->txd;
+    memset(&d, 0, sizeof(d));
+    d.m1 = mp;
+    d.np = np;
+    d.nint = D.ndocc + D.nactv;
+    d.ms = mp + 1;
+    for (int sp = 0; sp < (same ? 1 : 2); sp++) {
+        const SpinDesc &S = D.s[sp];
+        const long long ns = S.gstart[S.ngrp];
+        TxSpin &x = d.s[sp];
+        x.mask = s->d_mask[sp];
+        x.off1 = h->d_off1[sp];
+        x.e1 = h->d_e1[sp];
+        x.goff1 = h->d_goff1[sp];
+        x.G = S.ngrp;
+        x.npair = S.nelec * (S.nelec - 1) / 2;
+        RCHECK(tx_upload(h, nullptr, sizeof(uint32_t) * (size_t)P->nlst[sp], (void **)&x.lst));
+        RCHECK(tx_upload(h, nullptr, sizeof(uint16_t) * (size_t)h->nexc1[sp], (void **)&x.rk));
+        RCHECK(tx_upload(h, nullptr, sizeof(int2) * (size_t)P->nkl[sp], (void **)&x.kl));
+        RCHECK(tx_upload(h, nullptr, sizeof(int2) * (size_t)ns * x.npair, (void **)&x.gl));
+        RCHECK(tx_upload(h, nullptr, sizeof(double) * (size_t)np * np, (void **)&x.w64));
+        RCHECK(tx_upload(h, nullptr, sizeof(float) * (size_t)np * np, (void **)&x.w32));
+        const size_t nrow = (size_t)mp + P->nint_parts[sp] + 1;
+        x.zrow = (int)nrow - 1;
+        RCHECK(tx_upload(h, nullptr, sizeof(double) * nrow * d.ms, (void **)&x.m64));
+        RCHECK(tx_upload(h, nullptr, sizeof(float) * nrow * d.ms, (void **)&x.m32));
+        TxList *dl = nullptr;
+        TxPairGroup *dp = nullptr;
+        JCI_CHECK(hipMallocAsync((void **)&dl, sizeof(TxList) * P->lists[sp].size(), c->stream));
+        JCI_CHECK(hipMallocAsync((void **)&dp, sizeof(TxPairGroup) * P->pg[sp].size(), c->stream));
+        JCI_CHECK(hipMemcpyAsync(dl, P->lists[sp].data(), sizeof(TxList) * P->lists[sp].size(),
+                                 hipMemcpyHostToDevice, c->stream));
+        JCI_CHECK(hipMemcpyAsync(dp, P->pg[sp].data(), sizeof(TxPairGroup) * P->pg[sp].size(),
+                                 hipMemcpyHostToDevice, c->stream));
+        RCHECK(jk_tx_fill(P->nlst[sp], (uint32_t *)x.lst, c->stream));
+        RCHECK(jk_tx_lists(s->d_desc, sp, ns, s->d_mask[sp], x.off1, x.e1, x.goff1, dl,
+                           (uint32_t *)x.lst, (uint16_t *)x.rk, c->stream));
+        RCHECK(jk_tx_pairs(s->d_desc, sp, ns, s->d_mask[sp], c->d_binom, dp, (int)P->pg[sp].size(),
+                           x.npair, (int2 *)x.kl, (int2 *)x.gl, c->stream));
+        RCHECK(jk_tx_w(n, S.nelec, h->d_m1, h->d_m2, (double *)x.w64, (float *)x.w32, c->stream));
+        RCHECK(jk_tx_rows(s->d_desc, D, sp, s->d_mask[sp], mp, h->d_m2sq, *P, (double *)x.m64,
+                          (float *)x.m32, c->stream));
+        JCI_CHECK(hipStreamSynchronize(c->stream));
+        hipFreeAsync(dl, c->stream);
+        hipFreeAsync(dp, c->stream);
+    }
+    if (same) d.s[1] = d.s[0];
+    // the small tables in one block
+    std::vector<unsigned char> blob;
+    auto put = [&](const void *p, size_t bytes) {
+        const size_t at = (blob.size() + 255) / 256 * 256;
+        blob.resize(at + bytes);
+        if (bytes) memcpy(blob.data() + at, p, bytes);
+        return at;
+    };
+#define TX_PUT(v) put(P->v.data(), P->v.size() * sizeof(P->v[0]))
+    const size_t o_task = TX_PUT(task), o_slot = TX_PUT(slot), o_ch = TX_PUT(chunk), o_item = TX_PUT(item), o_out = TX_PUT(out),
+                 o_src = TX_PUT(src), o_pt = TX_PUT(ptask), o_pi = TX_PUT(pitem), o_po = TX_PUT(pout),
+                 o_q = TX_PUT(q);
+#undef TX_PUT
+    std::vector<long long> tt(D.nblk + 1, 0);
+    for (int b = 0; b < D.nblk; b++) {
+        const long long na = D.s[0].gn[D.bp[b]], nq = D.s[1].gn[D.bq[b]];
+        tt[b + 1] = tt[b] + ((na + 15) / 16) * ((nq + 15) / 16);
+    }
+    h->nttx = tt[D.nblk];
+    const size_t o_tt = put(tt.data(), sizeof(long long) * tt.size());
+    unsigned char *m;
+    RCHECK(tx_upload(h, blob.data(), blob.size(), (void **)&m));
+    d.task = (const TxTask *)(m + o_task);
+    d.slot = (const TxSlot *)(m + o_slot);
+    d.chunk = (const TxChunk *)(m + o_ch);
+    d.item = (const TxItem *)(m + o_item);
+    d.out = (const TxOut *)(m + o_out);
+    d.src = (const TxSrc *)(m + o_src);
+    d.ptask = (const TxPairTask *)(m + o_pt);
+    d.pitem = (const TxPairItem *)(m + o_pi);
+    d.pout = (const TxPairOut *)(m + o_po);
+    d.q = (const int *)(m + o_q);
+    h->d_ttx = (long long *)(m + o_tt);
+    if (D.ndets <= TX_NOALLOC_DETS) RCHECK(tx_buffers(h, 1, true));
+    return 0;
+}
+
+// y = H x in the contraction form: vector k at x + k xk (element stride xs) -> y + k yk (ys)
+static int tx_sigma(jci_ham *h, int prec, int nvec, const double *x, long long xs, long long xk,
+                    double *y, long long ys, long long yk)
+{
+    jci_ctx *c = h->sp->ctx;
+    const long long N = h->sp->h.ndets;
+    const bool copy = prec == 32 || xs != 1;
+    RCHECK(jk_tx_in(prec, nvec, N, h->sp->d_desc, h->d_ttx, h->nttx, x, xs, xk,
+                    copy ? h->d_txv : nullptr, h->d_txT, c->stream));
+    TxVec v;
+    v.x0 = copy ? h->d_txv : (const void *)x;
+    v.ldx0 = copy ? N : xk;
+    v.x1 = h->d_txT;
+    v.ldx1 = N;
+    v.y0 = y;
+    v.ys0 = ys;
+    v.yk0 = yk;
+    v.y1 = (double *)h->d_txy;
+    v.ys1 = 1;
+    v.yk1 = N;
+    RCHECK(jk_tx_run(prec, nvec, h->txd, *h->tx, v, h->d_txE, c->stream));
+    return jk_tx_out(nvec, N, h->sp->d_desc, h->d_ttx, h->nttx, (const double *)h->d_txy, y, ys, yk,
+                     c->stream);
+}
+
+// excitation tables and launch maps of the table kernels.  Spaces that take the contraction
+// form build the doubles tables and the maps only when a table kernel is asked for.
+static int ensure_tables(jci_ham *h);
+
+static int build_fast(jci_ham *h, int W)
+{
+    jci_space *s = h->sp;
+    jci_ctx *c = s->ctx;
+    const SpaceDesc &D = s->h;
+    const bool multi = D.nblk > 1;
+    RCHECK(build_exc(h, multi ? 1 : 3));
+    const int n = D.norbs, mp = n * (n + 1) / 2;
     JCI_CHECK(hipMalloc(&h->d_m2sq, sizeof(double) * (size_t)mp * mp));
     RCHECK(jk_m2_square(mp, h->d_m2, h->d_m2sq, c->stream));
+    h->fast_w = multi ? 3 : W == 64 ? 0 : W == 128 ? 1 : 2;
+    h->fast_split = multi ? 2 : 0;
+    // tiles chunk-major, in runs of 64 per XCD (16e/60o FP64 pass: 9.8 s string-major,
+    // 7.8 s chunk-major, 7.5 s chunk-major in runs of 64)
+    h->fast_cm = 1;
+    h->fast_xg = 64;
+    const int widths[3] = {64, 128, 256};
+    for (int wi = 0; wi < 3; wi++) h->fast[wi].W = widths[wi];
+    if (multi) RCHECK(build_tx(h));
+    h->have_fast = 1;
+    if (!h->tx) RCHECK(ensure_tables(h));
+    return multi ? 0 : build_gf(h);
+}
+
+static int ensure_tables(jci_ham *h)
+{
+    if (h->have_tables) return 0;
+    jci_space *s = h->sp;
+    jci_ctx *c = s->ctx;
+    const SpaceDesc &D = s->h;
+    if (!h->d_off2[0]) {
+        const int rc = build_exc(h, 2);
+        if (rc) {
+            hipStreamSynchronize(c->stream);
+            free_doubles(h);
+            return rc;
+        }
+    }
+    const int mp = D.norbs * (D.norbs + 1) / 2;
     const int widths[3] = {64, 128, 256};
     for (int wi = 0; wi < 3; wi++) {
         int Wd = widths[wi];
@@ -599,7 +836,6 @@ static int build_fast(jci_ham *h, int W)
         a.tout = 0;
         a.src_t = 0;
         a.ntiles = toff[D.nblk];
-        if (Wd == W) h->fast_w = wi;
     }
     // transposed space for the beta-side pass
     {
@@ -640,13 +876,6 @@ static int build_fast(jci_ham *h, int W)
             t.tout = 1;
             t.src_t = 1;
         }
-        h->fast_split = D.nblk > 1 ? 2 : 0;
-        // tiles chunk-major, in runs of 64 per XCD (16e/60o FP64 pass: 9.8 s string-major,
-        // 7.8 s chunk-major, 7.5 s chunk-major in runs of 64)
-        h->fast_cm = 1;
-        h->fast_xg = 64;
-        // spaces of several blocks: per-block widths (set below) by default
-        const bool multi = D.nblk > 1;
         // width classes: rows of nq strings go to the launch of the smallest width >= nq
         // (512 above 256)
         const int cw[4] = {64, 128, 256, 512};
@@ -667,12 +896,10 @@ static int build_fast(jci_ham *h, int W)
             h->fcls[ci].tile_off = h->d_cls_off[ci];
             h->fcls[ci].ntiles = toff[D.nblk];
         }
-        if (multi) h->fast_w = 3;
         for (int i = 0; i < 16; i++)
             JCI_CHECK(hipMalloc(&h->d_ooff[i], sizeof(long long) * (D.nblk + 1)));
         RCHECK(set_orient(h));
     }
-    h->have_fast = 1;
     if (D.nblk == 1 && D.norbs <= FCI_MAXORB) {
         FciArgs &f = h->fci;
         f.ma = s->d_mask[0];
@@ -689,7 +916,9 @@ static int build_fast(jci_ham *h, int W)
         long long maxs = (long long)std::max(s->na, s->nb) * (D.norbs - std::min(s->na, s->nb));
         h->have_fci = (D.s[0].gstart[0] == 0 && D.s[1].gstart[0] == 0 && maxs <= FCI_MAXSINGLES);
     }
-    return build_gf(h);
+    JCI_CHECK(hipStreamSynchronize(c->stream));
+    h->have_tables = 1;
+    return 0;
 }
 
 JCI_API int jci_ham_create(jci_space *s, const double *m1, const double *m2, int flags,
@@ -727,14 +956,16 @@ JCI_API void jci_ham_destroy(jci_ham *h)
     if (!h) return;
     hipSetDevice(h->sp->ctx->device);
     hipStreamSynchronize(h->sp->ctx->stream);
+    for (int i = 0; i < h->tx_nmem; i++) hipFree(h->tx_mem[i]);
+    hipFree(h->d_txE); hipFree(h->d_txv); hipFree(h->d_txT); hipFree(h->d_txy);
+    delete h->tx;
+    free_doubles(h);
     hipFree(h->d_m1); hipFree(h->d_m2); hipFree(h->d_hd);
     hipFree(h->d_rowptr); hipFree(h->d_col); hipFree(h->d_val64); hipFree(h->d_val32);
     hipFree(h->d_xf);
     for (int sp = 0; sp < 2; sp++) {
         if (sp == 1 && h->d_off1[1] == h->d_off1[0]) break;
-        hipFree(h->d_off1[sp]); hipFree(h->d_off2[sp]); hipFree(h->d_e1[sp]);
-        hipFree(h->d_goff1[sp]); hipFree(h->d_goff2[sp]);
-        hipFree(h->d_e2[sp]); hipFree(h->d_v1[sp]); hipFree(h->d_v2[sp]);
+        hipFree(h->d_off1[sp]); hipFree(h->d_e1[sp]); hipFree(h->d_goff1[sp]); hipFree(h->d_v1[sp]);
     }
     hipFree(h->d_m2sq);
     for (int wi = 0; wi < 3; wi++) hipFree(h->d_tile_off[wi]);
@@ -775,6 +1006,7 @@ JCI_API long long jci_ham_string_excitations(jci_ham *h, int spin, long long str
     if (string < 0 || string >= n) { jci_set_error("string_excitations: string out of range"); return -1; }
     jci_ctx *c = h->sp->ctx;
     JCI_CHECK(hipSetDevice(c->device));
+    if (kind == 2) RCHECK(ensure_tables(h));
     const long long *off = kind == 1 ? h->d_off1[spin] : h->d_off2[spin];
     long long b[2];
     JCI_CHECK(hipMemcpyAsync(b, off + string, sizeof(b), hipMemcpyDeviceToHost, c->stream));
@@ -1024,6 +1256,24 @@ static int fast_run(jci_ham *h, int method, int nvec, const double *x, double *y
     const long long N = h->sp->h.ndets;
     if (!h->have_fast) { jci_set_error("sigma: no excitation tables (JCI_DIRECT_TABLES)"); return -1; }
     const int prec = method == JCI_SIGMA_FAST64 ? 64 : 32;
+    if (h->tx && !h->tx_off) {
+        const long long ys = ldy ? 1 : nvec, yk = ldy ? ldy : 1;
+        if (!s) {
+            RCHECK(tx_buffers(h, nvec, prec == 32 || nvec > 1));
+            return tx_sigma(h, prec, nvec, x, nvec, 1, y, ys, yk);
+        }
+        // allocation-free: the staging of the table kernels bounds the sizes taken, the vectors
+        // go one at a time through the buffers kept from the start
+        float *xf;
+        void *xT;
+        if (prec == 32) RCHECK(ensure_xf(h, N * nvec, s, &xf));
+        RCHECK(jci_scratch_carve(s, (size_t)N * nvec * (prec == 64 ? sizeof(double) : sizeof(float)),
+                                 &xT, "the transposed input"));
+        for (int k = 0; k < nvec; k++)
+            RCHECK(tx_sigma(h, prec, 1, x + k, nvec, 1, y + k * yk, ys, yk));
+        return 0;
+    }
+    RCHECK(ensure_tables(h));
     const void *xin = x;
     if (prec == 32) {
         float *xf;
@@ -1255,6 +1505,13 @@ JCI_API int jci_ham_autotune(jci_ham *h, int nvec, int reps, int *best64, int *b
     double best_w_ms = 1e300;
     int best_w = h->fast_w;
     if (h->have_fast) {
+        double tx_ms = 1e300;
+        if (h->tx) {
+            h->tx_off = 0;
+            RCHECK(jci_bench_sigma(h, JCI_SIGMA_FAST64, nvec, reps, &tx_ms));
+        }
+        RCHECK(ensure_tables(h));
+        h->tx_off = 1;
         // beta tile width x alpha chunk of the table kernel
         int best_a = 0, best_split = h->fast_split;
         const int chunks[4] = {0, 1, 2, 4};
@@ -1279,7 +1536,8 @@ JCI_API int jci_ham_autotune(jci_ham *h, int nvec, int reps, int *best64, int *b
             RCHECK(set_orient(h));
         }
         for (int w2 = 0; w2 < 3; w2++) h->fast[w2].A = best_a;
-        t[JCI_SIGMA_FAST64] = best_w_ms;
+        if (tx_ms <= best_w_ms) h->tx_off = 0;
+        t[JCI_SIGMA_FAST64] = std::min(tx_ms, best_w_ms);
         RCHECK(jci_bench_sigma(h, JCI_SIGMA_FAST32, nvec, reps, &t[JCI_SIGMA_FAST32]));
     }
     if (h->have_fci) {
@@ -1326,9 +1584,19 @@ JCI_API int jci_ham_autotune(jci_ham *h, int nvec, int reps, int *best64, int *b
     return 0;
 }
 
+// the FAST methods run the table kernels from here on, in the shape the caller sets
+static int use_tables(jci_ham *h)
+{
+    JCI_CHECK(hipSetDevice(h->sp->ctx->device));
+    RCHECK(ensure_tables(h));
+    h->tx_off = 1;
+    return 0;
+}
+
 JCI_API int jci_ham_fast_tiles(jci_ham *h, int *width, int *chunk)
 {
     if (!h->have_fast) { jci_set_error("ham: no excitation tables"); return -1; }
+    if ((width && *width >= 0) || (chunk && *chunk >= 0)) RCHECK(use_tables(h));
     if (width && *width >= 0) {
         int wi = *width == 64 ? 0 : *width == 128 ? 1 : *width == 256 ? 2 : *width == 0 ? 3 : -1;
         if (wi < 0) {
@@ -1353,6 +1621,7 @@ JCI_API int jci_ham_fast_split(jci_ham *h, int *split)
 {
     if (!h->have_fast) { jci_set_error("ham: no excitation tables"); return -1; }
     if (split && *split > 3) { jci_set_error("ham: split mode %d not 0 .. 3", *split); return -1; }
+    if (split && *split >= 0) RCHECK(use_tables(h));
     if (split && *split >= 0 && *split != h->fast_split) {
         h->fast_split = *split;
         RCHECK(set_orient(h));
@@ -1364,6 +1633,7 @@ JCI_API int jci_ham_fast_split(jci_ham *h, int *split)
 JCI_API int jci_ham_fast_xcd(jci_ham *h, int *group, int *chunk_major)
 {
     if (!h->have_fast) { jci_set_error("ham: no excitation tables"); return -1; }
+    if ((group && *group >= 0) || (chunk_major && *chunk_major >= 0)) RCHECK(use_tables(h));
     if (group && *group >= 0) {
         if (*group > 4096) { jci_set_error("ham: XCD run of %d tiles too long", *group); return -1; }
         h->fast_xg = *group;
@@ -2037,6 +2307,10 @@ static int ham_sigma_cols(void *self, int method, int k, const double *V, long l
     jci_ham *h = (jci_ham *)self;
     method = resolve_method(h, method, 0);
     if (method == JCI_SIGMA_FAST64 || method == JCI_SIGMA_FAST32) {
+        if (h->have_fast && h->tx && !h->tx_off) {
+            RCHECK(tx_buffers(h, k, method == JCI_SIGMA_FAST32));
+            return tx_sigma(h, method == JCI_SIGMA_FAST64 ? 64 : 32, k, V, 1, ldv, S, 1, lds);
+        }
         // the table sigma reads determinant-major input and writes the columns directly
         RCHECK(jk_pack(k, h->sp->h.ndets, V, ldv, stage, h->sp->ctx->stream));
         return fast_run(h, method, k, stage, S, lds, nullptr);
@@ -2114,6 +2388,7 @@ int jci_ham_solve_op(jci_ham *h, const double *d_pre, SolveOp *op)
 int jci_ham_fastargs(jci_ham *h, FastArgs *out)
 {
     if (!h->have_fast) { jci_set_error("batch: the Hamiltonian has no excitation tables"); return -1; }
+    RCHECK(ensure_tables(h));
     *out = h->fast[2];            // the batched sigma uses 256-string beta tiles
     return 0;
 }

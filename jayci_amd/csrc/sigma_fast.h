@@ -50,10 +50,11 @@ struct FciArgs {
 };
 int jk_sigma_fci(int prec, int nvec, const FciArgs &a, const void *x, double *y, hipStream_t st);
 
-int jk_exc_count(const SpaceDesc *d, int spin, long long nstr, const uint64_t *M,
+// tables of the singles (kind 1), the doubles (2) or both (3)
+int jk_exc_count(int kind, const SpaceDesc *d, int spin, long long nstr, const uint64_t *M,
                  const unsigned long long *binom, long long *cnt1, long long *cnt2,
                  int *goff1, int *goff2, hipStream_t st);
-int jk_exc_fill(const SpaceDesc *d, int spin, long long nstr, const uint64_t *M,
+int jk_exc_fill(int kind, const SpaceDesc *d, int spin, long long nstr, const uint64_t *M,
                 const unsigned long long *binom, const double *m1, const double *m2,
                 const long long *off1, const long long *off2, const int *goff1,
                 const int *goff2, int2 *e1, double *v1, int2 *e2, double *v2, hipStream_t st);

@@ -59,7 +59,8 @@ __device__ __forceinline__ long long str_index2(const SpaceDesc *d, int s, uint6
 // Counting pass: per-string totals and per-target-group offsets (goff rows of G+1);
 // fill pass: entries written grouped by target group, in (i, f) enumeration order inside
 // a group.
-template <bool FILL>
+// KIND: 1 singles, 2 doubles, 3 both.
+template <bool FILL, int KIND>
 __global__ void k_exc(const SpaceDesc *__restrict__ d, int spin, long long nstr,
                       const uint64_t *__restrict__ M, const unsigned long long *__restrict__ binom,
                       const double *__restrict__ m1, const double *__restrict__ m2,
@@ -77,12 +78,12 @@ __global__ void k_exc(const SpaceDesc *__restrict__ d, int spin, long long nstr,
     for (int g = 0; g <= G; g++) { c1[g] = 0; c2[g] = 0; }
     if (FILL) {
         for (int g = 0; g <= G; g++) {
-            c1[g] = goff1[I * (G + 1) + g];
-            c2[g] = goff2[I * (G + 1) + g];
+            if (KIND & 1) c1[g] = goff1[I * (G + 1) + g];
+            if (KIND & 2) c2[g] = goff2[I * (G + 1) + g];
         }
     }
-    const long long b1 = FILL ? off1[I] : 0, b2 = FILL ? off2[I] : 0;
-    for (uint64_t x = m; x; x &= x - 1) {
+    const long long b1 = FILL && (KIND & 1) ? off1[I] : 0, b2 = FILL && (KIND & 2) ? off2[I] : 0;
+    for (uint64_t x = KIND & 1 ? m : 0; x; x &= x - 1) {
         int i = jci_ctz(x);
         for (uint64_t y = vir; y; y &= y - 1) {
             int f = jci_ctz(y);
@@ -104,7 +105,7 @@ __global__ void k_exc(const SpaceDesc *__restrict__ d, int spin, long long nstr,
             c1[g]++;
         }
     }
-    for (uint64_t x0 = m; x0; x0 &= x0 - 1) {
+    for (uint64_t x0 = KIND & 2 ? m : 0; x0; x0 &= x0 - 1) {
         int i0 = jci_ctz(x0);
         for (uint64_t x1 = x0 & (x0 - 1); x1; x1 &= x1 - 1) {
             int i1 = jci_ctz(x1);
@@ -132,39 +133,56 @@ __global__ void k_exc(const SpaceDesc *__restrict__ d, int spin, long long nstr,
     }
     if (!FILL) {
         long long t1 = 0, t2 = 0;
-        for (int g = 0; g < G; g++) {
-            goff1[I * (G + 1) + g] = (int)t1;
-            goff2[I * (G + 1) + g] = (int)t2;
+        for (int g = 0; g <= G; g++) {
+            if (KIND & 1) goff1[I * (G + 1) + g] = (int)t1;
+            if (KIND & 2) goff2[I * (G + 1) + g] = (int)t2;
             t1 += c1[g];
             t2 += c2[g];
         }
-        goff1[I * (G + 1) + G] = (int)t1;
-        goff2[I * (G + 1) + G] = (int)t2;
-        cnt1[I] = t1;
-        cnt2[I] = t2;
+        if (KIND & 1) cnt1[I] = t1;
+        if (KIND & 2) cnt2[I] = t2;
     }
 }
 
-int jk_exc_count(const SpaceDesc *d, int spin, long long nstr, const uint64_t *M,
+int jk_exc_count(int kind, const SpaceDesc *d, int spin, long long nstr, const uint64_t *M,
                  const unsigned long long *binom, long long *cnt1, long long *cnt2,
                  int *goff1, int *goff2, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_exc<false>, dim3(gridn(nstr, 64)), dim3(64), 0, st, d, spin, nstr, M,
-                       binom, (const double *)nullptr, (const double *)nullptr, cnt1, cnt2,
-                       goff1, goff2, (const long long *)nullptr, (const long long *)nullptr,
-                       (int2 *)nullptr, (double *)nullptr, (int2 *)nullptr, (double *)nullptr);
+    const dim3 g(gridn(nstr, 64)), b(64);
+    const double *nd = nullptr;
+    const long long *no = nullptr;
+    if (kind == 1)
+        hipLaunchKernelGGL((k_exc<false, 1>), g, b, 0, st, d, spin, nstr, M, binom, nd, nd, cnt1, cnt2,
+                           goff1, goff2, no, no, (int2 *)nullptr, (double *)nullptr, (int2 *)nullptr,
+                           (double *)nullptr);
+    else if (kind == 2)
+        hipLaunchKernelGGL((k_exc<false, 2>), g, b, 0, st, d, spin, nstr, M, binom, nd, nd, cnt1, cnt2,
+                           goff1, goff2, no, no, (int2 *)nullptr, (double *)nullptr, (int2 *)nullptr,
+                           (double *)nullptr);
+    else
+        hipLaunchKernelGGL((k_exc<false, 3>), g, b, 0, st, d, spin, nstr, M, binom, nd, nd, cnt1, cnt2,
+                           goff1, goff2, no, no, (int2 *)nullptr, (double *)nullptr, (int2 *)nullptr,
+                           (double *)nullptr);
     LAUNCH_CHECK2();
     return 0;
 }
 
-int jk_exc_fill(const SpaceDesc *d, int spin, long long nstr, const uint64_t *M,
+int jk_exc_fill(int kind, const SpaceDesc *d, int spin, long long nstr, const uint64_t *M,
                 const unsigned long long *binom, const double *m1, const double *m2,
                 const long long *off1, const long long *off2, const int *goff1,
                 const int *goff2, int2 *e1, double *v1, int2 *e2, double *v2, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_exc<true>, dim3(gridn(nstr, 64)), dim3(64), 0, st, d, spin, nstr, M,
-                       binom, m1, m2, (long long *)nullptr, (long long *)nullptr,
-                       (int *)goff1, (int *)goff2, off1, off2, e1, v1, e2, v2);
+    const dim3 g(gridn(nstr, 64)), b(64);
+    long long *nc = nullptr;
+    if (kind == 1)
+        hipLaunchKernelGGL((k_exc<true, 1>), g, b, 0, st, d, spin, nstr, M, binom, m1, m2, nc, nc,
+                           (int *)goff1, (int *)goff2, off1, off2, e1, v1, e2, v2);
+    else if (kind == 2)
+        hipLaunchKernelGGL((k_exc<true, 2>), g, b, 0, st, d, spin, nstr, M, binom, m1, m2, nc, nc,
+                           (int *)goff1, (int *)goff2, off1, off2, e1, v1, e2, v2);
+    else
+        hipLaunchKernelGGL((k_exc<true, 3>), g, b, 0, st, d, spin, nstr, M, binom, m1, m2, nc, nc,
+                           (int *)goff1, (int *)goff2, off1, off2, e1, v1, e2, v2);
     LAUNCH_CHECK2();
     return 0;
 }

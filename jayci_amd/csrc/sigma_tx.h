@@ -1,0 +1,354 @@
+// Contraction form of the sigma on truncated spaces (several group blocks).
+//
+// Both parts of the Hamiltonian are written as products of dense integral blocks with
+// gathered vector rows, so that the matrix cores do the work and an entry of the vector is
+// read a few dozen times instead of once per connected pair.
+//
+// Same-spin part (one-electron part and diagonal included).  With K2 a string of N - 2
+// electrons and a pair p = (i < j) of its empty orbitals,
+//
+//   D[q][K2, J'] = sign X(K2 + q, J')                 (rows of the vector)
+//   E[p][K2, J'] = sum_q W(p, q) D[q][K2, J']         (MFMA; rows and columns: the pairs of
+//                                                      K2 whose strings the block allows)
+//   sigma(I, J') += sum_{p in I} sign E[p][I - p, J'] (a string has N (N - 1) / 2 pairs)
+//   W((i,j),(k,l)) = (ik|jl) - (il|jk)
+//                    + (h_ik d_jl - h_il d_jk - h_jk d_il + h_jl d_ik) / (N - 1)
+//
+// Two strings that differ by a double share one K2, by a single N - 1 and equal ones
+// N (N - 1) / 2 of them, which is how often the spectators of their elements are counted.
+// J' is the other spin's string, so the vector's rows are contiguous: alpha on the vector,
+// beta on its block-transposed copy.
+//
+// Opposite-spin part.  Each connection (p, q) <- (p1, q1) of group blocks is contracted with
+// one spin first and the other last, through strings (last spin of the source, first spin of
+// the target), whichever order has the fewer of them:
+//
+//   D[Q][JL, IF] = sum_{JF: <IF|B_Q|JF> != 0} sign X(JL, JF)
+//   E[P][JL, IF] = sum_Q (P|Q) D[Q][JL, IF]
+//   sigma(IL, IF) += sum_{(JL, P) in the singles of IL} sign E[P][JL, IF]
+//
+// with B_Q = E_kl + E_lk of the pair Q = (k, l) and the diagonal pairs for the Coulomb terms.
+// The connections that share (JL's group, IF's group) and their source groups form one task.
+// A task's columns are the strings of IF's group, taken 16 internal (doubly occupied + active)
+// parts at a time for one external part: all of them reach the same short list of pairs Q
+// (the internal pairs, and those of the external part's orbitals), which is the reduction
+// index.  The rows are the singles of JL towards the target groups, plus one for JL's own
+// diagonal pairs together.
+//
+// Against the table kernels (one gather per connected entry, sigma_fast.hip), whole products:
+// MRCI-SD 16e/28o FP64 one vector 304 -> 206 ms, 16e/20o FP64 three vectors 108 -> 84 ms, FP32
+// two vectors 56 -> 43 ms, 7a6b/17o two vectors 3.3 -> 2.0 ms, 4a4b/10o 260 -> 74 us; error
+// against 64 bits 2.4e-15 -> 3.3e-16 (FP64) and 1.2e-6 -> 8e-8 (FP32) at 16e/20o.
+#pragma once
+#include "jci_internal.h"
+#include "sigma_fast.h"
+
+#define TX_MAXG2 64          // groups of N - 2 electron strings per spin
+#define TX_MAXSEC 8          // target groups of a single excitation (7), or the diagonal
+#define TX_NTYPE 6           // orbital-pair types dd, da, dv, aa, av, vv
+#define TX_KC 96             // reduction depth of one LDS tile (four waves: 50 KB in FP64)
+#define TX_ROWS64 32         // rows of E a wave holds integral fragments for, FP64 ...
+#define TX_ROWS32 48         // ... and FP32
+#define TX_PAD 0x7FF00000u   // list entry of a padded row or column (no position, string 0)
+
+// list entry of the first spin: target string in its group (bits 0..19), position of the pair
+// in its class (20..30), sign (31)
+#define TX_JBITS 20
+#define TX_KMAX 0x7FF
+
+// lists of one first-spin group: per external part `rows` rows of nIp entries, the sections
+// (target groups, then the diagonal pairs) each padded to a multiple of four rows
+struct TxList {
+    long long base;                  // first entry
+    int rows, nI, nIp, nsv;
+    int nsec;
+    int grp[TX_MAXSEC + 1];          // target group of the section, -1: the diagonal pairs
+    int row0[TX_MAXSEC + 1], cnt[TX_MAXSEC + 1];
+};
+
+// four list rows of a task's chunk: where their targets sit in the vector and in the chunk.
+// The rows' positions [k0, k0 + len) of their class are steps [base, base + len) of the chunk.
+struct TxSlot {
+    long long xb;                    // block offset of (JL's group, target group)
+    int nb;                          // strings of the target group (stride of JL)
+    int lrow;                        // first list row
+    int kinfo;                       // base | len << 8 | k0 << 16
+    int pad;
+};
+// at most TX_KC steps of a task's reduction; the chunks of a task add to E one after another
+struct TxChunk {
+    int KS;                          // reduction steps of 4 (a multiple of 4)
+    int slot0, nslot;
+    int q0;                          // pair Q of step s of external part w: q[q0 + w * 4 KS + s]
+};
+
+struct TxTask {
+    int o;                           // 0: beta first, alpha last (the vector); 1: the reverse
+    int l1, f;                       // groups of JL and IF
+    int na, ls0;                     // strings of JL's group, the first one
+    int nI, nIp, nsv;                // internal parts of IF's group (padded to 16), external
+    int La;                          // rows of E
+    int ch0, nch;                    // chunks of the reduction
+    int lrows;                       // rows of the list
+    int diag;                        // last row: JL's diagonal pairs
+    int nsec, sg[TX_MAXSEC], sr0[TX_MAXSEC];   // target groups and their first rows
+    int iI0, nsvL;                   // first internal part of l1 in the diagonal-row table,
+                                     // external parts of JL's group
+    long long lbase;
+};
+
+// one task's share of a round (a range of columns small enough that E fits its buffer)
+struct TxItem {
+    int task, w0, nw, t0, nt;        // external parts, column tiles
+    int rg[2];                       // row groups (FP64, FP32)
+    long long item0[2];              // first item of the round's launch: (JL, w, row group)
+    long long ebase;                 // first element in E
+};
+
+// target block of a round's gather: sources are consecutive entries of the TxSrc table
+struct TxOut {
+    int o, p, f;                     // last-spin group, first-spin group
+    int na, ls0, nI, nIp, nsv;
+    int w0, nw, t0, nt;
+    int src0, nsrc;
+    int nb;                          // strings of the first-spin group
+    long long yb;                    // block offset
+    long long blk0;                  // first work-group of the launch
+    int cblk;                        // work-groups per string
+};
+struct TxSrc {
+    int l1, ls0, La, r0, diag;       // JL's group and its first string, rows, first row of this
+                                     // target (-1: none); diag 1: also JL = IL
+    long long ebase;
+};
+
+// ---- same-spin part ----
+struct TxPairGroup {                 // group of N - 2 electron strings
+    int d, a, v;
+    long long n, base;               // strings; first list entry
+    int R;                           // list entries per string
+    int off[TX_NTYPE], cnt[TX_NTYPE], tgt[TX_NTYPE];   // per pair type: first, count, group (-1)
+};
+struct TxPairTask {
+    int o, g2, f;                    // orientation, N - 2 group, column group
+    int R;                           // pairs (rows and reduction index)
+    int nsec, so[TX_NTYPE], sc[TX_NTYPE], sr[TX_NTYPE];  // list offset, count, first row
+    long long sx[TX_NTYPE];          // vector offset of the section's strings
+    long long lbase;                 // list base of the group
+    int Rfull, n, nb;
+};
+struct TxPairItem {
+    int task, c0, nc, ncp;           // columns of the round, padded to 16
+    int rg, ct;                      // row groups of 64, column blocks of 64
+    long long item0, ebase;
+};
+struct TxPairOut {
+    int o, p, f, na, ls0, nb;
+    int c0, nc, ncp, cblk;
+    long long yb, blk0;
+    int nsec, np[TX_NTYPE], r0[TX_NTYPE], R[TX_NTYPE];   // pairs of I per type, rows of E
+    long long eb[TX_NTYPE];
+};
+
+// one spin's lists (device)
+struct TxSpin {
+    const uint64_t *mask;
+    const long long *off1;
+    const int2 *e1;
+    const int *goff1;
+    const uint32_t *lst;             // TxList lists of all groups
+    const uint16_t *rk;              // per entry of e1: its reverse's position among the
+                                     // target's singles towards this string's group
+    const int2 *kl;                  // per N - 2 string: pairs {string in its group,
+                                     // pair | sign << 31}
+    const int2 *gl;                  // per string: its pairs {N - 2 string in its group,
+                                     // position in the type | sign << 31}
+    int npair;                       // N (N - 1) / 2
+    int G;
+    const double *w64;               // W, np x np
+    const float *w32;
+    // integral rows of ms = m1 + 1 elements, the last one zero: (P|.) of every pair, then per
+    // internal part the sum of (kk|.) over its electrons, then a row of zeros
+    const double *m64;
+    const float *m32;
+    int zrow;                        // the row of zeros
+};
+
+struct TxDev {
+    TxSpin s[2];
+    const TxTask *task;
+    const TxSlot *slot;
+    const TxChunk *chunk;
+    const TxItem *item;
+    const TxOut *out;
+    const TxSrc *src;
+    const TxPairTask *ptask;
+    const TxPairItem *pitem;
+    const TxPairOut *pout;
+    const int *q;
+    int m1, ms, np, nint;
+};
+
+// one launch pair (E, gather) of either part
+struct TxRound {
+    int i0, ni, o0, no;              // items and outputs in their tables
+    long long items[2], blocks;      // waves (opposite spin; FP64, FP32) or work-groups; gather
+                                     // work-groups
+    long long elems;                 // elements of E
+};
+
+// index arithmetic shared by the device kernels and host checks -------------------------------
+#include "slater.h"
+
+// orbital subspace of orbital x: 0 doubly occupied, 1 active, 2 external
+JCI_HD int tx_sub(const SpaceDesc *d, int x)
+{
+    return x < d->ndocc ? 0 : x < d->ndocc + d->nactv ? 1 : 2;
+}
+JCI_HD uint64_t tx_submask(const SpaceDesc *d, int s)
+{
+    return s == 0 ? d->dmask : s == 1 ? d->amask : d->vmask;
+}
+JCI_HD uint64_t tx_below(int x) { return (1ULL << x) - 1ULL; }
+JCI_HD int tx_type(int s0, int s1)   // s0 <= s1
+{
+    return s0 == 0 ? s1 : s0 == 1 ? 2 + s1 : 5;
+}
+
+// position of the single excitation x -> y of string m among its singles towards their target
+// group (enumeration order of the excitation tables: x ascending, then y ascending)
+JCI_HD int tx_single_rank(const SpaceDesc *d, uint64_t m, int x, int y)
+{
+    const int sx = tx_sub(d, x), sy = tx_sub(d, y);
+    const uint64_t mx = tx_submask(d, sx), my = tx_submask(d, sy);
+    const int occ = jci_popc(m & mx & tx_below(x));
+    const int emp = jci_popc(~m & my & tx_below(y));
+    int r = occ * jci_popc(~m & my & d->allmask) + emp;
+    if (sx == sy)   // the three subspaces' own replacements share the target group
+        for (int s = 0; s < sx; s++) {
+            const uint64_t ms = tx_submask(d, s);
+            r += jci_popc(m & ms) * jci_popc(~m & ms & d->allmask);
+        }
+    return r;
+}
+
+// position of the pair (x, y) in its class for a string with external part ext: internal
+// pairs; pairs of an external orbital of the string with any external one (class of equal
+// external count); external orbital of the string with an internal one (target with one
+// external orbital less); any external with an internal one (one more)
+JCI_HD int tx_kpos(const SpaceDesc *d, uint64_t ext, int dv, int x, int y)
+{
+    const int nint = d->ndocc + d->nactv, nv = d->nvirt;
+    const int hi = x > y ? x : y, lo = x > y ? y : x;
+    if (hi < nint) return hi * (hi + 1) / 2 + lo;
+    if (dv > 0) return (hi - nint) * nint + lo;
+    if (dv < 0) return jci_popc(ext & tx_below(hi)) * nint + lo;
+    const int b = (ext >> hi) & 1 ? hi : lo, c = b == hi ? lo : hi;
+    return nint * (nint + 1) / 2 + jci_popc(ext & tx_below(b)) * nv + (c - nint);
+}
+
+// inverse of tx_kpos: pair index tri of position s of a class (dv as above), or -1
+JCI_HD int tx_kpair(int nint, int nv, const int *extorb, int next, int dv, int s)
+{
+    const int m1int = nint * (nint + 1) / 2;
+    if (dv == 0) {
+        if (s < m1int) return s;
+        const int r = (s - m1int) / nv, c = nint + (s - m1int) % nv;
+        return r < next ? (int)jci_tri(extorb[r], c) : -1;
+    }
+    if (dv < 0) {
+        const int r = s / nint;
+        return r < next ? (int)jci_tri(extorb[r], s % nint) : -1;
+    }
+    const int c = s / nint;
+    return c < nv ? (int)jci_tri(nint + c, s % nint) : -1;
+}
+
+JCI_HD int tx_class_size(int nint, int nv, int v, int dv, int own)
+{
+    if (dv == 0) return nint * (nint + 1) / 2 + (own ? v * nv : 0);
+    return dv < 0 ? v * nint : nv * nint;
+}
+
+// pair i < j of string m: the N - 2 string's mask, the pair's type, its position in the type's
+// section of that string's list and the sign of a_j a_i
+JCI_HD void tx_pair(const SpaceDesc *d, uint64_t m, int i, int j, uint64_t *k2, int *type,
+                    int *idx, int *neg)
+{
+    const uint64_t k = m & ~(1ULL << i) & ~(1ULL << j);
+    const int si = tx_sub(d, i), sj = tx_sub(d, j);
+    const uint64_t mi = tx_submask(d, si), mj = tx_submask(d, sj);
+    const int ei = jci_popc(~k & mi & tx_below(i)), ej = jci_popc(~k & mj & tx_below(j));
+    *k2 = k;
+    *type = tx_type(si, sj);
+    *idx = si == sj ? ej * (ej - 1) / 2 + ei : ei * jci_popc(~k & mj & d->allmask) + ej;
+    *neg = (jci_popc(m & tx_below(i)) + jci_popc(m & tx_below(j)) + 1) & 1;
+}
+
+// index of an N - 2 string in its group
+JCI_HD long long tx_pair_rank(const SpaceDesc *d, uint64_t k, const unsigned long long *binom)
+{
+    const int nd = jci_popc(k & d->dmask), na = jci_popc(k & d->amask), nv = jci_popc(k & d->vmask);
+    const int si = d->ndocc + d->nactv;
+    const long long rd = jci_lex_rank(k & d->dmask, d->ndocc, nd, binom);
+    const long long ra = jci_lex_rank(d->ndocc >= 64 ? 0 : (k & d->amask) >> d->ndocc, d->nactv, na, binom);
+    const long long rv = jci_lex_rank(si >= 64 ? 0 : (k & d->vmask) >> si, d->nvirt, nv, binom);
+    return (rd * (long long)binom[d->nactv * 65 + na] + ra) * (long long)binom[d->nvirt * 65 + nv] + rv;
+}
+
+// host tables of the contraction form: lists, tasks and rounds (tx_plan.cpp)
+#include <vector>
+struct TxPlan {
+    std::vector<TxList> lists[2];          // per spin and group
+    long long nlst[2];                     // list entries per spin
+    std::vector<TxPairGroup> pg[2];
+    long long nkl[2];                      // pair-list entries per spin
+    std::vector<TxTask> task;
+    std::vector<TxSlot> slot;
+    std::vector<TxChunk> chunk;
+    std::vector<TxItem> item;
+    std::vector<TxOut> out;
+    std::vector<TxSrc> src;
+    std::vector<TxPairTask> ptask;
+    std::vector<TxPairItem> pitem;
+    std::vector<TxPairOut> pout;
+    std::vector<int> q;
+    std::vector<TxRound> ab, ss;           // rounds of the two parts
+    long long elems;                       // largest E of a round
+    int ldt, rmax;                         // deepest reduction chunk; most pairs of a task
+    long long nint_parts[2];               // internal parts over all groups
+    int iI0[2][JCI_MAXG];
+};
+// 0: built; 1: the space is outside what the lists can index (the caller keeps the tables)
+int tx_plan(const SpaceDesc &D, const SpaceDesc &T, long long budget, TxPlan *P);
+
+// ---- kernels (sigma_tx.hip) ----
+int jk_tx_lists(const SpaceDesc *d, int spin, long long nstr, const uint64_t *mask,
+                const long long *off1, const int2 *e1, const int *goff1, const TxList *lists,
+                uint32_t *lst, uint16_t *rk, hipStream_t st);
+int jk_tx_fill(long long n, uint32_t *p, hipStream_t st);
+int jk_tx_pairs(const SpaceDesc *d, int spin, long long nstr, const uint64_t *mask,
+                const unsigned long long *binom, const TxPairGroup *pg, int npg, int npair,
+                int2 *kl, int2 *gl, hipStream_t st);
+int jk_tx_w(int norb, int nelec, const double *m1, const double *m2, double *w64, float *w32,
+            hipStream_t st);
+int jk_tx_rows(const SpaceDesc *d, const SpaceDesc &h, int spin, const uint64_t *mask, int m1,
+               const double *m2sq, const TxPlan &P, double *m64, float *m32, hipStream_t st);
+// x (vector k at x + k * xk, element n at n * xs) -> xT (every block transposed) and, unless
+// xv is null, xv, both vector-major of stride N in the arithmetic type
+int jk_tx_in(int prec, int nvec, long long N, const SpaceDesc *d, const long long *tt, long long ntt,
+             const double *x, long long xs, long long xk, void *xv, void *xT, hipStream_t st);
+// y += the transposed blocks of yT
+int jk_tx_out(int nvec, long long N, const SpaceDesc *d, const long long *tt, long long ntt,
+              const double *yT, double *y, long long ys, long long yk, hipStream_t st);
+// the rounds of both parts; X: vector of orientation 0 (element stride 1, vector stride ldx)
+// and its block-transposed copy (vector stride N), Y likewise (y: element stride ys, vector
+// stride yk; yT: N)
+struct TxVec {
+    const void *x0, *x1;
+    long long ldx0, ldx1;
+    double *y0, *y1;
+    long long ys0, yk0, ys1, yk1;
+};
+int jk_tx_run(int prec, int nvec, const TxDev &D, const TxPlan &P, const TxVec &V, void *E,
+              hipStream_t st);

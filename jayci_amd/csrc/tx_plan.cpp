@@ -1,0 +1,577 @@
+// Host tables of the contraction form of the truncated-space sigma (see sigma_tx.h): lists,
+// tasks, and the rounds that keep the intermediates inside a buffer.
+#include "sigma_tx.h"
+#include <algorithm>
+#include <map>
+#include <set>
+#include <string.h>
+
+typedef long long ll;
+
+static ll choose(int n, int k)
+{
+    if (k < 0 || n < 0 || k > n) return 0;
+    ll r = 1;
+    for (int i = 1; i <= k; i++) r = r * (n - k + i) / i;
+    return r;
+}
+
+// singles of one string of group g to strings of group h of the same spin; -1: no single
+// excitation leads there
+static ll singles(const SpaceDesc &D, const SpinDesc &S, int g, int h)
+{
+    const int size[3] = {D.ndocc, D.nactv, D.nvirt};
+    const int o[3] = {S.gd[g], S.ga[g], S.gv[g]}, t[3] = {S.gd[h], S.ga[h], S.gv[h]};
+    if (g == h) return o[0] * (size[0] - o[0]) + o[1] * (size[1] - o[1]) + o[2] * (size[2] - o[2]);
+    int from = -1, to = -1;
+    for (int s = 0; s < 3; s++) {
+        if (t[s] == o[s]) continue;
+        if (t[s] == o[s] - 1 && from < 0) from = s;
+        else if (t[s] == o[s] + 1 && to < 0) to = s;
+        else return -1;
+    }
+    if (from < 0 || to < 0) return -1;
+    return (ll)o[from] * (size[to] - o[to]);
+}
+
+static ll up(ll n, ll m) { return (n + m - 1) / m * m; }
+
+// lists of one spin as the first spin of a task
+static int plan_lists(const SpaceDesc &D, const SpinDesc &S, std::vector<TxList> &L, ll *total)
+{
+    ll base = 0;
+    for (int g = 0; g < S.ngrp; g++) {
+        TxList t;
+        memset(&t, 0, sizeof(t));
+        t.base = base;
+        t.nsv = (int)std::max(1LL, S.nsv[g]);
+        t.nI = (int)(S.gn[g] / t.nsv);
+        t.nIp = (int)up(t.nI, 16);
+        for (int h = 0; h < S.ngrp; h++) {
+            if (!S.gn[h] || !S.gn[g]) continue;
+            const ll c = singles(D, S, g, h);
+            if (c <= 0) continue;
+            if (t.nsec >= TX_MAXSEC) return 1;
+            t.grp[t.nsec] = h;
+            t.row0[t.nsec] = t.rows;
+            t.cnt[t.nsec] = (int)c;
+            t.rows += (int)up(c, 4);
+            t.nsec++;
+        }
+        t.grp[t.nsec] = -1;
+        t.row0[t.nsec] = t.rows;
+        t.cnt[t.nsec] = S.nelec;
+        t.rows += (int)up(S.nelec, 4);
+        t.nsec++;
+        if (S.gn[g] >= (1LL << TX_JBITS)) return 1;
+        base += (ll)t.nsv * t.rows * t.nIp;
+        L.push_back(t);
+    }
+    *total = base;
+    return 0;
+}
+
+// groups of N - 2 electron strings of one spin
+static int plan_pairs(const SpaceDesc &D, const SpinDesc &S, std::vector<TxPairGroup> &P, ll *total)
+{
+    const int size[3] = {D.ndocc, D.nactv, D.nvirt};
+    static const int ts[TX_NTYPE][2] = {{0, 0}, {0, 1}, {0, 2}, {1, 1}, {1, 2}, {2, 2}};
+    ll base = 0;
+    for (int g = 0; g < S.ngrp; g++) {
+        if (!S.gn[g]) continue;
+        for (int t = 0; t < TX_NTYPE; t++) {
+            int o[3] = {S.gd[g], S.ga[g], S.gv[g]};
+            o[ts[t][0]]--;
+            o[ts[t][1]]--;
+            if (o[0] < 0 || o[1] < 0 || o[2] < 0) continue;
+            bool have = false;
+            for (const TxPairGroup &k : P) have = have || (k.d == o[0] && k.a == o[1] && k.v == o[2]);
+            if (have) continue;
+            if ((int)P.size() >= TX_MAXG2) return 1;
+            TxPairGroup k;
+            memset(&k, 0, sizeof(k));
+            k.d = o[0];
+            k.a = o[1];
+            k.v = o[2];
+            k.n = choose(size[0], o[0]) * choose(size[1], o[1]) * choose(size[2], o[2]);
+            k.base = base;
+            for (int u = 0; u < TX_NTYPE; u++) {
+                int f[3] = {o[0], o[1], o[2]};
+                const int s0 = ts[u][0], s1 = ts[u][1];
+                const int e0 = size[s0] - o[s0], e1 = size[s1] - o[s1];
+                f[s0]++;
+                f[s1]++;
+                k.off[u] = k.R;
+                k.tgt[u] = -1;
+                for (int h = 0; h < S.ngrp; h++)
+                    if (S.gn[h] && S.gd[h] == f[0] && S.ga[h] == f[1] && S.gv[h] == f[2]) k.tgt[u] = h;
+                if (k.tgt[u] < 0) continue;
+                k.cnt[u] = s0 == s1 ? e0 * (e0 - 1) / 2 : e0 * e1;
+                k.R += k.cnt[u];
+            }
+            if (k.n >= (1LL << 31)) return 1;
+            base += k.n * k.R;
+            P.push_back(k);
+        }
+    }
+    *total = base;
+    return 0;
+}
+
+namespace {
+struct Builder {
+    const SpaceDesc *dd[2];
+    ll budget;
+    TxPlan *P;
+    // tasks by (orientation, first-spin group)
+    std::vector<int> by[2][JCI_MAXG], pby[2][JCI_MAXG];
+    std::map<std::vector<int>, int> qtab;
+    unsigned long long binom[65 * 65];
+
+    // a chunk's steps: consecutive positions of one or more classes
+    struct Seg { int dv, k0, len, base; };
+
+    // reduction-index table of a chunk for first-spin group f: its first entry
+    int pair_table(const SpaceDesc &D, int f, const std::vector<Seg> &seg, int depth)
+    {
+        const SpinDesc &S = D.s[1];
+        std::vector<int> key = {S.gv[f], depth};
+        for (const Seg &g : seg) key.insert(key.end(), {g.dv, g.k0, g.len});
+        auto it = qtab.find(key);
+        if (it != qtab.end()) return it->second;
+        const int nint = D.ndocc + D.nactv, v = S.gv[f];
+        const int at = (int)P->q.size();
+        const int none = D.norbs * (D.norbs + 1) / 2;   // the zero column
+        const int nsv = (int)std::max(1LL, S.nsv[f]);
+        for (int w = 0; w < nsv; w++) {
+            int ext[64], n = 0;
+            for (uint64_t m = v ? jci_lex_unrank(w, D.nvirt, v, binom) : 0; m; m &= m - 1)
+                ext[n++] = nint + jci_ctz(m);
+            int put = 0;
+            for (const Seg &g : seg)
+                for (int s = 0; s < g.len; s++, put++) {
+                    const int Q = tx_kpair(nint, D.nvirt, ext, n, g.dv, g.k0 + s);
+                    P->q.push_back(Q < 0 ? none : Q);
+                }
+            for (; put < depth; put++) P->q.push_back(none);
+        }
+        qtab[key] = at;
+        return at;
+    }
+
+    int tasks()
+    {
+        // every connection of group blocks goes to the orientation with fewer intermediates
+        std::map<std::vector<int>, std::map<int, std::set<int>>> T;   // (o, l1, f) -> l -> f1 set
+        const SpaceDesc &D = *dd[0];
+        auto linked = [&](const SpinDesc &S, int a, int b) { return a == b || singles(D, S, a, b) > 0; };
+        for (int b = 0; b < D.nblk; b++)
+            for (int c = 0; c < D.nblk; c++) {
+                const int p = D.bp[b], q = D.bq[b], p1 = D.bp[c], q1 = D.bq[c];
+                if (!linked(D.s[0], p, p1) || !linked(D.s[1], q, q1)) continue;
+                const ll n0 = D.s[0].gn[p1] * D.s[1].gn[q], n1 = D.s[0].gn[p] * D.s[1].gn[q1];
+                if (n0 <= n1) T[{0, p1, q}][p].insert(q1);
+                else T[{1, q1, p}][q].insert(p1);
+            }
+        for (auto &kv : T) {
+            const int o = kv.first[0], l1 = kv.first[1], f = kv.first[2];
+            const SpaceDesc &O = *dd[o];
+            const SpinDesc &L = O.s[0], &F = O.s[1];
+            // targets with the same source set form one task
+            std::map<std::set<int>, std::vector<int>> groups;
+            for (auto &t : kv.second) groups[t.second].push_back(t.first);
+            const TxList &li = P->lists[o == 0 ? 1 : 0][f];
+            for (auto &gr : groups) {
+                TxTask t;
+                memset(&t, 0, sizeof(t));
+                t.o = o;
+                t.l1 = l1;
+                t.f = f;
+                t.na = (int)L.gn[l1];
+                t.ls0 = (int)L.gstart[l1];
+                t.nI = li.nI;
+                t.nIp = li.nIp;
+                t.nsv = li.nsv;
+                t.lrows = li.rows;
+                t.lbase = li.base;
+                t.nsvL = (int)std::max(1LL, L.nsv[l1]);
+                t.iI0 = P->iI0[o == 0 ? 0 : 1][l1];
+                for (int l : gr.second) {
+                    const ll c = singles(O, L, l1, l);
+                    if (c <= 0) continue;
+                    if (t.nsec >= TX_MAXSEC) return 1;
+                    t.sg[t.nsec] = l;
+                    t.sr0[t.nsec] = t.La;
+                    t.nsec++;
+                    t.La += (int)c;
+                }
+                for (int l : gr.second) if (l == l1) { t.diag = 1; t.La++; break; }
+                if (!t.La) continue;
+                // reduction index: the classes of the sources, in chunks of at most TX_KC
+                // steps; a class that does not fit what is left of a chunk opens the next
+                // one, and one deeper than a chunk is split evenly
+                const int own = gr.first.count(f) ? 1 : 0;
+                int has[3] = {0, 0, 0};
+                const int v = F.gv[f], nint = O.ndocc + O.nactv;
+                for (int f1 : gr.first) has[F.gv[f1] - v + 1] = 1;
+                std::vector<std::vector<Seg>> chunks(1);
+                int depth = 0;
+                for (int dv : {0, -1, 1}) {
+                    if (!has[dv + 1]) continue;
+                    if (tx_class_size(nint, O.nvirt, v, dv, 1) >= TX_KMAX) return 1;
+                    const int m = tx_class_size(nint, O.nvirt, v, dv, own);
+                    const int np = (m + TX_KC - 1) / TX_KC, len = np ? (m + np - 1) / np : 0;
+                    for (int k0 = 0; k0 < m; k0 += len) {
+                        const int n = std::min(len, m - k0);
+                        if (depth + n > TX_KC) {
+                            chunks.push_back(std::vector<Seg>());
+                            depth = 0;
+                        }
+                        chunks.back().push_back(Seg{dv, k0, n, depth});
+                        depth += n;
+                    }
+                }
+                t.ch0 = (int)P->chunk.size();
+                for (const std::vector<Seg> &seg : chunks) {
+                    TxChunk ch;
+                    memset(&ch, 0, sizeof(ch));
+                    int d = 0;
+                    for (const Seg &g : seg) d += g.len;
+                    const int kc = (int)up(d, 16);
+                    ch.KS = kc / 4;
+                    P->ldt = std::max(P->ldt, kc);
+                    ch.q0 = pair_table(O, f, seg, kc);
+                    ch.slot0 = (int)P->slot.size();
+                    for (const Seg &g : seg)
+                        for (int s = 0; s < li.nsec; s++) {
+                            const int f1 = li.grp[s] < 0 ? f : li.grp[s];
+                            if (!gr.first.count(f1) || F.gv[f1] - v != g.dv) continue;
+                            const int blk = O.blkid[l1][f1];
+                            if (blk < 0) return 1;
+                            for (int r = 0; r < li.cnt[s]; r += 4) {
+                                TxSlot w;
+                                memset(&w, 0, sizeof(w));
+                                w.xb = O.boff[blk];
+                                w.nb = (int)F.gn[f1];
+                                w.lrow = li.row0[s] + r;
+                                w.kinfo = g.base | g.len << 8 | g.k0 << 16;
+                                P->slot.push_back(w);
+                            }
+                        }
+                    ch.nslot = (int)P->slot.size() - ch.slot0;
+                    if (!ch.nslot) continue;
+                    P->chunk.push_back(ch);
+                    t.nch++;
+                }
+                if (!t.nch) continue;
+                by[o][f].push_back((int)P->task.size());
+                P->task.push_back(t);
+            }
+        }
+        return 0;
+    }
+
+    // one piece of a round: external parts [w0, w0 + nw) and column tiles [t0, t0 + nt) of
+    // first-spin group f
+    void piece(int o, int f, int w0, int nw, int t0, int nt, TxRound &R)
+    {
+        const SpaceDesc &O = *dd[o];
+        const SpinDesc &L = O.s[0];
+        std::vector<ll> eb;
+        for (int ti : by[o][f]) {
+            const TxTask &t = P->task[ti];
+            TxItem it;
+            memset(&it, 0, sizeof(it));
+            it.task = ti;
+            it.w0 = w0;
+            it.nw = nw;
+            it.t0 = t0;
+            it.nt = nt;
+            const int rows[2] = {TX_ROWS64, TX_ROWS32};
+            for (int p = 0; p < 2; p++) {
+                it.rg[p] = (t.La + rows[p] - 1) / rows[p];
+                it.item0[p] = R.items[p];
+                R.items[p] += (ll)t.na * nw * it.rg[p];
+            }
+            it.ebase = R.elems;
+            eb.push_back(R.elems);
+            R.elems += (ll)t.na * nw * t.La * nt * 16;
+            P->item.push_back(it);
+            R.ni++;
+        }
+        for (int l = 0; l < L.ngrp; l++) {
+            const int blk = O.blkid[l][f];
+            if (blk < 0) continue;
+            TxOut u;
+            memset(&u, 0, sizeof(u));
+            u.src0 = (int)P->src.size();
+            for (size_t i = 0; i < by[o][f].size(); i++) {
+                const TxTask &t = P->task[by[o][f][i]];
+                TxSrc s;
+                memset(&s, 0, sizeof(s));
+                s.l1 = t.l1;
+                s.ls0 = t.ls0;
+                s.La = t.La;
+                s.r0 = -1;
+                s.ebase = eb[i];
+                for (int k = 0; k < t.nsec; k++) if (t.sg[k] == l) s.r0 = t.sr0[k];
+                s.diag = t.diag && t.l1 == l;
+                if (s.r0 < 0 && !s.diag) continue;
+                P->src.push_back(s);
+                u.nsrc++;
+            }
+            if (!u.nsrc) continue;
+            const TxTask &t = P->task[by[o][f][0]];
+            u.o = o;
+            u.p = l;
+            u.f = f;
+            u.na = (int)L.gn[l];
+            u.ls0 = (int)L.gstart[l];
+            u.nI = t.nI;
+            u.nIp = t.nIp;
+            u.nsv = t.nsv;
+            u.w0 = w0;
+            u.nw = nw;
+            u.t0 = t0;
+            u.nt = nt;
+            u.nb = (int)O.s[1].gn[f];
+            u.yb = O.boff[blk];
+            u.blk0 = R.blocks;
+            u.cblk = (nw * nt * 16 + 255) / 256;
+            R.blocks += (ll)u.na * u.cblk;
+            P->out.push_back(u);
+            R.no++;
+        }
+    }
+
+    void rounds()
+    {
+        TxRound R;
+        auto open = [&]() {
+            memset(&R, 0, sizeof(R));
+            R.i0 = (int)P->item.size();
+            R.o0 = (int)P->out.size();
+        };
+        auto close = [&]() {
+            if (R.ni) {
+                P->ab.push_back(R);
+                P->elems = std::max(P->elems, R.elems);
+            }
+            open();
+        };
+        open();
+        for (int o = 0; o < 2; o++)
+            for (int f = 0; f < dd[o]->s[1].ngrp; f++) {
+                if (by[o][f].empty()) continue;
+                ll tile = 0;                     // elements of one column tile
+                for (int ti : by[o][f]) tile += (ll)P->task[ti].na * P->task[ti].La * 16;
+                const TxTask &t = P->task[by[o][f][0]];
+                const int nt = t.nIp / 16;
+                if (tile * nt <= budget) {
+                    for (int w = 0; w < t.nsv;) {
+                        ll room = (budget - R.elems) / (tile * nt);
+                        if (room <= 0) {
+                            close();
+                            continue;
+                        }
+                        const int n = (int)std::min<ll>(room, t.nsv - w);
+                        piece(o, f, w, n, 0, nt, R);
+                        w += n;
+                    }
+                } else {
+                    for (int w = 0; w < t.nsv; w++)
+                        for (int c = 0; c < nt;) {
+                            ll room = (budget - R.elems) / tile;
+                            if (room <= 0 && R.elems) {
+                                close();
+                                continue;
+                            }
+                            const int n = (int)std::min<ll>(std::max(1LL, room), nt - c);
+                            piece(o, f, w, 1, c, n, R);
+                            c += n;
+                        }
+                }
+            }
+        close();
+    }
+
+    void pair_tasks()
+    {
+        for (int o = 0; o < 2; o++) {
+            const SpaceDesc &O = *dd[o];
+            const SpinDesc &F = O.s[1];
+            const std::vector<TxPairGroup> &pg = P->pg[o];
+            for (int f = 0; f < F.ngrp; f++) {
+                if (!F.gn[f]) continue;
+                for (size_t g = 0; g < pg.size(); g++) {
+                    TxPairTask t;
+                    memset(&t, 0, sizeof(t));
+                    t.o = o;
+                    t.g2 = (int)g;
+                    t.f = f;
+                    for (int u = 0; u < TX_NTYPE; u++) {
+                        if (pg[g].tgt[u] < 0 || !pg[g].cnt[u]) continue;
+                        const int blk = O.blkid[pg[g].tgt[u]][f];
+                        if (blk < 0) continue;
+                        t.so[t.nsec] = pg[g].off[u];
+                        t.sc[t.nsec] = pg[g].cnt[u];
+                        t.sr[t.nsec] = t.R;
+                        t.sx[t.nsec] = O.boff[blk];
+                        t.nsec++;
+                        t.R += pg[g].cnt[u];
+                    }
+                    if (!t.R) continue;
+                    t.lbase = pg[g].base;
+                    t.Rfull = pg[g].R;
+                    t.n = (int)pg[g].n;
+                    t.nb = (int)F.gn[f];
+                    P->rmax = std::max(P->rmax, t.R);
+                    pby[o][f].push_back((int)P->ptask.size());
+                    P->ptask.push_back(t);
+                }
+            }
+        }
+    }
+
+    void pair_piece(int o, int f, int c0, int nc, TxRound &R)
+    {
+        static const int ts[TX_NTYPE][2] = {{0, 0}, {0, 1}, {0, 2}, {1, 1}, {1, 2}, {2, 2}};
+        const SpaceDesc &O = *dd[o];
+        const SpinDesc &L = O.s[0];
+        const int ncp = (int)up(nc, 16);
+        std::vector<ll> eb;
+        for (int ti : pby[o][f]) {
+            const TxPairTask &t = P->ptask[ti];
+            TxPairItem it;
+            memset(&it, 0, sizeof(it));
+            it.task = ti;
+            it.c0 = c0;
+            it.nc = nc;
+            it.ncp = ncp;
+            it.rg = (t.R + 63) / 64;
+            it.ct = (nc + 63) / 64;
+            it.item0 = R.items[0];
+            R.items[0] += (ll)t.n * it.rg * it.ct;
+            it.ebase = R.elems;
+            eb.push_back(R.elems);
+            R.elems += (ll)t.n * t.R * ncp;
+            P->pitem.push_back(it);
+            R.ni++;
+        }
+        R.items[1] = R.items[0];
+        for (int l = 0; l < L.ngrp; l++) {
+            const int blk = O.blkid[l][f];
+            if (blk < 0) continue;
+            TxPairOut u;
+            memset(&u, 0, sizeof(u));
+            u.o = o;
+            u.p = l;
+            u.f = f;
+            u.na = (int)L.gn[l];
+            u.ls0 = (int)L.gstart[l];
+            u.nb = (int)O.s[1].gn[f];
+            u.c0 = c0;
+            u.nc = nc;
+            u.ncp = ncp;
+            u.cblk = (nc + 255) / 256;
+            u.yb = O.boff[blk];
+            u.blk0 = R.blocks;
+            R.blocks += (ll)u.na * u.cblk;
+            const int e[3] = {L.gd[l], L.ga[l], L.gv[l]};
+            for (int k = 0; k < TX_NTYPE; k++) {
+                const int s0 = ts[k][0], s1 = ts[k][1];
+                const int n = s0 == s1 ? e[s0] * (e[s0] - 1) / 2 : e[s0] * e[s1];
+                if (n <= 0) continue;
+                int o3[3] = {e[0], e[1], e[2]};
+                o3[s0]--;
+                o3[s1]--;
+                for (size_t i = 0; i < pby[o][f].size(); i++) {
+                    const TxPairTask &t = P->ptask[pby[o][f][i]];
+                    const TxPairGroup &g = P->pg[o][t.g2];
+                    if (g.d != o3[0] || g.a != o3[1] || g.v != o3[2]) continue;
+                    u.np[u.nsec] = n;
+                    u.R[u.nsec] = t.R;
+                    u.eb[u.nsec] = eb[i];
+                    for (int s = 0; s < t.nsec; s++)
+                        if (t.so[s] == g.off[k] && t.sc[s] == g.cnt[k]) u.r0[u.nsec] = t.sr[s];
+                    u.nsec++;
+                }
+            }
+            P->pout.push_back(u);
+            R.no++;
+        }
+    }
+
+    void pair_rounds()
+    {
+        TxRound R;
+        auto open = [&]() {
+            memset(&R, 0, sizeof(R));
+            R.i0 = (int)P->pitem.size();
+            R.o0 = (int)P->pout.size();
+        };
+        auto close = [&]() {
+            if (R.ni) {
+                P->ss.push_back(R);
+                P->elems = std::max(P->elems, R.elems);
+            }
+            open();
+        };
+        open();
+        for (int o = 0; o < 2; o++)
+            for (int f = 0; f < dd[o]->s[1].ngrp; f++) {
+                if (pby[o][f].empty()) continue;
+                ll col = 0;                      // elements of 16 columns
+                for (int ti : pby[o][f]) col += (ll)P->ptask[ti].n * P->ptask[ti].R * 16;
+                const int nb = P->ptask[pby[o][f][0]].nb;
+                for (int c = 0; c < nb;) {
+                    const ll room = (budget - R.elems) / col * 16;
+                    // whole 64-column blocks, the rest of the group if it fits, at least one
+                    // block in an empty round
+                    ll n = room >= nb - c ? nb - c : room / 64 * 64;
+                    if (n <= 0) {
+                        if (R.elems) {
+                            close();
+                            continue;
+                        }
+                        n = std::min<ll>(64, nb - c);
+                    }
+                    pair_piece(o, f, c, (int)n, R);
+                    c += (int)n;
+                }
+            }
+        close();
+    }
+};
+}
+
+int tx_plan(const SpaceDesc &D, const SpaceDesc &T, ll budget, TxPlan *P)
+{
+    if (D.s[0].nelec < 2 || D.s[1].nelec < 2 || D.norbs < 2) return 1;
+    P->elems = 0;
+    P->ldt = P->rmax = 0;
+    for (int s = 0; s < 2; s++) {
+        if (plan_lists(D, D.s[s], P->lists[s], &P->nlst[s])) return 1;
+        if (plan_pairs(D, D.s[s], P->pg[s], &P->nkl[s])) return 1;
+        ll n = 0;
+        for (int g = 0; g < D.s[s].ngrp; g++) {
+            P->iI0[s][g] = (int)n;
+            n += P->lists[s][g].nI;
+        }
+        P->nint_parts[s] = n;
+    }
+    Builder *B = new Builder();
+    B->dd[0] = &D;
+    B->dd[1] = &T;
+    B->budget = budget;
+    B->P = P;
+    jci_binom_table(B->binom);
+    int rc = B->tasks();
+    if (!rc) {
+        B->rounds();
+        B->pair_tasks();
+        B->pair_rounds();
+    }
+    delete B;
+    return rc;
+}
