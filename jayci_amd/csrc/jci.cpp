@@ -308,8 +308,8 @@ struct jci_ham {
     void *tx_mem[24];           // device arrays behind txd
     int tx_nmem;
     long long *d_ttx, nttx;     // 16 x 16 transpose tiles per block
-    void *d_txE, *d_txv, *d_txT, *d_txy;
-    size_t txE_bytes, txv_bytes, txT_bytes, txy_bytes;
+    void *d_txE, *d_txx, *d_txy;
+    size_t txE_bytes, txx_bytes, txy_bytes;
     int have_tables;            // doubles tables and launch maps of the table kernels built
     int have_fci;               // single-block space with n <= 16: FCI kernel usable
     FciArgs fci;
@@ -603,19 +603,19 @@ static void free_doubles(jci_ham *h)
 // vectors up to this many determinants keep one vector's buffers of the contraction form from
 // the start, for the allocation-free entry point (its own staging bounds the larger ones out)
 #define TX_NOALLOC_DETS (16LL << 20)
-// elements of the intermediate per vector and round: 32M (256 MB in FP64)
-#define TX_ELEMS (32LL << 20)
+// elements of the intermediate per vector and round: 256M (2 GB in FP64).  Fewer, longer rounds
+// beat an intermediate that stays in the last-level cache: 16e/28o one vector 107 ms at 32M,
+// 97 at 128M, 93 at 256M.
+#define TX_ELEMS (256LL << 20)
 
 static int grow(void **p, size_t *have, size_t want, const char *what);
 
-// buffers of nvec vectors; copy: the input is converted or gathered into vector-major form
-static int tx_buffers(jci_ham *h, int nvec, bool copy)
+static int tx_buffers(jci_ham *h, int nvec, int prec)
 {
-    const size_t N = (size_t)h->sp->h.ndets;
-    RCHECK(grow(&h->d_txE, &h->txE_bytes, sizeof(double) * nvec * (size_t)h->tx->elems, "the intermediate"));
-    if (copy) RCHECK(grow(&h->d_txv, &h->txv_bytes, sizeof(double) * nvec * N, "the input vectors"));
-    RCHECK(grow(&h->d_txT, &h->txT_bytes, sizeof(double) * nvec * N, "the transposed input"));
-    return grow(&h->d_txy, &h->txy_bytes, sizeof(double) * nvec * N, "the transposed result");
+    const size_t N = (size_t)h->sp->h.ndets, sz = prec == 64 ? sizeof(double) : sizeof(float);
+    RCHECK(grow(&h->d_txE, &h->txE_bytes, sz * nvec * (size_t)h->tx->elems, "the intermediate"));
+    RCHECK(grow(&h->d_txx, &h->txx_bytes, sz * 2 * nvec * N, "the input vectors"));
+    return grow(&h->d_txy, &h->txy_bytes, sizeof(double) * 2 * nvec * N, "the result vectors");
 }
 
 static int tx_upload(jci_ham *h, const void *src, size_t bytes, void **out)
@@ -672,8 +672,8 @@ static int build_tx(jci_ham *h)
         RCHECK(tx_upload(h, nullptr, sizeof(uint16_t) * (size_t)h->nexc1[sp], (void **)&x.rk));
         RCHECK(tx_upload(h, nullptr, sizeof(int2) * (size_t)P->nkl[sp], (void **)&x.kl));
         RCHECK(tx_upload(h, nullptr, sizeof(int2) * (size_t)ns * x.npair, (void **)&x.gl));
-        RCHECK(tx_upload(h, nullptr, sizeof(double) * (size_t)np * np, (void **)&x.w64));
-        RCHECK(tx_upload(h, nullptr, sizeof(float) * (size_t)np * np, (void **)&x.w32));
+        RCHECK(tx_upload(h, nullptr, sizeof(double) * (size_t)(np + 1) * (np + 1), (void **)&x.w64));
+        RCHECK(tx_upload(h, nullptr, sizeof(float) * (size_t)(np + 1) * (np + 1), (void **)&x.w32));
         const size_t nrow = (size_t)mp + P->nint_parts[sp] + 1;
         x.zrow = (int)nrow - 1;
         RCHECK(tx_upload(h, nullptr, sizeof(double) * nrow * d.ms, (void **)&x.m64));
@@ -691,7 +691,8 @@ static int build_tx(jci_ham *h)
                            (uint32_t *)x.lst, (uint16_t *)x.rk, c->stream));
         RCHECK(jk_tx_pairs(s->d_desc, sp, ns, s->d_mask[sp], c->d_binom, dp, (int)P->pg[sp].size(),
                            x.npair, (int2 *)x.kl, (int2 *)x.gl, c->stream));
-        RCHECK(jk_tx_w(n, S.nelec, h->d_m1, h->d_m2, (double *)x.w64, (float *)x.w32, c->stream));
+        RCHECK(jk_tx_w(s->d_desc, n, S.nelec, h->d_m1, h->d_m2, (double *)x.w64, (float *)x.w32,
+                       c->stream));
         RCHECK(jk_tx_rows(s->d_desc, D, sp, s->d_mask[sp], mp, h->d_m2sq, *P, (double *)x.m64,
                           (float *)x.m32, c->stream));
         JCI_CHECK(hipStreamSynchronize(c->stream));
@@ -714,8 +715,8 @@ static int build_tx(jci_ham *h)
 #undef TX_PUT
     std::vector<long long> tt(D.nblk + 1, 0);
     for (int b = 0; b < D.nblk; b++) {
-        const long long na = D.s[0].gn[D.bp[b]], nq = D.s[1].gn[D.bq[b]];
-        tt[b + 1] = tt[b] + ((na + 15) / 16) * ((nq + 15) / 16);
+        const TxList &la = P->lists[0][D.bp[b]], &lb = P->lists[1][D.bq[b]];
+        tt[b + 1] = tt[b] + (long long)(la.nIp / 16) * la.nsv * (lb.nIp / 16) * lb.nsv;
     }
     h->nttx = tt[D.nblk];
     const size_t o_tt = put(tt.data(), sizeof(long long) * tt.size());
@@ -732,7 +733,7 @@ static int build_tx(jci_ham *h)
     d.pout = (const TxPairOut *)(m + o_po);
     d.q = (const int *)(m + o_q);
     h->d_ttx = (long long *)(m + o_tt);
-    if (D.ndets <= TX_NOALLOC_DETS) RCHECK(tx_buffers(h, 1, true));
+    if (D.ndets <= TX_NOALLOC_DETS) RCHECK(tx_buffers(h, 1, 64));
     return 0;
 }
 
@@ -742,23 +743,16 @@ static int tx_sigma(jci_ham *h, int prec, int nvec, const double *x, long long x
 {
     jci_ctx *c = h->sp->ctx;
     const long long N = h->sp->h.ndets;
-    const bool copy = prec == 32 || xs != 1;
-    RCHECK(jk_tx_in(prec, nvec, N, h->sp->d_desc, h->d_ttx, h->nttx, x, xs, xk,
-                    copy ? h->d_txv : nullptr, h->d_txT, c->stream));
     TxVec v;
-    v.x0 = copy ? h->d_txv : (const void *)x;
-    v.ldx0 = copy ? N : xk;
-    v.x1 = h->d_txT;
-    v.ldx1 = N;
-    v.y0 = y;
-    v.ys0 = ys;
-    v.yk0 = yk;
-    v.y1 = (double *)h->d_txy;
-    v.ys1 = 1;
-    v.yk1 = N;
+    v.x0 = h->d_txx;
+    v.x1 = (const char *)h->d_txx + (size_t)nvec * N * (prec == 64 ? sizeof(double) : sizeof(float));
+    v.y0 = (double *)h->d_txy;
+    v.y1 = v.y0 + (size_t)nvec * N;
+    v.N = N;
+    RCHECK(jk_tx_in(prec, nvec, N, h->sp->d_desc, h->d_ttx, h->nttx, x, xs, xk, (void *)v.x0,
+                    (void *)v.x1, c->stream));
     RCHECK(jk_tx_run(prec, nvec, h->txd, *h->tx, v, h->d_txE, c->stream));
-    return jk_tx_out(nvec, N, h->sp->d_desc, h->d_ttx, h->nttx, (const double *)h->d_txy, y, ys, yk,
-                     c->stream);
+    return jk_tx_out(nvec, N, h->sp->d_desc, h->d_ttx, h->nttx, v.y0, v.y1, y, ys, yk, c->stream);
 }
 
 // excitation tables and launch maps of the table kernels.  Spaces that take the contraction
@@ -957,7 +951,7 @@ JCI_API void jci_ham_destroy(jci_ham *h)
     hipSetDevice(h->sp->ctx->device);
     hipStreamSynchronize(h->sp->ctx->stream);
     for (int i = 0; i < h->tx_nmem; i++) hipFree(h->tx_mem[i]);
-    hipFree(h->d_txE); hipFree(h->d_txv); hipFree(h->d_txT); hipFree(h->d_txy);
+    hipFree(h->d_txE); hipFree(h->d_txx); hipFree(h->d_txy);
     delete h->tx;
     free_doubles(h);
     hipFree(h->d_m1); hipFree(h->d_m2); hipFree(h->d_hd);
@@ -1259,7 +1253,7 @@ static int fast_run(jci_ham *h, int method, int nvec, const double *x, double *y
     if (h->tx && !h->tx_off) {
         const long long ys = ldy ? 1 : nvec, yk = ldy ? ldy : 1;
         if (!s) {
-            RCHECK(tx_buffers(h, nvec, prec == 32 || nvec > 1));
+            RCHECK(tx_buffers(h, nvec, prec));
             return tx_sigma(h, prec, nvec, x, nvec, 1, y, ys, yk);
         }
         // allocation-free: the staging of the table kernels bounds the sizes taken, the vectors
@@ -2308,7 +2302,7 @@ static int ham_sigma_cols(void *self, int method, int k, const double *V, long l
     method = resolve_method(h, method, 0);
     if (method == JCI_SIGMA_FAST64 || method == JCI_SIGMA_FAST32) {
         if (h->have_fast && h->tx && !h->tx_off) {
-            RCHECK(tx_buffers(h, k, method == JCI_SIGMA_FAST32));
+            RCHECK(tx_buffers(h, k, method == JCI_SIGMA_FAST64 ? 64 : 32));
             return tx_sigma(h, method == JCI_SIGMA_FAST64 ? 64 : 32, k, V, 1, ldv, S, 1, lds);
         }
         // the table sigma reads determinant-major input and writes the columns directly

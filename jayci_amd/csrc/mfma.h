@@ -29,6 +29,7 @@ template <> struct Mf<double> {
         return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
     static __device__ __forceinline__ int row(int l, int v) { return l / 16 + 4 * v; }
+    static constexpr int LROW = 1, VROW = 4;   // row(l, v) = LROW (l / 16) + VROW v
 };
 template <> struct Mf<float> {
     typedef v4f acc;
@@ -38,4 +39,5 @@ template <> struct Mf<float> {
         return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
     static __device__ __forceinline__ int row(int l, int v) { return 4 * (l / 16) + v; }
+    static constexpr int LROW = 4, VROW = 1;
 };

@@ -36,34 +36,56 @@
 // diagonal pairs together.
 //
 // Against the table kernels (one gather per connected entry, sigma_fast.hip), whole products:
-// MRCI-SD 16e/28o FP64 one vector 304 -> 206 ms, 16e/20o FP64 three vectors 108 -> 84 ms, FP32
-// two vectors 56 -> 43 ms, 7a6b/17o two vectors 3.3 -> 2.0 ms, 4a4b/10o 260 -> 74 us; error
-// against 64 bits 2.4e-15 -> 3.3e-16 (FP64) and 1.2e-6 -> 8e-8 (FP32) at 16e/20o.
+// MRCI-SD 16e/28o FP64 one vector 304 -> 93 ms, 16e/20o FP64 three vectors 108 -> 54 ms, FP32
+// two vectors 56 -> 22.7 ms, 7a6b/17o two vectors 3.3 -> 1.37 ms, 4a4b/10o 259 -> 56 us; error
+// against 64 bits 2.4e-15 -> 3.3e-16 (FP64) and 1.2e-6 -> 7.9e-8 (FP32) at 16e/20o.
 #pragma once
 #include "jci_internal.h"
 #include "sigma_fast.h"
 
 #define TX_MAXG2 64          // groups of N - 2 electron strings per spin
-#define TX_MAXSEC 8          // target groups of a single excitation (7), or the diagonal
+#define TX_MAXSEC 8          // target groups of a single excitation (7)
 #define TX_NTYPE 6           // orbital-pair types dd, da, dv, aa, av, vv
 #define TX_KC 96             // reduction depth of one LDS tile (four waves: 50 KB in FP64)
+// column tiles x chunks of one wave's item at most (about): fragments are loaded once per item,
+// and short items let a launch end evenly (8, 64 and no limit were 1 - 4 % slower)
+#define TX_PASSES 32
 #define TX_ROWS64 32         // rows of E a wave holds integral fragments for, FP64 ...
 #define TX_ROWS32 48         // ... and FP32
 #define TX_PAD 0x7FF00000u   // list entry of a padded row or column (no position, string 0)
 
-// list entry of the first spin: target string in its group (bits 0..19), position of the pair
-// in its class (20..30), sign (31)
+// Order of the vectors' columns.  Inside a block's row the strings of the first spin are kept
+// external part outermost (column w * nI + internal part, tx_col below), so that the targets of
+// a column tile, which share few external parts, are neighbours in memory; the vectors are
+// brought into this order, and their transpose likewise, on the way in, and back on the way out.
+
+// list entry of the first spin: column of the target string in its group (bits 0..19), position
+// of the pair in its class (20..30), sign (31)
 #define TX_JBITS 20
 #define TX_KMAX 0x7FF
 
-// lists of one first-spin group: per external part `rows` rows of nIp entries, the sections
-// (target groups, then the diagonal pairs) each padded to a multiple of four rows
+// Classes of orbital pairs that a string's replacements reach: internal pairs; pairs of an
+// external orbital of the string with any external one; an external orbital of the string with
+// an internal one (the target has one external electron less); any external orbital with an
+// internal one (one more).  A section of a list holds the replacements of one class towards one
+// target group.
+#define TX_II 0
+#define TX_EE 1
+#define TX_DEC 2
+#define TX_INC 3
+
+// lists of one first-spin group: per external part `rows` rows of nIp entries, every section
+// padded to a multiple of four rows
 struct TxList {
     long long base;                  // first entry
     int rows, nI, nIp, nsv;
     int nsec;
-    int grp[TX_MAXSEC + 1];          // target group of the section, -1: the diagonal pairs
-    int row0[TX_MAXSEC + 1], cnt[TX_MAXSEC + 1];
+    int grp[TX_MAXSEC + 4], cls[TX_MAXSEC + 4];
+    int own[TX_MAXSEC + 4];          // 1: the diagonal pairs (k, k) of the string's electrons
+    int first[TX_MAXSEC + 4];        // first single of the section towards its group, in table order
+    int row0[TX_MAXSEC + 4], cnt[TX_MAXSEC + 4];
+    int nf;                          // TX_INC: external orbitals to go to; a section's rows run
+                                     // over them with the leaving orbital inside
 };
 
 // four list rows of a task's chunk: where their targets sit in the vector and in the chunk.
@@ -99,7 +121,8 @@ struct TxTask {
 
 // one task's share of a round (a range of columns small enough that E fits its buffer)
 struct TxItem {
-    int task, w0, nw, t0, nt;        // external parts, column tiles
+    int task, w0, nw, t0, nt;        // external parts, column tiles of the item
+    int p0, pn;                      // column tiles of the whole piece (rows of E)
     int rg[2];                       // row groups (FP64, FP32)
     long long item0[2];              // first item of the round's launch: (JL, w, row group)
     long long ebase;                 // first element in E
@@ -137,9 +160,11 @@ struct TxPairTask {
     long long lbase;                 // list base of the group
     int Rfull, n, nb;
 };
+#define TX_RMAX 64           // pairs up to which a work-group keeps all of W in LDS
 struct TxPairItem {
     int task, c0, nc, ncp;           // columns of the round, padded to 16
-    int rg, ct;                      // row groups of 64, column blocks of 64
+    int rg, cb, ct;                  // row groups of 64, column blocks of 64 per work-group,
+                                     // work-groups across
     long long item0, ebase;
 };
 struct TxPairOut {
@@ -165,7 +190,7 @@ struct TxSpin {
                                      // position in the type | sign << 31}
     int npair;                       // N (N - 1) / 2
     int G;
-    const double *w64;               // W, np x np
+    const double *w64;               // W, (np + 1) x (np + 1), the last row and column zero
     const float *w32;
     // integral rows of ms = m1 + 1 elements, the last one zero: (P|.) of every pair, then per
     // internal part the sum of (kk|.) over its electrons, then a row of zeros
@@ -215,6 +240,9 @@ JCI_HD int tx_type(int s0, int s1)   // s0 <= s1
     return s0 == 0 ? s1 : s0 == 1 ? 2 + s1 : 5;
 }
 
+// column of string loc of a group of nI internal x nsv external parts
+JCI_HD long long tx_col(long long loc, int nI, int nsv) { return loc % nsv * nI + loc / nsv; }
+
 // position of the single excitation x -> y of string m among its singles towards their target
 // group (enumeration order of the excitation tables: x ascending, then y ascending)
 JCI_HD int tx_single_rank(const SpaceDesc *d, uint64_t m, int x, int y)
@@ -232,42 +260,71 @@ JCI_HD int tx_single_rank(const SpaceDesc *d, uint64_t m, int x, int y)
     return r;
 }
 
-// position of the pair (x, y) in its class for a string with external part ext: internal
-// pairs; pairs of an external orbital of the string with any external one (class of equal
-// external count); external orbital of the string with an internal one (target with one
-// external orbital less); any external with an internal one (one more)
-JCI_HD int tx_kpos(const SpaceDesc *d, uint64_t ext, int dv, int x, int y)
+// position of the pair (x, y) in its class for a string with external part ext
+JCI_HD int tx_kpos(const SpaceDesc *d, uint64_t ext, int cls, int x, int y)
 {
-    const int nint = d->ndocc + d->nactv, nv = d->nvirt;
+    const int nint = d->ndocc + d->nactv;
     const int hi = x > y ? x : y, lo = x > y ? y : x;
-    if (hi < nint) return hi * (hi + 1) / 2 + lo;
-    if (dv > 0) return (hi - nint) * nint + lo;
-    if (dv < 0) return jci_popc(ext & tx_below(hi)) * nint + lo;
+    if (cls == TX_II) return hi * (hi + 1) / 2 + lo;
+    if (cls == TX_INC) return (hi - nint) * nint + lo;
+    if (cls == TX_DEC) return jci_popc(ext & tx_below(hi)) * nint + lo;
     const int b = (ext >> hi) & 1 ? hi : lo, c = b == hi ? lo : hi;
-    return nint * (nint + 1) / 2 + jci_popc(ext & tx_below(b)) * nv + (c - nint);
+    return jci_popc(ext & tx_below(b)) * d->nvirt + (c - nint);
 }
 
-// inverse of tx_kpos: pair index tri of position s of a class (dv as above), or -1
-JCI_HD int tx_kpair(int nint, int nv, const int *extorb, int next, int dv, int s)
+// its inverse: pair index tri of position s of a class for the external orbitals extorb
+JCI_HD int tx_kpair(int nint, int nv, const int *extorb, int cls, int s)
 {
-    const int m1int = nint * (nint + 1) / 2;
-    if (dv == 0) {
-        if (s < m1int) return s;
-        const int r = (s - m1int) / nv, c = nint + (s - m1int) % nv;
-        return r < next ? (int)jci_tri(extorb[r], c) : -1;
-    }
-    if (dv < 0) {
-        const int r = s / nint;
-        return r < next ? (int)jci_tri(extorb[r], s % nint) : -1;
-    }
-    const int c = s / nint;
-    return c < nv ? (int)jci_tri(nint + c, s % nint) : -1;
+    if (cls == TX_II) return s;
+    if (cls == TX_EE) return (int)jci_tri(extorb[s / nv], nint + s % nv);
+    if (cls == TX_DEC) return (int)jci_tri(extorb[s / nint], s % nint);
+    return (int)jci_tri(nint + s / nint, s % nint);
 }
 
-JCI_HD int tx_class_size(int nint, int nv, int v, int dv, int own)
+// positions of a class for a string with v external electrons
+JCI_HD int tx_class_size(int nint, int nv, int v, int cls)
 {
-    if (dv == 0) return nint * (nint + 1) / 2 + (own ? v * nv : 0);
-    return dv < 0 ? v * nint : nv * nint;
+    return cls == TX_II ? nint * (nint + 1) / 2 : cls == TX_EE ? v * nv : cls == TX_DEC ? v * nint : nv * nint;
+}
+
+// Numbering of orbital pairs i < j by type, the second orbital fastest in the mixed types: the
+// pairs a string's list walks in order are then mostly consecutive columns of W.
+JCI_HD int tx_pair_id(const SpaceDesc *d, int i, int j)
+{
+    const int n[3] = {d->ndocc, d->nactv, d->nvirt}, o[3] = {0, d->ndocc, d->ndocc + d->nactv};
+    const int si = tx_sub(d, i), sj = tx_sub(d, j), a = i - o[si], b = j - o[sj];
+    int base = 0;
+    for (int s = 0; s < 3; s++)
+        for (int t = s; t < 3; t++) {
+            if (s == si && t == sj) return base + (s == t ? b * (b - 1) / 2 + a : a * n[t] + b);
+            base += s == t ? n[s] * (n[s] - 1) / 2 : n[s] * n[t];
+        }
+    return -1;
+}
+
+// its inverse
+JCI_HD void tx_pair_orbs(const SpaceDesc *d, int P, int *i, int *j)
+{
+    const int n[3] = {d->ndocc, d->nactv, d->nvirt}, o[3] = {0, d->ndocc, d->ndocc + d->nactv};
+    for (int s = 0; s < 3; s++)
+        for (int t = s; t < 3; t++) {
+            const int c = s == t ? n[s] * (n[s] - 1) / 2 : n[s] * n[t];
+            if (P >= c) {
+                P -= c;
+                continue;
+            }
+            if (s != t) {
+                *i = o[s] + P / n[t];
+                *j = o[t] + P % n[t];
+                return;
+            }
+            int b = 1;
+            while ((b + 1) * b / 2 <= P) b++;
+            *i = o[s] + P - b * (b - 1) / 2;
+            *j = o[s] + b;
+            return;
+        }
+    *i = *j = 0;
 }
 
 // pair i < j of string m: the N - 2 string's mask, the pair's type, its position in the type's
@@ -330,25 +387,24 @@ int jk_tx_fill(long long n, uint32_t *p, hipStream_t st);
 int jk_tx_pairs(const SpaceDesc *d, int spin, long long nstr, const uint64_t *mask,
                 const unsigned long long *binom, const TxPairGroup *pg, int npg, int npair,
                 int2 *kl, int2 *gl, hipStream_t st);
-int jk_tx_w(int norb, int nelec, const double *m1, const double *m2, double *w64, float *w32,
-            hipStream_t st);
+int jk_tx_w(const SpaceDesc *d, int norb, int nelec, const double *m1, const double *m2,
+            double *w64, float *w32, hipStream_t st);
 int jk_tx_rows(const SpaceDesc *d, const SpaceDesc &h, int spin, const uint64_t *mask, int m1,
                const double *m2sq, const TxPlan &P, double *m64, float *m32, hipStream_t st);
-// x (vector k at x + k * xk, element n at n * xs) -> xT (every block transposed) and, unless
-// xv is null, xv, both vector-major of stride N in the arithmetic type
+// x (vector k at x + k * xk, element n at n * xs) -> x0 and x1 (every block transposed), both in
+// the arithmetic type, vectors of stride N, columns in tx_col order; tt: first 16 x 16 tile of
+// each block (tx_tiles)
 int jk_tx_in(int prec, int nvec, long long N, const SpaceDesc *d, const long long *tt, long long ntt,
-             const double *x, long long xs, long long xk, void *xv, void *xT, hipStream_t st);
-// y += the transposed blocks of yT
+             const double *x, long long xs, long long xk, void *x0, void *x1, hipStream_t st);
+// y = y0 and the transposed blocks of y1, in the caller's order
 int jk_tx_out(int nvec, long long N, const SpaceDesc *d, const long long *tt, long long ntt,
-              const double *yT, double *y, long long ys, long long yk, hipStream_t st);
-// the rounds of both parts; X: vector of orientation 0 (element stride 1, vector stride ldx)
-// and its block-transposed copy (vector stride N), Y likewise (y: element stride ys, vector
-// stride yk; yT: N)
+              const double *y0, const double *y1, double *y, long long ys, long long yk,
+              hipStream_t st);
+// the rounds of both parts on vectors of stride N
 struct TxVec {
     const void *x0, *x1;
-    long long ldx0, ldx1;
     double *y0, *y1;
-    long long ys0, yk0, ys1, yk1;
+    long long N;
 };
 int jk_tx_run(int prec, int nvec, const TxDev &D, const TxPlan &P, const TxVec &V, void *E,
               hipStream_t st);

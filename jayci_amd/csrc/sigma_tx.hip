@@ -1,6 +1,7 @@
 // Contraction form of the truncated-space sigma on MFMA (see sigma_tx.h).
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <type_traits>
 #include "mfma.h"
 #include "sigma_tx.h"
 
@@ -34,24 +35,25 @@ __global__ void k_tx_lists(const SpaceDesc *__restrict__ d, int spin, long long 
     const uint64_t m = M[I], ext = m & d->vmask;
     uint32_t *out = lst + t.base + w * t.rows * t.nIp + iI;
     for (int s = 0; s < t.nsec; s++) {
-        const int h = t.grp[s];
-        if (h < 0) {
-            int r = t.row0[s];
-            for (uint64_t x = m; x; x &= x - 1, r++) {
+        const int h = t.grp[s], cls = t.cls[s], n = t.cnt[s];
+        if (t.own[s]) {
+            int r = 0;
+            for (uint64_t x = cls == TX_II ? m & ~d->vmask : ext; x && r < n; x &= x - 1, r++) {
                 const int k = jci_ctz(x);
-                out[(long long)r * t.nIp] = (uint32_t)loc | ((uint32_t)tx_kpos(d, ext, 0, k, k) << TX_JBITS);
+                out[(long long)(t.row0[s] + r) * t.nIp] =
+                    (uint32_t)tx_col(loc, t.nI, t.nsv) | ((uint32_t)tx_kpos(d, ext, cls, k, k) << TX_JBITS);
             }
             continue;
         }
-        const int dv = S.gv[h] == S.gv[g] ? 0 : S.gv[h] < S.gv[g] ? -1 : 1;
-        const long long e0 = off1[I] + goff1[I * (S.ngrp + 1) + h];
-        const int n = goff1[I * (S.ngrp + 1) + h + 1] - goff1[I * (S.ngrp + 1) + h];
-        for (int k = 0; k < n && k < t.cnt[s]; k++) {
+        const long long e0 = off1[I] + goff1[I * (S.ngrp + 1) + h] + t.first[s];
+        const int left = goff1[I * (S.ngrp + 1) + h + 1] - goff1[I * (S.ngrp + 1) + h] - t.first[s];
+        for (int k = 0; k < n && k < left; k++) {
             const int2 en = e1[e0 + k];
             const int i = en.y & 63, f = (en.y >> 6) & 63;
-            out[(long long)(t.row0[s] + k) * t.nIp] =
-                (uint32_t)(en.x - S.gstart[h]) |
-                ((uint32_t)tx_kpos(d, ext, dv, i, f) << TX_JBITS) |
+            const int r = cls == TX_INC ? k % t.nf * (n / t.nf) + k / t.nf : k;
+            out[(long long)(t.row0[s] + r) * t.nIp] =
+                (uint32_t)tx_col(en.x - S.gstart[h], lists[h].nI, lists[h].nsv) |
+                ((uint32_t)tx_kpos(d, ext, cls, i, f) << TX_JBITS) |
                 ((uint32_t)((en.y >> 12) & 1) << 31);
             rk[e0 + k] = (uint16_t)tx_single_rank(d, m ^ (1ULL << i) ^ (1ULL << f), f, i);
         }
@@ -120,7 +122,7 @@ __global__ void k_tx_pairs(const SpaceDesc *__restrict__ d, int spin, long long 
                     gl[I * npair + at++] = make_int2((int)K, idx | (int)((unsigned)neg << 31));
                     kl[pg[q].base + K * pg[q].R + pg[q].off[ty] + idx] =
                         make_int2((int)(I - S.gstart[g]),
-                                  (j * (j - 1) / 2 + i) | (int)((unsigned)neg << 31));
+                                  tx_pair_id(d, i, j) | (int)((unsigned)neg << 31));
                 }
             }
         }
@@ -136,40 +138,35 @@ int jk_tx_pairs(const SpaceDesc *d, int spin, long long nstr, const uint64_t *ma
     return 0;
 }
 
-__device__ __forceinline__ void pair_of(int P, int *i, int *j)
-{
-    int b = (int)((1.0 + sqrt(1.0 + 8.0 * P)) * 0.5);
-    while (b * (b - 1) / 2 > P) b--;
-    while ((b + 1) * b / 2 <= P) b++;
-    *j = b;
-    *i = P - b * (b - 1) / 2;
-}
-
-__global__ void k_tx_w(int np, double sc, const double *__restrict__ m1,
+__global__ void k_tx_w(const SpaceDesc *__restrict__ d, int np, double sc, const double *__restrict__ m1,
                        const double *__restrict__ m2, double *__restrict__ w64,
                        float *__restrict__ w32)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)np * np) return;
-    int i, j, k, l;
-    pair_of((int)(t / np), &i, &j);
-    pair_of((int)(t % np), &k, &l);
-    double v = jci_eri(m2, i, k, j, l) - jci_eri(m2, i, l, j, k);
-    double h = 0.0;
-    if (j == l) h += jci_h1(m1, i, k);
-    if (i == l) h -= jci_h1(m1, j, k);
-    if (j == k) h -= jci_h1(m1, i, l);
-    if (i == k) h += jci_h1(m1, j, l);
-    v += h * sc;
+    const int ws = np + 1, P = (int)(t / ws), Q = (int)(t % ws);
+    if (P > np) return;
+    double v = 0.0;
+    if (P < np && Q < np) {
+        int i, j, k, l;
+        tx_pair_orbs(d, P, &i, &j);
+        tx_pair_orbs(d, Q, &k, &l);
+        v = jci_eri(m2, i, k, j, l) - jci_eri(m2, i, l, j, k);
+        double h = 0.0;
+        if (j == l) h += jci_h1(m1, i, k);
+        if (i == l) h -= jci_h1(m1, j, k);
+        if (j == k) h -= jci_h1(m1, i, l);
+        if (i == k) h += jci_h1(m1, j, l);
+        v += h * sc;
+    }
     w64[t] = v;
     w32[t] = (float)v;
 }
 
-int jk_tx_w(int norb, int nelec, const double *m1, const double *m2, double *w64, float *w32,
-            hipStream_t st)
+int jk_tx_w(const SpaceDesc *d, int norb, int nelec, const double *m1, const double *m2,
+            double *w64, float *w32, hipStream_t st)
 {
     const int np = norb * (norb - 1) / 2;
-    hipLaunchKernelGGL(k_tx_w, dim3((unsigned)(((long long)np * np + 255) / 256)), dim3(256), 0, st, np,
+    hipLaunchKernelGGL(k_tx_w, dim3((unsigned)(((long long)(np + 1) * (np + 1) + 255) / 256)), dim3(256), 0, st, d, np,
                        1.0 / (nelec - 1), m1, m2, w64, w32);
     TX_CHECK();
     return 0;
@@ -233,91 +230,167 @@ __device__ __forceinline__ int tx_block(const long long *__restrict__ off, int n
     return lo;
 }
 
-// 16 x 16 element tiles of the blocks (tt: first tile of each block): the vector in the
-// arithmetic type (xv, may be null) and its block-transposed copy.  Bound by memory: one read
-// and one or two writes of the vector.
-template <typename T>
-__global__ __launch_bounds__(256) void k_tx_in(long long N, const SpaceDesc *__restrict__ d,
-                                               const long long *__restrict__ tt,
-                                               const double *__restrict__ x, long long xs,
-                                               long long xk, T *__restrict__ xv, T *__restrict__ xT)
+// work-groups in runs of `run` consecutive ones per XCD (they are dealt to the 8 XCDs round
+// robin), so that neighbours share an L2; the grid is a multiple of 8 run
+#define TX_RUN 16
+__device__ __forceinline__ long long tx_xcd(long long b)
 {
-    __shared__ T t[16][17];
-    const int b = tx_block(tt, d->nblk, blockIdx.x);
-    const long long na = d->s[0].gn[d->bp[b]], nb = d->s[1].gn[d->bq[b]];
-    const long long ntc = (nb + 15) / 16, rel = blockIdx.x - tt[b];
-    const long long r0 = rel / ntc * 16, c0 = rel % ntc * 16, off = d->boff[b];
-    const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
-    const long long k = blockIdx.y;
-    if (r0 + ty < na && c0 + tx < nb) {
-        const long long n = off + (r0 + ty) * nb + c0 + tx;
-        const T v = (T)x[n * xs + k * xk];
-        t[ty][tx] = v;
-        if (xv) xv[k * N + n] = v;
-    }
-    __syncthreads();
-    if (c0 + ty < nb && r0 + tx < na) xT[k * N + off + (c0 + ty) * na + r0 + tx] = t[tx][ty];
+    const long long q = b / (8 * TX_RUN), r = b % (8 * TX_RUN);
+    return q * (8 * TX_RUN) + (r & 7) * TX_RUN + (r >> 3);
+}
+static inline unsigned tx_grid(long long n)
+{
+    return (unsigned)((n + 8 * TX_RUN - 1) / (8 * TX_RUN) * (8 * TX_RUN));
 }
 
-__global__ __launch_bounds__(256) void k_tx_out(long long N, const SpaceDesc *__restrict__ d,
-                                                const long long *__restrict__ tt,
-                                                const double *__restrict__ yT,
-                                                double *__restrict__ y, long long ys, long long yk)
+// one 16 x 16 tile of a block: internal parts ia0 .. of external part wa, and so for columns
+struct TxTile {
+    int b, ia0, wa, ib0, wb, nIa, nsa, nIb, nsb;
+    long long na, nb, off;
+};
+__device__ __forceinline__ TxTile tx_tile(const SpaceDesc *__restrict__ d,
+                                          const long long *__restrict__ tt, long long u)
 {
-    __shared__ double t[16][17];
-    const int b = tx_block(tt, d->nblk, blockIdx.x);
-    const long long na = d->s[0].gn[d->bp[b]], nb = d->s[1].gn[d->bq[b]];
-    const long long ntc = (nb + 15) / 16, rel = blockIdx.x - tt[b];
-    const long long r0 = rel / ntc * 16, c0 = rel % ntc * 16, off = d->boff[b];
+    TxTile t;
+    t.b = tx_block(tt, d->nblk, u);
+    const int p = d->bp[t.b], q = d->bq[t.b];
+    t.na = d->s[0].gn[p];
+    t.nb = d->s[1].gn[q];
+    t.nsa = (int)(d->s[0].nsv[p] > 1 ? d->s[0].nsv[p] : 1);
+    t.nsb = (int)(d->s[1].nsv[q] > 1 ? d->s[1].nsv[q] : 1);
+    t.nIa = (int)(t.na / t.nsa);
+    t.nIb = (int)(t.nb / t.nsb);
+    const int ntc = (t.nIb + 15) / 16 * t.nsb;
+    const long long rel = u - tt[t.b];
+    const int rt = (int)(rel / ntc), ct = (int)(rel % ntc);
+    t.wa = rt % t.nsa;
+    t.ia0 = rt / t.nsa * 16;
+    t.wb = ct % t.nsb;
+    t.ib0 = ct / t.nsb * 16;
+    t.off = d->boff[t.b];
+    return t;
+}
+
+// The vector into tx_col order, straight and block-transposed.  Bound by memory: one read (in
+// runs of 16 external parts of a string, neighbouring tiles sharing the lines) and two writes.
+template <typename T>
+__global__ __launch_bounds__(256) void k_tx_in(long long N, long long ntt, const SpaceDesc *__restrict__ d,
+                                               const long long *__restrict__ tt,
+                                               const double *__restrict__ x, long long xs,
+                                               long long xk, T *__restrict__ x0, T *__restrict__ x1)
+{
+    __shared__ T s[16][17];
+    const long long u = tx_xcd(blockIdx.x);
+    if (u >= ntt) return;
+    const TxTile t = tx_tile(d, tt, u);
     const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
     const long long k = blockIdx.y;
-    if (c0 + ty < nb && r0 + tx < na) t[ty][tx] = yT[k * N + off + (c0 + ty) * na + r0 + tx];
+    if (t.ia0 + ty < t.nIa && t.ib0 + tx < t.nIb) {
+        const long long r = (long long)(t.ia0 + ty) * t.nsa + t.wa, c = (long long)(t.ib0 + tx) * t.nsb + t.wb;
+        const T v = (T)x[(t.off + r * t.nb + c) * xs + k * xk];
+        s[ty][tx] = v;
+        x0[k * N + t.off + r * t.nb + (long long)t.wb * t.nIb + t.ib0 + tx] = v;
+    }
     __syncthreads();
-    if (r0 + ty < na && c0 + tx < nb) {
-        const long long n = off + (r0 + ty) * nb + c0 + tx;
-        y[n * ys + k * yk] += t[tx][ty];
+    if (t.ib0 + ty < t.nIb && t.ia0 + tx < t.nIa) {
+        const long long c = (long long)(t.ib0 + ty) * t.nsb + t.wb;
+        x1[k * N + t.off + c * t.na + (long long)t.wa * t.nIa + t.ia0 + tx] = s[tx][ty];
+    }
+}
+
+__global__ __launch_bounds__(256) void k_tx_out(long long N, long long ntt, const SpaceDesc *__restrict__ d,
+                                                const long long *__restrict__ tt,
+                                                const double *__restrict__ y0,
+                                                const double *__restrict__ y1,
+                                                double *__restrict__ y, long long ys, long long yk)
+{
+    __shared__ double s[16][17];
+    const long long u = tx_xcd(blockIdx.x);
+    if (u >= ntt) return;
+    const TxTile t = tx_tile(d, tt, u);
+    const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
+    const long long k = blockIdx.y;
+    if (t.ib0 + ty < t.nIb && t.ia0 + tx < t.nIa) {
+        const long long c = (long long)(t.ib0 + ty) * t.nsb + t.wb;
+        s[ty][tx] = y1[k * N + t.off + c * t.na + (long long)t.wa * t.nIa + t.ia0 + tx];
+    }
+    __syncthreads();
+    if (t.ia0 + ty < t.nIa && t.ib0 + tx < t.nIb) {
+        const long long r = (long long)(t.ia0 + ty) * t.nsa + t.wa, c = (long long)(t.ib0 + tx) * t.nsb + t.wb;
+        y[(t.off + r * t.nb + c) * ys + k * yk] =
+            y0[k * N + t.off + r * t.nb + (long long)t.wb * t.nIb + t.ib0 + tx] + s[tx][ty];
     }
 }
 
 int jk_tx_in(int prec, int nvec, long long N, const SpaceDesc *d, const long long *tt, long long ntt,
-             const double *x, long long xs, long long xk, void *xv, void *xT, hipStream_t st)
+             const double *x, long long xs, long long xk, void *x0, void *x1, hipStream_t st)
 {
-    const dim3 g((unsigned)ntt, (unsigned)nvec);
+    const dim3 g(tx_grid(ntt), (unsigned)nvec);
     if (prec == 64)
-        hipLaunchKernelGGL(k_tx_in<double>, g, dim3(256), 0, st, N, d, tt, x, xs, xk, (double *)xv,
-                           (double *)xT);
+        hipLaunchKernelGGL(k_tx_in<double>, g, dim3(256), 0, st, N, ntt, d, tt, x, xs, xk, (double *)x0,
+                           (double *)x1);
     else
-        hipLaunchKernelGGL(k_tx_in<float>, g, dim3(256), 0, st, N, d, tt, x, xs, xk, (float *)xv,
-                           (float *)xT);
+        hipLaunchKernelGGL(k_tx_in<float>, g, dim3(256), 0, st, N, ntt, d, tt, x, xs, xk, (float *)x0,
+                           (float *)x1);
     TX_CHECK();
     return 0;
 }
 
 int jk_tx_out(int nvec, long long N, const SpaceDesc *d, const long long *tt, long long ntt,
-              const double *yT, double *y, long long ys, long long yk, hipStream_t st)
+              const double *y0, const double *y1, double *y, long long ys, long long yk,
+              hipStream_t st)
 {
-    hipLaunchKernelGGL(k_tx_out, dim3((unsigned)ntt, (unsigned)nvec), dim3(256), 0, st, N, d, tt, yT, y,
-                       ys, yk);
+    hipLaunchKernelGGL(k_tx_out, dim3(tx_grid(ntt), (unsigned)nvec), dim3(256), 0, st, N, ntt, d, tt, y0,
+                       y1, y, ys, yk);
     TX_CHECK();
     return 0;
 }
 
 // ---- same-spin part ----------------------------------------------------------------------------
 
+// element i of an array of less than 4 GB: a uniform base and a 32-bit offset per lane
+template <typename T> __device__ __forceinline__ T tx_at(const T *p, uint32_t i)
+{
+    return *(const T *)((const char *)p + i * (uint32_t)sizeof(T));
+}
+
+template <typename T> __device__ __forceinline__ void tx_put(T *p, uint32_t i, T v)
+{
+    *(T *)((char *)p + i * (uint32_t)sizeof(T)) = v;
+}
+
+__device__ __forceinline__ void tx_load4(double *v, const double *p)
+{
+    const double2 a = *(const double2 *)p, b = *(const double2 *)(p + 2);
+    v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
+}
+__device__ __forceinline__ void tx_load4(float *v, const float *p)
+{
+    const float4 a = *(const float4 *)p;
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+}
 template <typename T> __device__ __forceinline__ const T *tx_w(const TxSpin &s);
 template <> __device__ __forceinline__ const double *tx_w<double>(const TxSpin &s) { return s.w64; }
 template <> __device__ __forceinline__ const float *tx_w<float>(const TxSpin &s) { return s.w32; }
 
 // E[p][K2, c] on 64 x 64 tiles (64 pairs of one N - 2 electron string, 64 columns): a wave owns
 // 16 columns and all four row tiles, its B operand comes straight from the vector (rows of 16
-// consecutive elements), the W tile is staged in LDS one 16-deep step ahead.
-template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_tx_ess(TxDev A, TxRound R, const T *__restrict__ x0,
-                                                long long ldx0, const T *__restrict__ x1,
-                                                long long ldx1, T *__restrict__ E)
+// consecutive elements).  Strings of up to TX_RMAX pairs (most of them, and few pairs at that)
+// keep their whole W block in LDS for several column blocks, without barriers in between; the
+// others stage W one 16-deep step ahead.  In a step lane group g takes the pairs
+// 4 g .. 4 g + 3, so that its four W entries of a row are one or two 16-byte reads.  The pair
+// list is padded to whole steps by the zero row of W.  Offsets are 32 bits while the vector is
+// below 4 GB (BIG: 64).  Bound by the E traffic: 16e/28o FP64 writes 32 GB in 19.7 ms (one
+// 64-column block per work-group: 23.1 ms).
+#define TX_WS (TX_RMAX + 4)          // row stride of the W tile: 16-byte reads, rows spread over the banks
+template <typename T, bool BIG>
+__global__ __launch_bounds__(256, 4) void k_tx_ess(TxDev A, TxRound R, long long N,
+                                                   const T *__restrict__ x0, const T *__restrict__ x1,
+                                                   T *__restrict__ E)
 {
+    typedef typename std::conditional<BIG, long long, uint32_t>::type O;
     extern __shared__ __align__(16) unsigned char tx_smem[];
-    __shared__ T As[2][16][65];
+    __shared__ __align__(16) T As[64][TX_WS];
     const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
     int lo = 0, hi = R.ni - 1;
     const TxPairItem *__restrict__ items = A.pitem + R.i0;
@@ -330,89 +403,145 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const TxPairTask &t = A.ptask[it.task];
     const int loc = (int)(u - it.item0), rg = loc % it.rg, ct = loc / it.rg % it.ct;
     const long long K2 = loc / (it.rg * it.ct);
-    const int Rr = t.R, r0 = rg * 64;
+    const int Rr = t.R, Rp = (Rr + 15) / 16 * 16, r0 = rg * 64, nc = it.nc, ncp = it.ncp;
     const TxSpin &S = A.s[t.o];
     const long long k = blockIdx.y;
-    const T *__restrict__ x = (t.o ? x1 + k * ldx1 : x0 + k * ldx0) + it.c0 + ct * 64;
-    long long *__restrict__ off = (long long *)tx_smem;
-    int *__restrict__ pr = (int *)(off + Rr);
-    for (int r = tid; r < Rr; r += 256) {
-        int s = 0;
-        while (s + 1 < t.nsec && t.sr[s + 1] <= r) s++;
-        const int2 en = S.kl[t.lbase + K2 * t.Rfull + t.so[s] + (r - t.sr[s])];
-        off[r] = t.sx[s] + (long long)en.x * t.nb;
-        pr[r] = en.y;
+    const int np = A.np, ws = np + 1;
+    // vector offset and W row of every pair, sign in bit 31
+    O *__restrict__ off = (O *)tx_smem;
+    int *__restrict__ pr = (int *)(off + Rp);
+    for (int r = tid; r < Rp; r += 256) {
+        int p = np;
+        O o = (O)t.sx[0];
+        if (r < Rr) {
+            int s = 0;
+            while (s + 1 < t.nsec && t.sr[s + 1] <= r) s++;
+            const int2 en = S.kl[t.lbase + K2 * t.Rfull + t.so[s] + (r - t.sr[s])];
+            o = (O)(t.sx[s] + (long long)en.x * t.nb);
+            p = en.y;
+        }
+        off[r] = o;
+        pr[r] = p;
     }
     __syncthreads();
-    const int np = A.np;
     const T *__restrict__ W = tx_w<T>(S);
-    const int ar = tid >> 2, ak = (tid & 3) * 4;
-    const bool aok = r0 + ar < Rr;
-    const T *__restrict__ Wr = W + (long long)(aok ? pr[r0 + ar] & 0x7FFFFFFF : 0) * np;
-    const int c = w * 16 + (l & 15), kk = l >> 4;
-    const bool cok = ct * 64 + c < it.nc;
+    // W tile: rows ar + 16 j, column ak (16 mostly consecutive columns of four rows a load)
+    const int ar = tid >> 4, ak = tid & 15, kk = l >> 4;
+    const int nrt = (std::min(64, Rr - r0) + 15) / 16;
+    uint32_t wrow[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int r = r0 + ar + 16 * j;
+        wrow[j] = (uint32_t)(r < Rp ? pr[r] & 0x7FFFFFFF : np) * ws;
+    }
+    const T *__restrict__ x = (t.o ? x1 : x0) + k * N + it.c0;
+    T *__restrict__ Ek = E + k * R.elems + it.ebase + (K2 * Rr + r0) * ncp;
+    const int cb0 = ct * it.cb, cb1 = std::min(cb0 + it.cb, (nc + 63) / 64);
     T ra[4], rb[4];
-    auto gload = [&](int k0) {
+    typename Mf<T>::acc acc[4];
+    auto load_w = [&](int k0) __attribute__((always_inline)) {
+        const int p = pr[k0 + ak];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (j < nrt) {
+                const T v = tx_at(W, wrow[j] + (uint32_t)(p & 0x7FFFFFFF));
+                ra[j] = p < 0 ? -v : v;
+            }
+    };
+    // the vector's rows of a step; columns past the end repeat the last one (their products are
+    // not read)
+    auto load_x = [&](int k0, uint32_t xc) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int q = k0 + ak + j;
-            ra[j] = aok && q < Rr ? Wr[pr[q] & 0x7FFFFFFF] : (T)0;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int q = k0 + j * 4 + kk;
-            const bool ok = cok && q < Rr;
-            const T v = ok ? x[off[ok ? q : 0] + c] : (T)0;
-            rb[j] = ok && pr[q] < 0 ? -v : v;
+            const O o = off[k0 + kk * 4 + j];
+            rb[j] = BIG ? x[(long long)o + xc] : tx_at(x, (uint32_t)o + xc);
         }
     };
-    typename Mf<T>::acc acc[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) acc[i] = Mf<T>::zero();
-    const int nrt = (std::min(64, Rr - r0) + 15) / 16;
-    gload(0);
-#pragma unroll
-    for (int j = 0; j < 4; j++) As[0][ak + j][ar] = ra[j];
-    __syncthreads();
-    int buf = 0;
-    for (int k0 = 0; k0 < Rr; k0 += 16) {
-        T b[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) b[j] = rb[j];
-        const bool more = k0 + 16 < Rr;
-        if (more) gload(k0 + 16);
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            if (i < nrt) {
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    acc[i] = Mf<T>::mma(As[buf][j * 4 + kk][i * 16 + (l & 15)], b[j], acc[i]);
-            }
-        if (more) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) As[buf ^ 1][ak + j][ar] = ra[j];
-        }
-        __syncthreads();
-        buf ^= 1;
-    }
-    if (ct * 64 + c < it.ncp) {
-        T *__restrict__ Er = E + k * R.elems + it.ebase + K2 * Rr * it.ncp + ct * 64 + c;
+    auto store = [&](int c) __attribute__((always_inline)) {
+        if (c >= ncp) return;
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const int r = r0 + i * 16 + Mf<T>::row(l, v);
-                if (r < Rr) Er[(long long)r * it.ncp] = acc[i][v];
+                const int r = i * 16 + Mf<T>::row(l, v);
+                if (r0 + r < Rr) Ek[(long long)r * ncp + c] = acc[i][v];
             }
+    };
+    const int cl = w * 16 + (l & 15);
+    if (Rp <= TX_RMAX) {
+        for (int k0 = 0; k0 < Rp; k0 += 16) {
+            load_w(k0);
+#pragma unroll
+            for (int j = 0; j < 4; j++) if (j < nrt) As[ar + 16 * j][k0 + ak] = ra[j];
+        }
+        __syncthreads();
+        for (int cb = cb0; cb < cb1; cb++) {
+            if (cb * 64 + w * 16 >= nc) break;
+            const uint32_t xc = (uint32_t)std::min(cb * 64 + cl, nc - 1);
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[i] = Mf<T>::zero();
+            load_x(0, xc);
+            for (int k0 = 0; k0 < Rp; k0 += 16) {
+                T b[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) b[j] = rb[j];
+                if (k0 + 16 < Rp) load_x(k0 + 16, xc);
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (i < nrt) {
+                        T a[4];
+                        tx_load4(a, &As[i * 16 + (l & 15)][k0 + kk * 4]);
+#pragma unroll
+                        for (int j = 0; j < 4; j++) acc[i] = Mf<T>::mma(a[j], b[j], acc[i]);
+                    }
+            }
+            store(cb * 64 + cl);
+        }
+        return;
     }
+    // two 16-deep W tiles side by side in As, columns 0 .. 15 and 32 .. 47
+    const uint32_t xc = (uint32_t)std::min(cb0 * 64 + cl, nc - 1);
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[i] = Mf<T>::zero();
+    load_w(0);
+    load_x(0, xc);
+#pragma unroll
+    for (int j = 0; j < 4; j++) if (j < nrt) As[ar + 16 * j][ak] = ra[j];
+    __syncthreads();
+    int buf = 0;
+    for (int k0 = 0; k0 < Rp; k0 += 16) {
+        T b[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) b[j] = rb[j];
+        const bool more = k0 + 16 < Rp;
+        if (more) {
+            load_w(k0 + 16);
+            load_x(k0 + 16, xc);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (i < nrt) {
+                T a[4];
+                tx_load4(a, &As[i * 16 + (l & 15)][buf + kk * 4]);
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[i] = Mf<T>::mma(a[j], b[j], acc[i]);
+            }
+        buf ^= 32;
+        if (more) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) if (j < nrt) As[ar + 16 * j][buf + ak] = ra[j];
+        }
+        __syncthreads();
+    }
+    store(cb0 * 64 + cl);
 }
 
 // the same-spin sums: y(I, c) = sum over the pairs of I, one E row each (coalesced); the first
 // writer of the result
 template <typename T>
-__global__ __launch_bounds__(256) void k_tx_gss(TxDev A, TxRound R, const T *__restrict__ E, double *y0,
-                                                long long ys0, long long yk0, double *y1,
-                                                long long ys1, long long yk1)
+__global__ __launch_bounds__(256) void k_tx_gss(TxDev A, TxRound R, long long N,
+                                                const T *__restrict__ E, double *__restrict__ y0,
+                                                double *__restrict__ y1)
 {
     int lo = 0, hi = R.no - 1;
     const TxPairOut *__restrict__ outs = A.pout + R.o0;
@@ -452,21 +581,20 @@ __global__ __launch_bounds__(256) void k_tx_gss(TxDev A, TxRound R, const T *__r
         g += t.np[s];
     }
     const long long n = t.yb + (long long)il * t.nb + t.c0 + c;
-    if (t.o) y1[n * ys1 + k * yk1] = (double)acc;
-    else y0[n * ys0 + k * yk0] = (double)acc;
+    (t.o ? y1 : y0)[k * N + n] = (double)acc;
 }
 
 // ---- opposite-spin part ------------------------------------------------------------------------
 
 template <typename T> struct TxV;
 template <> struct TxV<double> {
-    static constexpr int VK = 2, PAD = 2, RT = TX_ROWS64 / 16, PREC = 0, EP = 12;
+    static constexpr int VK = 2, PAD = 2, RT = TX_ROWS64 / 16, PREC = 0, EP = 4, WPE = 3;
     typedef double2 vec;
     static __device__ __forceinline__ double at(const vec &v, int q) { return q ? v.y : v.x; }
     static __device__ __forceinline__ const double *rows(const TxSpin &s) { return s.m64; }
 };
 template <> struct TxV<float> {
-    static constexpr int VK = 4, PAD = 4, RT = TX_ROWS32 / 16, PREC = 1, EP = 12;
+    static constexpr int VK = 4, PAD = 4, RT = TX_ROWS32 / 16, PREC = 1, EP = 8, WPE = 3;
     typedef float4 vec;
     static __device__ __forceinline__ float at(const vec &v, int q)
     {
@@ -492,6 +620,7 @@ __device__ __forceinline__ void tx_mma(typename Mf<T>::acc *acc, const T (*a)[KS
 #pragma unroll
             for (int i = 0; i < NR; i++)
                 acc[i] = Mf<T>::mma(a[i][g * VK + q], TxV<T>::at(b[g & 1], q), acc[i]);
+        __builtin_amdgcn_sched_barrier(0);   // one group of B vectors ahead, no more
     }
 }
 
@@ -502,13 +631,8 @@ __device__ __forceinline__ void tx_wave_sync()
     __builtin_amdgcn_wave_barrier();
 }
 
-// element i of an array of less than 4 GB: a uniform base and a 32-bit offset per lane
-template <typename T> __device__ __forceinline__ T tx_at(const T *p, uint32_t i)
-{
-    return *(const T *)((const char *)p + i * (uint32_t)sizeof(T));
-}
-
 // a value that all lanes share, in scalar registers
+__device__ __forceinline__ int tx_uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ long long tx_uni(long long v)
 {
     const unsigned lo = __builtin_amdgcn_readfirstlane((int)v);
@@ -524,129 +648,180 @@ struct TxUnit {
 // one chunk of the reduction for every column tile and vector of the wave
 template <typename T, int KS>
 __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const TxTask &t,
-                                       const TxChunk &ch, const TxUnit &u, bool add,
+                                       const TxChunk &ch, TxUnit u, bool add,
                                        const T *__restrict__ x, long long ldx, T *__restrict__ Eo,
                                        long long lde, T *__restrict__ Dt)
 {
     constexpr int RT = TxV<T>::RT, EP = TxV<T>::EP, KC = 4 * KS, LDC = KC + TxV<T>::PAD;
     typedef typename TxV<T>::vec V;
-    const TxSpin &SL = A.s[t.o], &SF = A.s[1 - t.o];
-    const int l = threadIdx.x & 63, col = l & 15, part = l >> 4;
-    const int m1 = A.m1, La = t.La;
-    const long long J = t.ls0 + u.ja;
+    // the lane and the unit made opaque here: what the reduction depths have in common would
+    // otherwise be computed ahead of the switch over them and held in registers all along
+    int l = threadIdx.x & 63;
+    asm volatile("" : "+v"(l), "+s"(u.ja), "+s"(u.w), "+s"(u.r0));
+    const int col = l & 15, part = l >> 4;
+    const int La = tx_uni(t.La), nIp = tx_uni(t.nIp);
 
     // integral fragments: row r0 + 16 i + col, steps part * KS .. part * KS + KS - 1
     T a[RT][KS];
     {
+        const TxSpin &SL = A.s[t.o];
+        const long long J = t.ls0 + u.ja;
         const long long e0 = SL.off1[J];
         const int *__restrict__ go = SL.goff1 + J * (SL.G + 1);
         const T *__restrict__ M = TxV<T>::rows(SL);
-        const int *__restrict__ qt = A.q + ch.q0 + (long long)u.w * KC + part * KS;
+        const int *__restrict__ qt = A.q + ch.q0 + (long long)u.w * KC;
         const uint32_t zero = (uint32_t)SL.zrow * A.ms;
-        uint32_t row[RT];
+        // the rows come through LDS, a row (a run of mostly consecutive pairs) per load
+        uint32_t Q[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) Q[h] = qt[std::min(l + 64 * h, KC - 1)];
 #pragma unroll
         for (int i = 0; i < RT; i++) {
             const int r = u.r0 + i * 16 + col;
-            row[i] = zero;
+            uint32_t row = zero;
             if (r < La - t.diag) {
                 int s = 0;
                 while (s + 1 < t.nsec && t.sr0[s + 1] <= r) s++;
-                row[i] = (uint32_t)((SL.e1[e0 + go[t.sg[s]] + r - t.sr0[s]].y >> 18) & 4095) * A.ms;
+                row = (uint32_t)((SL.e1[e0 + go[t.sg[s]] + r - t.sr0[s]].y >> 18) & 4095) * A.ms;
             } else if (r < La) {
-                row[i] = (uint32_t)(m1 + t.iI0 + u.ja / t.nsvL) * A.ms;
+                row = (uint32_t)(A.m1 + t.iI0 + u.ja / t.nsvL) * A.ms;
             }
-        }
 #pragma unroll
-        for (int s = 0; s < KS; s++) {
-            const uint32_t Q = qt[s];
+            for (int g = 0; g < 16; g += 8) {
+                T v[8][2];
 #pragma unroll
-            for (int i = 0; i < RT; i++) a[i][s] = tx_at(M, row[i] + Q);
-            if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-        }
-        if (u.dr >= 0 && u.dr < RT * 16)
-            // the external electrons of JL add to its diagonal row
-            for (uint64_t z = A.nint >= 64 ? 0 : SL.mask[J] >> A.nint << A.nint; z; z &= z - 1) {
-                const int o = jci_ctz(z);
+                for (int j = 0; j < 8; j++) {
+                    const T *__restrict__ Mr = M + (uint32_t)__builtin_amdgcn_readlane((int)row, g + j);
 #pragma unroll
-                for (int i = 0; i < RT; i++)
-                    row[i] = i * 16 + col == u.dr ? (uint32_t)jci_tri(o, o) * A.ms : zero;
-#pragma unroll
-                for (int s = 0; s < KS; s++) {
-                    const uint32_t Q = qt[s];
-#pragma unroll
-                    for (int i = 0; i < RT; i++) a[i][s] += tx_at(M, row[i] + Q);
-                    if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                    for (int h = 0; h < (KC > 64 ? 2 : 1); h++) v[j][h] = tx_at(Mr, Q[h]);
                 }
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+#pragma unroll
+                    for (int h = 0; h < (KC > 64 ? 2 : 1); h++)
+                        if (l + 64 * h < KC) Dt[(g + j) * LDC + l + 64 * h] = v[j][h];
             }
+            tx_wave_sync();
+            if (u.dr >> 4 == i && u.dr >= 0) {
+                // the external electrons of JL add to its diagonal row
+                for (uint64_t z = A.nint >= 64 ? 0 : SL.mask[J] >> A.nint << A.nint; z; z &= z - 1) {
+                    const int o = jci_ctz(z);
+                    const T *__restrict__ Mr = M + (uint32_t)jci_tri(o, o) * A.ms;
+#pragma unroll
+                    for (int h = 0; h < (KC > 64 ? 2 : 1); h++)
+                        if (l + 64 * h < KC) Dt[(u.dr & 15) * LDC + l + 64 * h] += tx_at(Mr, Q[h]);
+                }
+                tx_wave_sync();
+            }
+#pragma unroll
+            for (int s = 0; s < KS; s += TxV<T>::VK) {
+                const V v = *(const V *)(Dt + col * LDC + part * KS + s);
+#pragma unroll
+                for (int q = 0; q < TxV<T>::VK; q++)
+#pragma unroll
+                    for (int ii = 0; ii < RT; ii++)
+                        if (ii == i) a[ii][s + q] = TxV<T>::at(v, q);
+            }
+            tx_wave_sync();
+        }
     }
 
-    const TxSlot *__restrict__ slots = A.slot + ch.slot0;
-    const int nsl = ch.nslot, nep = std::min(nsl, EP);
-    const uint32_t *__restrict__ lst =
-        SF.lst + t.lbase + (long long)u.w * t.lrows * t.nIp + part * t.nIp + col;
-    // vector base, list row and chunk steps of the first slots, in scalar registers
-    long long xo[EP];
-    int lo[EP], ki[EP];
-#pragma unroll
-    for (int j = 0; j < EP; j++) {
-        const TxSlot &q = slots[j < nsl ? j : 0];
-        xo[j] = tx_uni(q.xb + (long long)u.ja * q.nb);
-        lo[j] = __builtin_amdgcn_readfirstlane(q.lrow * t.nIp);
-        ki[j] = __builtin_amdgcn_readfirstlane(q.kinfo);
+    // list of external part w; a lane reads row `part` of four, column `col` of a tile
+    const uint32_t *__restrict__ lst = A.s[1 - t.o].lst + tx_uni(t.lbase + (long long)u.w * t.lrows * nIp);
+    const uint32_t lofs = (uint32_t)(part * nIp + col);
+    // vector base, list row and chunk steps of slot j in lane j (chunks hold at most 64 slots)
+    const int nsl = tx_uni(ch.nslot);
+    int vxl, vxh, vlo, vki;
+    {
+        const TxSlot &q = A.slot[ch.slot0 + std::min(l, nsl - 1)];
+        const long long xo = q.xb + (long long)u.ja * q.nb;
+        vxl = (int)xo;
+        vxh = (int)(xo >> 32);
+        vlo = q.lrow * nIp;
+        vki = l < nsl ? q.kinfo : 0;
     }
-    auto put = [&](int k, uint32_t e, T v) __attribute__((always_inline)) {
-        const int s = (int)((e >> TX_JBITS) & TX_KMAX) - (k >> 16);
-        if ((unsigned)s < (unsigned)((k >> 8) & 0xFF)) Dt[col * LDC + s + (k & 0xFF)] = e >> 31 ? -v : v;
-    };
+    T *Dc = Dt + col * LDC;
     const uint32_t jm = (1u << TX_JBITS) - 1;
-    const int tile1 = it.t0 + it.nt, ntc = it.nt * 16;
-    uint32_t le[EP], ln[EP];
-    T xv[EP];
+    const int tile0 = tx_uni(it.t0), tile1 = tile0 + tx_uni(it.nt);
+    const int p0 = tx_uni(it.p0), ntc = tx_uni(it.pn) * 16;
+    // a lane's rows are LROW * part + VROW v + 16 i from r0: one offset per lane, the rest scalar
+    const uint32_t eofs = (uint32_t)(Mf<T>::LROW * part * ntc + col);
+    const int rleft = La - u.r0 - Mf<T>::LROW * part;
+    Eo += (long long)u.r0 * ntc;
+    const T *__restrict__ xk = x;
+    // four slots at a time (the slots past the last one repeat it and write nothing)
+    auto entries = [&](int j0, int tile, uint32_t *e) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            e[j] = tx_at(lst + (__builtin_amdgcn_readlane(vlo, j0 + j) + tile * 16), lofs);
+    };
+    auto values = [&](int j0, const uint32_t *e, T *v) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const long long xo = (long long)__builtin_amdgcn_readlane(vxh, j0 + j) << 32 |
+                                 (unsigned)__builtin_amdgcn_readlane(vxl, j0 + j);
+            v[j] = tx_at(xk + xo, e[j] & jm);
+        }
+    };
+    auto puts = [&](int j0, const uint32_t *e, const T *v) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int k = __builtin_amdgcn_readlane(vki, j0 + j);
+            const int s = (int)((e[j] >> TX_JBITS) & TX_KMAX) - (k >> 16);
+            if ((unsigned)s < (unsigned)((k >> 8) & 0xFF)) Dc[s + (k & 0xFF)] = e[j] >> 31 ? -v[j] : v[j];
+        }
+    };
+    constexpr int NP = EP / 4;                     // groups of slots loaded one tile ahead
+    uint32_t le[EP + 1], ln[EP + 1];
+    T xv[EP + 1];
     V zv = {};
     for (int k = u.k0; k < u.k1; k++) {
-        const T *__restrict__ xk = x + k * ldx;
+        xk = x + k * ldx;
 #pragma unroll
-        for (int j = 0; j < EP; j++) le[j] = j < nep ? lst[lo[j] + it.t0 * 16] : TX_PAD;
+        for (int g = 0; g < NP; g++)
+            if (4 * g < nsl) entries(4 * g, tile0, le + 4 * g);
 #pragma unroll
-        for (int j = 0; j < EP; j++) xv[j] = j < nep ? tx_at(xk + xo[j], le[j] & jm) : (T)0;
-#pragma unroll
-        for (int j = 0; j < EP; j++)
-            ln[j] = j < nep && it.t0 + 1 < tile1 ? lst[lo[j] + (it.t0 + 1) * 16] : TX_PAD;
-        for (int tile = it.t0; tile < tile1; tile++) {
+        for (int g = 0; g < NP; g++)
+            if (4 * g < nsl) {
+                values(4 * g, le + 4 * g, xv + 4 * g);
+                if (tile0 + 1 < tile1) entries(4 * g, tile0 + 1, ln + 4 * g);
+            }
+        for (int tile = tile0; tile < tile1; tile++) {
             for (int z = l; z < LDC * (int)sizeof(T); z += 64) ((V *)Dt)[z] = zv;
             tx_wave_sync();
 #pragma unroll
-            for (int j = 0; j < EP; j++)
-                if (j < nep) put(ki[j], le[j], xv[j]);
-            for (int j = EP; j < nsl; j++) {
-                const TxSlot &q = slots[j];
-                const uint32_t e = lst[q.lrow * t.nIp + tile * 16];
-                put(q.kinfo, e, tx_at(xk + q.xb + (long long)u.ja * q.nb, e & jm));
+            for (int g = 0; g < NP; g++)
+                if (4 * g < nsl) puts(4 * g, le + 4 * g, xv + 4 * g);
+            for (int j = EP; j < nsl; j += 4) {
+                uint32_t e[4];
+                T v[4];
+                entries(j, tile, e);
+                values(j, e, v);
+                puts(j, e, v);
             }
             tx_wave_sync();
             // entries and vector elements of the next tile, behind the products below
 #pragma unroll
-            for (int j = 0; j < EP; j++) {
-                le[j] = ln[j];
-                if (j < nep && tile + 1 < tile1) {
-                    xv[j] = tx_at(xk + xo[j], le[j] & jm);
-                    if (tile + 2 < tile1) ln[j] = lst[lo[j] + (tile + 2) * 16];
+            for (int g = 0; g < NP; g++)
+                if (4 * g < nsl && tile + 1 < tile1) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) le[4 * g + j] = ln[4 * g + j];
+                    values(4 * g, le + 4 * g, xv + 4 * g);
+                    if (tile + 2 < tile1) entries(4 * g, tile + 2, ln + 4 * g);
                 }
-            }
-            T *__restrict__ Et = Eo + k * lde + (tile - it.t0) * 16 + col;
+            T *__restrict__ Et = Eo + k * lde + (tile - p0) * 16;
             typename Mf<T>::acc acc[RT];
 #pragma unroll
             for (int i = 0; i < RT; i++) {
                 acc[i] = Mf<T>::zero();
                 if (add) {
 #pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        const int r = u.r0 + i * 16 + Mf<T>::row(l, v);
-                        if (r < La) acc[i][v] = Et[(long long)r * ntc];
-                    }
+                    for (int v = 0; v < 4; v++)
+                        if (i * 16 + Mf<T>::VROW * v < rleft)
+                            acc[i][v] = tx_at(Et + (i * 16 + Mf<T>::VROW * v) * (long long)ntc, eofs);
                 }
             }
-            const T *b0 = Dt + col * LDC + part * KS;
+            const T *b0 = Dc + part * KS;
             if (u.nrt == 1) tx_mma<T, 1, KS>(acc, a, b0);
             else if (u.nrt == 2) tx_mma<T, 2, KS>(acc, a, b0);
             else if (RT > 2) tx_mma<T, RT, KS>(acc, a, b0);
@@ -654,10 +829,9 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
 #pragma unroll
             for (int i = 0; i < RT; i++)
 #pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int r = u.r0 + i * 16 + Mf<T>::row(l, v);
-                    if (r < La) Et[(long long)r * ntc] = acc[i][v];
-                }
+                for (int v = 0; v < 4; v++)
+                    if (i * 16 + Mf<T>::VROW * v < rleft)
+                        tx_put(Et + (i * 16 + Mf<T>::VROW * v) * (long long)ntc, eofs, acc[i][v]);
         }
     }
 }
@@ -668,14 +842,14 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
 // another and the products of one overlap the list walks of the next.  The vector entries of
 // the next column tile are loaded during the products of this one.
 template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_tx_eab(
-    TxDev A, TxRound R, int nvec, int kper, const T *__restrict__ x0, long long ldx0,
-    const T *__restrict__ x1, long long ldx1, T *__restrict__ E, int ldt)
+__global__ __launch_bounds__(256, TxV<T>::WPE) void k_tx_eab(
+    TxDev A, TxRound R, int nvec, int kper, long long N, const T *__restrict__ x0,
+    const T *__restrict__ x1, T *__restrict__ E, int ldt)
 {
     constexpr int RT = TxV<T>::RT, PREC = TxV<T>::PREC;
     extern __shared__ __align__(16) unsigned char tx_smem2[];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const long long u = (long long)blockIdx.x * 4 + wv;
+    const long long u = tx_xcd(blockIdx.x) * 4 + wv;
     if (u >= R.items[PREC]) return;
     T *Dt = (T *)tx_smem2 + (size_t)wv * 16 * ldt;
     const TxItem *__restrict__ items = A.item + R.i0;
@@ -697,18 +871,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     n.nrt = std::min(RT, (t.La - n.r0 + 15) / 16);
     n.dr = t.diag ? t.La - 1 - n.r0 : -1;
     const T *__restrict__ x = t.o ? x1 : x0;
-    const long long ldx = t.o ? ldx1 : ldx0, lde = R.elems;
-    T *__restrict__ Eo = E + it.ebase + ((long long)n.ja * it.nw + (n.w - it.w0)) * t.La * it.nt * 16;
+    const long long lde = R.elems;
+    T *__restrict__ Eo = E + it.ebase + ((long long)n.ja * it.nw + (n.w - it.w0)) * t.La * it.pn * 16;
     static_assert(TX_KC == 96, "reduction depths below cover chunks of up to 96");
     for (int c = 0; c < t.nch; c++) {
         const TxChunk &ch = A.chunk[t.ch0 + c];
         switch (ch.KS) {
-        case 4: tx_eab<T, 4>(A, it, t, ch, n, c > 0, x, ldx, Eo, lde, Dt); break;
-        case 8: tx_eab<T, 8>(A, it, t, ch, n, c > 0, x, ldx, Eo, lde, Dt); break;
-        case 12: tx_eab<T, 12>(A, it, t, ch, n, c > 0, x, ldx, Eo, lde, Dt); break;
-        case 16: tx_eab<T, 16>(A, it, t, ch, n, c > 0, x, ldx, Eo, lde, Dt); break;
-        case 20: tx_eab<T, 20>(A, it, t, ch, n, c > 0, x, ldx, Eo, lde, Dt); break;
-        default: tx_eab<T, 24>(A, it, t, ch, n, c > 0, x, ldx, Eo, lde, Dt); break;
+        case 4: tx_eab<T, 4>(A, it, t, ch, n, c > 0, x, N, Eo, lde, Dt); break;
+        case 8: tx_eab<T, 8>(A, it, t, ch, n, c > 0, x, N, Eo, lde, Dt); break;
+        case 12: tx_eab<T, 12>(A, it, t, ch, n, c > 0, x, N, Eo, lde, Dt); break;
+        case 16: tx_eab<T, 16>(A, it, t, ch, n, c > 0, x, N, Eo, lde, Dt); break;
+        case 20: tx_eab<T, 20>(A, it, t, ch, n, c > 0, x, N, Eo, lde, Dt); break;
+        default: tx_eab<T, 24>(A, it, t, ch, n, c > 0, x, N, Eo, lde, Dt); break;
         }
     }
 }
@@ -716,9 +890,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // y(IL, w, column) += sum over the singles of IL that a task covers, one E row each; 256
 // columns of one string per work-group, eight loads in flight per lane
 template <typename T>
-__global__ __launch_bounds__(256) void k_tx_gab(TxDev A, TxRound R, const T *__restrict__ E, double *y0,
-                                                long long ys0, long long yk0, double *y1,
-                                                long long ys1, long long yk1)
+__global__ __launch_bounds__(256) void k_tx_gab(TxDev A, TxRound R, long long N,
+                                                const T *__restrict__ E, double *__restrict__ y0,
+                                                double *__restrict__ y1)
 {
     int lo = 0, hi = R.no - 1;
     const TxOut *__restrict__ outs = A.out + R.o0;
@@ -764,9 +938,8 @@ __global__ __launch_bounds__(256) void k_tx_gab(TxDev A, TxRound R, const T *__r
         }
         if (q.diag) acc += Es[(long long)il * st + (long long)(q.La - 1) * ntc];
     }
-    const long long n = t.yb + (long long)il * t.nb + (long long)ib * t.nsv + t.w0 + wi;
-    if (t.o) y1[n * ys1 + k * yk1] += (double)acc;
-    else y0[n * ys0 + k * yk0] += (double)acc;
+    const long long n = t.yb + (long long)il * t.nb + (long long)(t.w0 + wi) * t.nI + ib;
+    (t.o ? y1 : y0)[k * N + n] += (double)acc;
 }
 
 template <typename T>
@@ -774,11 +947,16 @@ static int tx_run(int nvec, const TxDev &D, const TxPlan &P, const TxVec &V, T *
 {
     const T *x0 = (const T *)V.x0, *x1 = (const T *)V.x1;
     for (const TxRound &R : P.ss) {
-        hipLaunchKernelGGL(k_tx_ess<T>, dim3((unsigned)R.items[0], nvec), dim3(256),
-                           (unsigned)P.rmax * 12, st, D, R, x0, V.ldx0, x1, V.ldx1, E);
+        const unsigned rp = (unsigned)(P.rmax + 15) / 16 * 16;
+        if ((unsigned long long)V.N * sizeof(T) < (1ULL << 32))
+            hipLaunchKernelGGL((k_tx_ess<T, false>), dim3((unsigned)R.items[0], nvec), dim3(256), rp * 8,
+                               st, D, R, V.N, x0, x1, E);
+        else
+            hipLaunchKernelGGL((k_tx_ess<T, true>), dim3((unsigned)R.items[0], nvec), dim3(256), rp * 12,
+                               st, D, R, V.N, x0, x1, E);
         TX_CHECK();
-        hipLaunchKernelGGL(k_tx_gss<T>, dim3((unsigned)R.blocks, nvec), dim3(256), 0, st, D, R, E, V.y0,
-                           V.ys0, V.yk0, V.y1, V.ys1, V.yk1);
+        hipLaunchKernelGGL(k_tx_gss<T>, dim3((unsigned)R.blocks, nvec), dim3(256), 0, st, D, R, V.N, E,
+                           V.y0, V.y1);
         TX_CHECK();
     }
     const int ldt = P.ldt + TxV<T>::PAD;
@@ -786,12 +964,12 @@ static int tx_run(int nvec, const TxDev &D, const TxPlan &P, const TxVec &V, T *
         // the vectors share a wave's fragments where there are waves enough without them
         const int kper = R.items[TxV<T>::PREC] >= 8192 ? nvec : 1;
         hipLaunchKernelGGL(k_tx_eab<T>,
-                           dim3((unsigned)((R.items[TxV<T>::PREC] + 3) / 4), (nvec + kper - 1) / kper),
-                           dim3(256), (unsigned)(64 * ldt * sizeof(T)), st, D, R, nvec, kper, x0, V.ldx0,
-                           x1, V.ldx1, E, ldt);
+                           dim3(tx_grid((R.items[TxV<T>::PREC] + 3) / 4), (nvec + kper - 1) / kper),
+                           dim3(256), (unsigned)(64 * ldt * sizeof(T)), st, D, R, nvec, kper, V.N, x0,
+                           x1, E, ldt);
         TX_CHECK();
-        hipLaunchKernelGGL(k_tx_gab<T>, dim3((unsigned)R.blocks, nvec), dim3(256), 0, st, D, R, E, V.y0,
-                           V.ys0, V.yk0, V.y1, V.ys1, V.yk1);
+        hipLaunchKernelGGL(k_tx_gab<T>, dim3((unsigned)R.blocks, nvec), dim3(256), 0, st, D, R, V.N, E,
+                           V.y0, V.y1);
         TX_CHECK();
     }
     return 0;

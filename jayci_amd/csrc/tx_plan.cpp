@@ -47,22 +47,35 @@ static int plan_lists(const SpaceDesc &D, const SpinDesc &S, std::vector<TxList>
         t.nsv = (int)std::max(1LL, S.nsv[g]);
         t.nI = (int)(S.gn[g] / t.nsv);
         t.nIp = (int)up(t.nI, 16);
+        const int v = S.gv[g], nint_e = S.nelec - v;
+        auto add = [&](int h, int cls, int own, int first, int cnt) {
+            if (cnt <= 0) return;
+            t.grp[t.nsec] = h;
+            t.cls[t.nsec] = cls;
+            t.own[t.nsec] = own;
+            t.first[t.nsec] = first;
+            t.row0[t.nsec] = t.rows;
+            t.cnt[t.nsec] = cnt;
+            t.rows += (int)up(cnt, 4);
+            t.nsec++;
+        };
+        t.nf = D.nvirt - v;
         for (int h = 0; h < S.ngrp; h++) {
             if (!S.gn[h] || !S.gn[g]) continue;
-            const ll c = singles(D, S, g, h);
+            const int c = (int)singles(D, S, g, h);
             if (c <= 0) continue;
             if (t.nsec >= TX_MAXSEC) return 1;
-            t.grp[t.nsec] = h;
-            t.row0[t.nsec] = t.rows;
-            t.cnt[t.nsec] = (int)c;
-            t.rows += (int)up(c, 4);
-            t.nsec++;
+            if (h == g) {
+                // table order: internal replacements, then the external ones
+                const int ee = v * (D.nvirt - v);
+                add(h, TX_II, 0, 0, c - ee);
+                add(h, TX_EE, 0, c - ee, ee);
+            } else {
+                add(h, S.gv[h] == v ? TX_II : S.gv[h] < v ? TX_DEC : TX_INC, 0, 0, c);
+            }
         }
-        t.grp[t.nsec] = -1;
-        t.row0[t.nsec] = t.rows;
-        t.cnt[t.nsec] = S.nelec;
-        t.rows += (int)up(S.nelec, 4);
-        t.nsec++;
+        add(g, TX_II, 1, 0, nint_e);
+        add(g, TX_EE, 1, nint_e, v);
         if (S.gn[g] >= (1LL << TX_JBITS)) return 1;
         base += (ll)t.nsv * t.rows * t.nIp;
         L.push_back(t);
@@ -129,14 +142,14 @@ struct Builder {
     unsigned long long binom[65 * 65];
 
     // a chunk's steps: consecutive positions of one or more classes
-    struct Seg { int dv, k0, len, base; };
+    struct Seg { int cls, k0, len, base; };
 
     // reduction-index table of a chunk for first-spin group f: its first entry
     int pair_table(const SpaceDesc &D, int f, const std::vector<Seg> &seg, int depth)
     {
         const SpinDesc &S = D.s[1];
         std::vector<int> key = {S.gv[f], depth};
-        for (const Seg &g : seg) key.insert(key.end(), {g.dv, g.k0, g.len});
+        for (const Seg &g : seg) key.insert(key.end(), {g.cls, g.k0, g.len});
         auto it = qtab.find(key);
         if (it != qtab.end()) return it->second;
         const int nint = D.ndocc + D.nactv, v = S.gv[f];
@@ -149,10 +162,8 @@ struct Builder {
                 ext[n++] = nint + jci_ctz(m);
             int put = 0;
             for (const Seg &g : seg)
-                for (int s = 0; s < g.len; s++, put++) {
-                    const int Q = tx_kpair(nint, D.nvirt, ext, n, g.dv, g.k0 + s);
-                    P->q.push_back(Q < 0 ? none : Q);
-                }
+                for (int s = 0; s < g.len; s++, put++)
+                    P->q.push_back(tx_kpair(nint, D.nvirt, ext, g.cls, g.k0 + s));
             for (; put < depth; put++) P->q.push_back(none);
         }
         qtab[key] = at;
@@ -209,25 +220,27 @@ struct Builder {
                 if (!t.La) continue;
                 // reduction index: the classes of the sources, in chunks of at most TX_KC
                 // steps; a class that does not fit what is left of a chunk opens the next
-                // one, and one deeper than a chunk is split evenly
-                const int own = gr.first.count(f) ? 1 : 0;
-                int has[3] = {0, 0, 0};
+                // one, and one deeper than a chunk is split (by external orbitals for TX_INC)
                 const int v = F.gv[f], nint = O.ndocc + O.nactv;
-                for (int f1 : gr.first) has[F.gv[f1] - v + 1] = 1;
+                int has[4] = {0, 0, 0, 0};
+                for (int s = 0; s < li.nsec; s++) if (gr.first.count(li.grp[s])) has[li.cls[s]] = 1;
                 std::vector<std::vector<Seg>> chunks(1);
                 int depth = 0;
-                for (int dv : {0, -1, 1}) {
-                    if (!has[dv + 1]) continue;
-                    if (tx_class_size(nint, O.nvirt, v, dv, 1) >= TX_KMAX) return 1;
-                    const int m = tx_class_size(nint, O.nvirt, v, dv, own);
-                    const int np = (m + TX_KC - 1) / TX_KC, len = np ? (m + np - 1) / np : 0;
+                for (int cls = 0; cls < 4; cls++) {
+                    if (!has[cls]) continue;
+                    const int m = tx_class_size(nint, O.nvirt, v, cls);
+                    if (m >= TX_KMAX) return 1;
+                    const int unit = cls == TX_INC ? nint : 1;
+                    if (unit > TX_KC) return 1;
+                    const int most = TX_KC / unit * unit, np = (m + most - 1) / most;
+                    const int len = np ? (int)up((m + np - 1) / np, unit) : 0;
                     for (int k0 = 0; k0 < m; k0 += len) {
                         const int n = std::min(len, m - k0);
                         if (depth + n > TX_KC) {
                             chunks.push_back(std::vector<Seg>());
                             depth = 0;
                         }
-                        chunks.back().push_back(Seg{dv, k0, n, depth});
+                        chunks.back().push_back(Seg{cls, k0, n, depth});
                         depth += n;
                     }
                 }
@@ -244,15 +257,23 @@ struct Builder {
                     ch.slot0 = (int)P->slot.size();
                     for (const Seg &g : seg)
                         for (int s = 0; s < li.nsec; s++) {
-                            const int f1 = li.grp[s] < 0 ? f : li.grp[s];
-                            if (!gr.first.count(f1) || F.gv[f1] - v != g.dv) continue;
-                            const int blk = O.blkid[l1][f1];
+                            if (li.cls[s] != g.cls || !gr.first.count(li.grp[s])) continue;
+                            const int blk = O.blkid[l1][li.grp[s]];
                             if (blk < 0) return 1;
-                            for (int r = 0; r < li.cnt[s]; r += 4) {
+                            // rows of the section that can reach the segment: all, or those of
+                            // its external orbitals (whose ranks among the free ones lag by up
+                            // to v)
+                            int r0 = 0, r1 = li.cnt[s];
+                            if (g.cls == TX_INC) {
+                                const int ni = li.cnt[s] / li.nf;
+                                r0 = std::max(0, g.k0 / nint - v) * ni / 4 * 4;
+                                r1 = std::min(li.nf, (g.k0 + g.len + nint - 1) / nint) * ni;
+                            }
+                            for (int r = r0; r < r1; r += 4) {
                                 TxSlot w;
                                 memset(&w, 0, sizeof(w));
                                 w.xb = O.boff[blk];
-                                w.nb = (int)F.gn[f1];
+                                w.nb = (int)F.gn[li.grp[s]];
                                 w.lrow = li.row0[s] + r;
                                 w.kinfo = g.base | g.len << 8 | g.k0 << 16;
                                 P->slot.push_back(w);
@@ -260,6 +281,7 @@ struct Builder {
                         }
                     ch.nslot = (int)P->slot.size() - ch.slot0;
                     if (!ch.nslot) continue;
+                    if (ch.nslot > 64) return 1;
                     P->chunk.push_back(ch);
                     t.nch++;
                 }
@@ -272,32 +294,34 @@ struct Builder {
     }
 
     // one piece of a round: external parts [w0, w0 + nw) and column tiles [t0, t0 + nt) of
-    // first-spin group f
-    void piece(int o, int f, int w0, int nw, int t0, int nt, TxRound &R)
+    // first-spin group f, for some of its tasks
+    void piece(int o, int f, const std::vector<int> &tasks, int w0, int nw, int t0, int nt, TxRound &R)
     {
         const SpaceDesc &O = *dd[o];
         const SpinDesc &L = O.s[0];
         std::vector<ll> eb;
-        for (int ti : by[o][f]) {
+        for (int ti : tasks) {
             const TxTask &t = P->task[ti];
             TxItem it;
             memset(&it, 0, sizeof(it));
             it.task = ti;
             it.w0 = w0;
             it.nw = nw;
-            it.t0 = t0;
-            it.nt = nt;
+            it.p0 = t0;
+            it.pn = nt;
             const int rows[2] = {TX_ROWS64, TX_ROWS32};
-            for (int p = 0; p < 2; p++) {
-                it.rg[p] = (t.La + rows[p] - 1) / rows[p];
-                it.item0[p] = R.items[p];
-                R.items[p] += (ll)t.na * nw * it.rg[p];
-            }
+            for (int p = 0; p < 2; p++) it.rg[p] = (t.La + rows[p] - 1) / rows[p];
             it.ebase = R.elems;
             eb.push_back(R.elems);
             R.elems += (ll)t.na * nw * t.La * nt * 16;
-            P->item.push_back(it);
-            R.ni++;
+            // long rows of tiles in several items: the launch's last work-groups end sooner
+            const int most = std::max(2, TX_PASSES / t.nch), parts = (nt + most - 1) / most;
+            for (int k = 0; k < parts; k++) {
+                it.t0 = t0 + nt * k / parts;
+                it.nt = t0 + nt * (k + 1) / parts - it.t0;
+                P->item.push_back(it);
+                R.ni++;
+            }
         }
         for (int l = 0; l < L.ngrp; l++) {
             const int blk = O.blkid[l][f];
@@ -305,8 +329,8 @@ struct Builder {
             TxOut u;
             memset(&u, 0, sizeof(u));
             u.src0 = (int)P->src.size();
-            for (size_t i = 0; i < by[o][f].size(); i++) {
-                const TxTask &t = P->task[by[o][f][i]];
+            for (size_t i = 0; i < tasks.size(); i++) {
+                const TxTask &t = P->task[tasks[i]];
                 TxSrc s;
                 memset(&s, 0, sizeof(s));
                 s.l1 = t.l1;
@@ -321,7 +345,7 @@ struct Builder {
                 u.nsrc++;
             }
             if (!u.nsrc) continue;
-            const TxTask &t = P->task[by[o][f][0]];
+            const TxTask &t = P->task[tasks[0]];
             u.o = o;
             u.p = l;
             u.f = f;
@@ -354,6 +378,23 @@ struct Builder {
         };
         auto close = [&]() {
             if (R.ni) {
+                // the longest items first, so that the launch ends on short ones
+                auto first = P->item.begin() + R.i0;
+                auto cost = [&](const TxItem &a) {
+                    const TxTask &t = P->task[a.task];
+                    ll c = 0;
+                    for (int i = 0; i < t.nch; i++)
+                        c += 4 * P->chunk[t.ch0 + i].KS * std::min(2, (t.La + 15) / 16) + 40 * P->chunk[t.ch0 + i].nslot;
+                    return c * a.nt;
+                };
+                std::stable_sort(first, first + R.ni,
+                                 [&](const TxItem &a, const TxItem &b) { return cost(a) > cost(b); });
+                for (int i = 0; i < R.ni; i++)
+                    for (int p = 0; p < 2; p++) {
+                        TxItem &a = first[i];
+                        a.item0[p] = R.items[p];
+                        R.items[p] += (ll)P->task[a.task].na * a.nw * a.rg[p];
+                    }
                 P->ab.push_back(R);
                 P->elems = std::max(P->elems, R.elems);
             }
@@ -363,33 +404,45 @@ struct Builder {
         for (int o = 0; o < 2; o++)
             for (int f = 0; f < dd[o]->s[1].ngrp; f++) {
                 if (by[o][f].empty()) continue;
-                ll tile = 0;                     // elements of one column tile
-                for (int ti : by[o][f]) tile += (ll)P->task[ti].na * P->task[ti].La * 16;
                 const TxTask &t = P->task[by[o][f][0]];
                 const int nt = t.nIp / 16;
-                if (tile * nt <= budget) {
-                    for (int w = 0; w < t.nsv;) {
-                        ll room = (budget - R.elems) / (tile * nt);
-                        if (room <= 0) {
-                            close();
-                            continue;
-                        }
-                        const int n = (int)std::min<ll>(room, t.nsv - w);
-                        piece(o, f, w, n, 0, nt, R);
-                        w += n;
-                    }
-                } else {
-                    for (int w = 0; w < t.nsv; w++)
-                        for (int c = 0; c < nt;) {
-                            ll room = (budget - R.elems) / tile;
-                            if (room <= 0 && R.elems) {
+                // elements of one external part for all tasks; where one alone exceeds the
+                // buffer the tasks go one by one (their sums add up in the result), a single
+                // one past the buffer by column tiles
+                ll all = 0;
+                for (int ti : by[o][f]) all += (ll)P->task[ti].na * P->task[ti].La * 16 * nt;
+                std::vector<std::vector<int>> sets;
+                if (all <= budget) sets.push_back(by[o][f]);
+                else for (int ti : by[o][f]) sets.push_back(std::vector<int>(1, ti));
+                for (const std::vector<int> &set : sets) {
+                    ll tile = 0;                 // elements of one column tile
+                    for (int ti : set) tile += (ll)P->task[ti].na * P->task[ti].La * 16;
+                    if (tile * nt <= budget) {
+                        for (int w = 0; w < t.nsv;) {
+                            const ll room = (budget - R.elems) / (tile * nt);
+                            if (room <= 0) {
                                 close();
                                 continue;
                             }
-                            const int n = (int)std::min<ll>(std::max(1LL, room), nt - c);
-                            piece(o, f, w, 1, c, n, R);
-                            c += n;
+                            const int n = (int)std::min<ll>(room, t.nsv - w);
+                            piece(o, f, set, w, n, 0, nt, R);
+                            w += n;
                         }
+                    } else {
+                        for (int w = 0; w < t.nsv; w++)
+                            for (int c = 0; c < nt;) {
+                                const ll room = (budget - R.elems) / tile;
+                                if (room <= 0 && R.elems) {
+                                    close();
+                                    continue;
+                                }
+                                const int n = (int)std::min<ll>(std::max(1LL, room), nt - c);
+                                piece(o, f, set, w, 1, c, n, R);
+                                c += n;
+                            }
+                    }
+                    // two pieces of one round may not add to the same results
+                    if (sets.size() > 1) close();
                 }
             }
         close();
@@ -449,7 +502,9 @@ struct Builder {
             it.nc = nc;
             it.ncp = ncp;
             it.rg = (t.R + 63) / 64;
-            it.ct = (nc + 63) / 64;
+            // few pairs: many columns per work-group, for the list and the W tile it sets up
+            it.cb = t.R <= 16 ? 16 : t.R <= 32 ? 8 : t.R <= TX_RMAX ? 4 : 1;
+            it.ct = (nc + 64 * it.cb - 1) / (64 * it.cb);
             it.item0 = R.items[0];
             R.items[0] += (ll)t.n * it.rg * it.ct;
             it.ebase = R.elems;
