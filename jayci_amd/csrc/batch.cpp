@@ -678,11 +678,10 @@ static int run_sigma_gf(jci_batch *b, const std::vector<int> &ids, int prec)
             t.y = s.S + (size_t)s.sig_first * s.ld;
             t.ldy = s.ld;
             t.E = (char *)b->epool + used;
-            t.lde = jk_gf_lde((long long)k * s.N);
             long long u[4];
             jk_gf_units(prec, prec == 64 ? b->bn64 : b->bn32, t, u);
             for (int q = 0; q < 4; q++) { t.base[q] = base[q]; base[q] += u[q]; }
-            used += ((size_t)s.g.La * (size_t)t.lde * esz + 255) / 256 * 256;
+            used += ((size_t)s.g.La * (size_t)jk_gf_lde((long long)k * s.N) * esz + 255) / 256 * 256;
             who.push_back(i);
             kk.push_back(k);
             n++;

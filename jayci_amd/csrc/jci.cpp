@@ -404,6 +404,7 @@ static int build_gf(jci_ham *h)
     // alpha lists: the singles and one entry for the occupied diagonal pairs together
     const int La = sa + (s->na > 0 ? 1 : 0), Lb = sb + s->nb;
     if (La > GF_MAXLIST || Lb > GF_MAXLIST) return 0;
+    const int Lp = ge_pitch(MP);
     JCI_CHECK(hipMalloc(&h->d_gfH64[0], sizeof(double) * na * na));
     JCI_CHECK(hipMalloc(&h->d_gfH32[0], sizeof(float) * na * na));
     RCHECK(jk_gf_dense(na, s->d_mask[0], h->d_off1[0], h->d_e1[0], h->d_v1[0], h->d_off2[0],
@@ -426,8 +427,8 @@ static int build_gf(jci_ham *h)
     JCI_CHECK(hipMalloc(&h->d_gfD32, sizeof(float) * na * MP));
     RCHECK(jk_gf_diagrows(na, MP, s->d_mask[0], h->d_gfM64, h->d_gfD64, h->d_gfD32, c->stream));
     JCI_CHECK(hipMalloc(&h->d_gfla, sizeof(uint32_t) * na * La));
-    JCI_CHECK(hipMalloc(&h->d_gflb, sizeof(uint32_t) * nb * Lb));
-    RCHECK(jk_gf_lists(nb, s->d_mask[1], h->d_off1[1], h->d_e1[1], Lb, 0, h->d_gflb, c->stream));
+    JCI_CHECK(hipMalloc(&h->d_gflb, sizeof(uint32_t) * nb * Lp));
+    RCHECK(jk_gf_lists(nb, s->d_mask[1], h->d_off1[1], h->d_e1[1], Lb, Lp, MP, 0, h->d_gflb, c->stream));
     {
         // alpha lists with the E row of each entry (the pair's position in the target's list)
         uint32_t *raw = nullptr;
@@ -436,7 +437,7 @@ static int build_gf(jci_ham *h)
         JCI_CHECK(hipMallocAsync((void **)&raw, sizeof(uint32_t) * na * La, c->stream));
         JCI_CHECK(hipMallocAsync((void **)&d_missing, sizeof(int), c->stream));
         JCI_CHECK(hipMemsetAsync(d_missing, 0, sizeof(int), c->stream));
-        int rc = jk_gf_lists(na, s->d_mask[0], h->d_off1[0], h->d_e1[0], La, 1, raw, c->stream);
+        int rc = jk_gf_lists(na, s->d_mask[0], h->d_off1[0], h->d_e1[0], La, La, 0, 1, raw, c->stream);
         if (!rc) rc = jk_gf_rank(na, La, raw, h->d_gfla, d_missing, c->stream);
         if (!rc && hipMemcpyAsync(&missing, d_missing, sizeof(int), hipMemcpyDeviceToHost, c->stream) != hipSuccess)
             rc = -2;
@@ -1180,7 +1181,6 @@ static int gf_run(jci_ham *h, int prec, int K, const double *x, long long ldx, d
             t.y = y + (size_t)b * ldy;
             t.ldy = ldy;
             t.E = E;
-            t.lde = jk_gf_lde((long long)k * N);
             hh.n = 1;
             const int bn = prec == 64 ? h->gf_bn64 : h->gf_bn32;
             jk_gf_units(prec, bn, t, hh.total);
@@ -1221,7 +1221,6 @@ static int gf_run(jci_ham *h, int prec, int K, const double *x, long long ldx, d
         t.y = y + (size_t)b * ldy;
         t.ldy = ldy;
         t.E = h->d_gfE;
-        t.lde = jk_gf_lde((long long)k * N);
         hh.n = 1;
         const int bn = prec == 64 ? h->gf_bn64 : h->gf_bn32;
         jk_gf_units(prec, bn, t, hh.total);

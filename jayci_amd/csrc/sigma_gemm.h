@@ -51,7 +51,7 @@ struct GemmFci {
     const float *H32[2];
     const double *M64;           // (P|Q), MP x MP, zero padded
     const float *M32;
-    const uint32_t *la, *lb;     // [Na][La], [Nb][Lb]
+    const uint32_t *la, *lb;     // [Na][La], [Nb][ge_pitch(MP)]
     const double *D64;           // [Na][MP]: the (P|Q) row of each alpha string's GF_PDIAG
     const float *D32;            // entry, sum of (kk|Q) over its occupied orbitals k
 };
@@ -68,12 +68,10 @@ struct GfTask {
     float *x32;                  // FP32 copies [K][N] (FP32 launches)
     double *y;                   // output columns, vector k at y + k*ldy (overwritten)
     long long ldy;
-    void *E;                     // intermediate, La rows of K*N elements, row stride lde
-    long long lde;               // K*N rounded up to GF_EALIGN elements (jk_gf_lde)
+    void *E;                     // intermediate [K][Na][La][Nb], in La * jk_gf_lde(K*N) elements
     long long base[4];           // first unit: conversion, same-spin, E, gather
 };
-// E rows start on 512-byte boundaries (FP64) / 256-byte (FP32): the tile stores of the E
-// kernel then write whole 64-byte sectors
+// room for the intermediate is counted in rows of K*N rounded up to GF_EALIGN elements
 #define GF_EALIGN 64
 static inline long long jk_gf_lde(long long ncols) { return (ncols + GF_EALIGN - 1) / GF_EALIGN * GF_EALIGN; }
 struct GfHeader {
@@ -85,9 +83,31 @@ struct GfHeader {
 #define GF_E 2
 #define GF_GA 3
 
-// column-tile width of the E kernel (autotuned): FP64 16 or 32, FP32 32 or 64
+// columns of a unit of the E kernel (autotuned): FP64 16 or 32, FP32 32 or 64
 #define GF_BN64_DEFAULT 32
 #define GF_BN32_DEFAULT 32
+// one row of E past full tiles of 16: left to the vector units
+__host__ __device__ inline bool ge_extra(int La) { return La > 1 && (La - 1) % 16 == 0; }
+// Tile edge of the same-spin product of K vectors: the one whose whole waves of work-groups on
+// 256 CUs take least.  A 32 x 32 tile reads twice as much per product as the larger ones.
+__host__ __device__ inline int gs_edge(long long na, long long nb, int K)
+{
+    if (na < 4 || nb < 4) return 32;
+    int best = 32;
+    double cost = 1e300;
+    for (int e = 128; e >= 32; e >>= 1) {
+        const long long tiles = (long long)K * ((na + e - 1) / e) * ((nb + e - 1) / e);
+        const double c = (double)((tiles + 255) / 256) * e * e * (e == 32 ? 1.4 : 1.0);
+        if (c < cost) {
+            cost = c;
+            best = e;
+        }
+    }
+    return best;
+}
+// pitch of the beta lists: 16-byte reads of four lanes, all alike, for the longest list
+// b (n - b + 1) of the orbital counts n that share MP
+__host__ __device__ constexpr int ge_pitch(int MP) { return MP <= 32 ? 16 : MP <= 64 ? 32 : MP == 80 ? 48 : 64; }
 int jk_gf_bn_valid(int prec, int bn);
 // work units of one task per kernel for the given precision and E tile width
 void jk_gf_units(int prec, int bn, const GfTask &t, long long units[4]);
@@ -103,8 +123,9 @@ int jk_gf_dense(long long nstr, const uint64_t *mask, const long long *off1, con
                 const double *m1, const double *m2, double *H, hipStream_t st);
 // replacement lists of one spin: the singles, then one entry per occupied diagonal pair
 // (diag_one = 0, beta) or one GF_PDIAG entry for all of them (diag_one = 1, alpha)
+// at pitch Lp, filled up with entries of string 0 and pair `pad`
 int jk_gf_lists(long long nstr, const uint64_t *mask, const long long *off1, const int2 *e1,
-                int L, int diag_one, uint32_t *out, hipStream_t st);
+                int L, int Lp, int pad, int diag_one, uint32_t *out, hipStream_t st);
 // alpha lists: out = in with bits 24..30 set to the E row of each entry; *missing (device)
 // counts entries whose pair is absent from the target's list (0 for a valid list)
 int jk_gf_rank(long long nstr, int L, const uint32_t *in, uint32_t *out, int *missing,

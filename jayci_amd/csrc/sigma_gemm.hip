@@ -1,6 +1,7 @@
 // Dense-string full-CI sigma on MFMA (see sigma_gemm.h for the decomposition).
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <type_traits>
 #include "mfma.h"
 #include "sigma_gemm.h"
 #include "slater.h"
@@ -53,11 +54,12 @@ __global__ void k_gf_dense(long long nstr, const uint64_t *__restrict__ mask,
 
 __global__ void k_gf_lists(long long nstr, const uint64_t *__restrict__ mask,
                            const long long *__restrict__ off1, const int2 *__restrict__ e1, int L,
-                           int diag_one, uint32_t *__restrict__ out)
+                           int Lp, uint32_t pad, int diag_one, uint32_t *__restrict__ out)
 {
     long long I = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (I >= nstr) return;
-    uint32_t *o = out + I * L;
+    uint32_t *o = out + I * Lp;
+    for (int i = L; i < Lp; i++) o[i] = pad << 16;
     int n = 0;
     for (long long e = off1[I]; e < off1[I + 1] && n < L; e++) {
         int2 en = e1[e];
@@ -178,311 +180,521 @@ __global__ __launch_bounds__(256) void k_gcv(const GfHeader *__restrict__ H,
     }
 }
 
-// C(64x64 tile at m0, n0) += A B over Kr, A row-major (lda), B row-major (ldb), M x N bounds.
-// Two LDS buffers: the global loads of step k0 + 16 are issued before the products of step
-// k0 and stored into the other buffer after them, one barrier per step.
-template <typename T>
-__device__ __forceinline__ void mma_tile(typename Mf<T>::acc (&acc)[2][2], const T *__restrict__ A,
-                                         long long lda, const T *__restrict__ B, long long ldb,
-                                         long long M, long long N, long long Kr, long long m0,
-                                         long long n0, T (*As)[16][65], T (*Bs)[16][65])
+// ---- same-spin products -----------------------------------------------------------------------
+// four consecutive elements at an address aligned to one
+template <typename T> struct Gs;
+template <> struct Gs<double> {
+    typedef double quad __attribute__((ext_vector_type(4), aligned(8)));
+    typedef double pair __attribute__((ext_vector_type(2), aligned(8)));
+    static constexpr int WPE = 1;                // waves per SIMD: 64 x 64 accumulators and operands
+};
+template <> struct Gs<float> {
+    typedef float quad __attribute__((ext_vector_type(4), aligned(4)));
+    typedef float pair __attribute__((ext_vector_type(2), aligned(4)));
+    static constexpr int WPE = 2;
+};
+typedef double GsOut __attribute__((ext_vector_type(2), aligned(8)));
+
+// operands of one 16-deep step of a wave's tile: rows m of A, columns n of B
+template <typename T, int RT> struct GsStep { T a[RT][4], b[4][RT]; };
+
+// acc += A B over reduction steps [s0, s1) of 16, A row-major (lda), B row-major (ldb): a wave's
+// tile of RT x RT 16 x 16 tiles straight from memory, without LDS.  Lane group l / 16 takes the
+// reduction indexes 4 (l / 16) .. + 3 of a step, four consecutive elements of a row of A; the
+// columns are dealt out so that lane l % 16 has RT consecutive ones, one wide read of a row of
+// B.  The operands of the next step are loaded during the products of this one.  Rows, columns
+// and the last reduction indexes past the end are moved back inside (their results equal the
+// ones that are stored twice; reduction indexes met before are taken with zero from A).
+template <typename T, int RT>
+__device__ __forceinline__ void gs_wave(typename Mf<T>::acc (&acc)[RT][RT], const T *A, int lda,
+                                        const T *B, int ldb, int Kr, const int (&m)[RT], int n, int s0,
+                                        int s1)
 {
-    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
-    const int wm = w >> 1, wn = w & 1;
-    const int ar = tid >> 2, ak = (tid & 3) * 4;
-    const int bk = tid >> 4, bc = (tid & 15) * 4;
-    const long long gm = m0 + ar;
+    typedef const __attribute__((address_space(1))) typename Gs<T>::quad *QP;
+    typedef const __attribute__((address_space(1))) typename Gs<T>::pair *PP;
+    const int part = (threadIdx.x & 63) >> 4;
     const auto Ag = gptr(A), Bg = gptr(B);
-    T ra[4], rb[4];
-    auto gload = [&](long long k0) {
+    uint32_t ao[RT];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const long long gk = k0 + ak + j;
-            ra[j] = (gm < M && gk < Kr) ? Ag[gm * lda + gk] : (T)0;
+    for (int i = 0; i < RT; i++) ao[i] = (uint32_t)m[i] * (uint32_t)lda;
+    auto load = [&](int s, GsStep<T, RT> &o) __attribute__((always_inline)) {
+        const int k = std::min(s * 16 + part * 4, Kr - 4);
+#pragma unroll
+        for (int i = 0; i < RT; i++) {
+            const typename Gs<T>::quad v = *(QP)(Ag + (ao[i] + (uint32_t)k));
+#pragma unroll
+            for (int j = 0; j < 4; j++) o.a[i][j] = v[j];
         }
-        const long long gk = k0 + bk;
+        const uint32_t bo = (uint32_t)k * (uint32_t)ldb + (uint32_t)n;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const long long gn = n0 + bc + j;
-            rb[j] = (gk < Kr && gn < N) ? Bg[gk * ldb + gn] : (T)0;
+            const auto row = Bg + (bo + (uint32_t)(j * ldb));
+            if constexpr (RT == 4) {
+                const typename Gs<T>::quad v = *(QP)row;
+#pragma unroll
+                for (int c = 0; c < 4; c++) o.b[j][c] = v[c];
+            } else {
+                const typename Gs<T>::pair v = *(PP)row;
+#pragma unroll
+                for (int c = 0; c < RT; c++) o.b[j][c] = v[c];
+            }
         }
     };
-    auto sstore = [&](int buf) {
+    auto mul = [&](GsStep<T, RT> &o) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            As[buf][ak + j][ar] = ra[j];
-            Bs[buf][bk][bc + j] = rb[j];
-        }
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int i = 0; i < RT; i++)
+#pragma unroll
+                for (int c = 0; c < RT; c++) acc[i][c] = Mf<T>::mma(o.a[i][j], o.b[j][c], acc[i][c]);
     };
-    gload(0);
-    sstore(0);
-    __syncthreads();
-    int buf = 0;
-    for (long long k0 = 0; k0 < Kr; k0 += 16) {
-        const bool more = k0 + 16 < Kr;
-        if (more) gload(k0 + 16);
+    // zero the reduction indexes of a moved quad that an earlier one has
+    auto trim = [&](int s, GsStep<T, RT> &o) __attribute__((always_inline)) {
+        const int over = s * 16 + part * 4 - (Kr - 4);
 #pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            const int kr = ks * 4 + l / 16;
-            const T a0 = As[buf][kr][wm * 32 + l % 16], a1 = As[buf][kr][wm * 32 + 16 + l % 16];
-            const T b0 = Bs[buf][kr][wn * 32 + l % 16], b1 = Bs[buf][kr][wn * 32 + 16 + l % 16];
-            acc[0][0] = Mf<T>::mma(a0, b0, acc[0][0]);
-            acc[0][1] = Mf<T>::mma(a0, b1, acc[0][1]);
-            acc[1][0] = Mf<T>::mma(a1, b0, acc[1][0]);
-            acc[1][1] = Mf<T>::mma(a1, b1, acc[1][1]);
-        }
-        if (more) sstore(buf ^ 1);
-        __syncthreads();
-        buf ^= 1;
+        for (int i = 0; i < RT; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (j < over) o.a[i][j] = (T)0;
+    };
+    if (s0 >= s1) return;
+    GsStep<T, RT> o[2];
+    load(s0, o[0]);
+    int s = s0;
+    for (; s + 2 < s1; s += 2) {
+        load(s + 1, o[1]);
+        mul(o[0]);
+        load(s + 2, o[0]);
+        mul(o[1]);
+    }
+    if (s + 1 < s1) {
+        load(s + 1, o[1]);
+        mul(o[0]);
+        trim(s + 1, o[1]);
+        mul(o[1]);
+    } else {
+        trim(s, o[0]);
+        mul(o[0]);
     }
 }
 
-// same-spin parts: y_k = Haa X_k + X_k Hbb on 64 x 64 tiles (k, alpha rows, beta columns).
-// Four blocks per CU (at most 128 registers, 33 KB of LDS in FP64): the 1024 tiles of a
-// 2002 x 2002 string space are then resident at once instead of running as 768 + 256.
-template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_gss(const GfHeader *__restrict__ H,
-                                             const GfTask *__restrict__ tasks)
+// y_k = Haa X_k + X_k Hbb on a tile of the block's (RT = 4: 64 x 64, RT = 2: 32 x 32), every
+// wave over a quarter of the two reductions, the four sums added in LDS
+template <typename T, int RT>
+__device__ __forceinline__ void gs_split(const GfTask &t, const T *X, double *y, int m0, int n0, T *red)
 {
-    __shared__ T As[2][16][65];
-    __shared__ T Bs[2][16][65];
+    const GemmFci &g = t.g;
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, na = (int)g.na, nb = (int)g.nb;
+    typename Mf<T>::acc acc[RT][RT];
+    int m[RT];
+#pragma unroll
+    for (int i = 0; i < RT; i++) {
+        m[i] = std::min(m0 + i * 16 + (l & 15), na - 1);
+#pragma unroll
+        for (int c = 0; c < RT; c++) acc[i][c] = Mf<T>::zero();
+    }
+    const int n = std::min(n0 + RT * (l & 15), nb - RT);
+    const int ka = (na + 15) / 16, kb = (nb + 15) / 16, q0 = (ka + kb) * w / 4, q1 = (ka + kb) * (w + 1) / 4;
+    gs_wave<T, RT>(acc, hmat<T>(g, 0), na, X, nb, na, m, n, q0, std::min(q1, ka));
+    gs_wave<T, RT>(acc, X, nb, hmat<T>(g, 1), nb, nb, m, n, std::max(q0 - ka, 0), q1 - ka);
+#pragma unroll
+    for (int c = 0; c < RT; c++) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < RT; i++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) red[((w * RT + i) * 4 + v) * 64 + l] = acc[i][c][v];
+        __syncthreads();
+        // wave w finishes element w of every row tile
+#pragma unroll
+        for (int i = 0; i < RT; i++) {
+            T sum = (T)0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) sum += red[((q * RT + i) * 4 + w) * 64 + l];
+            const int r = std::min(m0 + i * 16 + Mf<T>::row(l, w), na - 1);
+            y[(long long)r * nb + n + c] = (double)sum;
+        }
+    }
+}
+
+// any shape with fewer than four strings of a spin: one element per lane
+template <typename T>
+__device__ __forceinline__ void gs_small(const GfTask &t, const T *X, double *y, int m0, int n0)
+{
+    const GemmFci &g = t.g;
+    const int na = (int)g.na, nb = (int)g.nb;
+    for (int e = threadIdx.x; e < 32 * 32; e += 256) {
+        const int r = m0 + e / 32, c = n0 + e % 32;
+        if (r >= na || c >= nb) continue;
+        const T *Ha = hmat<T>(g, 0), *Hb = hmat<T>(g, 1);
+        T sum = (T)0;
+        for (int k = 0; k < na; k++) sum += Ha[(long long)r * na + k] * X[(long long)k * nb + c];
+        for (int k = 0; k < nb; k++) sum += X[(long long)r * nb + k] * Hb[(long long)k * nb + c];
+        y[(long long)r * nb + c] = (double)sum;
+    }
+}
+
+// Same-spin parts: y_k = Haa X_k + X_k Hbb on tiles (k, alpha rows, beta columns) of the edge
+// that gs_edge chooses.  128: four waves of 64 x 64 each over both reductions whole; 64 and 32:
+// the four waves share the reductions of one tile.
+//
+// Bound by the matrix cores (FP64 88 % busy, FP32 73 % at 1.8 GHz).  Operands straight from
+// memory: a 16-deep step of a 64 x 64 tile is 16 (FP64) or 8 wide loads for 64 products, which
+// the caches keep up with, and no wave waits at a barrier.  5a5b in 14 orbitals: FP64 one vector
+// 720 -> 589 us, FP32 four vectors 2390 -> 1573 us against 64 x 64 tiles staged through LDS;
+// 4a4b in 12 orbitals, where 64 x 64 tiles occupy a quarter of the chip, 67 -> 16 us.
+template <typename T>
+__global__ __launch_bounds__(256, Gs<T>::WPE) void k_gss(const GfHeader *__restrict__ H,
+                                                         const GfTask *__restrict__ tasks)
+{
+    __shared__ T red[4 * 4 * 4 * 64];
     const int n = H->n;
     const long long total = H->total[GF_SS];
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int wm = w >> 1, wn = w & 1;
     for (long long u = blockIdx.x; u < total; u += gridDim.x) {
         const GfTask &t = tasks[find_task(tasks, n, u, GF_SS)];
         const GemmFci &g = t.g;
-        const long long na = g.na, nb = g.nb;
-        const long long tn = (nb + 63) / 64, tm = (na + 63) / 64;
-        const long long loc = u - t.base[GF_SS];
-        const int k = (int)(loc / (tm * tn));
-        const long long rem = loc - (long long)k * tm * tn;
-        const long long m0 = (rem / tn) * 64, n0 = (rem % tn) * 64;
+        const int na = (int)g.na, nb = (int)g.nb, edge = gs_edge(g.na, g.nb, t.K);
+        const int tn = (nb + edge - 1) / edge, tm = (na + edge - 1) / edge;
+        const int loc = (int)(u - t.base[GF_SS]), k = loc / (tm * tn), rem = loc - k * tm * tn;
+        const int m0 = rem / tn * edge, n0 = rem % tn * edge;
         const T *X = xin<T>(t, k);
-        typename Mf<T>::acc acc[2][2];
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) acc[i][j] = Mf<T>::zero();
-        mma_tile<T>(acc, hmat<T>(g, 0), na, X, nb, na, nb, na, m0, n0, As, Bs);
-        mma_tile<T>(acc, X, nb, hmat<T>(g, 1), nb, na, nb, nb, m0, n0, As, Bs);
         double *y = t.y + (long long)k * t.ldy;
+        if (na < 4 || nb < 4) {
+            gs_small<T>(t, X, y, m0, n0);
+        } else if (edge == 32) {
+            gs_split<T, 2>(t, X, y, m0, n0, red);
+        } else if (edge == 64) {
+            gs_split<T, 4>(t, X, y, m0, n0, red);
+        } else {
+            typename Mf<T>::acc acc[4][4];
+            int m[4];
+            const int mw = m0 + (w >> 1) * 64;
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+            for (int i = 0; i < 4; i++) {
+                m[i] = std::min(mw + i * 16 + (l & 15), na - 1);
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+                for (int c = 0; c < 4; c++) acc[i][c] = Mf<T>::zero();
+            }
+            const int c0 = std::min(n0 + (w & 1) * 64 + 4 * (l & 15), nb - 4);
+            gs_wave<T, 4>(acc, hmat<T>(g, 0), na, X, nb, na, m, c0, 0, (na + 15) / 16);
+            gs_wave<T, 4>(acc, X, nb, hmat<T>(g, 1), nb, nb, m, c0, 0, (nb + 15) / 16);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
-                    const long long r = m0 + wm * 32 + i * 16 + Mf<T>::row(l, v);
-                    const long long c = n0 + wn * 32 + j * 16 + l % 16;
-                    if (r < na && c < nb) y[r * nb + c] = (double)acc[i][j][v];
+                    const int r = std::min(mw + i * 16 + Mf<T>::row(l, v), na - 1);
+                    const auto o = gptr_w(y + (long long)r * nb + c0);
+#pragma unroll
+                    for (int c = 0; c < 4; c += 2)
+                        *(__attribute__((address_space(1))) GsOut *)(o + c) =
+                            (GsOut){(double)acc[i][c][v], (double)acc[i][c + 1][v]};
                 }
+        }
     }
 }
 
-// The D tile sits in LDS column-major, Dt[column][Q], and the reduction index of the
-// products is permuted: step ks, lane group kk = l / 16 takes Q = kk * KS + ks (the (P|Q)
-// fragments use the same order).  A lane's B values for VK consecutive steps are then
-// adjacent and come in one 16-byte LDS read.  Row stride GF_LDT elements (a multiple of
-// 16 bytes, 4 banks past a multiple of 64 banks).
+// ---- opposite-spin products -------------------------------------------------------------------
 template <typename T> struct GeL;
 template <> struct GeL<double> {
-    static constexpr int LDT = GF_MAXMP + 2;
-    static constexpr int VK = 2;
-    typedef double2 vec;
-    static __device__ __forceinline__ double at(const vec &v, int q) { return q ? v.y : v.x; }
-};
-template <> struct GeL<float> {
-    static constexpr int LDT = GF_MAXMP + 4;
-    static constexpr int VK = 4;
-    typedef float4 vec;
-    static __device__ __forceinline__ float at(const vec &v, int q)
+    // row padding, elements of a 16-byte read; waves per SIMD (work-groups per CU), their LDS
+    static constexpr int PAD = 2, VK = 2, WPE = 1, LDS = 160 << 10;
+    typedef double vec __attribute__((ext_vector_type(2)));
+    static __device__ __forceinline__ double sgn(double v, uint32_t e)
     {
-        return q == 0 ? v.x : q == 1 ? v.y : q == 2 ? v.z : v.w;
+        return __hiloint2double(__double2hiint(v) ^ (int)(e & 0x80000000u), __double2loint(v));
     }
 };
-
-// Products of one D tile for the wave's row tile: acc[j] += A . D(column tile j) over the
-// KS reduction steps, straight-line code, the B vectors of the next group of steps read
-// while the products of the current group run (group gi = steps gi*VK .. gi*VK + VK - 1).
-template <typename T, int BN, int KS>
-__device__ __forceinline__ void gE_mma(typename Mf<T>::acc (&acc)[BN / 16],
-                                       const T (&a)[GF_MAXMP / 4], const T (*Dt)[GeL<T>::LDT],
-                                       int l)
+template <> struct GeL<float> {
+    static constexpr int PAD = 4, VK = 4, WPE = 2, LDS = 80 << 10;
+    typedef float vec __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ float sgn(float v, uint32_t e)
+    {
+        return __int_as_float(__float_as_int(v) ^ (int)(e & 0x80000000u));
+    }
+};
+__device__ __forceinline__ void gf_wave_sync()
 {
-    constexpr int NCT = BN / 16, VK = GeL<T>::VK, NG = KS / VK;
-    typedef typename GeL<T>::vec V;
-    const int kk = l / 16;
-    V b[2][NCT];
-#pragma unroll
-    for (int j = 0; j < NCT; j++) b[0][j] = *(const V *)&Dt[j * 16 + l % 16][kk * KS];
-#pragma unroll
-    for (int gi = 0; gi < NG; gi++) {
-        const int cb = gi & 1;
-        if (gi + 1 < NG) {
-#pragma unroll
-            for (int j = 0; j < NCT; j++)
-                b[cb ^ 1][j] = *(const V *)&Dt[j * 16 + l % 16][kk * KS + (gi + 1) * VK];
-        }
-#pragma unroll
-        for (int q = 0; q < VK; q++)
-#pragma unroll
-            for (int j = 0; j < NCT; j++)
-                acc[j] = Mf<T>::mma(a[gi * VK + q], GeL<T>::at(b[cb][j], q), acc[j]);
+    // LDS accesses of one wave execute in order; this keeps the compiler from moving them
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// a value that all lanes share, in scalar registers (divisions leave theirs in vector registers)
+__device__ __forceinline__ int gf_uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ long long gf_uni(long long v)
+{
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)v);
+    return (long long)(int)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | lo;
+}
+
+// element i past a uniform pointer, by a 32-bit offset per lane
+template <typename T>
+__device__ __forceinline__ void gf_put(__attribute__((address_space(1))) T *p, uint32_t i, T v)
+{
+    *(__attribute__((address_space(1))) T *)((__attribute__((address_space(1))) char *)p + i * (uint32_t)sizeof(T)) = v;
+}
+
+typedef uint32_t GfQuad __attribute__((ext_vector_type(4)));
+
+// f(integral constant i) for i = A .. B - 1, written out
+template <int A, int B, typename F> __device__ __forceinline__ void gf_each(F f)
+{
+    if constexpr (A < B) {
+        f(std::integral_constant<int, A>{});
+        gf_each<A + 1, B>(f);
     }
 }
 
-// the reduction depth KS = MP / 4 is a multiple of 4 up to GF_MAXMP / 4
-template <typename T, int BN>
-__device__ __forceinline__ void gE_mma_ks(int KS, typename Mf<T>::acc (&acc)[BN / 16],
-                                          const T (&a)[GF_MAXMP / 4], const T (*Dt)[GeL<T>::LDT],
-                                          int l)
+// E rows of alpha string Ja, vector k, column tiles tile0 .. tile1 - 1, by one wave: the (P|Q)
+// fragments of its RT row tiles stay in registers, the D tile of 16 columns is in the wave's
+// own part of LDS.  D sits column-major and the reduction index is permuted: step ks, lane
+// group l / 16 takes Q = (l / 16) * KS + ks, so that a lane's B values of consecutive steps
+// come in one 16-byte read.  A lane scatters a quarter of one column's list (4 entries per
+// 16 bytes).
+//
+// A matrix product occupies the matrix core for 64 (FP64) or 32 cycles, in which the wave may
+// issue other work: everything else a tile needs is cut into single operations that are dealt
+// out between the products, in this order: the list of the tile after next (F), the clearing of
+// the next tile's D (Z, the other of two buffers), the stores of the previous tile's results
+// (S), the reads of the next tile's values (G) and their scatter (P).  Rows and columns past the
+// end repeat the last one, results and all, so that nothing needs a mask; a span's first tile
+// stores zeros where its results follow.
+template <typename T, int KS, int RT, bool EX, bool ST>
+__device__ __forceinline__ void gE_span(const GfTask &t, long long r, int Ja, int tile0, int tile1,
+                                        int xo, const T *xg, int dofs)
+{
+    constexpr int KC = 4 * KS, LDC = KC + GeL<T>::PAD, VK = GeL<T>::VK, NG = KS / VK;
+    constexpr int Lp = ge_pitch(KC), NL = Lp / 4, NZ = (LDC * (int)sizeof(T) + 63) / 64;
+    typedef typename GeL<T>::vec V;
+    typedef const __attribute__((address_space(1))) V *VP;
+    typedef const __attribute__((address_space(1))) char *CP;
+    typedef const __attribute__((address_space(1))) GfQuad *QP;
+    // the lane and the row made opaque here: what the cases of the switch over the shapes have
+    // in common would otherwise be computed ahead of it and held in registers all along
+    int l = threadIdx.x & 63;
+    asm volatile("" : "+v"(l));
+    asm volatile("" : "+s"(r));
+    asm volatile("" : "+s"(Ja));
+    asm volatile("" : "+s"(tile0));
+    asm volatile("" : "+s"(xo));
+    asm volatile("" : "+s"(dofs));
+    const int col = l & 15, part = l >> 4;
+    extern __shared__ __align__(16) unsigned char gf_smem[];
+    T *Dt = (T *)gf_smem + dofs;                   // two tiles of 16 columns, the extra row of (P|Q)
+    const T *xs = (const T *)gf_smem + xo;         // staged row (ST; else gathered from memory)
+    const GemmFci &g = t.g;
+    const int La = gf_uni(g.La), nb = gf_uni((int)g.nb);
+    T a[RT][KS];
+#pragma unroll
+    for (int i = 0; i < RT; i++) {
+        const int p = std::min(i * 16 + col, La - 1 - (int)EX);
+        const int P = (int)((gptr(g.la)[(long long)Ja * La + p] >> 16) & 0xFFu);
+        const auto row = gptr(P == GF_PDIAG ? drows<T>(g) + (long long)Ja * KC : mpad<T>(g) + P * KC) + part * KS;
+#pragma unroll
+        for (int s = 0; s < NG; s++) {
+            const V v = *(VP)(row + s * VK);
+#pragma unroll
+            for (int q = 0; q < VK; q++) a[i][s * VK + q] = v[q];
+        }
+    }
+    if (EX) {
+        const auto row = gptr(drows<T>(g) + (long long)Ja * KC);
+        for (int i = l; i < KC; i += 64) Dt[32 * LDC + i] = row[i];
+    }
+    const auto lb = gptr((const uint32_t *)gf_uni((long long)g.lb));
+    const auto xr = gptr((const T *)gf_uni((long long)xg));
+    const auto E = gptr_w((T *)gf_uni((long long)t.E)) + r * La * nb;
+    // rows of a lane: LROW * part + VROW * v, in the last row tile up to the last one
+    const uint32_t eofs = (uint32_t)(Mf<T>::LROW * part * nb);
+    uint32_t elast[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+        elast[v] = (uint32_t)(std::min((RT - 1) * 16 + Mf<T>::LROW * part + Mf<T>::VROW * v, La - 1 - (int)EX) * nb);
+    uint32_t e[NL], en[NL];
+    T v[NL];
+    typename Mf<T>::acc acc[RT], res[RT];
+    T d, dres = (T)0;                              // the extra row: a dot product per column
+    uint32_t cres = 0;                             // column of res
+    auto fetch = [&](int tile, int i) __attribute__((always_inline)) {
+        const uint32_t o = ((uint32_t)std::min(tile * 16 + col, nb - 1) * Lp + (uint32_t)part * 4) * 4;
+        const GfQuad q = *(QP)((CP)lb + o + i * 64);
+#pragma unroll
+        for (int j = 0; j < 4; j++) en[4 * i + j] = q[j];
+    };
+    auto clear = [&](T *D, int z) __attribute__((always_inline)) {
+        const V zv = {};
+        if (z * 64 + 64 <= LDC * (int)sizeof(T) || z * 64 + l < LDC * (int)sizeof(T)) ((V *)D)[z * 64 + l] = zv;
+    };
+    auto get = [&](int j) __attribute__((always_inline)) { v[j] = ST ? xs[e[j] & 0xFFFFu] : xr[e[j] & 0xFFFFu]; };
+    auto put = [&](T *Dc, int j) __attribute__((always_inline)) {
+        Dc[(e[j] >> 16) & 0xFFu] = GeL<T>::sgn(v[j], e[j]);
+    };
+    auto store = [&](int i, int q) __attribute__((always_inline)) {
+        if (i + 1 < RT) gf_put(E + (i * 16 + Mf<T>::VROW * q) * nb, eofs + cres, res[i][q]);
+        else gf_put(E, elast[q] + cres, res[i][q]);
+    };
+    // operation m of the M that go with a tile's products (order above)
+    constexpr int GL = NL / 2, M = NL / 4 + NZ + 4 * RT + 2 * NL, NM = KS * RT;
+    auto op = [&](auto mc, T *D, int tile) __attribute__((always_inline)) {
+        constexpr int m = decltype(mc)::value, z = m - NL / 4, st = z - NZ, f = st - 4 * RT;
+        T *Dc = D + col * LDC;
+        if constexpr (z < 0) fetch(std::min(tile + 2, tile1 - 1), m);
+        else if constexpr (st < 0) clear(D, z);
+        else if constexpr (f < 0) store(st >> 2, st & 3);
+        // half the reads, then a write and a read in turn, then the other writes
+        else if constexpr (f < GL) get(f);
+        else if constexpr (f >= GL + NL) put(Dc, f - NL);
+        else if constexpr ((f - GL) & 1) get(GL + (f - GL) / 2);
+        else put(Dc, (f - GL) / 2);
+    };
+#pragma unroll
+    for (int i = 0; i < NL / 4; i++) fetch(tile0, i);
+#pragma unroll
+    for (int i = 0; i < NZ; i++) clear(Dt, i);
+#pragma unroll
+    for (int i = 0; i < NL; i++) e[i] = en[i];
+#pragma unroll
+    for (int i = 0; i < NL / 4; i++) fetch(std::min(tile0 + 1, tile1 - 1), i);
+#pragma unroll
+    for (int j = 0; j < NL; j++) get(j);
+    gf_wave_sync();
+#pragma unroll
+    for (int j = 0; j < NL; j++) put(Dt + col * LDC, j);
+#pragma unroll
+    for (int i = 0; i < RT; i++) res[i] = Mf<T>::zero();
+    cres = (uint32_t)std::min(tile0 * 16 + col, nb - 1);
+    int cur = 0;
+    for (int tile = tile0; tile < tile1; tile++) {
+        gf_wave_sync();
+        const T *b0 = Dt + cur + col * LDC + part * KS;
+        T *Dn = Dt + (16 * LDC - cur);
+#pragma unroll
+        for (int i = 0; i < NL; i++) e[i] = en[i];
+#pragma unroll
+        for (int i = 0; i < RT; i++) acc[i] = Mf<T>::zero();
+        d = (T)0;
+        V b[2], y[2];
+        b[0] = *(const V *)b0;
+        if (EX) y[0] = *(const V *)(Dt + 32 * LDC + part * KS);
+        gf_each<0, NM>([&](auto kc) __attribute__((always_inline)) {
+            constexpr int k = decltype(kc)::value, i = k % RT, st = k / RT, s = st / VK, q = st % VK;
+            if constexpr (k % (RT * VK) == 0 && s + 1 < NG) {
+                b[(s + 1) & 1] = *(const V *)(b0 + (s + 1) * VK);
+                if (EX) y[(s + 1) & 1] = *(const V *)(Dt + 32 * LDC + part * KS + (s + 1) * VK);
+            }
+            acc[i] = Mf<T>::mma(a[i][st], b[s & 1][q], acc[i]);
+            gf_each<(k * M + NM - 1) / NM, ((k + 1) * M + NM - 1) / NM>(
+                [&](auto mc) __attribute__((always_inline)) { op(mc, Dn, tile); });
+            if constexpr (EX && i == RT - 1) d += b[s & 1][q] * y[s & 1][q];
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        if (EX) {
+            // the previous tile's extra row, and this one's sum over the four lane groups
+            gf_put(E + (La - 1) * nb, cres, dres);
+            d += __shfl_xor(d, 16);
+            dres = d + __shfl_xor(d, 32);
+        }
+        cres = (uint32_t)std::min(tile * 16 + col, nb - 1);
+#pragma unroll
+        for (int i = 0; i < RT; i++) res[i] = acc[i];
+        cur = 16 * LDC - cur;
+    }
+    if (EX) gf_put(E + (La - 1) * nb, cres, dres);
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) store(i, q);
+}
+
+// The depths KS, row tiles and extra rows that alpha lists of n <= 15 orbitals have
+// (La = a (n - a) + 1 rows, KS = MP / 4); only n = 15 has rows too long to stage.
+template <typename T>
+__device__ __forceinline__ void gE_shape(const GfTask &t, long long r, int Ja, bool ex, int tile0,
+                                         int tile1, int xo, const T *xg, int dofs)
 {
     static_assert(GF_MAXMP == 128, "reduction depths below cover MP <= 128");
-    switch (KS) {
-    case 4: gE_mma<T, BN, 4>(acc, a, Dt, l); break;
-    case 8: gE_mma<T, BN, 8>(acc, a, Dt, l); break;
-    case 12: gE_mma<T, BN, 12>(acc, a, Dt, l); break;
-    case 16: gE_mma<T, BN, 16>(acc, a, Dt, l); break;
-    case 20: gE_mma<T, BN, 20>(acc, a, Dt, l); break;
-    case 24: gE_mma<T, BN, 24>(acc, a, Dt, l); break;
-    case 28: gE_mma<T, BN, 28>(acc, a, Dt, l); break;
-    default: gE_mma<T, BN, 32>(acc, a, Dt, l); break;
+#define GE_CASE(KS, RT, EX) \
+    case (KS) * 16 + (RT) * 2 + (EX): \
+        gE_span<T, KS, RT, EX, true>(t, r, Ja, tile0, tile1, xo, xg, dofs); break
+#define GE_CASE2(KS, RT) \
+    case (KS) * 16 + (RT) * 2: \
+        if (xo >= 0) gE_span<T, KS, RT, false, true>(t, r, Ja, tile0, tile1, xo, xg, dofs); \
+        else gE_span<T, KS, RT, false, false>(t, r, Ja, tile0, tile1, xo, xg, dofs); \
+        break
+    switch (t.g.MP / 4 * 16 + (t.g.La - ex + 15) / 16 * 2 + ex) {
+    GE_CASE(4, 1, 0);                                                      // n <= 5
+    GE_CASE(8, 1, 0);                                                      // 6, 7
+    GE_CASE(12, 1, 0); GE_CASE(12, 1, 1); GE_CASE(12, 2, 0);               // 8, 9
+    GE_CASE(16, 1, 0); GE_CASE(16, 1, 1); GE_CASE(16, 2, 0);               // 10
+    GE_CASE(20, 1, 0); GE_CASE(20, 2, 0); GE_CASE(20, 2, 1); GE_CASE(20, 3, 0);   // 11, 12
+    GE_CASE(24, 1, 0); GE_CASE(24, 2, 0); GE_CASE(24, 3, 0);               // 13
+    GE_CASE(28, 1, 0); GE_CASE(28, 2, 0); GE_CASE(28, 3, 0); GE_CASE(28, 3, 1); GE_CASE(28, 4, 0);   // 14
+    GE_CASE2(32, 1); GE_CASE2(32, 2); GE_CASE2(32, 3); GE_CASE2(32, 4);    // 15
     }
+#undef GE_CASE
+#undef GE_CASE2
 }
 
 // E[p][c] = sum_Q (P_p|Q) D[Q][c] over columns c = (k, Ja, Ib), for the La rows p of the
-// alpha string Ja (P_p = pair of entry p of Ja's alpha list).  A column tile holds BN beta
-// strings of one row (k, Ja), so the tile shares Ja: wave w keeps the (P|Q) fragments of
-// rows 16w .. 16w+15 of Ja in registers (La <= 64: at most four row tiles, one per wave),
-// reloaded when the row changes, and the row X_k[Ja] is staged in LDS (rows of up to
-// GF_XROW_BYTES: 2048 strings FP64, 4096 FP32) for the beta-list gathers.  The tile of D is built in LDS from the beta
-// lists (each (Q, column) receives at most one entry); columns past the end of the row
-// repeat its last column (their products are not stored).
-#define GF_XROW_BYTES 16384
-template <typename T, int BN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_gE(
-    const GfHeader *__restrict__ H, const GfTask *__restrict__ tasks)
+// alpha string Ja (P_p = pair of entry p of Ja's alpha list).  Every wave works on its own 16
+// columns of one row (k, Ja) and all of that string's row tiles, without barriers.  A row past
+// the last full tile (a (n - a) a multiple of 16) is a dot product on the vector units instead
+// of a tile.  The vector's rows that a work-group needs next are staged in LDS for the list
+// gathers (as many as fit beside the D tiles; longer rows are gathered from memory).  A unit
+// is `bn` columns of one row; work-groups take equal consecutive ranges of units.
+//
+// Bound by the matrix cores (70 % busy at the clock the power limit leaves, about 2 GHz).  FP64
+// keeps one wave per SIMD: two D tiles a wave fill the LDS, and the fragments of four row tiles
+// take half the registers.  5a5b in 14 orbitals: FP64 one vector 1362 -> 936 us, FP32 four
+// vectors 3232 -> 1884 us against a work-group per tile with three barriers and a row tile per
+// wave (the fourth wave idle at 46 rows); waves by themselves, two per SIMD and one D tile each,
+// reached 1017 and 2220 us, two D tiles without the dealt-out order 1083 and 2151 us.  4a4b in
+// 12 orbitals (33 rows): 81 -> 45 us.
+template <typename T>
+__global__ __launch_bounds__(256, GeL<T>::WPE) void k_gE(const GfHeader *__restrict__ H,
+                                                         const GfTask *__restrict__ tasks, int bn)
 {
-    constexpr int LDT = GeL<T>::LDT;
-    __shared__ __align__(16) T Dt[BN][LDT];
-    constexpr int XROW = GF_XROW_BYTES / (int)sizeof(T);
-    __shared__ T xs[XROW];
-    constexpr int NCT = BN / 16, PARTS = 256 / BN, KSMAX = GF_MAXMP / 4;
-    constexpr int EMAX = (GF_MAXLIST + PARTS - 1) / PARTS;   // list entries per thread
-    const int tid = threadIdx.x, l = tid & 63;
+    extern __shared__ __align__(16) unsigned char gf_smem[];
+    const int tid = threadIdx.x, S = bn >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = H->n;
     const long long total = H->total[GF_E];
-    const int col = tid % BN, part = tid / BN;
     const long long u0 = total * blockIdx.x / gridDim.x, u1 = total * (blockIdx.x + 1) / gridDim.x;
-    if (u0 >= u1) return;
-    for (int idx = tid; idx < BN * LDT; idx += 256) (&Dt[0][0])[idx] = (T)0;
-    // task of the current tile and the first unit past it
-    int ti = find_task(tasks, n, u0, GF_E);
-    long long tend = ti + 1 < n ? tasks[ti + 1].base[GF_E] : total;
-    // tile u of a task: row r = (k, Ja) = k * Na + Ja, beta strings Ib0 .. Ib0 + ncol - 1
-    auto geom = [](const GfTask &t, long long u, long long &r, int &Ib0, int &ncol) {
-        const long long tpr = (t.g.nb + BN - 1) / BN, q = u - t.base[GF_E];
-        r = q / tpr;
-        Ib0 = (int)(q - r * tpr) * BN;
-        ncol = (int)std::min<long long>(BN, t.g.nb - Ib0);
-    };
-    // beta-list entries of this thread's column for a tile (issued one tile ahead, so their
-    // global loads overlap the products of the current tile); entry i is e = part + i*PARTS
-    uint32_t lcur[EMAX], lnxt[EMAX];
-    auto fetch = [&](long long u, uint32_t (&dst)[EMAX]) {
-        if (u >= u1) return;
-        const GfTask &t = tasks[u < tend ? ti : find_task(tasks, n, u, GF_E)];
-        long long r;
-        int Ib0, ncol;
-        geom(t, u, r, Ib0, ncol);
-        const long long Ib = Ib0 + std::min(col, ncol - 1);
-        const auto lst = gptr(t.g.lb + Ib * t.g.Lb);
-#pragma unroll
-        for (int i = 0; i < EMAX; i++) {
-            const int e = part + i * PARTS;
-            if (e < t.g.Lb) dst[i] = lst[e];
-        }
-    };
-    fetch(u0, lcur);
-    T a[KSMAX];
-    long long arow = -1;          // (task, row) of the fragments in a[] and of the row in xs
-    for (long long u = u0; u < u1; u++) {
-        if (u >= tend) {
-            ti = find_task(tasks, n, u, GF_E);
-            tend = ti + 1 < n ? tasks[ti + 1].base[GF_E] : total;
-        }
+    for (long long u = u0; u < u1;) {
+        const int ti = find_task(tasks, n, u, GF_E);
         const GfTask &t = tasks[ti];
         const GemmFci &g = t.g;
-        const int MP = g.MP, KS = MP / 4, Lb = g.Lb, La = g.La;
-        const bool active = 16 * w < La;
-        long long r;
-        int Ib0, ncol;
-        geom(t, u, r, Ib0, ncol);
-        const long long Nb = g.nb, k = r / g.na, Ja = r - k * g.na;
-        const bool staged_row = Nb <= XROW;
-        const long long key = ((long long)ti << 40) + r;
-        if (key != arow) {
-            // A fragment of step ks for row p = 16w + l%16 of Ja: (P_p | Q) at column
-            // Q = (l/16)*KS + ks; for the GF_PDIAG entry, Ja's row of sums of (kk | Q)
-            const int p = 16 * w + l % 16;
-            const bool ok = active && p < La;
-            const int P = ok ? (int)((gptr(g.la)[Ja * La + p] >> 16) & 0xFFu) : 0;
-            const T *Arow = P == GF_PDIAG ? drows<T>(g) + Ja * MP : mpad<T>(g) + (long long)P * MP;
-#pragma unroll
-            for (int ks = 0; ks < KSMAX; ks++)
-                a[ks] = (ok && ks < KS) ? Arow[(l / 16) * KS + ks] : (T)0;
-            if (staged_row) {
-                const T *__restrict__ xr = xin<T>(t, (int)k) + Ja * Nb;
-                for (int i = tid; i < Nb; i += 256) xs[i] = xr[i];
+        const bool ex = ge_extra(g.La);
+        const int nct = (int)(g.nb + 15) / 16, per = (nct + S - 1) / S;
+        const long long base = t.base[GF_E];
+        const long long r0 = (u - base) / per;
+        const int dw = (32 + ex) * (g.MP + GeL<T>::PAD);          // one wave's D tiles
+        T *xs = (T *)gf_smem + 4 * dw;
+        const int room = (GeL<T>::LDS / (int)sizeof(T) - 4 * dw) / (int)g.nb;
+        long long end = std::min(u1, ti + 1 < n ? tasks[ti + 1].base[GF_E] : total);
+        if (room > 0) end = std::min(end, base + (r0 + room) * per);
+        __syncthreads();   // the rows and tiles of the previous stage are read
+        if (room > 0) {
+            for (long long r = r0; r <= (end - 1 - base) / per; r++) {
+                const long long k = r / g.na;
+                const auto xr = gptr(xin<T>(t, (int)k) + (r - k * g.na) * g.nb);
+                for (int i = tid; i < g.nb; i += 256) xs[(r - r0) * g.nb + i] = xr[i];
             }
-            arow = key;
+            __syncthreads();
         }
-        __syncthreads();   // row staged; the previous tile's entries are cleared
-        {
-            // all reads first (independent, one wait), then the scatter into the D tile
-            T v[EMAX];
-            if (staged_row) {
-#pragma unroll
-                for (int i = 0; i < EMAX; i++)
-                    if (part + i * PARTS < Lb) v[i] = xs[lcur[i] & 0xFFFFu];
-            } else {
-                const auto xr = gptr(xin<T>(t, (int)k) + Ja * Nb);
-#pragma unroll
-                for (int i = 0; i < EMAX; i++)
-                    if (part + i * PARTS < Lb) v[i] = xr[lcur[i] & 0xFFFFu];
-            }
-#pragma unroll
-            for (int i = 0; i < EMAX; i++)
-                if (part + i * PARTS < Lb)
-                    Dt[col][(lcur[i] >> 16) & 0xFFu] = (lcur[i] >> 31) ? -v[i] : v[i];
+        const long long w1 = u + ((end - u) * (w + 1) >> 2);
+        for (long long q = u + ((end - u) * w >> 2); q < w1;) {
+            const long long r = gf_uni((q - base) / per);
+            const int k = gf_uni((int)(r / g.na)), Ja = gf_uni((int)(r - k * g.na));
+            const int un = (int)(q - base - r * per), m = (int)std::min<long long>(w1 - q, per - un);
+            const int xo = gf_uni(room > 0 ? 4 * dw + (int)(r - r0) * (int)g.nb : -1);
+            const T *xg = xin<T>(t, k) + Ja * g.nb;
+            const int t0 = gf_uni(un * S), t1 = gf_uni(std::min(nct, (un + m) * S)), dofs = gf_uni(w * dw);
+            gE_shape<T>(t, r, Ja, ex, t0, t1, xo, xg, dofs);
+            q += m;
         }
-        __syncthreads();   // D tile complete
-        fetch(u + 1, lnxt);
-        if (active) {
-            typename Mf<T>::acc acc[NCT];
-#pragma unroll
-            for (int j = 0; j < NCT; j++) acc[j] = Mf<T>::zero();
-            gE_mma_ks<T, BN>(KS, acc, a, Dt, l);
-            const auto E = gptr_w((T *)t.E);
-            const long long c0 = r * Nb + Ib0;
-#pragma unroll
-            for (int j = 0; j < NCT; j++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int p = 16 * w + Mf<T>::row(l, v), cj = j * 16 + l % 16;
-                    if (p < La && cj < ncol) E[(long long)p * t.lde + c0 + cj] = acc[j][v];
-                }
-        }
-        __syncthreads();   // the products have read the D tile
-        // clear exactly the entries this thread wrote (the rest of Dt stays zero)
-#pragma unroll
-        for (int i = 0; i < EMAX; i++)
-            if (part + i * PARTS < Lb) Dt[col][(lcur[i] >> 16) & 0xFFu] = (T)0;
-#pragma unroll
-        for (int i = 0; i < EMAX; i++) lcur[i] = lnxt[i];
+        u = end;
     }
 }
 
@@ -497,29 +709,30 @@ __global__ __launch_bounds__(256) void k_gga(const GfHeader *__restrict__ H,
     for (long long u = blockIdx.x; u < total; u += gridDim.x) {
         const GfTask &t = tasks[find_task(tasks, n, u, GF_GA)];
         const GemmFci &g = t.g;
-        const long long Nb = g.nb, N = g.na * g.nb, ncols = N * t.K, lde = t.lde;
+        const long long Nb = g.nb, N = g.na * g.nb, ncols = N * t.K;
+        const int La = g.La;
         const long long idx = (u - t.base[GF_GA]) * 256 + threadIdx.x;
         if (idx >= ncols) continue;
         const long long k = idx / N, rem = idx - k * N;
         const long long Ia = rem / Nb, Ib = rem - Ia * Nb;
-        const auto lst = gptr(g.la + Ia * g.La);
-        const auto Ek = gptr((const T *)t.E + k * N + Ib);
+        const auto lst = gptr(g.la + Ia * La);
+        const auto Ek = gptr((const T *)t.E + k * N * La + Ib);
         T acc = (T)0;
         int e = 0;
         // eight independent loads in flight per lane
-        for (; e + 8 <= g.La; e += 8) {
+        for (; e + 8 <= La; e += 8) {
             T v[8];
 #pragma unroll
             for (int q = 0; q < 8; q++) {
                 const uint32_t wd = lst[e + q];
-                v[q] = Ek[(long long)((wd >> 24) & 0x7Fu) * lde + (long long)(wd & 0xFFFFu) * Nb];
+                v[q] = Ek[(long long)((wd & 0xFFFFu) * (uint32_t)La + ((wd >> 24) & 0x7Fu)) * Nb];
             }
 #pragma unroll
             for (int q = 0; q < 8; q++) acc += (lst[e + q] >> 31) ? -v[q] : v[q];
         }
-        for (; e < g.La; e++) {
+        for (; e < La; e++) {
             const uint32_t wd = lst[e];
-            const T v = Ek[(long long)((wd >> 24) & 0x7Fu) * lde + (long long)(wd & 0xFFFFu) * Nb];
+            const T v = Ek[(long long)((wd & 0xFFFFu) * (uint32_t)La + ((wd >> 24) & 0x7Fu)) * Nb];
             acc += (wd >> 31) ? -v : v;
         }
         t.y[k * t.ldy + rem] += (double)acc;
@@ -542,10 +755,10 @@ int jk_gf_dense(long long nstr, const uint64_t *mask, const long long *off1, con
 }
 
 int jk_gf_lists(long long nstr, const uint64_t *mask, const long long *off1, const int2 *e1,
-                int L, int diag_one, uint32_t *out, hipStream_t st)
+                int L, int Lp, int pad, int diag_one, uint32_t *out, hipStream_t st)
 {
     hipLaunchKernelGGL(k_gf_lists, dim3((unsigned)((nstr + 127) / 128)), dim3(128), 0, st, nstr,
-                       mask, off1, e1, L, diag_one, out);
+                       mask, off1, e1, L, Lp, (uint32_t)pad, diag_one, out);
     GF_CHECK();
     return 0;
 }
@@ -587,13 +800,23 @@ void jk_gf_units(int prec, int bn, const GfTask &t, long long units[4])
 {
     const long long na = t.g.na, nb = t.g.nb, N = na * nb, cols = N * t.K;
     units[GF_CV] = prec == 64 ? 0 : (cols + 255) / 256;
-    units[GF_SS] = (long long)t.K * ((na + 63) / 64) * ((nb + 63) / 64);
-    units[GF_E] = (long long)t.K * na * ((nb + bn - 1) / bn);
+    const int edge = gs_edge(na, nb, t.K);
+    units[GF_SS] = (long long)t.K * ((na + edge - 1) / edge) * ((nb + edge - 1) / edge);
+    units[GF_E] = t.g.La ? (long long)t.K * na * ((nb + bn - 1) / bn) : 0;
     units[GF_GA] = (cols + 255) / 256;
 }
 
 // persistent grid caps of the grid-stride kernels (conversion, gather)
 static const long long gf_cap[4] = {4096, 2048, 2048, 4096};
+
+static long long device_cus()
+{
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return 256;
+    return cus;
+}
 
 // blocks of 256 threads of a kernel resident on the whole device at once
 static long long resident_blocks(const void *kernel)
@@ -606,24 +829,27 @@ static long long resident_blocks(const void *kernel)
     return (long long)cus * per;
 }
 
-template <typename T, int BN>
-static int gf_group_t(const GfHeader *d_hdr, const GfTask *d_tasks, const GfHeader *hh,
+template <typename T>
+static int gf_group_t(int bn, const GfHeader *d_hdr, const GfTask *d_tasks, const GfHeader *hh,
                       hipStream_t st)
 {
-    // The E kernel splits its units into equal consecutive ranges, one per block, and the
-    // same-spin kernel walks whole 64 x 64 tiles: both run one wave of resident blocks
-    // (a grid past residency leaves a last, partly filled wave of blocks)
-    static const long long cap_e = std::max(256LL, resident_blocks((const void *)k_gE<T, BN>));
+    // The same-spin kernel walks whole 64 x 64 tiles, the E kernel equal consecutive ranges of
+    // its units, one per work-group: both run one wave of resident blocks (a grid past
+    // residency leaves a last, partly filled wave of blocks)
+    static const long long cap_e = device_cus() * GeL<T>::WPE;
     static const long long cap_ss = std::max(256LL, resident_blocks((const void *)k_gss<T>));
     const long long cap[4] = {gf_cap[GF_CV], cap_ss, cap_e, gf_cap[GF_GA]};
     unsigned g[4];
-    for (int i = 0; i < 4; i++)
-        g[i] = (unsigned)(hh ? std::max<long long>(1, std::min(hh->total[i], cap[i])) : cap[i]);
+    for (int i = 0; i < 4; i++) {
+        // E: a unit is one wave's, four to a work-group
+        const long long units = !hh ? cap[i] : i == GF_E ? (hh->total[i] + 3) / 4 : hh->total[i];
+        g[i] = (unsigned)std::max<long long>(1, std::min(units, cap[i]));
+    }
     if (sizeof(T) == 4) {
         hipLaunchKernelGGL(k_gcv, dim3(g[GF_CV]), dim3(256), 0, st, d_hdr, d_tasks);
         GF_CHECK();
     }
-    hipLaunchKernelGGL((k_gE<T, BN>), dim3(g[GF_E]), dim3(256), 0, st, d_hdr, d_tasks);
+    hipLaunchKernelGGL(k_gE<T>, dim3(g[GF_E]), dim3(256), GeL<T>::LDS, st, d_hdr, d_tasks, bn);
     GF_CHECK();
     hipLaunchKernelGGL(k_gss<T>, dim3(g[GF_SS]), dim3(256), 0, st, d_hdr, d_tasks);
     GF_CHECK();
@@ -635,13 +861,10 @@ static int gf_group_t(const GfHeader *d_hdr, const GfTask *d_tasks, const GfHead
 int jk_gf_group(int prec, int bn, const GfHeader *d_hdr, const GfTask *d_tasks,
                 const GfHeader *hdr_host, hipStream_t st)
 {
-    if (prec == 64) {
-        if (bn == 16) return gf_group_t<double, 16>(d_hdr, d_tasks, hdr_host, st);
-        if (bn == 32) return gf_group_t<double, 32>(d_hdr, d_tasks, hdr_host, st);
-    } else {
-        if (bn == 32) return gf_group_t<float, 32>(d_hdr, d_tasks, hdr_host, st);
-        if (bn == 64) return gf_group_t<float, 64>(d_hdr, d_tasks, hdr_host, st);
+    if (!jk_gf_bn_valid(prec, bn)) {
+        jci_set_error("gf_sigma: E tile width %d not available for FP%d", bn, prec);
+        return -1;
     }
-    jci_set_error("gf_sigma: E tile width %d not available for FP%d", bn, prec);
-    return -1;
+    if (prec == 64) return gf_group_t<double>(bn, d_hdr, d_tasks, hdr_host, st);
+    return gf_group_t<float>(bn, d_hdr, d_tasks, hdr_host, st);
 }

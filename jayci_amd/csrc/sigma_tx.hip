@@ -657,7 +657,10 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
     // the lane and the unit made opaque here: what the reduction depths have in common would
     // otherwise be computed ahead of the switch over them and held in registers all along
     int l = threadIdx.x & 63;
-    asm volatile("" : "+v"(l), "+s"(u.ja), "+s"(u.w), "+s"(u.r0));
+    asm volatile("" : "+v"(l));
+    asm volatile("" : "+s"(u.ja));
+    asm volatile("" : "+s"(u.w));
+    asm volatile("" : "+s"(u.r0));
     const int col = l & 15, part = l >> 4;
     const int La = tx_uni(t.La), nIp = tx_uni(t.nIp);
 
