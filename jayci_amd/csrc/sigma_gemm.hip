@@ -186,12 +186,10 @@ template <typename T> struct Gs;
 template <> struct Gs<double> {
     typedef double quad __attribute__((ext_vector_type(4), aligned(8)));
     typedef double pair __attribute__((ext_vector_type(2), aligned(8)));
-    static constexpr int WPE = 1;                // waves per SIMD: 64 x 64 accumulators and operands
 };
 template <> struct Gs<float> {
     typedef float quad __attribute__((ext_vector_type(4), aligned(4)));
     typedef float pair __attribute__((ext_vector_type(2), aligned(4)));
-    static constexpr int WPE = 2;
 };
 typedef double GsOut __attribute__((ext_vector_type(2), aligned(8)));
 
@@ -344,14 +342,15 @@ __device__ __forceinline__ void gs_small(const GfTask &t, const T *X, double *y,
 // 720 -> 589 us, FP32 four vectors 2390 -> 1573 us against 64 x 64 tiles staged through LDS;
 // 4a4b in 12 orbitals, where 64 x 64 tiles occupy a quarter of the chip, 67 -> 16 us.
 template <typename T>
-__global__ __launch_bounds__(256, Gs<T>::WPE) void k_gss(const GfHeader *__restrict__ H,
-                                                         const GfTask *__restrict__ tasks)
+__device__ __forceinline__ void gf_same(const GfHeader *__restrict__ H, const GfTask *__restrict__ tasks,
+                                        int block, int blocks)
 {
-    __shared__ T red[4 * 4 * 4 * 64];
+    extern __shared__ __align__(16) unsigned char gf_smem[];
+    T *red = (T *)gf_smem;                         // 4 x 4 x 4 x 64
     const int n = H->n;
     const long long total = H->total[GF_SS];
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (long long u = blockIdx.x; u < total; u += gridDim.x) {
+    for (long long u = block; u < total; u += blocks) {
         const GfTask &t = tasks[find_task(tasks, n, u, GF_SS)];
         const GemmFci &g = t.g;
         const int na = (int)g.na, nb = (int)g.nb, edge = gs_edge(g.na, g.nb, t.K);
@@ -652,15 +651,16 @@ __device__ __forceinline__ void gE_shape(const GfTask &t, long long r, int Ja, b
 // reached 1017 and 2220 us, two D tiles without the dealt-out order 1083 and 2151 us.  4a4b in
 // 12 orbitals (33 rows): 81 -> 45 us.
 template <typename T>
-__global__ __launch_bounds__(256, GeL<T>::WPE) void k_gE(const GfHeader *__restrict__ H,
-                                                         const GfTask *__restrict__ tasks, int bn)
+__device__ __forceinline__ void gf_opposite(const GfHeader *__restrict__ H,
+                                            const GfTask *__restrict__ tasks, int bn, int block,
+                                            int blocks)
 {
     extern __shared__ __align__(16) unsigned char gf_smem[];
     const int tid = threadIdx.x, S = bn >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = H->n;
     const long long total = H->total[GF_E];
-    const long long u0 = total * blockIdx.x / gridDim.x, u1 = total * (blockIdx.x + 1) / gridDim.x;
+    const long long u0 = total * block / blocks, u1 = total * (block + 1) / blocks;
     for (long long u = u0; u < u1;) {
         const int ti = find_task(tasks, n, u, GF_E);
         const GfTask &t = tasks[ti];
@@ -696,6 +696,20 @@ __global__ __launch_bounds__(256, GeL<T>::WPE) void k_gE(const GfHeader *__restr
         }
         u = end;
     }
+}
+
+// Both parts in one launch, the first `eblocks` work-groups on the opposite-spin products: they
+// are independent of each other, and the one's last work-groups run beside the other's first.
+// Small spaces, of which either part leaves most of the chip idle, take the time of the longer
+// one and a launch less: 3a3b in 8 orbitals FP64 15.0 -> 10.3 us; 1 % or less from 4a4b in 12
+// orbitals on.
+template <typename T>
+__global__ __launch_bounds__(256, GeL<T>::WPE) void k_gprod(const GfHeader *__restrict__ H,
+                                                            const GfTask *__restrict__ tasks, int bn,
+                                                            int eblocks)
+{
+    if ((int)blockIdx.x < eblocks) gf_opposite<T>(H, tasks, bn, blockIdx.x, eblocks);
+    else gf_same<T>(H, tasks, blockIdx.x - eblocks, gridDim.x - eblocks);
 }
 
 // y_k[Ia][Ib] += sum over the alpha list of Ia of sign * E[p][k, Ja, Ib], p the entry's E row
@@ -807,7 +821,7 @@ void jk_gf_units(int prec, int bn, const GfTask &t, long long units[4])
 }
 
 // persistent grid caps of the grid-stride kernels (conversion, gather)
-static const long long gf_cap[4] = {4096, 2048, 2048, 4096};
+static const long long gf_cap[4] = {4096, 0, 0, 4096};
 
 static long long device_cus()
 {
@@ -818,30 +832,17 @@ static long long device_cus()
     return cus;
 }
 
-// blocks of 256 threads of a kernel resident on the whole device at once
-static long long resident_blocks(const void *kernel)
-{
-    int dev = 0, cus = 0, per = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, 256, 0) != hipSuccess)
-        return 0;
-    return (long long)cus * per;
-}
-
 template <typename T>
 static int gf_group_t(int bn, const GfHeader *d_hdr, const GfTask *d_tasks, const GfHeader *hh,
                       hipStream_t st)
 {
-    // The same-spin kernel walks whole 64 x 64 tiles, the E kernel equal consecutive ranges of
-    // its units, one per work-group: both run one wave of resident blocks (a grid past
-    // residency leaves a last, partly filled wave of blocks)
-    static const long long cap_e = device_cus() * GeL<T>::WPE;
-    static const long long cap_ss = std::max(256LL, resident_blocks((const void *)k_gss<T>));
-    const long long cap[4] = {gf_cap[GF_CV], cap_ss, cap_e, gf_cap[GF_GA]};
+    // Opposite-spin units go in equal consecutive ranges, one per work-group, same-spin tiles one
+    // after another: each part as many work-groups as the device holds
+    static const long long cap_p = device_cus() * GeL<T>::WPE;
+    const long long cap[4] = {gf_cap[GF_CV], cap_p, cap_p, gf_cap[GF_GA]};
     unsigned g[4];
     for (int i = 0; i < 4; i++) {
-        // E: a unit is one wave's, four to a work-group
+        // an opposite-spin unit is one wave's, four to a work-group
         const long long units = !hh ? cap[i] : i == GF_E ? (hh->total[i] + 3) / 4 : hh->total[i];
         g[i] = (unsigned)std::max<long long>(1, std::min(units, cap[i]));
     }
@@ -849,9 +850,8 @@ static int gf_group_t(int bn, const GfHeader *d_hdr, const GfTask *d_tasks, cons
         hipLaunchKernelGGL(k_gcv, dim3(g[GF_CV]), dim3(256), 0, st, d_hdr, d_tasks);
         GF_CHECK();
     }
-    hipLaunchKernelGGL(k_gE<T>, dim3(g[GF_E]), dim3(256), GeL<T>::LDS, st, d_hdr, d_tasks, bn);
-    GF_CHECK();
-    hipLaunchKernelGGL(k_gss<T>, dim3(g[GF_SS]), dim3(256), 0, st, d_hdr, d_tasks);
+    hipLaunchKernelGGL(k_gprod<T>, dim3(g[GF_E] + g[GF_SS]), dim3(256), GeL<T>::LDS, st, d_hdr, d_tasks,
+                       bn, (int)g[GF_E]);
     GF_CHECK();
     hipLaunchKernelGGL(k_gga<T>, dim3(g[GF_GA]), dim3(256), 0, st, d_hdr, d_tasks);
     GF_CHECK();
