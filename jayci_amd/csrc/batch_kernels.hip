@@ -11,6 +11,7 @@
 #include "slater.h"
 #include "sigma_fast.h"
 #include "batch.h"
+#include "davidson_tiles.h"
 
 #define BLAUNCH_CHECK()                                                  \
     do {                                                                 \
@@ -33,88 +34,24 @@ __device__ __forceinline__ int find_inst(const BDesc *__restrict__ d, int n, lon
 }
 
 // ---- Gram: out = A^T B (m x k), A and B vector-major with leading dimension ld ----------
-// FP64 MFMA 16x16x4 on 32-row LDS tiles (operand layout as k_gram); partial per block.
-// MAXM bounds m and k over the launch (checked by the host): the LDS tiles, the staging
-// registers and the (MAXM/16)^2 output tiles spread over the four waves are sized to it.
-#define BG_ROWS 32
-template <int MAXM>
+// The work-group's sum over its rows (gram_block), partial per block.  MT bounds the column
+// tiles of m and k over the launch (checked by the host); most products have one tile of k.
+template <int MT>
 __global__ __launch_bounds__(256) void k_bgram(const BHeader *__restrict__ H,
                                                const BDesc *__restrict__ D,
                                                double *__restrict__ partial)
 {
-    constexpr int NT = ((MAXM / 16) * (MAXM / 16) + 3) / 4;   // output tiles per wave
-    __shared__ double sA[BG_ROWS][MAXM + 1];
-    __shared__ double sB[BG_ROWS][MAXM + 1];
+    __shared__ double red[1024];
     const int n = H->n;
     const long long total = H->total;
     for (long long blk = blockIdx.x; blk < total; blk += gridDim.x) {
-    __syncthreads();
-    const int inst = find_inst(D, n, blk);
-    const BDesc &d = D[inst];
-    const int b = (int)(blk - d.blk0);
-    const int m = d.m, w = d.k;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int mt = (m + 15) / 16, wt = (w + 15) / 16, ntile = mt * wt;
-    const long long chunk = (d.N + d.nblk - 1) / d.nblk;
-    const long long r0 = (long long)b * chunk;
-    const long long r1 = r0 + chunk < d.N ? r0 + chunk : d.N;
-    typedef double v4d __attribute__((ext_vector_type(4)));
-    v4d acc[NT];
-    for (int t = 0; t < NT; t++) acc[t] = (v4d){0.0, 0.0, 0.0, 0.0};
-    // the chunk's values this thread stages (element idx = tid + 256 q: column idx / BG_ROWS,
-    // row idx % BG_ROWS), loaded into registers one chunk ahead so that the loads of the
-    // next chunk are in flight during the products of this one
-    constexpr int QA = BG_ROWS * MAXM / 256, QB = BG_ROWS * MAXM / 256;
-    double ra[QA], rb[QB];
-    auto gload = [&](long long base) {
-        const int rows = (int)((r1 - base) < BG_ROWS ? (r1 - base) : BG_ROWS);
-#pragma unroll
-        for (int q = 0; q < QA; q++) {
-            const int idx = tid + 256 * q, c = idx / BG_ROWS, r = idx % BG_ROWS;
-            ra[q] = (idx < BG_ROWS * mt * 16 && c < m && r < rows) ? d.A[(long long)c * d.ld + base + r] : 0.0;
-        }
-#pragma unroll
-        for (int q = 0; q < QB; q++) {
-            const int idx = tid + 256 * q, c = idx / BG_ROWS, r = idx % BG_ROWS;
-            rb[q] = (idx < BG_ROWS * wt * 16 && c < w && r < rows) ? d.B[(long long)c * d.ld + base + r] : 0.0;
-        }
-    };
-    if (r0 < r1) gload(r0);
-    for (long long base = r0; base < r1; base += BG_ROWS) {
-#pragma unroll
-        for (int q = 0; q < QA; q++) {
-            const int idx = tid + 256 * q;
-            if (idx < BG_ROWS * mt * 16) sA[idx % BG_ROWS][idx / BG_ROWS] = ra[q];
-        }
-#pragma unroll
-        for (int q = 0; q < QB; q++) {
-            const int idx = tid + 256 * q;
-            if (idx < BG_ROWS * wt * 16) sB[idx % BG_ROWS][idx / BG_ROWS] = rb[q];
-        }
-        __syncthreads();
-        if (base + BG_ROWS < r1) gload(base + BG_ROWS);
-        for (int t = 0; t < NT; t++) {
-            int tile = wave + 4 * t;
-            if (tile >= ntile) break;
-            int ti = tile / wt, tj = tile % wt;
-            for (int k0 = 0; k0 < BG_ROWS; k0 += 4) {
-                double a = sA[k0 + lane / 16][ti * 16 + lane % 16];
-                double bb = sB[k0 + lane / 16][tj * 16 + lane % 16];
-                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bb, acc[t], 0, 0, 0);
-            }
-        }
-        __syncthreads();
-    }
-    double *out = partial + d.pofs + (long long)b * m * w;
-    for (int t = 0; t < NT; t++) {
-        int tile = wave + 4 * t;
-        if (tile >= ntile) break;
-        int ti = tile / wt, tj = tile % wt;
-        for (int v = 0; v < 4; v++) {
-            int i = ti * 16 + lane / 16 + 4 * v, j = tj * 16 + lane % 16;
-            if (i < m && j < w) out[i * w + j] = acc[t][v];
-        }
-    }
+        const BDesc &d = D[find_inst(D, n, blk)];
+        const int b = (int)(blk - d.blk0), m = d.m, w = d.k;
+        const long long chunk = (d.N + d.nblk - 1) / d.nblk;
+        const long long r0 = (long long)b * chunk, r1 = r0 + chunk < d.N ? r0 + chunk : d.N;
+        double *out = partial + d.pofs + (long long)b * m * w;
+        if (MT == 1 || w <= 16) gram_block<MT, 1>(m, w, d.A, d.ld, d.B, d.ld, r0, r1, out, w, red);
+        else gram_block<MT, MT>(m, w, d.A, d.ld, d.B, d.ld, r0, r1, out, w, red);
     }
 }
 
@@ -141,13 +78,13 @@ int jb_gram(const BHeader *h, const BDesc *dD, int n_cap, int mmax, double *part
 {
     if (mmax > JCI_MAXBASIS) return -1;
     if (mmax <= 16)
-        hipLaunchKernelGGL(k_bgram<16>, dim3(JB_GRID), dim3(256), 0, st, h, dD, partial);
+        hipLaunchKernelGGL(k_bgram<1>, dim3(JB_GRID), dim3(256), 0, st, h, dD, partial);
     else if (mmax <= 32)
-        hipLaunchKernelGGL(k_bgram<32>, dim3(JB_GRID), dim3(256), 0, st, h, dD, partial);
+        hipLaunchKernelGGL(k_bgram<2>, dim3(JB_GRID), dim3(256), 0, st, h, dD, partial);
     else if (mmax <= 48)
-        hipLaunchKernelGGL(k_bgram<48>, dim3(JB_GRID), dim3(256), 0, st, h, dD, partial);
+        hipLaunchKernelGGL(k_bgram<3>, dim3(JB_GRID), dim3(256), 0, st, h, dD, partial);
     else
-        hipLaunchKernelGGL(k_bgram<JCI_MAXBASIS>, dim3(JB_GRID), dim3(256), 0, st, h, dD, partial);
+        hipLaunchKernelGGL(k_bgram<4>, dim3(JB_GRID), dim3(256), 0, st, h, dD, partial);
     hipLaunchKernelGGL(k_bpartial_sum, dim3(n_cap, BPS_SPLIT), dim3(256), 0, st, h, dD,
                        (const double *)partial);
     BLAUNCH_CHECK();
@@ -164,7 +101,9 @@ template <int MAXM>
 __global__ __launch_bounds__(256) void k_bcombine(const BHeader *__restrict__ H,
                                                   const BDesc *__restrict__ D)
 {
-    __shared__ double sC[MAXM * MAXM];   // k <= m <= MAXM (checked by the host)
+    // k <= m <= MAXM (checked by the host); [j][i], zero past m, so that two coefficients come in
+    // one read and the sums need no bounds
+    __shared__ __align__(16) double sC[MAXM * MAXM];
     const int n = H->n;
     const long long total = H->total;
     int cur = -1;
@@ -173,7 +112,10 @@ __global__ __launch_bounds__(256) void k_bcombine(const BHeader *__restrict__ H,
         const BDesc &d = D[inst];
         if (inst != cur) {
             __syncthreads();
-            for (int t = threadIdx.x; t < d.m * d.k; t += blockDim.x) sC[t] = d.C[t];
+            for (int t = threadIdx.x; t < MAXM * d.k; t += blockDim.x) {
+                const int j = t / MAXM, i = t - j * MAXM;
+                sC[t] = i < d.m ? d.C[i * d.k + j] : 0.0;
+            }
             __syncthreads();
             cur = inst;
         }
@@ -181,13 +123,15 @@ __global__ __launch_bounds__(256) void k_bcombine(const BHeader *__restrict__ H,
         if (r >= d.N) continue;
         double a[MAXM];
 #pragma unroll
-        for (int i = 0; i < MAXM; i++)
-            if (i < d.m) a[i] = d.A[(long long)i * d.ld + r];
+        for (int i = 0; i < MAXM; i++) a[i] = i < d.m ? d.A[(long long)i * d.ld + r] : 0.0;
         for (int j = 0; j < d.k; j++) {
             double s = d.beta == 0.0 ? 0.0 : d.beta * d.O[(long long)j * d.ld + r];
 #pragma unroll
-            for (int i = 0; i < MAXM; i++)
-                if (i < d.m) s += a[i] * sC[i * d.k + j];
+            for (int i = 0; i < MAXM; i += 2) {
+                const double2 c = *(const double2 *)&sC[j * MAXM + i];
+                s += a[i] * c.x;
+                s += a[i + 1] * c.y;
+            }
             d.O[(long long)j * d.ld + r] = s;
         }
     }
@@ -214,60 +158,23 @@ __global__ __launch_bounds__(256) void k_bresidual(const BHeader *__restrict__ H
                                                    const BDesc *__restrict__ D,
                                                    double *__restrict__ partial)
 {
-    __shared__ double sC[JCI_MAXBASIS * JCI_MAXK];
-    __shared__ double sT[JCI_MAXK];
-    __shared__ double red[JCI_MAXK][256];
+    __shared__ double sC[JCI_MAXBASIS * JCI_MAXK], sT[JCI_MAXK], red[4 * JCI_MAXK];
     const int n = H->n;
     const long long total = H->total;
     for (long long blk = blockIdx.x; blk < total; blk += gridDim.x) {
-    const int inst = find_inst(D, n, blk);
-    const BDesc &d = D[inst];
-    const int m = d.m, k = d.k;
-    __syncthreads();
-    for (int t = threadIdx.x; t < m * k; t += blockDim.x) sC[t] = d.C[t];
-    if (threadIdx.x < k) sT[threadIdx.x] = d.th[threadIdx.x];
-    __syncthreads();
-    const int b = (int)(blk - d.blk0);
-    const long long chunk = (d.N + d.nblk - 1) / d.nblk;
-    const long long r0 = (long long)b * chunk, r1 = r0 + chunk < d.N ? r0 + chunk : d.N;
-    double nrm[JCI_MAXK];
-    for (int r = 0; r < k; r++) nrm[r] = 0.0;
-    for (long long row = r0 + threadIdx.x; row < r1; row += 256) {
-        double res[JCI_MAXK];
-        for (int r = 0; r < k; r++) res[r] = 0.0;
-        // four basis vectors per step: their eight loads are issued together
-        int i = 0;
-        for (; i + 4 <= m; i += 4) {
-            double a[4], sv[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                a[q] = d.A[(long long)(i + q) * d.ld + row];
-                sv[q] = d.B[(long long)(i + q) * d.ld + row];
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                for (int r = 0; r < k; r++) res[r] += sC[(i + q) * k + r] * (sv[q] - sT[r] * a[q]);
-        }
-        for (; i < m; i++) {
-            double a = d.A[(long long)i * d.ld + row], sv = d.B[(long long)i * d.ld + row];
-            for (int r = 0; r < k; r++) res[r] += sC[i * k + r] * (sv - sT[r] * a);
-        }
-        double h = d.hd[row];
-        for (int r = 0; r < k; r++) {
-            nrm[r] += res[r] * res[r];
-            double den = h - sT[r];
-            if (fabs(den) < 1e-8) den = den < 0 ? -1e-8 : 1e-8;
-            d.O[(long long)r * d.ld + row] = -res[r] / den;
-        }
-    }
-    for (int r = 0; r < k; r++) red[r][threadIdx.x] = nrm[r];
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s)
-            for (int r = 0; r < k; r++) red[r][threadIdx.x] += red[r][threadIdx.x + s];
+        const BDesc &d = D[find_inst(D, n, blk)];
+        const int m = d.m, k = d.k;
         __syncthreads();
-    }
-    if (threadIdx.x < k) partial[d.pofs + (long long)b * k + threadIdx.x] = red[threadIdx.x][0];
+        for (int t = threadIdx.x; t < m * k; t += 256) sC[t] = d.C[t];
+        if (threadIdx.x < k) sT[threadIdx.x] = d.th[threadIdx.x];
+        __syncthreads();
+        const int b = (int)(blk - d.blk0);
+        const long long chunk = (d.N + d.nblk - 1) / d.nblk;
+        const long long r0 = (long long)b * chunk, r1 = r0 + chunk < d.N ? r0 + chunk : d.N;
+        with_k(k, [&](auto kc) __attribute__((always_inline)) {
+            residual_block<decltype(kc)::value>(m, d.A, d.B, d.ld, r0, r1, sC, sT, d.hd, d.O,
+                                                partial + d.pofs + (long long)b * k, red);
+        });
     }
 }
 

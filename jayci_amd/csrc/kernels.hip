@@ -10,6 +10,7 @@
 //   determinant lists ..... k_list_* (the O(N^2) screen of source/cimapping.c:92 on explicit lists)
 #include "jci_internal.h"
 #include "slater.h"
+#include "davidson_tiles.h"
 
 #define LAUNCH_CHECK()                                                   \
     do {                                                                 \
@@ -573,77 +574,18 @@ int jk_to_f32(const double *x, float *y, long long n, hipStream_t st)
 // Davidson vector kernels.  Basis vectors are stored one after another (leading
 // dimension ld >= N).
 
-// G = V^T W on MFMA (v_mfma_f64_16x16x4f64).  Each work-group stages 64-row tiles of V and
-// W in LDS (coalesced), each wavefront owns 16x16 output tiles and accumulates over the
-// row tiles of its work-group; per-work-group partials are reduced in a fixed order by
-// k_gram_reduce, so the result is deterministic.
-//
-// Operand layout of the 16x16x4 f64 MFMA (lane l, 64 lanes):
-//   A (16x4):  lane l holds A[l % 16][l / 16]
-//   B (4x16):  lane l holds B[l / 16][l % 16]
-//   D (16x16): lane l, register v holds D[l / 16 + 4 * v][l % 16]
-#define GRAM_ROWS 32
+// G = V^T W on MFMA: per work-group the sum over its rows (gram_block), the work-groups' sums
+// added in a fixed order by k_gram_reduce, so the result is deterministic.
+template <int MT, int WT>
 __global__ __launch_bounds__(256) void k_gram(int m, int w, long long N,
                                               const double *__restrict__ V, long long ldv,
                                               const double *__restrict__ W, long long ldw,
                                               double *__restrict__ partial, long long chunk)
 {
-    __shared__ double sV[GRAM_ROWS][JCI_MAXBASIS + 1];
-    __shared__ double sW[GRAM_ROWS][JCI_MAXBASIS + 1];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int mt = (m + 15) / 16, wt = (w + 15) / 16, ntile = mt * wt;
-    typedef double v4d __attribute__((ext_vector_type(4)));
-    v4d acc[4];
-    for (int t = 0; t < 4; t++) acc[t] = (v4d){0.0, 0.0, 0.0, 0.0};
-    long long r0 = (long long)blockIdx.x * chunk;
-    long long r1 = r0 + chunk < N ? r0 + chunk : N;
-    // stage: element (vector c, row r) -> sV[r][c], zero-padded to multiples of 16; element
-    // idx = tid + 256 q of the chunk is column idx / GRAM_ROWS, row idx % GRAM_ROWS.  The
-    // values are loaded into registers one chunk ahead, so the loads of the next chunk are
-    // in flight during the products of this one.
-    constexpr int Q = GRAM_ROWS * JCI_MAXBASIS / 256;
-    double rv[Q], rw[Q];
-    auto gload = [&](long long base) {
-        const int rows = (int)((r1 - base) < GRAM_ROWS ? (r1 - base) : GRAM_ROWS);
-#pragma unroll
-        for (int q = 0; q < Q; q++) {
-            const int idx = tid + 256 * q, c = idx / GRAM_ROWS, r = idx % GRAM_ROWS;
-            rv[q] = (idx < GRAM_ROWS * mt * 16 && c < m && r < rows) ? V[(long long)c * ldv + base + r] : 0.0;
-            rw[q] = (idx < GRAM_ROWS * wt * 16 && c < w && r < rows) ? W[(long long)c * ldw + base + r] : 0.0;
-        }
-    };
-    if (r0 < r1) gload(r0);
-    for (long long base = r0; base < r1; base += GRAM_ROWS) {
-#pragma unroll
-        for (int q = 0; q < Q; q++) {
-            const int idx = tid + 256 * q;
-            if (idx < GRAM_ROWS * mt * 16) sV[idx % GRAM_ROWS][idx / GRAM_ROWS] = rv[q];
-            if (idx < GRAM_ROWS * wt * 16) sW[idx % GRAM_ROWS][idx / GRAM_ROWS] = rw[q];
-        }
-        __syncthreads();
-        if (base + GRAM_ROWS < r1) gload(base + GRAM_ROWS);
-        for (int t = 0; t < 4; t++) {
-            int tile = wave + 4 * t;
-            if (tile >= ntile) break;
-            int ti = tile / wt, tj = tile % wt;
-            for (int k0 = 0; k0 < GRAM_ROWS; k0 += 4) {
-                double a = sV[k0 + lane / 16][ti * 16 + lane % 16];
-                double b = sW[k0 + lane / 16][tj * 16 + lane % 16];
-                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[t], 0, 0, 0);
-            }
-        }
-        __syncthreads();
-    }
-    double *out = partial + (long long)blockIdx.x * JCI_MAXBASIS * JCI_MAXBASIS;
-    for (int t = 0; t < 4; t++) {
-        int tile = wave + 4 * t;
-        if (tile >= ntile) break;
-        int ti = tile / wt, tj = tile % wt;
-        for (int v = 0; v < 4; v++) {
-            int i = ti * 16 + lane / 16 + 4 * v, j = tj * 16 + lane % 16;
-            if (i < m && j < w) out[i * JCI_MAXBASIS + j] = acc[t][v];
-        }
-    }
+    __shared__ double red[1024];
+    const long long r0 = (long long)blockIdx.x * chunk, r1 = r0 + chunk < N ? r0 + chunk : N;
+    gram_block<MT, WT>(m, w, V, ldv, W, ldw, r0, r1,
+                       partial + (long long)blockIdx.x * JCI_MAXBASIS * JCI_MAXBASIS, JCI_MAXBASIS, red);
 }
 
 // one wavefront per output element: lanes take the partials b = lane, lane + 64, ... and a
@@ -661,11 +603,11 @@ __global__ void k_gram_reduce(int m, int w, int nblocks, const double *__restric
     if (lane == 0) out[i * w + j] = s;
 }
 
-// reduction work-groups: 2048 rows each (the chunks are walked sequentially, so shorter
-// chunks put more independent loads in flight), at most `cap`
+// reduction work-groups: 512 rows each (a few steps per wave or rows per thread: vectors of
+// 100,000 rows then occupy most of the chip), at most `cap`
 static int reduction_blocks(long long N, int cap)
 {
-    long long b = (N + 2047) / 2048;
+    long long b = (N + 511) / 512;
     if (b > cap) b = cap;
     return (int)(b < 1 ? 1 : b);
 }
@@ -677,39 +619,70 @@ int jk_gram(int m, int w, long long N, const double *V, long long ldv, const dou
         jci_set_error("gram: dimensions out of range");
         return -1;
     }
-    if ((m + 15) / 16 * ((w + 15) / 16) > 16) {
-        jci_set_error("gram: at most 16 output tiles");
-        return -1;
-    }
     nblocks = reduction_blocks(N, nblocks);
     long long chunk = (N + nblocks - 1) / nblocks;
-    chunk = (chunk + GRAM_ROWS - 1) / GRAM_ROWS * GRAM_ROWS;
+    chunk = (chunk + 63) / 64 * 64;                // whole steps of the four waves
     int nb = (int)((N + chunk - 1) / chunk);
     if (nb < 1) nb = 1;
-    hipLaunchKernelGGL(k_gram, dim3(nb), dim3(256), 0, st, m, w, N, V, ldv, W, ldw, partial, chunk);
+    static_assert(JCI_MAXBASIS == 64, "tiles of 16 columns below");
+    const int mt = (m + 15) / 16, wt = (w + 15) / 16;
+#define GRAM_WT(MT)                                                                                  \
+    switch (wt) {                                                                                    \
+    case 1: GRAM_GO(MT, 1);                                                                          \
+    case 2: GRAM_GO(MT, 2);                                                                          \
+    case 3: GRAM_GO(MT, 3);                                                                          \
+    default: GRAM_GO(MT, 4);                                                                         \
+    }                                                                                                \
+    break
+#define GRAM_GO(MT, WT)                                                                              \
+    hipLaunchKernelGGL((k_gram<MT, WT>), dim3(nb), dim3(256), 0, st, m, w, N, V, ldv, W, ldw,        \
+                       partial, chunk);                                                              \
+    break
+    switch (mt) {
+    case 1: GRAM_WT(1);
+    case 2: GRAM_WT(2);
+    case 3: GRAM_WT(3);
+    default: GRAM_WT(4);
+    }
+#undef GRAM_GO
+#undef GRAM_WT
     hipLaunchKernelGGL(k_gram_reduce, dim3(grid_for(m * w, 4)), dim3(256), 0, st, m, w, nb,
                        partial, out_dev);
     LAUNCH_CHECK();
     return 0;
 }
 
-// out_j = beta * out_j + sum_i V_i * Y[i*k + j]   (j < k, i < m)
-__global__ void k_combine(int m, int k, long long N, const double *__restrict__ V, long long ldv,
-                          const double *__restrict__ Y, double *__restrict__ out, long long ldo,
-                          double beta)
+// out_j = beta * out_j + sum_i V_i * Y[i*K + j]   (j < K, i < m), eight vectors' loads at a time
+template <int K>
+__global__ __launch_bounds__(256) void k_combine(int m, long long N, const double *__restrict__ V,
+                                                 long long ldv, const double *__restrict__ Y,
+                                                 double *__restrict__ out, long long ldo, double beta)
 {
-    __shared__ double sY[JCI_MAXBASIS * JCI_MAXK];
-    for (int t = threadIdx.x; t < m * k; t += blockDim.x) sY[t] = Y[t];
+    __shared__ double sY[JCI_MAXBASIS * K];
+    for (int t = threadIdx.x; t < m * K; t += blockDim.x) sY[t] = Y[t];
     __syncthreads();
-    long long n = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long n = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
-    double acc[JCI_MAXK];
-    for (int j = 0; j < k; j++) acc[j] = beta == 0.0 ? 0.0 : beta * out[(long long)j * ldo + n];
-    for (int i = 0; i < m; i++) {
-        double vi = V[(long long)i * ldv + n];
-        for (int j = 0; j < k; j++) acc[j] += vi * sY[i * k + j];
+    double acc[K];
+#pragma unroll
+    for (int j = 0; j < K; j++) acc[j] = beta == 0.0 ? 0.0 : beta * out[(long long)j * ldo + n];
+    int i = 0;
+    for (; i + 8 <= m; i += 8) {
+        double v[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = V[(long long)(i + q) * ldv + n];
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+#pragma unroll
+            for (int j = 0; j < K; j++) acc[j] += v[q] * sY[(i + q) * K + j];
     }
-    for (int j = 0; j < k; j++) out[(long long)j * ldo + n] = acc[j];
+    for (; i < m; i++) {
+        const double v = V[(long long)i * ldv + n];
+#pragma unroll
+        for (int j = 0; j < K; j++) acc[j] += v * sY[i * K + j];
+    }
+#pragma unroll
+    for (int j = 0; j < K; j++) out[(long long)j * ldo + n] = acc[j];
 }
 
 int jk_combine(int m, int k, long long N, const double *V, long long ldv, const double *Y,
@@ -720,8 +693,10 @@ int jk_combine(int m, int k, long long N, const double *V, long long ldv, const 
         jci_set_error("combine: dimensions out of range");
         return -1;
     }
-    hipLaunchKernelGGL(k_combine, dim3(grid_for(N, 256)), dim3(256), 0, st, m, k, N, V, ldv, Y,
-                       out, ldo, beta);
+    with_k(k, [&](auto kc) {
+        hipLaunchKernelGGL((k_combine<decltype(kc)::value>), dim3(grid_for(N, 256)), dim3(256), 0, st, m, N,
+                           V, ldv, Y, out, ldo, beta);
+    });
     LAUNCH_CHECK();
     return 0;
 }
@@ -729,7 +704,8 @@ int jk_combine(int m, int k, long long N, const double *V, long long ldv, const 
 // Residuals and preconditioned corrections for k roots:
 //   R_r = sum_i Y[i*k+r] (S_i - theta_r V_i),  T_r = -R_r / (hd - theta_r),
 // partial[b*k + r] = sum over the block's rows of R_r^2 (fixed-order block reduction).
-__global__ __launch_bounds__(256) void k_residual(int m, int k, long long N,
+template <int K>
+__global__ __launch_bounds__(256) void k_residual(int m, long long N,
                                                   const double *__restrict__ V,
                                                   const double *__restrict__ S, long long ld,
                                                   const double *__restrict__ Y,
@@ -738,51 +714,12 @@ __global__ __launch_bounds__(256) void k_residual(int m, int k, long long N,
                                                   double *__restrict__ T,
                                                   double *__restrict__ partial, long long chunk)
 {
-    __shared__ double sY[JCI_MAXBASIS * JCI_MAXK];
-    __shared__ double sT[JCI_MAXK];
-    __shared__ double red[JCI_MAXK][256];
-    for (int t = threadIdx.x; t < m * k; t += blockDim.x) sY[t] = Y[t];
-    if (threadIdx.x < k) sT[threadIdx.x] = theta[threadIdx.x];
+    __shared__ double sY[JCI_MAXBASIS * K], sT[K], red[4 * K];
+    for (int t = threadIdx.x; t < m * K; t += 256) sY[t] = Y[t];
+    if (threadIdx.x < K) sT[threadIdx.x] = theta[threadIdx.x];
     __syncthreads();
-    double nrm[JCI_MAXK];
-    for (int r = 0; r < k; r++) nrm[r] = 0.0;
-    long long r0 = (long long)blockIdx.x * chunk, r1 = r0 + chunk < N ? r0 + chunk : N;
-    for (long long n = r0 + threadIdx.x; n < r1; n += blockDim.x) {
-        double res[JCI_MAXK];
-        for (int r = 0; r < k; r++) res[r] = 0.0;
-        // four basis vectors per step: their eight loads are issued together
-        int i = 0;
-        for (; i + 4 <= m; i += 4) {
-            double vi[4], si[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                vi[q] = V[(long long)(i + q) * ld + n];
-                si[q] = S[(long long)(i + q) * ld + n];
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                for (int r = 0; r < k; r++) res[r] += sY[(i + q) * k + r] * (si[q] - sT[r] * vi[q]);
-        }
-        for (; i < m; i++) {
-            double vi = V[(long long)i * ld + n], si = S[(long long)i * ld + n];
-            for (int r = 0; r < k; r++) res[r] += sY[i * k + r] * (si - sT[r] * vi);
-        }
-        double h = hd[n];
-        for (int r = 0; r < k; r++) {
-            nrm[r] += res[r] * res[r];
-            double den = h - sT[r];
-            if (fabs(den) < 1e-8) den = den < 0 ? -1e-8 : 1e-8;
-            T[(long long)r * ld + n] = -res[r] / den;
-        }
-    }
-    for (int r = 0; r < k; r++) red[r][threadIdx.x] = nrm[r];
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s)
-            for (int r = 0; r < k; r++) red[r][threadIdx.x] += red[r][threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x < k) partial[(long long)blockIdx.x * JCI_MAXK + threadIdx.x] = red[threadIdx.x][0];
+    const long long r0 = (long long)blockIdx.x * chunk, r1 = r0 + chunk < N ? r0 + chunk : N;
+    residual_block<K>(m, V, S, ld, r0, r1, sY, sT, hd, T, partial + (long long)blockIdx.x * JCI_MAXK, red);
 }
 
 // out[r] = sum_b partial[b*JCI_MAXK + r], one wavefront per r (fixed order)
@@ -808,8 +745,10 @@ int jk_residual(int m, int k, long long N, const double *V, const double *S, lon
     nblocks = reduction_blocks(N, nblocks);
     long long chunk = (N + nblocks - 1) / nblocks;
     int nb = (int)((N + chunk - 1) / chunk);
-    hipLaunchKernelGGL(k_residual, dim3(nb), dim3(256), 0, st, m, k, N, V, S, ld, Y, theta, hd,
-                       T, partial, chunk);
+    with_k(k, [&](auto kc) {
+        hipLaunchKernelGGL((k_residual<decltype(kc)::value>), dim3(nb), dim3(256), 0, st, m, N, V, S, ld, Y,
+                           theta, hd, T, partial, chunk);
+    });
     hipLaunchKernelGGL(k_partial_reduce, dim3(k), dim3(64), 0, st, k, nb, partial, norms_dev);
     LAUNCH_CHECK();
     return 0;
