@@ -37,7 +37,7 @@
 //
 // Against the table kernels (one gather per connected entry, sigma_fast.hip), whole products:
 // MRCI-SD 16e/28o FP64 one vector 304 -> 93 ms, 16e/20o FP64 three vectors 108 -> 54 ms, FP32
-// two vectors 56 -> 22.7 ms, 7a6b/17o two vectors 3.3 -> 1.37 ms, 4a4b/10o 259 -> 56 us; error
+// two vectors 56 -> 22.0 ms, 7a6b/17o two vectors 3.3 -> 1.37 ms, 4a4b/10o 259 -> 56 us; error
 // against 64 bits 2.4e-15 -> 3.3e-16 (FP64) and 1.2e-6 -> 7.9e-8 (FP32) at 16e/20o.
 #pragma once
 #include "jci_internal.h"
@@ -50,8 +50,10 @@
 // column tiles x chunks of one wave's item at most (about): fragments are loaded once per item,
 // and short items let a launch end evenly (8, 64 and no limit were 1 - 4 % slower)
 #define TX_PASSES 32
-#define TX_ROWS64 32         // rows of E a wave holds integral fragments for, FP64 ...
-#define TX_ROWS32 48         // ... and FP32
+// rows of E a wave holds integral fragments for: two row tiles leave three (FP64) or four waves
+// a SIMD.  More rows per scattered tile at two waves: 16e/28o FP64 93 -> 97 ms; 48 at three in
+// FP32, two vectors 16e/20o: 22.0 -> 22.7 ms
+#define TX_ROWS 32
 #define TX_PAD 0x7FF00000u   // list entry of a padded row or column (no position, string 0)
 
 // Order of the vectors' columns.  Inside a block's row the strings of the first spin are kept
@@ -123,8 +125,8 @@ struct TxTask {
 struct TxItem {
     int task, w0, nw, t0, nt;        // external parts, column tiles of the item
     int p0, pn;                      // column tiles of the whole piece (rows of E)
-    int rg[2];                       // row groups (FP64, FP32)
-    long long item0[2];              // first item of the round's launch: (JL, w, row group)
+    int rg;                          // row groups
+    long long item0;                 // first item of the round's launch: (JL, w, row group)
     long long ebase;                 // first element in E
 };
 
@@ -217,7 +219,7 @@ struct TxDev {
 // one launch pair (E, gather) of either part
 struct TxRound {
     int i0, ni, o0, no;              // items and outputs in their tables
-    long long items[2], blocks;      // waves (opposite spin; FP64, FP32) or work-groups; gather
+    long long items, blocks;         // waves (opposite spin) or work-groups (same spin); gather
                                      // work-groups
     long long elems;                 // elements of E
 };

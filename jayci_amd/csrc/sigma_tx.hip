@@ -588,13 +588,13 @@ __global__ __launch_bounds__(256) void k_tx_gss(TxDev A, TxRound R, long long N,
 
 template <typename T> struct TxV;
 template <> struct TxV<double> {
-    static constexpr int VK = 2, PAD = 2, RT = TX_ROWS64 / 16, PREC = 0, EP = 4, WPE = 3;
+    static constexpr int VK = 2, PAD = 2, EP = 4, WPE = 3;
     typedef double2 vec;
     static __device__ __forceinline__ double at(const vec &v, int q) { return q ? v.y : v.x; }
     static __device__ __forceinline__ const double *rows(const TxSpin &s) { return s.m64; }
 };
 template <> struct TxV<float> {
-    static constexpr int VK = 4, PAD = 4, RT = TX_ROWS32 / 16, PREC = 1, EP = 8, WPE = 3;
+    static constexpr int VK = 4, PAD = 4, EP = 4, WPE = 4;
     typedef float4 vec;
     static __device__ __forceinline__ float at(const vec &v, int q)
     {
@@ -652,7 +652,7 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
                                        const T *__restrict__ x, long long ldx, T *__restrict__ Eo,
                                        long long lde, T *__restrict__ Dt)
 {
-    constexpr int RT = TxV<T>::RT, EP = TxV<T>::EP, KC = 4 * KS, LDC = KC + TxV<T>::PAD;
+    constexpr int RT = TX_ROWS / 16, EP = TxV<T>::EP, KC = 4 * KS, LDC = KC + TxV<T>::PAD;
     typedef typename TxV<T>::vec V;
     // the lane and the unit made opaque here: what the reduction depths have in common would
     // otherwise be computed ahead of the switch over them and held in registers all along
@@ -826,8 +826,7 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
             }
             const T *b0 = Dc + part * KS;
             if (u.nrt == 1) tx_mma<T, 1, KS>(acc, a, b0);
-            else if (u.nrt == 2) tx_mma<T, 2, KS>(acc, a, b0);
-            else if (RT > 2) tx_mma<T, RT, KS>(acc, a, b0);
+            else if (u.nrt == 2) tx_mma<T, RT, KS>(acc, a, b0);
             tx_wave_sync();
 #pragma unroll
             for (int i = 0; i < RT; i++)
@@ -849,24 +848,24 @@ __global__ __launch_bounds__(256, TxV<T>::WPE) void k_tx_eab(
     TxDev A, TxRound R, int nvec, int kper, long long N, const T *__restrict__ x0,
     const T *__restrict__ x1, T *__restrict__ E, int ldt)
 {
-    constexpr int RT = TxV<T>::RT, PREC = TxV<T>::PREC;
+    constexpr int RT = TX_ROWS / 16;
     extern __shared__ __align__(16) unsigned char tx_smem2[];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long long u = tx_xcd(blockIdx.x) * 4 + wv;
-    if (u >= R.items[PREC]) return;
+    if (u >= R.items) return;
     T *Dt = (T *)tx_smem2 + (size_t)wv * 16 * ldt;
     const TxItem *__restrict__ items = A.item + R.i0;
     int lo = 0, hi = R.ni - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if (items[mid].item0[PREC] <= u) lo = mid; else hi = mid - 1;
+        if (items[mid].item0 <= u) lo = mid; else hi = mid - 1;
     }
     const TxItem &it = items[lo];
     const TxTask &t = A.task[it.task];
-    int loc = (int)(u - it.item0[PREC]);
+    int loc = (int)(u - it.item0);
     TxUnit n;
-    n.r0 = loc % it.rg[PREC] * RT * 16;
-    loc /= it.rg[PREC];
+    n.r0 = loc % it.rg * RT * 16;
+    loc /= it.rg;
     n.ja = loc / it.nw;
     n.w = it.w0 + loc % it.nw;
     n.k0 = blockIdx.y * kper;
@@ -952,10 +951,10 @@ static int tx_run(int nvec, const TxDev &D, const TxPlan &P, const TxVec &V, T *
     for (const TxRound &R : P.ss) {
         const unsigned rp = (unsigned)(P.rmax + 15) / 16 * 16;
         if ((unsigned long long)V.N * sizeof(T) < (1ULL << 32))
-            hipLaunchKernelGGL((k_tx_ess<T, false>), dim3((unsigned)R.items[0], nvec), dim3(256), rp * 8,
+            hipLaunchKernelGGL((k_tx_ess<T, false>), dim3((unsigned)R.items, nvec), dim3(256), rp * 8,
                                st, D, R, V.N, x0, x1, E);
         else
-            hipLaunchKernelGGL((k_tx_ess<T, true>), dim3((unsigned)R.items[0], nvec), dim3(256), rp * 12,
+            hipLaunchKernelGGL((k_tx_ess<T, true>), dim3((unsigned)R.items, nvec), dim3(256), rp * 12,
                                st, D, R, V.N, x0, x1, E);
         TX_CHECK();
         hipLaunchKernelGGL(k_tx_gss<T>, dim3((unsigned)R.blocks, nvec), dim3(256), 0, st, D, R, V.N, E,
@@ -965,9 +964,9 @@ static int tx_run(int nvec, const TxDev &D, const TxPlan &P, const TxVec &V, T *
     const int ldt = P.ldt + TxV<T>::PAD;
     for (const TxRound &R : P.ab) {
         // the vectors share a wave's fragments where there are waves enough without them
-        const int kper = R.items[TxV<T>::PREC] >= 8192 ? nvec : 1;
+        const int kper = R.items >= 8192 ? nvec : 1;
         hipLaunchKernelGGL(k_tx_eab<T>,
-                           dim3(tx_grid((R.items[TxV<T>::PREC] + 3) / 4), (nvec + kper - 1) / kper),
+                           dim3(tx_grid((R.items + 3) / 4), (nvec + kper - 1) / kper),
                            dim3(256), (unsigned)(64 * ldt * sizeof(T)), st, D, R, nvec, kper, V.N, x0,
                            x1, E, ldt);
         TX_CHECK();

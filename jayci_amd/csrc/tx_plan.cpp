@@ -309,8 +309,7 @@ struct Builder {
             it.nw = nw;
             it.p0 = t0;
             it.pn = nt;
-            const int rows[2] = {TX_ROWS64, TX_ROWS32};
-            for (int p = 0; p < 2; p++) it.rg[p] = (t.La + rows[p] - 1) / rows[p];
+            it.rg = (t.La + TX_ROWS - 1) / TX_ROWS;
             it.ebase = R.elems;
             eb.push_back(R.elems);
             R.elems += (ll)t.na * nw * t.La * nt * 16;
@@ -389,12 +388,11 @@ struct Builder {
                 };
                 std::stable_sort(first, first + R.ni,
                                  [&](const TxItem &a, const TxItem &b) { return cost(a) > cost(b); });
-                for (int i = 0; i < R.ni; i++)
-                    for (int p = 0; p < 2; p++) {
-                        TxItem &a = first[i];
-                        a.item0[p] = R.items[p];
-                        R.items[p] += (ll)P->task[a.task].na * a.nw * a.rg[p];
-                    }
+                for (int i = 0; i < R.ni; i++) {
+                    TxItem &a = first[i];
+                    a.item0 = R.items;
+                    R.items += (ll)P->task[a.task].na * a.nw * a.rg;
+                }
                 P->ab.push_back(R);
                 P->elems = std::max(P->elems, R.elems);
             }
@@ -505,15 +503,14 @@ struct Builder {
             // few pairs: many columns per work-group, for the list and the W tile it sets up
             it.cb = t.R <= 16 ? 16 : t.R <= 32 ? 8 : t.R <= TX_RMAX ? 4 : 1;
             it.ct = (nc + 64 * it.cb - 1) / (64 * it.cb);
-            it.item0 = R.items[0];
-            R.items[0] += (ll)t.n * it.rg * it.ct;
+            it.item0 = R.items;
+            R.items += (ll)t.n * it.rg * it.ct;
             it.ebase = R.elems;
             eb.push_back(R.elems);
             R.elems += (ll)t.n * t.R * ncp;
             P->pitem.push_back(it);
             R.ni++;
         }
-        R.items[1] = R.items[0];
         for (int l = 0; l < L.ngrp; l++) {
             const int blk = O.blkid[l][f];
             if (blk < 0) continue;
