@@ -74,10 +74,10 @@ struct BInst {
 // rewritten only after the event recorded behind its last upload has completed, so the host
 // never waits for the whole stream just to refill a buffer
 #define JB_STAGES 4
+// pinned staging of one launch: the descriptors end where the coefficients begin (desc_area), here
+// and in the device copy, so that both go up together
 struct Stage {
-    BHeader *hH;
-    BDesc *hD;
-    double *hcoef;
+    BDesc *hD;         // desc_cap descriptors, then the coefficients
     hipEvent_t ev;
     int used;
 };
@@ -95,14 +95,14 @@ struct jci_batch {
     int m1max;      // largest orbital-pair count (LDS sizing)
     // device / pinned arenas
     BHeader *dH, *hH;
-    BDesc *dD, *hD;
+    BDesc *dD, *hD;    // of the current launch (desc_area)
+    BDesc *dD0;        // device copy of a staging area
     BSigma *dS, *hS;
     double *dcoef, *hcoef;
     size_t coef_cap;
     Stage stg[JB_STAGES];
     int stg_cur;
     int desc_cap;      // descriptors per launch (dD and every stage's hD)
-    BHeader *hHs;      // header of the current stage
     double *dout, *hout;
     size_t out_cap;
     double *dpartial;
@@ -173,36 +173,37 @@ JCI_API int jci_batch_create(jci_ctx *c, int capacity, int max_norbs, jci_batch 
     b->W = 256;
     b->m1max = max_norbs * (max_norbs + 1) / 2;
     b->use_graphs = 1;
-    JCI_CHECK(hipMalloc(&b->dH, sizeof(BHeader) * 8));
-    JCI_CHECK(hipHostMalloc(&b->hH, sizeof(BHeader) * 8, 0));
+    JCI_CHECK(hipMalloc(&b->dH, sizeof(BHeader)));
+    JCI_CHECK(hipHostMalloc(&b->hH, sizeof(BHeader), 0));
     // descriptors per launch: at most two per instance (V and S rotated together)
     b->desc_cap = 2 * capacity + 8;
-    JCI_CHECK(hipMalloc(&b->dD, sizeof(BDesc) * b->desc_cap));
     JCI_CHECK(hipMalloc(&b->dS, sizeof(BSigma) * capacity * 2));
     JCI_CHECK(hipHostMalloc(&b->hS, sizeof(BSigma) * capacity * 2, 0));
     b->coef_cap = (size_t)capacity * (JCI_MAXBASIS * JCI_MAXBASIS + JCI_MAXK);
-    JCI_CHECK(hipMalloc(&b->dcoef, sizeof(double) * b->coef_cap));
+    const size_t area = sizeof(BDesc) * b->desc_cap + sizeof(double) * b->coef_cap;
+    JCI_CHECK(hipMalloc(&b->dD0, area));
+    b->dcoef = (double *)(b->dD0 + b->desc_cap);
     for (int i = 0; i < JB_STAGES; i++) {
         Stage &g = b->stg[i];
-        JCI_CHECK(hipHostMalloc(&g.hH, sizeof(BHeader) * (1 + JB_NCLASS), 0));
-        JCI_CHECK(hipHostMalloc(&g.hD, sizeof(BDesc) * b->desc_cap, 0));
-        JCI_CHECK(hipHostMalloc(&g.hcoef, sizeof(double) * b->coef_cap, 0));
+        JCI_CHECK(hipHostMalloc(&g.hD, area, 0));
         JCI_CHECK(hipEventCreateWithFlags(&g.ev, hipEventDisableTiming));
         g.used = 0;
     }
     b->stg_cur = 0;
     b->hD = b->stg[0].hD;
-    b->hcoef = b->stg[0].hcoef;
-    b->hHs = b->stg[0].hH;
+    b->dD = b->dD0;
+    b->hcoef = (double *)(b->hD + b->desc_cap);
     b->out_cap = (size_t)capacity * JCI_MAXBASIS * JCI_MAXBASIS;
     JCI_CHECK(hipMalloc(&b->dout, sizeof(double) * b->out_cap));
     JCI_CHECK(hipHostMalloc(&b->hout, sizeof(double) * b->out_cap, 0));
     b->partial_cap = (size_t)1 << 22;
     JCI_CHECK(hipMalloc(&b->dpartial, sizeof(double) * b->partial_cap));
-    JCI_CHECK(hipMalloc(&b->dGH, sizeof(GfHeader)));
-    JCI_CHECK(hipHostMalloc(&b->hGH, sizeof(GfHeader), 0));
-    JCI_CHECK(hipMalloc(&b->dGT, sizeof(GfTask) * capacity));
-    JCI_CHECK(hipHostMalloc(&b->hGT, sizeof(GfTask) * capacity, 0));
+    // header, then (64 bytes on) the tasks: one upload
+    static_assert(sizeof(GfHeader) <= 64, "header before the tasks");
+    JCI_CHECK(hipMalloc(&b->dGH, 64 + sizeof(GfTask) * capacity));
+    JCI_CHECK(hipHostMalloc(&b->hGH, 64 + sizeof(GfTask) * capacity, 0));
+    b->dGT = (GfTask *)((char *)b->dGH + 64);
+    b->hGT = (GfTask *)((char *)b->hGH + 64);
     b->epool = nullptr;
     b->epool_bytes = 0;
     b->epool_want = (size_t)24 << 30;
@@ -280,17 +281,15 @@ JCI_API void jci_batch_destroy(jci_batch *b)
     hipFree(b->gscr);
     for (auto &g : b->graphs) hipGraphExecDestroy(g.exec);
     hipFree(b->dH); hipHostFree(b->hH);
-    hipFree(b->dD);
+    hipFree(b->dD0);
     for (int i = 0; i < JB_STAGES; i++) {
-        hipHostFree(b->stg[i].hH); hipHostFree(b->stg[i].hD); hipHostFree(b->stg[i].hcoef);
+        hipHostFree(b->stg[i].hD);
         hipEventDestroy(b->stg[i].ev);
     }
     hipFree(b->dS); hipHostFree(b->hS);
-    hipFree(b->dcoef);
     hipFree(b->dout); hipHostFree(b->hout);
     hipFree(b->dpartial);
     hipFree(b->dGH); hipHostFree(b->hGH);
-    hipFree(b->dGT); hipHostFree(b->hGT);
     hipFree(b->epool);
     delete b;
 }
@@ -460,8 +459,7 @@ static int stage_next(jci_batch *b)
     if (g.used) JCI_CHECK(hipEventSynchronize(g.ev));
     g.used = 0;
     b->hD = g.hD;
-    b->hcoef = g.hcoef;
-    b->hHs = g.hH;
+    b->hcoef = (double *)(g.hD + b->desc_cap);
     return 0;
 }
 
@@ -474,25 +472,31 @@ static int stage_done(jci_batch *b)
     return 0;
 }
 
-// hslot < 0: descriptors only (the launches read per-class headers, upload_class_headers)
-static int upload_desc(jci_batch *b, int n, long long total, int hslot = 0)
+// hD and dD for the n descriptors of the current area's launch, which end at the coefficients
+static int desc_area(jci_batch *b, int n)
 {
     if (n > b->desc_cap) { jci_set_error("batch: %d descriptors above %d", n, b->desc_cap); return -1; }
-    b->hHs->n = n;
-    b->hHs->total = total;
-    if (hslot >= 0)
-        JCI_CHECK(hipMemcpyAsync(b->dH + hslot, b->hHs, sizeof(BHeader), hipMemcpyHostToDevice,
-                                 b->c->stream));
-    if (n > 0)
-        JCI_CHECK(hipMemcpyAsync(b->dD, b->hD, sizeof(BDesc) * n, hipMemcpyHostToDevice, b->c->stream));
+    b->hD = b->stg[b->stg_cur].hD + (b->desc_cap - n);
+    b->dD = b->dD0 + (b->desc_cap - n);
     return 0;
 }
 
-static int upload_coef(jci_batch *b, size_t len)
+// the n descriptors and `coef` coefficients of the current area
+static int upload_desc(jci_batch *b, int n, size_t coef)
 {
-    if (len) JCI_CHECK(hipMemcpyAsync(b->dcoef, b->hcoef, sizeof(double) * len, hipMemcpyHostToDevice,
-                                      b->c->stream));
+    if (n > 0)
+        JCI_CHECK(hipMemcpyAsync(b->dD, b->hD, sizeof(BDesc) * n + sizeof(double) * coef,
+                                 hipMemcpyHostToDevice, b->c->stream));
     return 0;
+}
+
+static BHeader header(int n, long long total)
+{
+    BHeader h;
+    memset(&h, 0, sizeof(h));
+    h.n = n;
+    h.total = total;
+    return h;
 }
 
 // Basis classes of the combine and Gram kernels: each class launches the instantiation
@@ -513,19 +517,6 @@ static void class_order(const std::vector<int> &cls, std::vector<int> &order, in
             if (cls[t] == c) order.push_back(t);
         cnt[c] = (int)order.size() - first[c];
     }
-}
-
-// one header per class into device slots JB_HCLASS.. (the descriptors go up with upload_desc)
-static int upload_class_headers(jci_batch *b, const int cnt[JB_NCLASS], const long long tot[JB_NCLASS])
-{
-    for (int c = 0; c < JB_NCLASS; c++) {
-        memset(&b->hHs[1 + c], 0, sizeof(BHeader));
-        b->hHs[1 + c].n = cnt[c];
-        b->hHs[1 + c].total = tot[c];
-    }
-    JCI_CHECK(hipMemcpyAsync(b->dH + JB_HCLASS, b->hHs + 1, sizeof(BHeader) * JB_NCLASS,
-                             hipMemcpyHostToDevice, b->c->stream));
-    return 0;
 }
 
 static int download_out(jci_batch *b, size_t len)
@@ -561,6 +552,7 @@ static int run_gram(jci_batch *b, const std::vector<int> &ids, std::vector<doubl
     }
     if (o > b->out_cap) { jci_set_error("batch: scratch too small"); return -1; }
     class_order(cls, order, first, cnt);
+    RCHECK(desc_area(b, n));
     for (int q = 0; q < n; q++) {
         const int t = order[q];
         BInst &s = b->in[ids[t]];
@@ -573,12 +565,11 @@ static int run_gram(jci_batch *b, const std::vector<int> &ids, std::vector<doubl
         pofs += (long long)d.nblk * m[t] * w[t];
     }
     RCHECK(ensure_partial(b, (size_t)pofs));
-    RCHECK(upload_desc(b, n, tot[0] + tot[1] + tot[2] + tot[3], -1));
-    RCHECK(upload_class_headers(b, cnt, tot));
+    RCHECK(upload_desc(b, n, 0));
     RCHECK(stage_done(b));
     for (int c = 0; c < JB_NCLASS; c++)
         if (cnt[c] > 0)
-            RCHECK(jb_gram(b->dH + JB_HCLASS + c, b->dD + first[c], cnt[c], kClassMax[c],
+            RCHECK(jb_gram(header(cnt[c], tot[c]), b->dD + first[c], cnt[c], kClassMax[c],
                            b->dpartial, b->c->stream));
     RCHECK(download_out(b, o));
     return 0;
@@ -606,6 +597,7 @@ static int run_combine(jci_batch *b, const std::vector<int> &ids, const std::vec
         cls[t] = basis_class(m[t]);
     }
     class_order(cls, order, first, cnt);
+    RCHECK(desc_area(b, n));
     for (int q = 0; q < n; q++) {
         const int t = order[q];
         BInst &s = b->in[ids[t]];
@@ -616,12 +608,10 @@ static int run_combine(jci_batch *b, const std::vector<int> &ids, const std::vec
         d.blk0 = tot[cls[t]]; d.nblk = nblk_rows(s.N);
         tot[cls[t]] += d.nblk;
     }
-    RCHECK(upload_coef(b, coef_len));
-    RCHECK(upload_desc(b, n, tot[0] + tot[1] + tot[2] + tot[3], -1));
-    RCHECK(upload_class_headers(b, cnt, tot));
+    RCHECK(upload_desc(b, n, coef_len));
     RCHECK(stage_done(b));
     for (int c = 0; c < JB_NCLASS; c++)
-        if (cnt[c] > 0 && jb_combine(b->dH + JB_HCLASS + c, b->dD + first[c], kClassMax[c],
+        if (cnt[c] > 0 && jb_combine(header(cnt[c], tot[c]), b->dD + first[c], kClassMax[c],
                                      b->c->stream))
             return -1;
     return 0;
@@ -696,8 +686,7 @@ static int run_sigma_gf(jci_batch *b, const std::vector<int> &ids, int prec)
         }
         b->hGH->n = n;
         for (int q = 0; q < 4; q++) b->hGH->total[q] = base[q];
-        JCI_CHECK(hipMemcpyAsync(b->dGH, b->hGH, sizeof(GfHeader), hipMemcpyHostToDevice, c->stream));
-        JCI_CHECK(hipMemcpyAsync(b->dGT, b->hGT, sizeof(GfTask) * n, hipMemcpyHostToDevice, c->stream));
+        JCI_CHECK(hipMemcpyAsync(b->dGH, b->hGH, 64 + sizeof(GfTask) * n, hipMemcpyHostToDevice, c->stream));
         double t0 = tnow();
         if (b->use_graphs) {
             hipGraphExec_t ex = find_graph(b, prec, -1);
@@ -777,6 +766,7 @@ static int run_sigma_tab(jci_batch *b, const std::vector<int> &ids, int prec)
     jci_ctx *c = b->c;
     JCI_CHECK(hipStreamSynchronize(c->stream));
     // pack V columns [sig_first, +cnt) into X (determinant-major), optionally FP32 copy
+    RCHECK(desc_area(b, n));
     long long blk = 0;
     int K = 1;
     for (int t = 0; t < n; t++) {
@@ -789,9 +779,9 @@ static int run_sigma_tab(jci_batch *b, const std::vector<int> &ids, int prec)
         K = std::max(K, s.sig_count);
     }
     if (K > JCI_MAXK) { jci_set_error("batch: more than %d pending sigma vectors", JCI_MAXK); return -1; }
-    RCHECK(upload_desc(b, n, blk, 0));
-    RCHECK(jb_pack(b->dH, b->dD, 1, c->stream));
-    // FP32 copy descriptors (A = X, O = X32) in header slot 1, descriptors after the pack's
+    RCHECK(upload_desc(b, n, 0));
+    RCHECK(jb_pack(header(n, blk), b->dD, 1, c->stream));
+    // FP32 copy descriptors (A = X, O = X32), over the pack's
     long long ntile = 0;
     for (int t = 0; t < n; t++) {
         BInst &s = b->in[ids[t]];
@@ -814,13 +804,12 @@ static int run_sigma_tab(jci_batch *b, const std::vector<int> &ids, int prec)
             d.blk0 = blk2; d.nblk = (int)((s.N * s.sig_count + 255) / 256);
             blk2 += d.nblk;
         }
-        RCHECK(upload_desc(b, n, blk2, 0));
-        RCHECK(jb_to32(b->dH, b->dD, c->stream));
+        RCHECK(upload_desc(b, n, 0));
+        RCHECK(jb_to32(header(n, blk2), b->dD, c->stream));
     }
-    b->hH[1].n = n;
-    b->hH[1].total = ntile;
-    b->hH[1].kmax = K;
-    JCI_CHECK(hipMemcpyAsync(b->dH + 1, b->hH + 1, sizeof(BHeader), hipMemcpyHostToDevice, c->stream));
+    *b->hH = header(n, ntile);
+    b->hH->kmax = K;
+    JCI_CHECK(hipMemcpyAsync(b->dH, b->hH, sizeof(BHeader), hipMemcpyHostToDevice, c->stream));
     JCI_CHECK(hipMemcpyAsync(b->dS, b->hS, sizeof(BSigma) * n, hipMemcpyHostToDevice, c->stream));
     int Kt = K <= 1 ? 1 : (K <= 2 ? 2 : (K <= 4 ? 4 : 8));
     double t0 = tnow();
@@ -830,7 +819,7 @@ static int run_sigma_tab(jci_batch *b, const std::vector<int> &ids, int prec)
             // record the persistent sigma launch once for this (precision, K)
             hipGraph_t g;
             JCI_CHECK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-            int rc = jb_sigma(prec, b->W, Kt, b->dH + 1, b->dS, b->m1max, c->stream);
+            int rc = jb_sigma(prec, b->W, Kt, b->dH, b->dS, b->m1max, c->stream);
             hipError_t e = hipStreamEndCapture(c->stream, &g);
             if (rc) return rc;
             if (e != hipSuccess) { jci_set_error("batch: graph capture failed: %s", hipGetErrorString(e)); return -2; }
@@ -840,7 +829,7 @@ static int run_sigma_tab(jci_batch *b, const std::vector<int> &ids, int prec)
         }
         JCI_CHECK(hipGraphLaunch(ex, c->stream));
     } else {
-        RCHECK(jb_sigma(prec, b->W, Kt, b->dH + 1, b->dS, b->m1max, c->stream));
+        RCHECK(jb_sigma(prec, b->W, Kt, b->dH, b->dS, b->m1max, c->stream));
     }
     JCI_CHECK(hipStreamSynchronize(c->stream));
     b->sigma_seconds += tnow() - t0;
@@ -856,8 +845,8 @@ static int run_sigma_tab(jci_batch *b, const std::vector<int> &ids, int prec)
         if (prec == 64) s.ns64 += s.sig_count; else s.ns32 += s.sig_count;
         s.sig_count = 0;
     }
-    RCHECK(upload_desc(b, n, blk, 0));
-    RCHECK(jb_pack(b->dH, b->dD, 0, c->stream));
+    RCHECK(upload_desc(b, n, 0));
+    RCHECK(jb_pack(header(n, blk), b->dD, 0, c->stream));
     JCI_CHECK(hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -937,6 +926,7 @@ JCI_API int jci_batch_step(jci_batch *b, int *nactive)
     std::vector<size_t> ofs(act.size());
     {
         RCHECK(stage_next(b));
+        RCHECK(desc_area(b, (int)act.size()));
         size_t co = 0, o = 0;
         long long blk = 0, pofs = 0;
         for (size_t t = 0; t < act.size(); t++) {
@@ -956,11 +946,10 @@ JCI_API int jci_batch_step(jci_batch *b, int *nactive)
             blk += d.nblk;
             pofs += (long long)d.nblk * k;
         }
-        RCHECK(upload_coef(b, co));
-        RCHECK(upload_desc(b, (int)act.size(), blk));
+        RCHECK(upload_desc(b, (int)act.size(), co));
         RCHECK(stage_done(b));
         RCHECK(ensure_partial(b, (size_t)pofs));
-        RCHECK(jb_residual(b->dH, b->dD, (int)act.size(), b->dpartial, c->stream));
+        RCHECK(jb_residual(header((int)act.size(), blk), b->dD, (int)act.size(), b->dpartial, c->stream));
         RCHECK(download_out(b, o));
     }
     // 4. decisions per instance

@@ -4,7 +4,8 @@
 #include "sigma_fast.h"
 #include "sigma_gemm.h"
 
-// launch header in device memory: the persistent kernels read their work counts here
+// launch header, the work counts of the persistent kernels: an argument of the vector kernels, in
+// device memory for the sigma
 struct BHeader {
     int n;                 // instances in the descriptor array
     long long total;       // flattened blocks (vector kernels) or tiles (sigma)
@@ -13,7 +14,6 @@ struct BHeader {
 
 #define JB_GRID 2048       // persistent work-groups of the vector kernels
 #define JB_NCLASS 4        // basis classes of the combine and Gram launches (16/32/48/64 vectors)
-#define JB_HCLASS 4        // first device header slot of the class launches (slots 4..7)
 #define JB_SGRID 1024      // persistent work-groups of the sigma kernel
 
 // descriptor of one instance for the batched vector kernels (meaning of the fields per
@@ -44,13 +44,13 @@ struct BSigma {
 
 // all launches use fixed grids; n_cap bounds the instance count (reduction grids)
 // MAXM-sized Gram launch: mmax bounds every descriptor's m and k (<= JCI_MAXBASIS)
-int jb_gram(const BHeader *h, const BDesc *dD, int n_cap, int mmax, double *partial,
+int jb_gram(const BHeader &h, const BDesc *dD, int n_cap, int mmax, double *partial,
             hipStream_t st);
 // mmax: the largest m of the launch's descriptors
-int jb_combine(const BHeader *h, const BDesc *dD, int mmax, hipStream_t st);
-int jb_residual(const BHeader *h, const BDesc *dD, int n_cap, double *partial, hipStream_t st);
-int jb_pack(const BHeader *h, const BDesc *dD, int pack, hipStream_t st);
-int jb_to32(const BHeader *h, const BDesc *dD, hipStream_t st);
+int jb_combine(const BHeader &h, const BDesc *dD, int mmax, hipStream_t st);
+int jb_residual(const BHeader &h, const BDesc *dD, int n_cap, double *partial, hipStream_t st);
+int jb_pack(const BHeader &h, const BDesc *dD, int pack, hipStream_t st);
+int jb_to32(const BHeader &h, const BDesc *dD, hipStream_t st);
 int jb_sigma(int prec, int W, int K, const BHeader *h, const BSigma *dS, int m1max,
              hipStream_t st);
 

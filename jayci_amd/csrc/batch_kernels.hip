@@ -1,7 +1,7 @@
 // Batched Davidson kernels: one launch serves every active CI instance.
 //
-// Each launch reads a header (work counts) and an array of per-instance descriptors
-// (BDesc / BSigma) from device memory.  Work is flattened over instances: instance i
+// Each launch takes a header (work counts; the sigma, which graphs record, reads it from device
+// memory) and reads an array of per-instance descriptors (BDesc / BSigma).  Work is flattened over instances: instance i
 // owns flattened blocks [blk0, blk0 + nblk) and a work-group finds its instance by binary
 // search over blk0.  The kernels are persistent: a fixed grid strides over the
 // flattened blocks, so launch parameters never change between iterations (only the
@@ -37,13 +37,13 @@ __device__ __forceinline__ int find_inst(const BDesc *__restrict__ d, int n, lon
 // The work-group's sum over its rows (gram_block), partial per block.  MT bounds the column
 // tiles of m and k over the launch (checked by the host); most products have one tile of k.
 template <int MT>
-__global__ __launch_bounds__(256) void k_bgram(const BHeader *__restrict__ H,
+__global__ __launch_bounds__(256) void k_bgram(BHeader H,
                                                const BDesc *__restrict__ D,
                                                double *__restrict__ partial)
 {
     __shared__ double red[1024];
-    const int n = H->n;
-    const long long total = H->total;
+    const int n = H.n;
+    const long long total = H.total;
     for (long long blk = blockIdx.x; blk < total; blk += gridDim.x) {
         const BDesc &d = D[find_inst(D, n, blk)];
         const int b = (int)(blk - d.blk0), m = d.m, w = d.k;
@@ -59,10 +59,10 @@ __global__ __launch_bounds__(256) void k_bgram(const BHeader *__restrict__ H,
 // blockIdx.x: instance; blockIdx.y: one of BPS_SPLIT blocks sharing its elements, one
 // element per wave at a time (the order of each element's sum does not depend on the split)
 #define BPS_SPLIT 16
-__global__ void k_bpartial_sum(const BHeader *__restrict__ H, const BDesc *__restrict__ D,
+__global__ void k_bpartial_sum(BHeader H, const BDesc *__restrict__ D,
                                const double *__restrict__ partial)
 {
-    if ((int)blockIdx.x >= H->n) return;
+    if ((int)blockIdx.x >= H.n) return;
     const BDesc &d = D[blockIdx.x];
     int cnt = d.m * d.k, lane = threadIdx.x & 63;
     for (int e = (int)blockIdx.y * 4 + (threadIdx.x >> 6); e < cnt; e += 4 * (int)gridDim.y) {
@@ -73,7 +73,7 @@ __global__ void k_bpartial_sum(const BHeader *__restrict__ H, const BDesc *__res
     }
 }
 
-int jb_gram(const BHeader *h, const BDesc *dD, int n_cap, int mmax, double *partial,
+int jb_gram(const BHeader &h, const BDesc *dD, int n_cap, int mmax, double *partial,
             hipStream_t st)
 {
     if (mmax > JCI_MAXBASIS) return -1;
@@ -98,14 +98,14 @@ int jb_gram(const BHeader *h, const BDesc *dD, int n_cap, int mmax, double *part
 // launch needs.  The coefficients are staged in LDS when the instance changes; every
 // descriptor has k <= m.
 template <int MAXM>
-__global__ __launch_bounds__(256) void k_bcombine(const BHeader *__restrict__ H,
+__global__ __launch_bounds__(256) void k_bcombine(BHeader H,
                                                   const BDesc *__restrict__ D)
 {
     // k <= m <= MAXM (checked by the host); [j][i], zero past m, so that two coefficients come in
     // one read and the sums need no bounds
     __shared__ __align__(16) double sC[MAXM * MAXM];
-    const int n = H->n;
-    const long long total = H->total;
+    const int n = H.n;
+    const long long total = H.total;
     int cur = -1;
     for (long long blk = blockIdx.x; blk < total; blk += gridDim.x) {
         const int inst = find_inst(D, n, blk);
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void k_bcombine(const BHeader *__restrict__ H,
     }
 }
 
-int jb_combine(const BHeader *h, const BDesc *dD, int mmax, hipStream_t st)
+int jb_combine(const BHeader &h, const BDesc *dD, int mmax, hipStream_t st)
 {
     if (mmax > JCI_MAXBASIS) return -1;
     if (mmax <= 16)
@@ -154,13 +154,13 @@ int jb_combine(const BHeader *h, const BDesc *dD, int mmax, hipStream_t st)
 
 // ---- residuals + preconditioned corrections -------------------------------------------------
 // R_r = sum_i C[i*k + r] (B_i - th_r A_i), O_r = -R_r / (hd - th_r); partial norms^2
-__global__ __launch_bounds__(256) void k_bresidual(const BHeader *__restrict__ H,
+__global__ __launch_bounds__(256) void k_bresidual(BHeader H,
                                                    const BDesc *__restrict__ D,
                                                    double *__restrict__ partial)
 {
     __shared__ double sC[JCI_MAXBASIS * JCI_MAXK], sT[JCI_MAXK], red[4 * JCI_MAXK];
-    const int n = H->n;
-    const long long total = H->total;
+    const int n = H.n;
+    const long long total = H.total;
     for (long long blk = blockIdx.x; blk < total; blk += gridDim.x) {
         const BDesc &d = D[find_inst(D, n, blk)];
         const int m = d.m, k = d.k;
@@ -179,10 +179,10 @@ __global__ __launch_bounds__(256) void k_bresidual(const BHeader *__restrict__ H
 }
 
 // sums of k entries per block (norms): out[r] = sum_b partial[b*k + r]
-__global__ void k_bpartial_vec(const BHeader *__restrict__ H, const BDesc *__restrict__ D,
+__global__ void k_bpartial_vec(BHeader H, const BDesc *__restrict__ D,
                                const double *__restrict__ partial)
 {
-    if ((int)blockIdx.x >= H->n) return;
+    if ((int)blockIdx.x >= H.n) return;
     const BDesc &d = D[blockIdx.x];
     const int lane = threadIdx.x & 63;
     // one wave per entry: lanes stride over the blocks, then a fixed shuffle tree
@@ -194,7 +194,7 @@ __global__ void k_bpartial_vec(const BHeader *__restrict__ H, const BDesc *__res
     }
 }
 
-int jb_residual(const BHeader *h, const BDesc *dD, int n_cap, double *partial, hipStream_t st)
+int jb_residual(const BHeader &h, const BDesc *dD, int n_cap, double *partial, hipStream_t st)
 {
     hipLaunchKernelGGL(k_bresidual, dim3(JB_GRID), dim3(256), 0, st, h, dD, partial);
     hipLaunchKernelGGL(k_bpartial_vec, dim3(n_cap), dim3(256), 0, st, h, dD,
@@ -207,11 +207,11 @@ int jb_residual(const BHeader *h, const BDesc *dD, int n_cap, double *partial, h
 // pack:   O[r*k + j] = A[(m + j)*ld + r]     (k columns starting at column m)
 // unpack: O[(m + j)*ld + r] = A[r*k + j]
 template <bool PACK>
-__global__ __launch_bounds__(256) void k_bpack(const BHeader *__restrict__ H,
+__global__ __launch_bounds__(256) void k_bpack(BHeader H,
                                                const BDesc *__restrict__ D)
 {
-    const int n = H->n;
-    const long long total = H->total;
+    const int n = H.n;
+    const long long total = H.total;
     for (long long blk = blockIdx.x; blk < total; blk += gridDim.x) {
         const int inst = find_inst(D, n, blk);
         const BDesc &d = D[inst];
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(256) void k_bpack(const BHeader *__restrict__ H,
     }
 }
 
-int jb_pack(const BHeader *h, const BDesc *dD, int pack, hipStream_t st)
+int jb_pack(const BHeader &h, const BDesc *dD, int pack, hipStream_t st)
 {
     if (pack) hipLaunchKernelGGL(k_bpack<true>, dim3(JB_GRID), dim3(256), 0, st, h, dD);
     else hipLaunchKernelGGL(k_bpack<false>, dim3(JB_GRID), dim3(256), 0, st, h, dD);
@@ -421,11 +421,11 @@ int jb_sigma(int prec, int W, int K, const BHeader *h, const BSigma *dS, int m1m
 
 // FP64 -> FP32 copy of every instance's packed block (N*k entries)
 // (flattened blocks cover N*k entries per instance)
-__global__ __launch_bounds__(256) void k_bto32(const BHeader *__restrict__ H,
+__global__ __launch_bounds__(256) void k_bto32(BHeader H,
                                                const BDesc *__restrict__ D)
 {
-    const int n = H->n;
-    const long long total = H->total;
+    const int n = H.n;
+    const long long total = H.total;
     for (long long blk = blockIdx.x; blk < total; blk += gridDim.x) {
         const int inst = find_inst(D, n, blk);
         const BDesc &d = D[inst];
@@ -434,7 +434,7 @@ __global__ __launch_bounds__(256) void k_bto32(const BHeader *__restrict__ H,
     }
 }
 
-int jb_to32(const BHeader *h, const BDesc *dD, hipStream_t st)
+int jb_to32(const BHeader &h, const BDesc *dD, hipStream_t st)
 {
     hipLaunchKernelGGL(k_bto32, dim3(JB_GRID), dim3(256), 0, st, h, dD);
     BLAUNCH_CHECK();
