@@ -189,7 +189,7 @@ PEAK_MFMA = {64: 78.6, 32: 157.3}   # MI355X dense MFMA peaks, TFLOP/s
 
 
 def roofline_dense(J, ctx, spec, seed):
-    """Dense-string sigma (k_gE + k_gss + k_gga, one vector) on one full-CI instance, FP64
+    """Dense-string sigma (k_gprod + k_gga, one vector) on one full-CI instance, FP64
     and FP32: algorithmic FLOPs 4*P_u + 2*N (two FMAs per unique connected pair, one per
     diagonal element) over the HIP-event time of one sigma.  Beside it, the FLOPs the GEMMs
     issue, 2*La*m1*N (opposite-spin product: La = a(n-a) + 1 rows per alpha string against
@@ -220,7 +220,7 @@ def roofline_dense(J, ctx, spec, seed):
         out[prec] = {"bound": "mfma", "achieved": ach, "peak": PEAK_MFMA[prec],
                      "unit": "TFLOP/s", "frac": ach / PEAK_MFMA[prec],
                      "traffic": traffic.get(prec),
-                     "kernel": "dense-string sigma %s (k_gE + k_gss + k_gga), N=%d (%da%db/%d)"
+                     "kernel": "dense-string sigma %s (k_gprod + k_gga), N=%d (%da%db/%d)"
                                % ("FP64" if prec == 64 else "FP32", N, spec["na"], spec["nb"], n),
                      "ms_per_launch": ms, "algorithmic_flops": flops,
                      "flop_count": "4*P_u + 2*N (P_u unique connected pairs)",
@@ -232,9 +232,9 @@ def roofline_dense(J, ctx, spec, seed):
 
 
 def roofline_table(J, ctx, spec, seed):
-    """Matrix-free table sigma (k_block_transpose, k_sigma_fast and k_sigma_fast_beta
-    launches of one pass, default settings), FP64 and FP32, one vector, on one MRCI-SD
-    instance of the stream.  HBM-bound by its governing definition: the compulsory bytes of
+    """Matrix-free sigma of a truncated space in contraction form (the k_tx launches of one
+    pass, default settings), FP64 and FP32, one vector, on one MRCI-SD instance of the
+    stream.  HBM-bound by its governing definition: the compulsory bytes of
     a pass that cannot materialise its pair list, N*(2*k*b + 8) (vector read, sigma
     written, diagonal read; b bytes per vector element), over the HIP-event time of one
     pass; the connected entries per second (N times the mean connections of 64 sampled
@@ -245,7 +245,7 @@ def roofline_table(J, ctx, spec, seed):
     rows = np.random.default_rng(0).integers(0, N, size=64)
     cbar = float(np.mean([len(c) for c, _, _, _ in h.rows(rows)]))
     traffic = {}
-    tpath = os.path.join(ROOT, "profiles", "sigma_tables_mrcisd_16e20o_traffic.json")
+    tpath = os.path.join(ROOT, "profiles", "sigma_contraction_mrcisd_16e20o_traffic.json")
     if os.path.exists(tpath):
         t = json.load(open(tpath))
         if t.get("ndets") == N:
@@ -257,8 +257,8 @@ def roofline_table(J, ctx, spec, seed):
         ach = byt / (ms * 1e-3) / 1e9
         out[prec] = {"bound": "hbm", "achieved": ach, "peak": PEAK_HBM / 1e9, "unit": "GB/s",
                      "frac": ach * 1e9 / PEAK_HBM, "traffic": traffic.get(prec),
-                     "kernel": "table sigma %s (k_block_transpose + k_sigma_fast + "
-                               "k_sigma_fast_beta), N=%d (MRCI-SD 16e/%do)"
+                     "kernel": "matrix-free sigma %s (k_tx_in/ess/gss/eab/gab/out), N=%d "
+                               "(MRCI-SD 16e/%do)"
                                % ("FP64" if prec == 64 else "FP32", N, spec["norbs"]),
                      "ms_per_launch": ms, "algorithmic_bytes": byt,
                      "byte_count": "N*(2*k*b + 8): vector read, sigma written, diagonal read",
@@ -467,7 +467,7 @@ def bench_mrci(J, ctx, args):
     excitation level 2, MRCI-SD rule: 603,651,972 determinants), synthetic integrals of seed
     1 (n = 60): plain FP64 solve and/or mixed precision (FP32 sigma until the residual is
     below 1e-4, then FP64) of the lowest args.roots roots, residual 1e-6 and |r|^2/gap below
-    1e-9, matrix-free table sigma.  With both precisions the per-root |dE| of the mixed solve
+    1e-9, matrix-free sigma.  With both precisions the per-root |dE| of the mixed solve
     against the FP64 one is reported (the FP64 GPU solve is this configuration's accuracy
     reference).  The sigma kernel's rate is reported as connected entries per second (N
     times the mean connections of 64 sampled rows, per vector) and as compulsory HBM bytes
@@ -488,10 +488,10 @@ def bench_mrci(J, ctx, args):
     from jayci_amd.serve import lane_solve_params
     nr = args.roots
     # the subspace as large as the device's free memory allows (a margin of 6 GiB kept;
-    # the diagonal and the excitation tables, 128 bytes per determinant in the lane's
-    # estimate, are allocated already)
+    # the diagonal and the lists, 32 bytes per determinant in the lane's estimate, are
+    # allocated already)
     free_b, total_b = J.device_memory(ctx.device)
-    kw = lane_solve_params({"nroots": nr}, N, 1e-6, budget=free_b - (6 << 30) + 128 * N,
+    kw = lane_solve_params({"nroots": nr}, N, 1e-6, budget=free_b - (6 << 30) + 32 * N,
                            kfac=args.mrci_kfac)
     nt = kw["nroots"] + kw["nbuffer"]
     log("device memory: %.1f GB free of %.1f GB; krymax %d" % (free_b / 1e9, total_b / 1e9,
@@ -504,7 +504,7 @@ def bench_mrci(J, ctx, args):
             sig["%s_k%d" % (name, k)] = {
                 "ms": ms, "entries_per_s": N * cbar * k / (ms * 1e-3),
                 "compulsory_GBps": N * (2 * k * (8 if name == "fp64" else 4) + 8) / (ms * 1e-3) / 1e9}
-            log("table sigma %s, %d vector(s): %.0f ms" % (name, k, ms))
+            log("matrix-free sigma %s, %d vector(s): %.0f ms" % (name, k, ms))
     precs = {"fp64": [J.PREC_FP64], "mixed": [J.PREC_MIXED],
              "both": [J.PREC_FP64, J.PREC_MIXED]}[args.precision]
     out = {}
@@ -717,11 +717,11 @@ def main():
     mrci = res.pop("_mrci", None)
     table = None
     if mrci is not None:
-        # with the MRCI-SD share the stream's time is the lane's table sigma: it is the
+        # with the MRCI-SD share the stream's time is the lane's sigma: it is the
         # dominant kernel, the dense-string sigma of the full-CI requests is reported beside it
         table = roofline_table(J, ctx, mrci[0], mrci[1])
         roof, roof32 = table[64], table[32]
-        log("table sigma FP64 %.3f ms per pass, %.2f GB/s compulsory (%.5f of HBM peak), "
+        log("matrix-free sigma FP64 %.3f ms per pass, %.2f GB/s compulsory (%.5f of HBM peak), "
             "%.3g entries/s" % (table[64]["ms_per_launch"], table[64]["achieved"],
                                 table[64]["frac"], table[64]["connected_entries_per_s"]))
     cpu = None

@@ -7,7 +7,7 @@ profiler run:
 
 Runs a 1 GiB device copy (the byte counters' calibration), then builds the string tables,
 the diagonal and the per-string excitation tables on the device,
-then applies the table sigma (two passes, per-block tile widths: the defaults) once to K
+then applies the matrix-free sigma (contraction form, the default) once to K
 seeded random vectors resident on the device (one untimed launch first) and prints the
 wall times of each stage; the kernels' own durations are read from the profiler.  Also
 prints the connections per row over a sample of rows (the entries/s figure) and the

@@ -72,10 +72,11 @@ def ndets_of(spec):
 
 def lane_vector_bytes(N, krymax, kb):
     """Device bytes of a lane solve over N determinants: basis and sigma vectors (2 krymax),
-    new directions and the determinant-major sigma input (2 kb), the block-transposed input
-    (kb, FP64) and its FP32 copy (kb), the diagonal, and the excitation tables (bounded by
-    120 bytes per determinant for excitation level 2: 104 at 16e/60o)."""
-    return N * (8 * (2 * krymax + 2 * kb) + 12 * kb + 8 + 120)
+    new directions and the determinant-major sigma input (2 kb), the sigma's reordered inputs
+    and results in both orientations (4 kb, FP64), its intermediate (kb times at most 2 GiB; 60
+    elements per determinant where all of it is less), the diagonal, and the lists of singles
+    and pairs (bounded by 24 bytes per determinant)."""
+    return N * (8 * (2 * krymax + 6 * kb) + 8 + 24) + kb * min(2 << 30, 480 * N)
 
 
 def lane_solve_params(spec, N, restol=1e-6, etol=1e-9, buftol=1e-3, budget=None, kfac=4):
