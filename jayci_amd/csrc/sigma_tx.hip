@@ -220,14 +220,19 @@ int jk_tx_rows(const SpaceDesc *d, const SpaceDesc &h, int spin, const uint64_t 
 
 // ---- vectors in and out ------------------------------------------------------------------------
 
-__device__ __forceinline__ int tx_block(const long long *__restrict__ off, int n, long long t)
+// the last i < n with at(i) <= u (at(0) <= u, ascending), by whole waves: 64 probes a round, one
+// round up to 64 entries, two up to 4096
+template <typename F> __device__ __forceinline__ int tx_find(int n, long long u, F at)
 {
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (off[mid] <= t) lo = mid; else hi = mid - 1;
+    const int l = threadIdx.x & 63;
+    int lo = 0;
+    while (n > 1) {
+        const int st = (n + 63) / 64, i = l * st;
+        const int c = __popcll(__ballot(i < n && at(lo + i) <= u)) - 1;
+        lo += c * st;
+        n = std::min(st, n - c * st);
     }
-    return lo;
+    return __builtin_amdgcn_readfirstlane(lo);
 }
 
 // work-groups in runs of `run` consecutive ones per XCD (they are dealt to the 8 XCDs round
@@ -252,7 +257,7 @@ __device__ __forceinline__ TxTile tx_tile(const SpaceDesc *__restrict__ d,
                                           const long long *__restrict__ tt, long long u)
 {
     TxTile t;
-    t.b = tx_block(tt, d->nblk, u);
+    t.b = tx_find(d->nblk, u, [&](int i) { return tt[i]; });
     const int p = d->bp[t.b], q = d->bq[t.b];
     t.na = d->s[0].gn[p];
     t.nb = d->s[1].gn[q];
@@ -392,14 +397,9 @@ __global__ __launch_bounds__(256, 4) void k_tx_ess(TxDev A, TxRound R, long long
     extern __shared__ __align__(16) unsigned char tx_smem[];
     __shared__ __align__(16) T As[64][TX_WS];
     const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
-    int lo = 0, hi = R.ni - 1;
     const TxPairItem *__restrict__ items = A.pitem + R.i0;
     const long long u = blockIdx.x;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (items[mid].item0 <= u) lo = mid; else hi = mid - 1;
-    }
-    const TxPairItem &it = items[lo];
+    const TxPairItem &it = items[tx_find(R.ni, u, [&](int i) { return items[i].item0; })];
     const TxPairTask &t = A.ptask[it.task];
     const int loc = (int)(u - it.item0), rg = loc % it.rg, ct = loc / it.rg % it.ct;
     const long long K2 = loc / (it.rg * it.ct);
@@ -536,50 +536,76 @@ __global__ __launch_bounds__(256, 4) void k_tx_ess(TxDev A, TxRound R, long long
     store(cb0 * 64 + cl);
 }
 
+// acc plus (or less, where the entry is complemented) E at the n offsets ent, each moved by w
+// times its step, eight loads in flight
+template <typename T>
+__device__ __forceinline__ T tx_sum(T acc, const T *__restrict__ E, const long long *ent, int n,
+                                    const int *step = nullptr, int w = 0)
+{
+    int m = 0;
+    for (; m + 8 <= n; m += 8) {
+        T v[8];
+        long long o[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            o[j] = ent[m + j];
+            v[j] = E[(o[j] ^ (o[j] >> 63)) + (step ? (long long)w * step[m + j] : 0)];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc += o[j] < 0 ? -v[j] : v[j];
+    }
+    // the rest together: entry 0 in place of those past the end, their values unused
+    if (m < n) {
+        T v[8];
+        long long o[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int i = m + j < n ? m + j : 0;
+            o[j] = ent[i];
+            v[j] = E[(o[j] ^ (o[j] >> 63)) + (step ? (long long)w * step[i] : 0)];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (m + j < n) acc += o[j] < 0 ? -v[j] : v[j];
+    }
+    return acc;
+}
+
 // the same-spin sums: y(I, c) = sum over the pairs of I, one E row each (coalesced); the first
-// writer of the result
+// writer of the result.  The rows' offsets are set up in LDS once for the string's columns.
+#define TX_ENT 512
+#define TX_SRC 64            // one wave's scan
 template <typename T>
 __global__ __launch_bounds__(256) void k_tx_gss(TxDev A, TxRound R, long long N,
                                                 const T *__restrict__ E, double *__restrict__ y0,
                                                 double *__restrict__ y1)
 {
-    int lo = 0, hi = R.no - 1;
+    __shared__ long long ent[TX_ENT];
     const TxPairOut *__restrict__ outs = A.pout + R.o0;
     const long long u = blockIdx.x;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (outs[mid].blk0 <= u) lo = mid; else hi = mid - 1;
-    }
-    const TxPairOut &t = outs[lo];
+    const TxPairOut &t = outs[tx_find(R.no, u, [&](int i) { return outs[i].blk0; })];
     const int loc = (int)(u - t.blk0), il = loc / t.cblk;
     const int c = (loc - il * t.cblk) * 256 + threadIdx.x;
-    if (c >= t.nc) return;
     const TxSpin &S = A.s[t.o];
     const int2 *__restrict__ g = S.gl + (long long)(t.ls0 + il) * S.npair;
     const long long k = blockIdx.y;
+    int np = 0;
+    for (int s = 0; s < t.nsec; s++) np += t.np[s];
     T acc = (T)0;
-    for (int s = 0; s < t.nsec; s++) {
-        const T *__restrict__ Es = E + k * R.elems + t.eb[s] + (long long)t.r0[s] * t.ncp + c;
-        const long long st = (long long)t.R[s] * t.ncp;
-        int m = 0;
-        for (; m + 4 <= t.np[s]; m += 4) {
-            T v[4];
-            int2 e[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                e[j] = g[m + j];
-                v[j] = Es[(long long)e[j].x * st + (long long)(e[j].y & 0x7FFFFFFF) * t.ncp];
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++) acc += e[j].y < 0 ? -v[j] : v[j];
+    for (int m0 = 0; m0 < np; m0 += TX_ENT) {
+        const int n = std::min(TX_ENT, np - m0);
+        if (m0) __syncthreads();
+        for (int m = threadIdx.x; m < n; m += 256) {
+            int s = 0, r = m0 + m;
+            while (r >= t.np[s]) r -= t.np[s++];
+            const int2 e = g[m0 + m];
+            const long long o = t.eb[s] + ((long long)e.x * t.R[s] + t.r0[s] + (e.y & 0x7FFFFFFF)) * t.ncp;
+            ent[m] = e.y < 0 ? ~o : o;
         }
-        for (; m < t.np[s]; m++) {
-            const int2 e = g[m];
-            const T v = Es[(long long)e.x * st + (long long)(e.y & 0x7FFFFFFF) * t.ncp];
-            acc += e.y < 0 ? -v : v;
-        }
-        g += t.np[s];
+        __syncthreads();
+        if (c < t.nc) acc = tx_sum(acc, E + k * R.elems + c, ent, n);
     }
+    if (c >= t.nc) return;
     const long long n = t.yb + (long long)il * t.nb + t.c0 + c;
     (t.o ? y1 : y0)[k * N + n] = (double)acc;
 }
@@ -680,41 +706,45 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
         for (int h = 0; h < 2; h++) Q[h] = qt[std::min(l + 64 * h, KC - 1)];
 #pragma unroll
         for (int i = 0; i < RT; i++) {
-            const int r = u.r0 + i * 16 + col;
-            uint32_t row = zero;
-            if (r < La - t.diag) {
-                int s = 0;
-                while (s + 1 < t.nsec && t.sr0[s + 1] <= r) s++;
-                row = (uint32_t)((SL.e1[e0 + go[t.sg[s]] + r - t.sr0[s]].y >> 18) & 4095) * A.ms;
-            } else if (r < La) {
-                row = (uint32_t)(A.m1 + t.iI0 + u.ja / t.nsvL) * A.ms;
-            }
-#pragma unroll
-            for (int g = 0; g < 16; g += 8) {
-                T v[8][2];
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const T *__restrict__ Mr = M + (uint32_t)__builtin_amdgcn_readlane((int)row, g + j);
-#pragma unroll
-                    for (int h = 0; h < (KC > 64 ? 2 : 1); h++) v[j][h] = tx_at(Mr, Q[h]);
+            // (past the last row tile the rows of the one before are read again, and not used:
+            // 20.4 -> 17 us at 4a4b/10o)
+            if (i == 0 || u.nrt > 1) {
+                const int r = u.r0 + i * 16 + col;
+                uint32_t row = zero;
+                if (r < La - t.diag) {
+                    int s = 0;
+                    while (s + 1 < t.nsec && t.sr0[s + 1] <= r) s++;
+                    row = (uint32_t)((SL.e1[e0 + go[t.sg[s]] + r - t.sr0[s]].y >> 18) & 4095) * A.ms;
+                } else if (r < La) {
+                    row = (uint32_t)(A.m1 + t.iI0 + u.ja / t.nsvL) * A.ms;
                 }
 #pragma unroll
-                for (int j = 0; j < 8; j++)
+                for (int g = 0; g < 16; g += 8) {
+                    T v[8][2];
 #pragma unroll
-                    for (int h = 0; h < (KC > 64 ? 2 : 1); h++)
-                        if (l + 64 * h < KC) Dt[(g + j) * LDC + l + 64 * h] = v[j][h];
-            }
-            tx_wave_sync();
-            if (u.dr >> 4 == i && u.dr >= 0) {
-                // the external electrons of JL add to its diagonal row
-                for (uint64_t z = A.nint >= 64 ? 0 : SL.mask[J] >> A.nint << A.nint; z; z &= z - 1) {
-                    const int o = jci_ctz(z);
-                    const T *__restrict__ Mr = M + (uint32_t)jci_tri(o, o) * A.ms;
+                    for (int j = 0; j < 8; j++) {
+                        const T *__restrict__ Mr = M + (uint32_t)__builtin_amdgcn_readlane((int)row, g + j);
 #pragma unroll
-                    for (int h = 0; h < (KC > 64 ? 2 : 1); h++)
-                        if (l + 64 * h < KC) Dt[(u.dr & 15) * LDC + l + 64 * h] += tx_at(Mr, Q[h]);
+                        for (int h = 0; h < (KC > 64 ? 2 : 1); h++) v[j][h] = tx_at(Mr, Q[h]);
+                    }
+#pragma unroll
+                    for (int j = 0; j < 8; j++)
+#pragma unroll
+                        for (int h = 0; h < (KC > 64 ? 2 : 1); h++)
+                            if (l + 64 * h < KC) Dt[(g + j) * LDC + l + 64 * h] = v[j][h];
                 }
                 tx_wave_sync();
+                if (u.dr >> 4 == i && u.dr >= 0) {
+                    // the external electrons of JL add to its diagonal row
+                    for (uint64_t z = A.nint >= 64 ? 0 : SL.mask[J] >> A.nint << A.nint; z; z &= z - 1) {
+                        const int o = jci_ctz(z);
+                        const T *__restrict__ Mr = M + (uint32_t)jci_tri(o, o) * A.ms;
+#pragma unroll
+                        for (int h = 0; h < (KC > 64 ? 2 : 1); h++)
+                            if (l + 64 * h < KC) Dt[(u.dr & 15) * LDC + l + 64 * h] += tx_at(Mr, Q[h]);
+                    }
+                    tx_wave_sync();
+                }
             }
 #pragma unroll
             for (int s = 0; s < KS; s += TxV<T>::VK) {
@@ -855,12 +885,7 @@ __global__ __launch_bounds__(256, TxV<T>::WPE) void k_tx_eab(
     if (u >= R.items) return;
     T *Dt = (T *)tx_smem2 + (size_t)wv * 16 * ldt;
     const TxItem *__restrict__ items = A.item + R.i0;
-    int lo = 0, hi = R.ni - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (items[mid].item0 <= u) lo = mid; else hi = mid - 1;
-    }
-    const TxItem &it = items[lo];
+    const TxItem &it = items[tx_find(R.ni, u, [&](int i) { return items[i].item0; })];
     const TxTask &t = A.task[it.task];
     int loc = (int)(u - it.item0);
     TxUnit n;
@@ -889,57 +914,79 @@ __global__ __launch_bounds__(256, TxV<T>::WPE) void k_tx_eab(
     }
 }
 
-// y(IL, w, column) += sum over the singles of IL that a task covers, one E row each; 256
-// columns of one string per work-group, eight loads in flight per lane
+// y(IL, w, column) += sum over the singles of IL that the round's tasks cover, one E row each;
+// 256 columns of one string per work-group.  The rows' offsets, over all sources, are set up in
+// LDS first: the sum is then one stream of loads, eight in flight per lane, at the copy rate for
+// large spaces, and small ones (chains of list loads before) take 16.2 -> 9.1 us at 4a4b/10o and
+// 0.22 -> 0.19 ms at 7a6b/17o.
 template <typename T>
 __global__ __launch_bounds__(256) void k_tx_gab(TxDev A, TxRound R, long long N,
                                                 const T *__restrict__ E, double *__restrict__ y0,
                                                 double *__restrict__ y1)
 {
-    int lo = 0, hi = R.no - 1;
+    // per source: first of the string's singles, rows before it in the list (its singles, then its
+    // diagonal row); the list's offsets and steps per external part
+    __shared__ int first[TX_SRC], base[TX_SRC + 1];
+    __shared__ long long ent[TX_ENT];
+    __shared__ int step[TX_ENT];
     const TxOut *__restrict__ outs = A.out + R.o0;
     const long long u = blockIdx.x;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (outs[mid].blk0 <= u) lo = mid; else hi = mid - 1;
-    }
-    const TxOut &t = outs[lo];
+    const TxOut &t = outs[tx_find(R.no, u, [&](int i) { return outs[i].blk0; })];
     const int loc = (int)(u - t.blk0), il = loc / t.cblk;
     const int c = (loc - il * t.cblk) * 256 + threadIdx.x, ntc = t.nt * 16;
     const int wi = c / ntc, ci = c - wi * ntc, ib = t.t0 * 16 + ci;
-    if (wi >= t.nw || ib >= t.nI) return;
+    const bool in = wi < t.nw && ib < t.nI;
     const TxSpin &S = A.s[t.o];
     const long long I = t.ls0 + il, k = blockIdx.y;
     const long long e00 = S.off1[I];
     const int *__restrict__ go = S.goff1 + I * (S.G + 1);
     T acc = (T)0;
-    for (int s = 0; s < t.nsrc; s++) {
-        const TxSrc &q = A.src[t.src0 + s];
-        const long long st = (long long)t.nw * q.La * ntc;
-        const T *__restrict__ Es = E + k * R.elems + q.ebase + (long long)wi * q.La * ntc + ci;
-        if (q.r0 >= 0) {
-            long long e = e00 + go[q.l1];
-            const long long e1 = e00 + go[q.l1 + 1];
-            const T *__restrict__ Er = Es + (long long)q.r0 * ntc;
-            for (; e + 8 <= e1; e += 8) {
-                T v[8];
-                int2 en[8];
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    en[j] = S.e1[e + j];
-                    v[j] = Er[(long long)(en[j].x - q.ls0) * st + (long long)S.rk[e + j] * ntc];
-                }
-#pragma unroll
-                for (int j = 0; j < 8; j++) acc += en[j].y & (1 << 12) ? -v[j] : v[j];
+    for (int s0 = 0; s0 < t.nsrc; s0 += TX_SRC) {
+        const int ns = std::min(TX_SRC, t.nsrc - s0);
+        if (s0) __syncthreads();
+        if (threadIdx.x < TX_SRC) {
+            int n = 0;
+            if ((int)threadIdx.x < ns) {
+                const TxSrc &q = A.src[t.src0 + s0 + threadIdx.x];
+                const int g0 = go[q.l1];
+                first[threadIdx.x] = g0;
+                n = (q.r0 >= 0 ? go[q.l1 + 1] - g0 : 0) + (q.diag ? 1 : 0);
             }
-            for (; e < e1; e++) {
-                const int2 en = S.e1[e];
-                const T v = Er[(long long)(en.x - q.ls0) * st + (long long)S.rk[e] * ntc];
-                acc += en.y & (1 << 12) ? -v : v;
+            for (int d = 1; d < 64; d <<= 1) {
+                const int o = __shfl_up(n, d);
+                if ((int)threadIdx.x >= d) n += o;
             }
+            base[threadIdx.x + 1] = n;
+            if (threadIdx.x == 0) base[0] = 0;
         }
-        if (q.diag) acc += Es[(long long)il * st + (long long)(q.La - 1) * ntc];
+        __syncthreads();
+        const int all = base[ns];
+        for (int m0 = 0; m0 < all; m0 += TX_ENT) {
+            const int n = std::min(TX_ENT, all - m0);
+            if (m0) __syncthreads();
+            for (int m = threadIdx.x; m < n; m += 256) {
+                int s = 0;
+                while (base[s + 1] <= m0 + m) s++;
+                const TxSrc &q = A.src[t.src0 + s0 + s];
+                const int i = m0 + m - base[s], rows = q.La * ntc;
+                long long J = il, row = q.La - 1;
+                bool neg = false;
+                if (!q.diag || m0 + m + 1 < base[s + 1]) {
+                    const long long e = e00 + first[s] + i;
+                    const int2 en = S.e1[e];
+                    J = en.x - q.ls0;
+                    row = q.r0 + S.rk[e];
+                    neg = en.y & (1 << 12);
+                }
+                const long long o = q.ebase + J * t.nw * rows + row * ntc;
+                ent[m] = neg ? ~o : o;
+                step[m] = rows;
+            }
+            __syncthreads();
+            if (in) acc = tx_sum(acc, E + k * R.elems + ci, ent, n, step, wi);
+        }
     }
+    if (!in) return;
     const long long n = t.yb + (long long)il * t.nb + (long long)(t.w0 + wi) * t.nI + ib;
     (t.o ? y1 : y0)[k * N + n] += (double)acc;
 }
