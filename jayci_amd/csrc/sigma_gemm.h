@@ -83,8 +83,10 @@ struct GfHeader {
 #define GF_E 2
 #define GF_GA 3
 
-// columns of a unit of the E kernel (autotuned): FP64 16 or 32, FP32 32 or 64
-#define GF_BN64_DEFAULT 32
+// columns of a unit of the E products (autotuned): FP64 16 or 32, FP32 32 or 64.  FP64: 16 spread
+// small spaces over more waves (3a3b in 8 orbitals 10.4 -> 9.4 us) and cost large ones nothing;
+// FP32 units of 16 were slower (4a4b in 12 orbitals 48.3 -> 51.4 us).
+#define GF_BN64_DEFAULT 16
 #define GF_BN32_DEFAULT 32
 // one row of E past full tiles of 16: left to the vector units
 __host__ __device__ inline bool ge_extra(int La) { return La > 1 && (La - 1) % 16 == 0; }

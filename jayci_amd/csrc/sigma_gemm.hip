@@ -480,7 +480,7 @@ __device__ __forceinline__ void gE_span(const GfTask &t, long long r, int Ja, in
     asm volatile("" : "+s"(dofs));
     const int col = l & 15, part = l >> 4;
     extern __shared__ __align__(16) unsigned char gf_smem[];
-    T *Dt = (T *)gf_smem + dofs;                   // two tiles of 16 columns, the extra row of (P|Q)
+    T *Dt = (T *)gf_smem + dofs;                   // two tiles of 16 columns
     const T *xs = (const T *)gf_smem + xo;         // staged row (ST; else gathered from memory)
     const GemmFci &g = t.g;
     const int La = gf_uni(g.La), nb = gf_uni((int)g.nb);
@@ -497,9 +497,15 @@ __device__ __forceinline__ void gE_span(const GfTask &t, long long r, int Ja, in
             for (int q = 0; q < VK; q++) a[i][s * VK + q] = v[q];
         }
     }
+    T ar[EX ? KS : 1];                             // the row past the last tile, at this lane's steps
     if (EX) {
-        const auto row = gptr(drows<T>(g) + (long long)Ja * KC);
-        for (int i = l; i < KC; i += 64) Dt[32 * LDC + i] = row[i];
+        const auto row = gptr(drows<T>(g) + (long long)Ja * KC) + part * KS;
+#pragma unroll
+        for (int s = 0; s < NG; s++) {
+            const V v = *(VP)(row + s * VK);
+#pragma unroll
+            for (int q = 0; q < VK; q++) ar[s * VK + q] = v[q];
+        }
     }
     const auto lb = gptr((const uint32_t *)gf_uni((long long)g.lb));
     const auto xr = gptr((const T *)gf_uni((long long)xg));
@@ -573,19 +579,15 @@ __device__ __forceinline__ void gE_span(const GfTask &t, long long r, int Ja, in
 #pragma unroll
         for (int i = 0; i < RT; i++) acc[i] = Mf<T>::zero();
         d = (T)0;
-        V b[2], y[2];
+        V b[2];
         b[0] = *(const V *)b0;
-        if (EX) y[0] = *(const V *)(Dt + 32 * LDC + part * KS);
         gf_each<0, NM>([&](auto kc) __attribute__((always_inline)) {
             constexpr int k = decltype(kc)::value, i = k % RT, st = k / RT, s = st / VK, q = st % VK;
-            if constexpr (k % (RT * VK) == 0 && s + 1 < NG) {
-                b[(s + 1) & 1] = *(const V *)(b0 + (s + 1) * VK);
-                if (EX) y[(s + 1) & 1] = *(const V *)(Dt + 32 * LDC + part * KS + (s + 1) * VK);
-            }
+            if constexpr (k % (RT * VK) == 0 && s + 1 < NG) b[(s + 1) & 1] = *(const V *)(b0 + (s + 1) * VK);
             acc[i] = Mf<T>::mma(a[i][st], b[s & 1][q], acc[i]);
             gf_each<(k * M + NM - 1) / NM, ((k + 1) * M + NM - 1) / NM>(
                 [&](auto mc) __attribute__((always_inline)) { op(mc, Dn, tile); });
-            if constexpr (EX && i == RT - 1) d += b[s & 1][q] * y[s & 1][q];
+            if constexpr (EX && i == RT - 1) d += b[s & 1][q] * ar[st];
             __builtin_amdgcn_sched_barrier(0);
         });
         if (EX) {
@@ -649,7 +651,8 @@ __device__ __forceinline__ void gE_shape(const GfTask &t, long long r, int Ja, b
 // vectors 3232 -> 1884 us against a work-group per tile with three barriers and a row tile per
 // wave (the fourth wave idle at 46 rows); waves by themselves, two per SIMD and one D tile each,
 // reached 1017 and 2220 us, two D tiles without the dealt-out order 1083 and 2151 us.  4a4b in
-// 12 orbitals (33 rows): 81 -> 45 us.
+// 12 orbitals (33 rows): 81 -> 45 us, and the whole product 70 -> 67 with the 33rd row of (P|Q)
+// in registers instead of LDS.
 template <typename T>
 __device__ __forceinline__ void gf_opposite(const GfHeader *__restrict__ H,
                                             const GfTask *__restrict__ tasks, int bn, int block,
@@ -669,7 +672,7 @@ __device__ __forceinline__ void gf_opposite(const GfHeader *__restrict__ H,
         const int nct = (int)(g.nb + 15) / 16, per = (nct + S - 1) / S;
         const long long base = t.base[GF_E];
         const long long r0 = (u - base) / per;
-        const int dw = (32 + ex) * (g.MP + GeL<T>::PAD);          // one wave's D tiles
+        const int dw = 32 * (g.MP + GeL<T>::PAD);                 // one wave's D tiles
         T *xs = (T *)gf_smem + 4 * dw;
         const int room = (GeL<T>::LDS / (int)sizeof(T) - 4 * dw) / (int)g.nb;
         long long end = std::min(u1, ti + 1 < n ? tasks[ti + 1].base[GF_E] : total);
