@@ -162,6 +162,8 @@ struct TxPairTask {
     long long lbase;                 // list base of the group
     int Rfull, n, nb;
 };
+#define TX_RSMALL 32         // pairs up to which a work-group has two row tiles, in rounds of at
+#define TX_SMALL_GROUPS 4096 // least so many such work-groups (fewer are not worth a launch)
 #define TX_RMAX 64           // pairs up to which a work-group keeps all of W in LDS
 struct TxPairItem {
     int task, c0, nc, ncp;           // columns of the round, padded to 16
@@ -219,6 +221,8 @@ struct TxDev {
 // one launch pair (E, gather) of either part
 struct TxRound {
     int i0, ni, o0, no;              // items and outputs in their tables
+    int nsmall;                      // same spin: first items, strings of up to TX_RSMALL pairs
+    long long small;                 // their work-groups
     long long items, blocks;         // waves (opposite spin) or work-groups (same spin); gather
                                      // work-groups
     long long elems;                 // elements of E

@@ -387,19 +387,23 @@ template <> __device__ __forceinline__ const float *tx_w<float>(const TxSpin &s)
 // list is padded to whole steps by the zero row of W.  Offsets are 32 bits while the vector is
 // below 4 GB (BIG: 64).  Bound by the E traffic: 16e/28o FP64 writes 32 GB in 19.7 ms (one
 // 64-column block per work-group: 23.1 ms).
-#define TX_WS (TX_RMAX + 4)          // row stride of the W tile: 16-byte reads, rows spread over the banks
-template <typename T, bool BIG>
-__global__ __launch_bounds__(256, 4) void k_tx_ess(TxDev A, TxRound R, long long N,
+// RT: row tiles of a work-group, 4, or 2 for strings of up to 32 pairs, whose work-groups are the
+// most and the shortest: with half the registers and a quarter of the LDS seven fit on a CU
+// instead of four (7a6b/17o two vectors 1.33 -> 1.28 ms, 16e/20o FP64 three 53.3 -> 51.8, 16e/28o
+// one 92.2 -> 90.0).
+template <typename T, bool BIG, int RT>
+__global__ __launch_bounds__(256, RT == 2 ? 6 : 4) void k_tx_ess(TxDev A, TxRound R, int i0, int ni, long long N,
                                                    const T *__restrict__ x0, const T *__restrict__ x1,
                                                    T *__restrict__ E)
 {
     typedef typename std::conditional<BIG, long long, uint32_t>::type O;
     extern __shared__ __align__(16) unsigned char tx_smem[];
-    __shared__ __align__(16) T As[64][TX_WS];
+    // row stride: 16-byte reads, rows spread over the banks
+    __shared__ __align__(16) T As[RT * 16][RT * 16 + 4];
     const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
-    const TxPairItem *__restrict__ items = A.pitem + R.i0;
+    const TxPairItem *__restrict__ items = A.pitem + i0;
     const long long u = blockIdx.x;
-    const TxPairItem &it = items[tx_find(R.ni, u, [&](int i) { return items[i].item0; })];
+    const TxPairItem &it = items[tx_find(ni, u, [&](int i) { return items[i].item0; })];
     const TxPairTask &t = A.ptask[it.task];
     const int loc = (int)(u - it.item0), rg = loc % it.rg, ct = loc / it.rg % it.ct;
     const long long K2 = loc / (it.rg * it.ct);
@@ -427,22 +431,22 @@ __global__ __launch_bounds__(256, 4) void k_tx_ess(TxDev A, TxRound R, long long
     const T *__restrict__ W = tx_w<T>(S);
     // W tile: rows ar + 16 j, column ak (16 mostly consecutive columns of four rows a load)
     const int ar = tid >> 4, ak = tid & 15, kk = l >> 4;
-    const int nrt = (std::min(64, Rr - r0) + 15) / 16;
-    uint32_t wrow[4];
+    const int nrt = (std::min(RT * 16, Rr - r0) + 15) / 16;
+    uint32_t wrow[RT];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < RT; j++) {
         const int r = r0 + ar + 16 * j;
         wrow[j] = (uint32_t)(r < Rp ? pr[r] & 0x7FFFFFFF : np) * ws;
     }
     const T *__restrict__ x = (t.o ? x1 : x0) + k * N + it.c0;
     T *__restrict__ Ek = E + k * R.elems + it.ebase + (K2 * Rr + r0) * ncp;
     const int cb0 = ct * it.cb, cb1 = std::min(cb0 + it.cb, (nc + 63) / 64);
-    T ra[4], rb[4];
-    typename Mf<T>::acc acc[4];
+    T ra[RT], rb[4];
+    typename Mf<T>::acc acc[RT];
     auto load_w = [&](int k0) __attribute__((always_inline)) {
         const int p = pr[k0 + ak];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < RT; j++)
             if (j < nrt) {
                 const T v = tx_at(W, wrow[j] + (uint32_t)(p & 0x7FFFFFFF));
                 ra[j] = p < 0 ? -v : v;
@@ -460,7 +464,7 @@ __global__ __launch_bounds__(256, 4) void k_tx_ess(TxDev A, TxRound R, long long
     auto store = [&](int c) __attribute__((always_inline)) {
         if (c >= ncp) return;
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < RT; i++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int r = i * 16 + Mf<T>::row(l, v);
@@ -468,18 +472,18 @@ __global__ __launch_bounds__(256, 4) void k_tx_ess(TxDev A, TxRound R, long long
             }
     };
     const int cl = w * 16 + (l & 15);
-    if (Rp <= TX_RMAX) {
+    if (RT == 2 || Rp <= TX_RMAX) {
         for (int k0 = 0; k0 < Rp; k0 += 16) {
             load_w(k0);
 #pragma unroll
-            for (int j = 0; j < 4; j++) if (j < nrt) As[ar + 16 * j][k0 + ak] = ra[j];
+            for (int j = 0; j < RT; j++) if (j < nrt) As[ar + 16 * j][k0 + ak] = ra[j];
         }
         __syncthreads();
         for (int cb = cb0; cb < cb1; cb++) {
             if (cb * 64 + w * 16 >= nc) break;
             const uint32_t xc = (uint32_t)std::min(cb * 64 + cl, nc - 1);
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc[i] = Mf<T>::zero();
+            for (int i = 0; i < RT; i++) acc[i] = Mf<T>::zero();
             load_x(0, xc);
             for (int k0 = 0; k0 < Rp; k0 += 16) {
                 T b[4];
@@ -487,7 +491,7 @@ __global__ __launch_bounds__(256, 4) void k_tx_ess(TxDev A, TxRound R, long long
                 for (int j = 0; j < 4; j++) b[j] = rb[j];
                 if (k0 + 16 < Rp) load_x(k0 + 16, xc);
 #pragma unroll
-                for (int i = 0; i < 4; i++)
+                for (int i = 0; i < RT; i++)
                     if (i < nrt) {
                         T a[4];
                         tx_load4(a, &As[i * 16 + (l & 15)][k0 + kk * 4]);
@@ -502,11 +506,11 @@ __global__ __launch_bounds__(256, 4) void k_tx_ess(TxDev A, TxRound R, long long
     // two 16-deep W tiles side by side in As, columns 0 .. 15 and 32 .. 47
     const uint32_t xc = (uint32_t)std::min(cb0 * 64 + cl, nc - 1);
 #pragma unroll
-    for (int i = 0; i < 4; i++) acc[i] = Mf<T>::zero();
+    for (int i = 0; i < RT; i++) acc[i] = Mf<T>::zero();
     load_w(0);
     load_x(0, xc);
 #pragma unroll
-    for (int j = 0; j < 4; j++) if (j < nrt) As[ar + 16 * j][ak] = ra[j];
+    for (int j = 0; j < RT; j++) if (j < nrt) As[ar + 16 * j][ak] = ra[j];
     __syncthreads();
     int buf = 0;
     for (int k0 = 0; k0 < Rp; k0 += 16) {
@@ -519,7 +523,7 @@ __global__ __launch_bounds__(256, 4) void k_tx_ess(TxDev A, TxRound R, long long
             load_x(k0 + 16, xc);
         }
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < RT; i++)
             if (i < nrt) {
                 T a[4];
                 tx_load4(a, &As[i * 16 + (l & 15)][buf + kk * 4]);
@@ -529,7 +533,7 @@ __global__ __launch_bounds__(256, 4) void k_tx_ess(TxDev A, TxRound R, long long
         buf ^= 32;
         if (more) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) if (j < nrt) As[ar + 16 * j][buf + ak] = ra[j];
+            for (int j = 0; j < RT; j++) if (j < nrt) As[ar + 16 * j][buf + ak] = ra[j];
         }
         __syncthreads();
     }
@@ -997,13 +1001,21 @@ static int tx_run(int nvec, const TxDev &D, const TxPlan &P, const TxVec &V, T *
     const T *x0 = (const T *)V.x0, *x1 = (const T *)V.x1;
     for (const TxRound &R : P.ss) {
         const unsigned rp = (unsigned)(P.rmax + 15) / 16 * 16;
-        if ((unsigned long long)V.N * sizeof(T) < (1ULL << 32))
-            hipLaunchKernelGGL((k_tx_ess<T, false>), dim3((unsigned)R.items, nvec), dim3(256), rp * 8,
-                               st, D, R, V.N, x0, x1, E);
-        else
-            hipLaunchKernelGGL((k_tx_ess<T, true>), dim3((unsigned)R.items, nvec), dim3(256), rp * 12,
-                               st, D, R, V.N, x0, x1, E);
-        TX_CHECK();
+        const bool big = (unsigned long long)V.N * sizeof(T) >= (1ULL << 32);
+        if (R.nsmall) {
+            const dim3 g((unsigned)R.small, nvec);
+            const unsigned rs = TX_RSMALL;
+            if (big) hipLaunchKernelGGL((k_tx_ess<T, true, 2>), g, dim3(256), rs * 12, st, D, R, R.i0, R.nsmall, V.N, x0, x1, E);
+            else hipLaunchKernelGGL((k_tx_ess<T, false, 2>), g, dim3(256), rs * 8, st, D, R, R.i0, R.nsmall, V.N, x0, x1, E);
+            TX_CHECK();
+        }
+        if (R.ni > R.nsmall) {
+            const dim3 g((unsigned)R.items, nvec);
+            const int i0 = R.i0 + R.nsmall, ni = R.ni - R.nsmall;
+            if (big) hipLaunchKernelGGL((k_tx_ess<T, true, 4>), g, dim3(256), rp * 12, st, D, R, i0, ni, V.N, x0, x1, E);
+            else hipLaunchKernelGGL((k_tx_ess<T, false, 4>), g, dim3(256), rp * 8, st, D, R, i0, ni, V.N, x0, x1, E);
+            TX_CHECK();
+        }
         hipLaunchKernelGGL(k_tx_gss<T>, dim3((unsigned)R.blocks, nvec), dim3(256), 0, st, D, R, V.N, E,
                            V.y0, V.y1);
         TX_CHECK();

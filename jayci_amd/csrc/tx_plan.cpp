@@ -564,6 +564,24 @@ struct Builder {
         };
         auto close = [&]() {
             if (R.ni) {
+                // strings of few pairs first, in a launch of their own where they fill one
+                auto groups = [&](const TxPairItem &it) { return (ll)P->ptask[it.task].n * it.rg * it.ct; };
+                auto few = [&](const TxPairItem &it) { return P->ptask[it.task].R <= TX_RSMALL; };
+                const auto first = P->pitem.begin() + R.i0, end = P->pitem.end();
+                ll small = 0;
+                for (auto it = first; it != end; ++it) if (few(*it)) small += groups(*it);
+                if (small >= TX_SMALL_GROUPS) {
+                    R.nsmall = (int)(std::stable_partition(first, end, few) - first);
+                    R.small = small;
+                    R.items -= small;
+                    ll at[2] = {0, 0};
+                    for (int q = 0; q < R.ni; q++) {
+                        TxPairItem &it = first[q];
+                        ll &p = at[q >= R.nsmall];
+                        it.item0 = p;
+                        p += groups(it);
+                    }
+                }
                 P->ss.push_back(R);
                 P->elems = std::max(P->elems, R.elems);
             }
