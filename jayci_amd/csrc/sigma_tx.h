@@ -36,8 +36,8 @@
 // diagonal pairs together.
 //
 // Against the table kernels (one gather per connected entry, sigma_fast.hip), whole products:
-// MRCI-SD 16e/28o FP64 one vector 304 -> 92 ms, 16e/20o FP64 three vectors 108 -> 53 ms, FP32
-// two vectors 56 -> 21 ms, 7a6b/17o two vectors 3.3 -> 1.33 ms, 4a4b/10o 259 -> 44 us; error
+// MRCI-SD 16e/28o FP64 one vector 304 -> 90 ms, 16e/20o FP64 three vectors 108 -> 52 ms, FP32
+// two vectors 56 -> 21 ms, 7a6b/17o two vectors 3.3 -> 1.28 ms, 4a4b/10o 259 -> 44 us; error
 // against 64 bits 2.4e-15 -> 3.3e-16 (FP64) and 1.2e-6 -> 7.9e-8 (FP32) at 16e/20o.
 #pragma once
 #include "jci_internal.h"

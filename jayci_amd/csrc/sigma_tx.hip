@@ -385,7 +385,7 @@ template <> __device__ __forceinline__ const float *tx_w<float>(const TxSpin &s)
 // others stage W one 16-deep step ahead.  In a step lane group g takes the pairs
 // 4 g .. 4 g + 3, so that its four W entries of a row are one or two 16-byte reads.  The pair
 // list is padded to whole steps by the zero row of W.  Offsets are 32 bits while the vector is
-// below 4 GB (BIG: 64).  Bound by the E traffic: 16e/28o FP64 writes 32 GB in 19.7 ms (one
+// below 4 GB (BIG: 64).  16e/28o FP64 writes 31 GB in 17.6 ms (one
 // 64-column block per work-group: 23.1 ms).
 // RT: row tiles of a work-group, 4, or 2 for strings of up to 32 pairs, whose work-groups are the
 // most and the shortest: with half the registers and a quarter of the LDS seven fit on a CU
