@@ -91,21 +91,22 @@ struct GfHeader {
 // one row of E past full tiles of 16: left to the vector units
 __host__ __device__ inline bool ge_extra(int La) { return La > 1 && (La - 1) % 16 == 0; }
 // Tile edge of the same-spin product of K vectors: the one whose whole waves of work-groups on
-// 256 CUs take least.  A 32 x 32 tile reads twice as much per product as the larger ones.
+// 256 CUs take least.  A 32 x 32 tile reads twice as much per product as the larger ones.  A tile
+// of 128 sums each reduction whole, the smaller ones in four quarters: whether to take 128 is
+// decided for one vector, so that a vector's sums do not depend on how many go with it (several
+// vectors at 128 gain nothing on four times as many tiles of 64, which is what they are compared
+// with); 64 and 32 add up alike, and the count chooses between them.
+__host__ __device__ inline double gs_cost(long long na, long long nb, int K, int e)
+{
+    const long long tiles = (long long)K * ((na + e - 1) / e) * ((nb + e - 1) / e);
+    return (double)((tiles + 255) / 256) * e * e * (e == 32 ? 1.4 : 1.0);
+}
 __host__ __device__ inline int gs_edge(long long na, long long nb, int K)
 {
     if (na < 4 || nb < 4) return 32;
-    int best = 32;
-    double cost = 1e300;
-    for (int e = 128; e >= 32; e >>= 1) {
-        const long long tiles = (long long)K * ((na + e - 1) / e) * ((nb + e - 1) / e);
-        const double c = (double)((tiles + 255) / 256) * e * e * (e == 32 ? 1.4 : 1.0);
-        if (c < cost) {
-            cost = c;
-            best = e;
-        }
-    }
-    return best;
+    const double whole = gs_cost(na, nb, 1, 128);
+    if (whole <= gs_cost(na, nb, 1, 64) && whole <= gs_cost(na, nb, 1, 32)) return 128;
+    return gs_cost(na, nb, K, 64) <= gs_cost(na, nb, K, 32) ? 64 : 32;
 }
 // pitch of the beta lists: 16-byte reads of four lanes, all alike, for the longest list
 // b (n - b + 1) of the orbital counts n that share MP

@@ -334,7 +334,8 @@ __device__ __forceinline__ void gs_small(const GfTask &t, const T *X, double *y,
 
 // Same-spin parts: y_k = Haa X_k + X_k Hbb on tiles (k, alpha rows, beta columns) of the edge
 // that gs_edge chooses.  128: four waves of 64 x 64 each over both reductions whole; 64 and 32:
-// the four waves share the reductions of one tile.
+// the four waves share the reductions of one tile, in the same four ranges, so that the two give
+// the same sums to the last bit.
 //
 // Bound by the matrix cores (FP64 88 % busy, FP32 73 % at 1.8 GHz).  Operands straight from
 // memory: a 16-deep step of a 64 x 64 tile is 16 (FP64) or 8 wide loads for 64 products, which
