@@ -384,7 +384,8 @@ template <> __device__ __forceinline__ const float *tx_w<float>(const TxSpin &s)
 // keep their whole W block in LDS for several column blocks, without barriers in between; the
 // others stage W one 16-deep step ahead.  In a step lane group g takes the pairs
 // 4 g .. 4 g + 3, so that its four W entries of a row are one or two 16-byte reads.  The pair
-// list is padded to whole steps by the zero row of W.  Offsets are 32 bits while the vector is
+// list is padded to whole steps by the zero row of W and by zeros in place of the vector's rows
+// (an infinite element would make NaN of the padding).  Offsets are 32 bits while the vector is
 // below 4 GB (BIG: 64).  16e/28o FP64 writes 31 GB in 17.6 ms (one
 // 64-column block per work-group: 23.1 ms).
 // RT: row tiles of a work-group, 4, or 2 for strings of up to 32 pairs, whose work-groups are the
@@ -461,6 +462,15 @@ __global__ __launch_bounds__(256, RT == 2 ? 6 : 4) void k_tx_ess(TxDev A, TxRoun
             rb[j] = BIG ? x[(long long)o + xc] : tx_at(x, (uint32_t)o + xc);
         }
     };
+    // the vector's operands of step k0
+    auto take = [&](int k0, T *b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) b[j] = rb[j];
+        if (k0 + 16 > Rr) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) if (k0 + kk * 4 + j >= Rr) b[j] = (T)0;
+        }
+    };
     auto store = [&](int c) __attribute__((always_inline)) {
         if (c >= ncp) return;
 #pragma unroll
@@ -487,8 +497,7 @@ __global__ __launch_bounds__(256, RT == 2 ? 6 : 4) void k_tx_ess(TxDev A, TxRoun
             load_x(0, xc);
             for (int k0 = 0; k0 < Rp; k0 += 16) {
                 T b[4];
-#pragma unroll
-                for (int j = 0; j < 4; j++) b[j] = rb[j];
+                take(k0, b);
                 if (k0 + 16 < Rp) load_x(k0 + 16, xc);
 #pragma unroll
                 for (int i = 0; i < RT; i++)
@@ -515,8 +524,7 @@ __global__ __launch_bounds__(256, RT == 2 ? 6 : 4) void k_tx_ess(TxDev A, TxRoun
     int buf = 0;
     for (int k0 = 0; k0 < Rp; k0 += 16) {
         T b[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) b[j] = rb[j];
+        take(k0, b);
         const bool more = k0 + 16 < Rp;
         if (more) {
             load_w(k0 + 16);
