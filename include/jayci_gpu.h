@@ -252,7 +252,8 @@ int jci_sigma(jci_ham *h, int method, int nvec, const double *x, double *y);
  * runs its vectors in as many passes as the array allows, one vector of up to about
  * 128 MiB / (8 La) determinants in FP64).  All calls on one GPU share the array, so calls
  * that overlap on one GPU race; results equal jci_sigma_dev's bit for bit.  (Truncated spaces
- * that this size admits keep one vector's buffers with the Hamiltonian besides.) */
+ * that this size admits hold buffers of their own for this from creation on; no other call moves
+ * or frees them but jci_ham_contraction with another *elems and jci_ham_destroy.) */
 int jci_sigma_dev_noalloc(jci_ham *h, int method, int nvec, const double *x_dev, double *y_dev);
 long long jci_sigma_noalloc_capacity(void);
 
@@ -360,6 +361,16 @@ int jci_ham_fast_split(jci_ham *h, int *split);
  * vector rows over the same columns); 0: the chunks of one string are consecutive.  -1
  * keeps; the values in use are returned */
 int jci_ham_fast_xcd(jci_ham *h, int *group, int *chunk_major);
+/* the two forms of the FAST methods on truncated spaces.  *use 1: products over the strings'
+ * replacements (the default where the space has that form), 0: the table kernels, as the three
+ * shapes above choose them; *elems > 0: that form in rounds of at most that many elements of its
+ * intermediate per vector, or of one string's where that is more (default 256M; plans anew and
+ * moves the buffers, so not while a captured graph uses them); *bytes > 0: bound on the block that
+ * calls of several vectors grow (beyond it, or where device memory ends, they go in passes).
+ * Other values keep.  Returned: the form in use, the elements of the largest round, the bytes
+ * of the buffers held, and the numbers of opposite-spin and same-spin rounds (0 without the form;
+ * any pointer may be NULL) */
+int jci_ham_contraction(jci_ham *h, int *use, long long *elems, long long *bytes, int rounds[2]);
 /* column-tile widths of the dense-string sigma's opposite-spin product (FP64: 16 or 32,
  * FP32: 32 or 64; the autotuner sets them): a positive *bn sets, then both are returned */
 int jci_ham_gemm_tiles(jci_ham *h, int *bn64, int *bn32);

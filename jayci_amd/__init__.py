@@ -95,6 +95,7 @@ _sig("jci_ham_fast_width", _i, [_P])
 _sig("jci_ham_fast_tiles", _i, [_P, ctypes.POINTER(_i), ctypes.POINTER(_i)])
 _sig("jci_ham_fast_split", _i, [_P, ctypes.POINTER(_i)])
 _sig("jci_ham_fast_xcd", _i, [_P, ctypes.POINTER(_i), ctypes.POINTER(_i)])
+_sig("jci_ham_contraction", _i, [_P, ctypes.POINTER(_i), ctypes.POINTER(_ll), ctypes.POINTER(_ll), _P])
 _sig("jci_batch_create", _i, [_P, _i, _i, ctypes.POINTER(_P)])
 _sig("jci_batch_destroy", None, [_P])
 _sig("jci_batch_set_graphs", _i, [_P, _i])
@@ -406,6 +407,15 @@ class Hamiltonian:
         v, c = _i(group), _i(chunk_major)
         _check(_L.jci_ham_fast_xcd(self._h, ctypes.byref(v), ctypes.byref(c)), "jci_ham_fast_xcd")
         return v.value, c.value
+
+    def contraction(self, use=-1, elems=0, nbytes=0):
+        """Form of the FAST methods on truncated spaces (jci_ham_contraction): use 1 / 0 chooses
+        the products over replacements / the table kernels, elems > 0 the largest round, nbytes >
+        0 the bound on grown buffers.  Returns (use, elems, bytes held, (rounds, rounds))."""
+        u, e, b, r = _i(use), _ll(elems), _ll(nbytes), (_i * 2)()
+        _check(_L.jci_ham_contraction(self._h, ctypes.byref(u), ctypes.byref(e), ctypes.byref(b), r),
+               "jci_ham_contraction")
+        return u.value, e.value, b.value, tuple(r)
 
     def gemm_tiles(self, bn64=0, bn32=0):
         """E tile widths of the dense-string sigma; positive arguments set them."""

@@ -308,8 +308,12 @@ struct jci_ham {
     void *tx_mem[24];           // device arrays behind txd
     int tx_nmem;
     long long *d_ttx, nttx;     // 16 x 16 transpose tiles per block
-    void *d_txE, *d_txx, *d_txy;
-    size_t txE_bytes, txx_bytes, txy_bytes;
+    // its buffers: one block from creation on that never moves (for the allocation-free entry
+    // point), and one that calls of more vectors grow, up to tx_cap bytes
+    void *d_txkeep, *d_txmore;
+    size_t txkeep_bytes, txmore_bytes, tx_cap;
+    long long tx_elems;         // bound on the intermediate of a round, elements per vector
+    void *d_txtab;              // the plan's tables
     int have_tables;            // doubles tables and launch maps of the table kernels built
     int have_fci;               // single-block space with n <= 16: FCI kernel usable
     FciArgs fci;
@@ -601,27 +605,100 @@ static void free_doubles(jci_ham *h)
     }
 }
 
-// vectors up to this many determinants keep one vector's buffers of the contraction form from
-// the start, for the allocation-free entry point (its own staging bounds the larger ones out)
+// Hamiltonians of up to this many determinants hold buffers of the contraction form from creation
+// on, for the allocation-free entry point (its own staging bounds the larger ones out): of one
+// vector, and of as many more as TX_KEEP_BYTES have room for, so that the first product of several
+// vectors of a small space allocates nothing
 #define TX_NOALLOC_DETS (16LL << 20)
+#define TX_KEEP_BYTES ((size_t)64 << 20)
 // elements of the intermediate per vector and round: 256M (2 GB in FP64).  Fewer, longer rounds
 // beat an intermediate that stays in the last-level cache: 16e/28o one vector 107 ms at 32M,
 // 97 at 128M, 93 at 256M.
 #define TX_ELEMS (256LL << 20)
 
-static int grow(void **p, size_t *have, size_t want, const char *what);
-
-static int tx_buffers(jci_ham *h, int nvec, int prec)
+// one block for nvec vectors: the intermediate, the inputs in both orders, the results in both
+static size_t tx_pieces(const jci_ham *h, int prec, int nvec, size_t at[3])
 {
     const size_t N = (size_t)h->sp->h.ndets, sz = prec == 64 ? sizeof(double) : sizeof(float);
-    RCHECK(grow(&h->d_txE, &h->txE_bytes, sz * nvec * (size_t)h->tx->elems, "the intermediate"));
-    RCHECK(grow(&h->d_txx, &h->txx_bytes, sz * 2 * nvec * N, "the input vectors"));
-    return grow(&h->d_txy, &h->txy_bytes, sizeof(double) * 2 * nvec * N, "the result vectors");
+    auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+    at[0] = 0;
+    at[1] = up(sz * nvec * (size_t)h->tx->elems);
+    at[2] = at[1] + up(sz * 2 * nvec * N);
+    return at[2] + sizeof(double) * 2 * nvec * N;
 }
 
-static int tx_upload(jci_ham *h, const void *src, size_t bytes, void **out)
+// vectors that a block of this size has room for
+static int tx_fit(const jci_ham *h, int prec, size_t bytes)
 {
-    jci_ctx *c = h->sp->ctx;
+    size_t at[3];
+    int k = 0;
+    while (k < JCI_MAXK && tx_pieces(h, prec, k + 1, at) <= bytes) k++;
+    return k;
+}
+
+static void tx_drop(void **p, size_t *bytes)
+{
+    if (*p) hipFree(*p);
+    *p = nullptr;
+    *bytes = 0;
+}
+
+static int tx_keep(jci_ham *h)
+{
+    size_t at[3];
+    tx_drop(&h->d_txkeep, &h->txkeep_bytes);
+    if (h->sp->h.ndets > TX_NOALLOC_DETS) return 0;
+    const size_t want = tx_pieces(h, 64, std::max(1, tx_fit(h, 64, TX_KEEP_BYTES)), at);
+    if (hipMalloc(&h->d_txkeep, want) != hipSuccess) {
+        (void)hipGetLastError();
+        h->d_txkeep = nullptr;
+        jci_set_error("sigma: out of device memory for the contraction form (%zu bytes)", want);
+        return -3;
+    }
+    h->txkeep_bytes = want;
+    return 0;
+}
+
+// the block for up to nvec vectors and how many go at a time: the kept one where it has room, else
+// one that is grown to as many of them as device memory allows (alloc 0: only the kept one)
+static int tx_block(jci_ham *h, int prec, int nvec, int alloc, void **block, int *per)
+{
+    size_t at[3];
+    const int keep = tx_fit(h, prec, h->txkeep_bytes);
+    int more = tx_fit(h, prec, h->txmore_bytes);
+    if (alloc && keep < nvec && more < nvec) {
+        size_t room = 0, total = 0;
+        JCI_CHECK(hipMemGetInfo(&room, &total));
+        room += h->txmore_bytes;
+        if (h->tx_cap && room > h->tx_cap) room = h->tx_cap;
+        int k = std::min(nvec, tx_fit(h, prec, room));
+        if (k > keep && k > more) {
+            tx_drop(&h->d_txmore, &h->txmore_bytes);   // (waits for the kernels that use it)
+            for (; k > keep; k--) {
+                const size_t want = tx_pieces(h, prec, k, at);
+                if (hipMalloc(&h->d_txmore, want) == hipSuccess) {
+                    h->txmore_bytes = want;
+                    break;
+                }
+                (void)hipGetLastError();
+                h->d_txmore = nullptr;
+            }
+            more = tx_fit(h, prec, h->txmore_bytes);
+        }
+    }
+    const bool kept = !alloc || keep >= nvec || keep >= more;
+    *block = kept ? h->d_txkeep : h->d_txmore;
+    *per = std::min(nvec, kept ? keep : more);
+    if (*per < 1 || !*block) {
+        jci_set_error("sigma: no device memory for one vector of the contraction form (%zu bytes)",
+                      tx_pieces(h, prec, 1, at));
+        return alloc ? -3 : -1;
+    }
+    return 0;
+}
+
+static int tx_alloc(jci_ham *h, size_t bytes, void **out)
+{
     void *d = nullptr;
     if (hipMalloc(&d, bytes ? bytes : 16) != hipSuccess) {
         (void)hipGetLastError();
@@ -630,10 +707,57 @@ static int tx_upload(jci_ham *h, const void *src, size_t bytes, void **out)
     }
     h->tx_mem[h->tx_nmem++] = d;
     *out = d;
-    if (src && bytes) {
-        JCI_CHECK(hipMemcpyAsync(d, src, bytes, hipMemcpyHostToDevice, c->stream));
-        JCI_CHECK(hipStreamSynchronize(c->stream));   // src is the caller's pageable memory
+    return 0;
+}
+
+// the plan's tables on the device, in one block
+static int tx_tables(jci_ham *h)
+{
+    jci_ctx *c = h->sp->ctx;
+    const SpaceDesc &D = h->sp->h;
+    const TxPlan *P = h->tx;
+    TxDev &d = h->txd;
+    std::vector<unsigned char> blob;
+    auto put = [&](const void *p, size_t bytes) {
+        const size_t at = (blob.size() + 255) / 256 * 256;
+        blob.resize(at + bytes);
+        if (bytes) memcpy(blob.data() + at, p, bytes);
+        return at;
+    };
+#define TX_PUT(v) put(P->v.data(), P->v.size() * sizeof(P->v[0]))
+    const size_t o_task = TX_PUT(task), o_slot = TX_PUT(slot), o_ch = TX_PUT(chunk), o_item = TX_PUT(item), o_out = TX_PUT(out),
+                 o_src = TX_PUT(src), o_pt = TX_PUT(ptask), o_pi = TX_PUT(pitem), o_po = TX_PUT(pout),
+                 o_q = TX_PUT(q);
+#undef TX_PUT
+    std::vector<long long> tt(D.nblk + 1, 0);
+    for (int b = 0; b < D.nblk; b++) {
+        const TxList &la = P->lists[0][D.bp[b]], &lb = P->lists[1][D.bq[b]];
+        tt[b + 1] = tt[b] + (long long)(la.nIp / 16) * la.nsv * (lb.nIp / 16) * lb.nsv;
     }
+    h->nttx = tt[D.nblk];
+    const size_t o_tt = put(tt.data(), sizeof(long long) * tt.size());
+    if (h->d_txtab) hipFree(h->d_txtab);
+    h->d_txtab = nullptr;
+    if (hipMalloc(&h->d_txtab, blob.size()) != hipSuccess) {
+        (void)hipGetLastError();
+        h->d_txtab = nullptr;
+        jci_set_error("contraction plan: out of device memory (%zu bytes)", blob.size());
+        return -3;
+    }
+    unsigned char *m = (unsigned char *)h->d_txtab;
+    JCI_CHECK(hipMemcpyAsync(m, blob.data(), blob.size(), hipMemcpyHostToDevice, c->stream));
+    JCI_CHECK(hipStreamSynchronize(c->stream));
+    d.task = (const TxTask *)(m + o_task);
+    d.slot = (const TxSlot *)(m + o_slot);
+    d.chunk = (const TxChunk *)(m + o_ch);
+    d.item = (const TxItem *)(m + o_item);
+    d.out = (const TxOut *)(m + o_out);
+    d.src = (const TxSrc *)(m + o_src);
+    d.ptask = (const TxPairTask *)(m + o_pt);
+    d.pitem = (const TxPairItem *)(m + o_pi);
+    d.pout = (const TxPairOut *)(m + o_po);
+    d.q = (const int *)(m + o_q);
+    h->d_ttx = (long long *)(m + o_tt);
     return 0;
 }
 
@@ -646,7 +770,8 @@ static int build_tx(jci_ham *h)
     SpaceDesc T;
     jci_transpose_desc(D, &T);
     TxPlan *P = new TxPlan();
-    if (tx_plan(D, T, TX_ELEMS, P)) {
+    h->tx_elems = TX_ELEMS;
+    if (tx_plan(D, T, h->tx_elems, P)) {
         delete P;
         return 0;
     }
@@ -669,16 +794,16 @@ static int build_tx(jci_ham *h)
         x.goff1 = h->d_goff1[sp];
         x.G = S.ngrp;
         x.npair = S.nelec * (S.nelec - 1) / 2;
-        RCHECK(tx_upload(h, nullptr, sizeof(uint32_t) * (size_t)P->nlst[sp], (void **)&x.lst));
-        RCHECK(tx_upload(h, nullptr, sizeof(uint16_t) * (size_t)h->nexc1[sp], (void **)&x.rk));
-        RCHECK(tx_upload(h, nullptr, sizeof(int2) * (size_t)P->nkl[sp], (void **)&x.kl));
-        RCHECK(tx_upload(h, nullptr, sizeof(int2) * (size_t)ns * x.npair, (void **)&x.gl));
-        RCHECK(tx_upload(h, nullptr, sizeof(double) * (size_t)(np + 1) * (np + 1), (void **)&x.w64));
-        RCHECK(tx_upload(h, nullptr, sizeof(float) * (size_t)(np + 1) * (np + 1), (void **)&x.w32));
+        RCHECK(tx_alloc(h, sizeof(uint32_t) * (size_t)P->nlst[sp], (void **)&x.lst));
+        RCHECK(tx_alloc(h, sizeof(uint16_t) * (size_t)h->nexc1[sp], (void **)&x.rk));
+        RCHECK(tx_alloc(h, sizeof(int2) * (size_t)P->nkl[sp], (void **)&x.kl));
+        RCHECK(tx_alloc(h, sizeof(int2) * (size_t)ns * x.npair, (void **)&x.gl));
+        RCHECK(tx_alloc(h, sizeof(double) * (size_t)(np + 1) * (np + 1), (void **)&x.w64));
+        RCHECK(tx_alloc(h, sizeof(float) * (size_t)(np + 1) * (np + 1), (void **)&x.w32));
         const size_t nrow = (size_t)mp + P->nint_parts[sp] + 1;
         x.zrow = (int)nrow - 1;
-        RCHECK(tx_upload(h, nullptr, sizeof(double) * nrow * d.ms, (void **)&x.m64));
-        RCHECK(tx_upload(h, nullptr, sizeof(float) * nrow * d.ms, (void **)&x.m32));
+        RCHECK(tx_alloc(h, sizeof(double) * nrow * d.ms, (void **)&x.m64));
+        RCHECK(tx_alloc(h, sizeof(float) * nrow * d.ms, (void **)&x.m32));
         TxList *dl = nullptr;
         TxPairGroup *dp = nullptr;
         JCI_CHECK(hipMallocAsync((void **)&dl, sizeof(TxList) * P->lists[sp].size(), c->stream));
@@ -701,59 +826,38 @@ static int build_tx(jci_ham *h)
         hipFreeAsync(dp, c->stream);
     }
     if (same) d.s[1] = d.s[0];
-    // the small tables in one block
-    std::vector<unsigned char> blob;
-    auto put = [&](const void *p, size_t bytes) {
-        const size_t at = (blob.size() + 255) / 256 * 256;
-        blob.resize(at + bytes);
-        if (bytes) memcpy(blob.data() + at, p, bytes);
-        return at;
-    };
-#define TX_PUT(v) put(P->v.data(), P->v.size() * sizeof(P->v[0]))
-    const size_t o_task = TX_PUT(task), o_slot = TX_PUT(slot), o_ch = TX_PUT(chunk), o_item = TX_PUT(item), o_out = TX_PUT(out),
-                 o_src = TX_PUT(src), o_pt = TX_PUT(ptask), o_pi = TX_PUT(pitem), o_po = TX_PUT(pout),
-                 o_q = TX_PUT(q);
-#undef TX_PUT
-    std::vector<long long> tt(D.nblk + 1, 0);
-    for (int b = 0; b < D.nblk; b++) {
-        const TxList &la = P->lists[0][D.bp[b]], &lb = P->lists[1][D.bq[b]];
-        tt[b + 1] = tt[b] + (long long)(la.nIp / 16) * la.nsv * (lb.nIp / 16) * lb.nsv;
-    }
-    h->nttx = tt[D.nblk];
-    const size_t o_tt = put(tt.data(), sizeof(long long) * tt.size());
-    unsigned char *m;
-    RCHECK(tx_upload(h, blob.data(), blob.size(), (void **)&m));
-    d.task = (const TxTask *)(m + o_task);
-    d.slot = (const TxSlot *)(m + o_slot);
-    d.chunk = (const TxChunk *)(m + o_ch);
-    d.item = (const TxItem *)(m + o_item);
-    d.out = (const TxOut *)(m + o_out);
-    d.src = (const TxSrc *)(m + o_src);
-    d.ptask = (const TxPairTask *)(m + o_pt);
-    d.pitem = (const TxPairItem *)(m + o_pi);
-    d.pout = (const TxPairOut *)(m + o_po);
-    d.q = (const int *)(m + o_q);
-    h->d_ttx = (long long *)(m + o_tt);
-    if (D.ndets <= TX_NOALLOC_DETS) RCHECK(tx_buffers(h, 1, 64));
-    return 0;
+    RCHECK(tx_tables(h));
+    return tx_keep(h);
 }
 
-// y = H x in the contraction form: vector k at x + k xk (element stride xs) -> y + k yk (ys)
+// y = H x in the contraction form: vector k at x + k xk (element stride xs) -> y + k yk (ys), in as
+// many passes as the buffers ask for (a vector's sums are the same in each)
 static int tx_sigma(jci_ham *h, int prec, int nvec, const double *x, long long xs, long long xk,
-                    double *y, long long ys, long long yk)
+                    double *y, long long ys, long long yk, int alloc)
 {
     jci_ctx *c = h->sp->ctx;
     const long long N = h->sp->h.ndets;
-    TxVec v;
-    v.x0 = h->d_txx;
-    v.x1 = (const char *)h->d_txx + (size_t)nvec * N * (prec == 64 ? sizeof(double) : sizeof(float));
-    v.y0 = (double *)h->d_txy;
-    v.y1 = v.y0 + (size_t)nvec * N;
-    v.N = N;
-    RCHECK(jk_tx_in(prec, nvec, N, h->sp->d_desc, h->d_ttx, h->nttx, x, xs, xk, (void *)v.x0,
-                    (void *)v.x1, c->stream));
-    RCHECK(jk_tx_run(prec, nvec, h->txd, *h->tx, v, h->d_txE, c->stream));
-    return jk_tx_out(nvec, N, h->sp->d_desc, h->d_ttx, h->nttx, v.y0, v.y1, y, ys, yk, c->stream);
+    void *block;
+    int per;
+    RCHECK(tx_block(h, prec, nvec, alloc, &block, &per));
+    for (int k0 = 0; k0 < nvec; k0 += per) {
+        const int k = std::min(per, nvec - k0);
+        size_t at[3];
+        tx_pieces(h, prec, k, at);
+        char *p = (char *)block;
+        TxVec v;
+        v.x0 = p + at[1];
+        v.x1 = p + at[1] + (size_t)k * N * (prec == 64 ? sizeof(double) : sizeof(float));
+        v.y0 = (double *)(p + at[2]);
+        v.y1 = v.y0 + (size_t)k * N;
+        v.N = N;
+        RCHECK(jk_tx_in(prec, k, N, h->sp->d_desc, h->d_ttx, h->nttx, x + k0 * xk, xs, xk,
+                        (void *)v.x0, (void *)v.x1, c->stream));
+        RCHECK(jk_tx_run(prec, k, h->txd, *h->tx, v, p, c->stream));
+        RCHECK(jk_tx_out(k, N, h->sp->d_desc, h->d_ttx, h->nttx, v.y0, v.y1, y + k0 * yk, ys, yk,
+                         c->stream));
+    }
+    return 0;
 }
 
 // excitation tables and launch maps of the table kernels.  Spaces that take the contraction
@@ -952,7 +1056,7 @@ JCI_API void jci_ham_destroy(jci_ham *h)
     hipSetDevice(h->sp->ctx->device);
     hipStreamSynchronize(h->sp->ctx->stream);
     for (int i = 0; i < h->tx_nmem; i++) hipFree(h->tx_mem[i]);
-    hipFree(h->d_txE); hipFree(h->d_txx); hipFree(h->d_txy);
+    hipFree(h->d_txtab); hipFree(h->d_txkeep); hipFree(h->d_txmore);
     delete h->tx;
     free_doubles(h);
     hipFree(h->d_m1); hipFree(h->d_m2); hipFree(h->d_hd);
@@ -1251,20 +1355,15 @@ static int fast_run(jci_ham *h, int method, int nvec, const double *x, double *y
     const int prec = method == JCI_SIGMA_FAST64 ? 64 : 32;
     if (h->tx && !h->tx_off) {
         const long long ys = ldy ? 1 : nvec, yk = ldy ? ldy : 1;
-        if (!s) {
-            RCHECK(tx_buffers(h, nvec, prec));
-            return tx_sigma(h, prec, nvec, x, nvec, 1, y, ys, yk);
-        }
+        if (!s) return tx_sigma(h, prec, nvec, x, nvec, 1, y, ys, yk, 1);
         // allocation-free: the staging of the table kernels bounds the sizes taken, the vectors
-        // go one at a time through the buffers kept from the start
+        // go through the buffers kept from the start
         float *xf;
         void *xT;
         if (prec == 32) RCHECK(ensure_xf(h, N * nvec, s, &xf));
         RCHECK(jci_scratch_carve(s, (size_t)N * nvec * (prec == 64 ? sizeof(double) : sizeof(float)),
                                  &xT, "the transposed input"));
-        for (int k = 0; k < nvec; k++)
-            RCHECK(tx_sigma(h, prec, 1, x + k, nvec, 1, y + k * yk, ys, yk));
-        return 0;
+        return tx_sigma(h, prec, nvec, x, nvec, 1, y, ys, yk, 0);
     }
     RCHECK(ensure_tables(h));
     const void *xin = x;
@@ -1634,6 +1733,48 @@ JCI_API int jci_ham_fast_xcd(jci_ham *h, int *group, int *chunk_major)
     if (chunk_major && *chunk_major >= 0) h->fast_cm = *chunk_major ? 1 : 0;
     if (group) *group = h->fast_xg;
     if (chunk_major) *chunk_major = h->fast_cm;
+    return 0;
+}
+
+JCI_API int jci_ham_contraction(jci_ham *h, int *use, long long *elems, long long *bytes, int rounds[2])
+{
+    if (!h->have_fast) { jci_set_error("ham: no excitation tables"); return -1; }
+    const int want = use ? *use : -1;
+    if (want > 1 || (want == 1 && !h->tx)) {
+        jci_set_error("ham: the space has no contraction form, or use %d not 0 or 1", want);
+        return -1;
+    }
+    if (h->tx && elems && *elems > 0 && *elems != h->tx_elems) {
+        JCI_CHECK(hipSetDevice(h->sp->ctx->device));
+        SpaceDesc T;
+        jci_transpose_desc(h->sp->h, &T);
+        TxPlan *P = new TxPlan();
+        if (tx_plan(h->sp->h, T, *elems, P)) {
+            delete P;
+            jci_set_error("ham: no plan with rounds of %lld elements", *elems);
+            return -1;
+        }
+        JCI_CHECK(hipStreamSynchronize(h->sp->ctx->stream));
+        delete h->tx;
+        h->tx = P;
+        h->tx_elems = *elems;
+        tx_drop(&h->d_txmore, &h->txmore_bytes);
+        RCHECK(tx_tables(h));
+        RCHECK(tx_keep(h));
+    }
+    if (bytes && *bytes > 0) {
+        h->tx_cap = (size_t)*bytes;
+        if (h->txmore_bytes > h->tx_cap) tx_drop(&h->d_txmore, &h->txmore_bytes);
+    }
+    if (want == 0) RCHECK(use_tables(h));
+    if (want == 1) h->tx_off = 0;
+    if (use) *use = h->tx && !h->tx_off;
+    if (elems) *elems = h->tx ? h->tx->elems : 0;
+    if (bytes) *bytes = (long long)(h->txkeep_bytes + h->txmore_bytes);
+    if (rounds) {
+        rounds[0] = h->tx ? (int)h->tx->ab.size() : 0;
+        rounds[1] = h->tx ? (int)h->tx->ss.size() : 0;
+    }
     return 0;
 }
 
@@ -2300,10 +2441,8 @@ static int ham_sigma_cols(void *self, int method, int k, const double *V, long l
     jci_ham *h = (jci_ham *)self;
     method = resolve_method(h, method, 0);
     if (method == JCI_SIGMA_FAST64 || method == JCI_SIGMA_FAST32) {
-        if (h->have_fast && h->tx && !h->tx_off) {
-            RCHECK(tx_buffers(h, k, method == JCI_SIGMA_FAST64 ? 64 : 32));
-            return tx_sigma(h, method == JCI_SIGMA_FAST64 ? 64 : 32, k, V, 1, ldv, S, 1, lds);
-        }
+        if (h->have_fast && h->tx && !h->tx_off)
+            return tx_sigma(h, method == JCI_SIGMA_FAST64 ? 64 : 32, k, V, 1, ldv, S, 1, lds, 1);
         // the table sigma reads determinant-major input and writes the columns directly
         RCHECK(jk_pack(k, h->sp->h.ndets, V, ldv, stage, h->sp->ctx->stream));
         return fast_run(h, method, k, stage, S, lds, nullptr);
