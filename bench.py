@@ -485,15 +485,21 @@ def bench_mrci(J, ctx, args):
     import numpy as np
     rows = np.random.default_rng(0).integers(0, N, size=64)
     cbar = float(np.mean([len(c) for c, _, _, _ in h.rows(rows)]))
-    from jayci_amd.serve import lane_solve_params
+    from jayci_amd.serve import (lane_solve_params, lane_vector_bytes, sigma_buffer_bytes,
+                                 sigma_elems)
     nr = args.roots
     # the subspace as large as the device's free memory allows (a margin of 6 GiB kept;
     # the diagonal and the lists, 32 bytes per determinant in the lane's estimate, are
-    # allocated already)
+    # allocated already); the sigma then takes as many vectors at a time as the rest holds
     free_b, total_b = J.device_memory(ctx.device)
-    kw = lane_solve_params({"nroots": nr}, N, 1e-6, budget=free_b - (6 << 30) + 32 * N,
-                           kfac=args.mrci_kfac)
+    spec = dict(na=8, nb=8, norbs=n, ndocc=4, nactv=8, xlvl=2, rule=J.RULE_MRCISD, nroots=nr)
+    budget = free_b - (6 << 30) + 32 * N
+    kw = lane_solve_params(spec, N, 1e-6, budget=budget, kfac=args.mrci_kfac, at_once=1)
     nt = kw["nroots"] + kw["nbuffer"]
+    elems = sigma_elems(spec, N)
+    at_once = max([k for k in range(1, nt + 1)
+                   if lane_vector_bytes(N, kw["krymax"], nt, elems, k) <= budget], default=1)
+    h.contraction(nbytes=sigma_buffer_bytes(N, at_once, elems))
     log("device memory: %.1f GB free of %.1f GB; krymax %d" % (free_b / 1e9, total_b / 1e9,
                                                               kw["krymax"]))
     kw.update(maxiter=args.mrci_maxiter, vectors=False, check=False)

@@ -364,13 +364,22 @@ int jci_ham_fast_xcd(jci_ham *h, int *group, int *chunk_major);
 /* the two forms of the FAST methods on truncated spaces.  *use 1: products over the strings'
  * replacements (the default where the space has that form), 0: the table kernels, as the three
  * shapes above choose them; *elems > 0: that form in rounds of at most that many elements of its
- * intermediate per vector, or of one string's where that is more (default 256M; plans anew and
- * moves the buffers, so not while a captured graph uses them); *bytes > 0: bound on the block that
+ * intermediate per vector, or of one string's where that is more (default 256M, or the
+ * determinants where they are more; plans anew and moves the buffers, so not while a captured
+ * graph uses them); *bytes > 0: bound on the block that
  * calls of several vectors grow (beyond it, or where device memory ends, they go in passes).
  * Other values keep.  Returned: the form in use, the elements of the largest round, the bytes
  * of the buffers held, and the numbers of opposite-spin and same-spin rounds (0 without the form;
  * any pointer may be NULL) */
 int jci_ham_contraction(jci_ham *h, int *use, long long *elems, long long *bytes, int rounds[2]);
+/* plan of that form for a space (arguments of jci_space_create; host only, no GPU needed): 1 when
+ * the FAST methods take it, 0 when they run the table kernels, < 0 on invalid arguments.  elems as
+ * above (0: default).  out (may be NULL): [0] elements per vector of the largest round's
+ * intermediate, [1] of all rounds together, [2] opposite-spin and [3] same-spin rounds, [4]
+ * work-groups of the largest launch, [5..9] pieces that start past the first external part, column
+ * tile, string (opposite spin), column and N - 2 electron string (same spin) */
+int jci_contraction_plan(int na, int nb, int norbs, int ndocc, int nactv, int xlvl, int rule,
+                         long long elems, long long out[10]);
 /* column-tile widths of the dense-string sigma's opposite-spin product (FP64: 16 or 32,
  * FP32: 32 or 64; the autotuner sets them): a positive *bn sets, then both are returned */
 int jci_ham_gemm_tiles(jci_ham *h, int *bn64, int *bn32);

@@ -95,6 +95,7 @@ _sig("jci_ham_fast_width", _i, [_P])
 _sig("jci_ham_fast_tiles", _i, [_P, ctypes.POINTER(_i), ctypes.POINTER(_i)])
 _sig("jci_ham_fast_split", _i, [_P, ctypes.POINTER(_i)])
 _sig("jci_ham_fast_xcd", _i, [_P, ctypes.POINTER(_i), ctypes.POINTER(_i)])
+_sig("jci_contraction_plan", _i, [_i] * 7 + [_ll, _P])
 _sig("jci_ham_contraction", _i, [_P, ctypes.POINTER(_i), ctypes.POINTER(_ll), ctypes.POINTER(_ll), _P])
 _sig("jci_batch_create", _i, [_P, _i, _i, ctypes.POINTER(_P)])
 _sig("jci_batch_destroy", None, [_P])
@@ -288,6 +289,19 @@ class Space:
 
     def index(self, a, b):
         return _L.jci_space_index(self._h, int(a), int(b))
+
+
+def contraction_plan(na, nb, norbs, ndocc=0, nactv=None, xlvl=0, rule=RULE_MRCISD, elems=0):
+    """Plan of the truncated-space sigma's contraction form (jci_contraction_plan, host only): a
+    dict, or None for spaces whose FAST methods run the table kernels."""
+    out = (_ll * 10)()
+    rc = _L.jci_contraction_plan(na, nb, norbs, ndocc, norbs if nactv is None else nactv, xlvl, rule,
+                                 elems, out)
+    if rc < 0:
+        raise JciError("jci_contraction_plan failed (%d): %s" % (rc, last_error()))
+    if rc == 0:
+        return None
+    return dict(elems=out[0], total=out[1], rounds=(out[2], out[3]), grid=out[4], split=tuple(out[5:10]))
 
 
 class Hamiltonian:

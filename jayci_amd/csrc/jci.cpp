@@ -611,10 +611,13 @@ static void free_doubles(jci_ham *h)
 // vectors of a small space allocates nothing
 #define TX_NOALLOC_DETS (16LL << 20)
 #define TX_KEEP_BYTES ((size_t)64 << 20)
-// elements of the intermediate per vector and round: 256M (2 GB in FP64).  Fewer, longer rounds
-// beat an intermediate that stays in the last-level cache: 16e/28o one vector 107 ms at 32M,
-// 97 at 128M, 93 at 256M.
+// elements of the intermediate per vector and round: 256M (2 GB in FP64), or as many as the vector
+// has where that is more (a fifth of its buffers).  Fewer, longer rounds beat an intermediate that
+// stays in the last-level cache: 16e/28o one vector 107 ms at 32M, 97 at 128M, 93 at 256M; 16e/60o
+// (604M determinants), whose column tiles are cut by strings below 1417M, 1.78 s at 256M, 1.72 at
+// 512M, 1.67 at 768M.
 #define TX_ELEMS (256LL << 20)
+static long long tx_bound(const SpaceDesc &D) { return std::max(TX_ELEMS, D.ndets); }
 
 // one block for nvec vectors: the intermediate, the inputs in both orders, the results in both
 static size_t tx_pieces(const jci_ham *h, int prec, int nvec, size_t at[3])
@@ -770,7 +773,7 @@ static int build_tx(jci_ham *h)
     SpaceDesc T;
     jci_transpose_desc(D, &T);
     TxPlan *P = new TxPlan();
-    h->tx_elems = TX_ELEMS;
+    h->tx_elems = tx_bound(D);
     if (tx_plan(D, T, h->tx_elems, P)) {
         delete P;
         return 0;
@@ -1734,6 +1737,27 @@ JCI_API int jci_ham_fast_xcd(jci_ham *h, int *group, int *chunk_major)
     if (group) *group = h->fast_xg;
     if (chunk_major) *chunk_major = h->fast_cm;
     return 0;
+}
+
+JCI_API int jci_contraction_plan(int na, int nb, int norbs, int ndocc, int nactv, int xlvl, int rule,
+                                 long long elems, long long out[10])
+{
+    SpaceDesc D, T;
+    if (out) for (int i = 0; i < 10; i++) out[i] = 0;
+    if (jci_build_desc(na, nb, norbs, ndocc, nactv, xlvl, rule, &D)) return -1;
+    if (D.nblk < 2) return 0;
+    jci_transpose_desc(D, &T);
+    TxPlan P;
+    if (tx_plan(D, T, elems > 0 ? elems : tx_bound(D), &P)) return 0;
+    if (out) {
+        out[0] = P.elems;
+        out[1] = P.total;
+        out[2] = (long long)P.ab.size();
+        out[3] = (long long)P.ss.size();
+        out[4] = P.grid;
+        for (int i = 0; i < 5; i++) out[5 + i] = P.split[i];
+    }
+    return 1;
 }
 
 JCI_API int jci_ham_contraction(jci_ham *h, int *use, long long *elems, long long *bytes, int rounds[2])

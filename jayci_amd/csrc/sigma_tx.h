@@ -54,6 +54,8 @@
 // a SIMD.  More rows per scattered tile at two waves: 16e/28o FP64 93 -> 97 ms; 48 at three in
 // FP32, two vectors 16e/20o: 22.0 -> 22.7 ms
 #define TX_ROWS 32
+// work-groups of a launch: 256 threads each, and a grid holds fewer than 2^32 threads
+#define TX_GRID ((1LL << 24) - 1024)
 #define TX_PAD 0x7FF00000u   // list entry of a padded row or column (no position, string 0)
 
 // Order of the vectors' columns.  Inside a block's row the strings of the first spin are kept
@@ -121,10 +123,12 @@ struct TxTask {
     long long lbase;
 };
 
-// one task's share of a round (a range of columns small enough that E fits its buffer)
+// one task's share of a round (a range of columns, of one column tile also a range of strings JL,
+// small enough that E fits its buffer)
 struct TxItem {
     int task, w0, nw, t0, nt;        // external parts, column tiles of the item
     int p0, pn;                      // column tiles of the whole piece (rows of E)
+    int j0, nj;                      // strings JL
     int rg;                          // row groups
     long long item0;                 // first item of the round's launch: (JL, w, row group)
     long long ebase;                 // first element in E
@@ -136,6 +140,7 @@ struct TxOut {
     int na, ls0, nI, nIp, nsv;
     int w0, nw, t0, nt;
     int src0, nsrc;
+    int part;                        // 1: a source holds some of its strings only
     int nb;                          // strings of the first-spin group
     long long yb;                    // block offset
     long long blk0;                  // first work-group of the launch
@@ -144,6 +149,7 @@ struct TxOut {
 struct TxSrc {
     int l1, ls0, La, r0, diag;       // JL's group and its first string, rows, first row of this
                                      // target (-1: none); diag 1: also JL = IL
+    int j0, nj;                      // strings of JL's group that the round holds
     long long ebase;
 };
 
@@ -167,6 +173,7 @@ struct TxPairTask {
 #define TX_RMAX 64           // pairs up to which a work-group keeps all of W in LDS
 struct TxPairItem {
     int task, c0, nc, ncp;           // columns of the round, padded to 16
+    int k0, nk;                      // N - 2 electron strings
     int rg, cb, ct;                  // row groups of 64, column blocks of 64 per work-group,
                                      // work-groups across
     long long item0, ebase;
@@ -174,8 +181,11 @@ struct TxPairItem {
 struct TxPairOut {
     int o, p, f, na, ls0, nb;
     int c0, nc, ncp, cblk;
+    int add, part;                   // 1: adds to the result; 1: not every N - 2 string is there
     long long yb, blk0;
     int nsec, np[TX_NTYPE], r0[TX_NTYPE], R[TX_NTYPE];   // pairs of I per type, rows of E
+    int g0[TX_NTYPE];                // first pair of the type in the string's list
+    int k0[TX_NTYPE], nk[TX_NTYPE];  // N - 2 strings that the round holds
     long long eb[TX_NTYPE];
 };
 
@@ -377,11 +387,16 @@ struct TxPlan {
     std::vector<TxPairOut> pout;
     std::vector<int> q;
     std::vector<TxRound> ab, ss;           // rounds of the two parts
-    long long elems;                       // largest E of a round
+    long long elems, total;                // largest E of a round, sum over the rounds
+    long long grid;                        // most work-groups of a launch
+    int split[5];                          // pieces that start past the first external part, column
+                                           // tile, JL (opposite spin), column, N - 2 string (same spin)
     int ldt, rmax;                         // deepest reduction chunk; most pairs of a task
     long long nint_parts[2];               // internal parts over all groups
     int iI0[2][JCI_MAXG];
 };
+// budget: bound on a round's E (what one string of a task needs for one column tile, or one N - 2
+// electron string for 64 columns, where that is more).
 // 0: built; 1: the space is outside what the lists can index (the caller keeps the tables)
 int tx_plan(const SpaceDesc &D, const SpaceDesc &T, long long budget, TxPlan *P);
 

@@ -407,7 +407,7 @@ __global__ __launch_bounds__(256, RT == 2 ? 6 : 4) void k_tx_ess(TxDev A, TxRoun
     const TxPairItem &it = items[tx_find(ni, u, [&](int i) { return items[i].item0; })];
     const TxPairTask &t = A.ptask[it.task];
     const int loc = (int)(u - it.item0), rg = loc % it.rg, ct = loc / it.rg % it.ct;
-    const long long K2 = loc / (it.rg * it.ct);
+    const long long k2 = loc / (it.rg * it.ct), K2 = it.k0 + k2;
     const int Rr = t.R, Rp = (Rr + 15) / 16 * 16, r0 = rg * 64, nc = it.nc, ncp = it.ncp;
     const TxSpin &S = A.s[t.o];
     const long long k = blockIdx.y;
@@ -440,7 +440,7 @@ __global__ __launch_bounds__(256, RT == 2 ? 6 : 4) void k_tx_ess(TxDev A, TxRoun
         wrow[j] = (uint32_t)(r < Rp ? pr[r] & 0x7FFFFFFF : np) * ws;
     }
     const T *__restrict__ x = (t.o ? x1 : x0) + k * N + it.c0;
-    T *__restrict__ Ek = E + k * R.elems + it.ebase + (K2 * Rr + r0) * ncp;
+    T *__restrict__ Ek = E + k * R.elems + it.ebase + (k2 * Rr + r0) * ncp;
     const int cb0 = ct * it.cb, cb1 = std::min(cb0 + it.cb, (nc + 63) / 64);
     T ra[RT], rb[4];
     typename Mf<T>::acc acc[RT];
@@ -583,8 +583,23 @@ __device__ __forceinline__ T tx_sum(T acc, const T *__restrict__ E, const long l
     return acc;
 }
 
+// of the work-group's 256 entries those to keep, in order: this thread's place and their number
+__device__ __forceinline__ int tx_place(bool keep, int *cnt, int *n)
+{
+    const uint64_t b = __ballot(keep);
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (l == 0) cnt[w] = __popcll(b);
+    __syncthreads();
+    int at = __popcll(b & ((1ULL << l) - 1ULL));
+    for (int i = 0; i < w; i++) at += cnt[i];
+    *n = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+    return at;
+}
+
 // the same-spin sums: y(I, c) = sum over the pairs of I, one E row each (coalesced); the first
-// writer of the result.  The rows' offsets are set up in LDS once for the string's columns.
+// writer of the result.  The rows' offsets are set up in LDS once for the string's columns.  Where
+// a round holds some of the N - 2 electron strings only, the entries of the others are left out and
+// the sums of its successors are added.
 #define TX_ENT 512
 #define TX_SRC 64            // one wave's scan
 template <typename T>
@@ -593,6 +608,7 @@ __global__ __launch_bounds__(256) void k_tx_gss(TxDev A, TxRound R, long long N,
                                                 double *__restrict__ y1)
 {
     __shared__ long long ent[TX_ENT];
+    __shared__ int cnt[4];
     const TxPairOut *__restrict__ outs = A.pout + R.o0;
     const long long u = blockIdx.x;
     const TxPairOut &t = outs[tx_find(R.no, u, [&](int i) { return outs[i].blk0; })];
@@ -604,22 +620,45 @@ __global__ __launch_bounds__(256) void k_tx_gss(TxDev A, TxRound R, long long N,
     int np = 0;
     for (int s = 0; s < t.nsec; s++) np += t.np[s];
     T acc = (T)0;
-    for (int m0 = 0; m0 < np; m0 += TX_ENT) {
-        const int n = std::min(TX_ENT, np - m0);
-        if (m0) __syncthreads();
-        for (int m = threadIdx.x; m < n; m += 256) {
-            int s = 0, r = m0 + m;
-            while (r >= t.np[s]) r -= t.np[s++];
-            const int2 e = g[m0 + m];
-            const long long o = t.eb[s] + ((long long)e.x * t.R[s] + t.r0[s] + (e.y & 0x7FFFFFFF)) * t.ncp;
-            ent[m] = e.y < 0 ? ~o : o;
+    // offset of entry r (complemented: less), false where its N - 2 string is not in the round
+    auto entry = [&](int r, long long &o) __attribute__((always_inline)) {
+        int s = 0;
+        while (r >= t.np[s]) r -= t.np[s++];
+        const int2 e = g[t.g0[s] + r];
+        const int K = e.x - t.k0[s];
+        o = t.eb[s] + ((long long)K * t.R[s] + t.r0[s] + (e.y & 0x7FFFFFFF)) * t.ncp;
+        if (e.y < 0) o = ~o;
+        return (unsigned)K < (unsigned)t.nk[s];
+    };
+    if (!t.part) {
+        for (int m0 = 0; m0 < np; m0 += TX_ENT) {
+            const int n = std::min(TX_ENT, np - m0);
+            if (m0) __syncthreads();
+            for (int m = threadIdx.x; m < n; m += 256) {
+                long long o;
+                entry(m0 + m, o);
+                ent[m] = o;
+            }
+            __syncthreads();
+            if (c < t.nc) acc = tx_sum(acc, E + k * R.elems + c, ent, n);
         }
-        __syncthreads();
-        if (c < t.nc) acc = tx_sum(acc, E + k * R.elems + c, ent, n);
+    } else {
+        for (int m0 = 0; m0 < np; m0 += 256) {
+            const int m = m0 + threadIdx.x;
+            long long o = 0;
+            const bool in = m < np && entry(m, o);
+            int n;
+            if (m0) __syncthreads();
+            const int at = tx_place(in, cnt, &n);
+            if (in) ent[at] = o;
+            __syncthreads();
+            if (c < t.nc) acc = tx_sum(acc, E + k * R.elems + c, ent, n);
+        }
     }
     if (c >= t.nc) return;
     const long long n = t.yb + (long long)il * t.nb + t.c0 + c;
-    (t.o ? y1 : y0)[k * N + n] = (double)acc;
+    double *y = (t.o ? y1 : y0) + (k * N + n);
+    *y = t.add ? *y + (double)acc : (double)acc;
 }
 
 // ---- opposite-spin part ------------------------------------------------------------------------
@@ -903,7 +942,8 @@ __global__ __launch_bounds__(256, TxV<T>::WPE) void k_tx_eab(
     TxUnit n;
     n.r0 = loc % it.rg * RT * 16;
     loc /= it.rg;
-    n.ja = loc / it.nw;
+    const int jl = loc / it.nw;
+    n.ja = it.j0 + jl;
     n.w = it.w0 + loc % it.nw;
     n.k0 = blockIdx.y * kper;
     n.k1 = std::min(nvec, n.k0 + kper);
@@ -911,7 +951,7 @@ __global__ __launch_bounds__(256, TxV<T>::WPE) void k_tx_eab(
     n.dr = t.diag ? t.La - 1 - n.r0 : -1;
     const T *__restrict__ x = t.o ? x1 : x0;
     const long long lde = R.elems;
-    T *__restrict__ Eo = E + it.ebase + ((long long)n.ja * it.nw + (n.w - it.w0)) * t.La * it.pn * 16;
+    T *__restrict__ Eo = E + it.ebase + ((long long)jl * it.nw + (n.w - it.w0)) * t.La * it.pn * 16;
     static_assert(TX_KC == 96, "reduction depths below cover chunks of up to 96");
     for (int c = 0; c < t.nch; c++) {
         const TxChunk &ch = A.chunk[t.ch0 + c];
@@ -930,7 +970,8 @@ __global__ __launch_bounds__(256, TxV<T>::WPE) void k_tx_eab(
 // 256 columns of one string per work-group.  The rows' offsets, over all sources, are set up in
 // LDS first: the sum is then one stream of loads, eight in flight per lane, at the copy rate for
 // large spaces, and small ones (chains of list loads before) take 16.2 -> 9.1 us at 4a4b/10o and
-// 0.22 -> 0.19 ms at 7a6b/17o.
+// 0.22 -> 0.19 ms at 7a6b/17o.  Where a round holds some of a source's strings JL only, the entries
+// of the others are left out.
 template <typename T>
 __global__ __launch_bounds__(256) void k_tx_gab(TxDev A, TxRound R, long long N,
                                                 const T *__restrict__ E, double *__restrict__ y0,
@@ -940,7 +981,7 @@ __global__ __launch_bounds__(256) void k_tx_gab(TxDev A, TxRound R, long long N,
     // diagonal row); the list's offsets and steps per external part
     __shared__ int first[TX_SRC], base[TX_SRC + 1];
     __shared__ long long ent[TX_ENT];
-    __shared__ int step[TX_ENT];
+    __shared__ int step[TX_ENT], cnt[4];
     const TxOut *__restrict__ outs = A.out + R.o0;
     const long long u = blockIdx.x;
     const TxOut &t = outs[tx_find(R.no, u, [&](int i) { return outs[i].blk0; })];
@@ -973,29 +1014,56 @@ __global__ __launch_bounds__(256) void k_tx_gab(TxDev A, TxRound R, long long N,
         }
         __syncthreads();
         const int all = base[ns];
-        for (int m0 = 0; m0 < all; m0 += TX_ENT) {
-            const int n = std::min(TX_ENT, all - m0);
-            if (m0) __syncthreads();
-            for (int m = threadIdx.x; m < n; m += 256) {
-                int s = 0;
-                while (base[s + 1] <= m0 + m) s++;
-                const TxSrc &q = A.src[t.src0 + s0 + s];
-                const int i = m0 + m - base[s], rows = q.La * ntc;
-                long long J = il, row = q.La - 1;
-                bool neg = false;
-                if (!q.diag || m0 + m + 1 < base[s + 1]) {
-                    const long long e = e00 + first[s] + i;
-                    const int2 en = S.e1[e];
-                    J = en.x - q.ls0;
-                    row = q.r0 + S.rk[e];
-                    neg = en.y & (1 << 12);
-                }
-                const long long o = q.ebase + J * t.nw * rows + row * ntc;
-                ent[m] = neg ? ~o : o;
-                step[m] = rows;
+        // offset and step of entry m of the list (complemented: less), false where its JL is not
+        // in the round
+        auto entry = [&](int m, long long &o, int &rows) __attribute__((always_inline)) {
+            int s = 0;
+            while (base[s + 1] <= m) s++;
+            const TxSrc &q = A.src[t.src0 + s0 + s];
+            rows = q.La * ntc;
+            long long J = il, row = q.La - 1;
+            bool neg = false;
+            if (!q.diag || m + 1 < base[s + 1]) {
+                const long long e = e00 + first[s] + (m - base[s]);
+                const int2 en = S.e1[e];
+                J = en.x - q.ls0;
+                row = q.r0 + S.rk[e];
+                neg = en.y & (1 << 12);
             }
-            __syncthreads();
-            if (in) acc = tx_sum(acc, E + k * R.elems + ci, ent, n, step, wi);
+            J -= q.j0;
+            o = q.ebase + J * t.nw * rows + row * ntc;
+            if (neg) o = ~o;
+            return (unsigned long long)J < (unsigned long long)q.nj;
+        };
+        if (!t.part) {
+            for (int m0 = 0; m0 < all; m0 += TX_ENT) {
+                const int n = std::min(TX_ENT, all - m0);
+                if (m0) __syncthreads();
+                for (int m = threadIdx.x; m < n; m += 256) {
+                    long long o;
+                    int rows;
+                    entry(m0 + m, o, rows);
+                    ent[m] = o;
+                    step[m] = rows;
+                }
+                __syncthreads();
+                if (in) acc = tx_sum(acc, E + k * R.elems + ci, ent, n, step, wi);
+            }
+        } else {
+            for (int m0 = 0; m0 < all; m0 += 256) {
+                const int m = m0 + threadIdx.x;
+                long long o = 0;
+                int rows = 0, n;
+                const bool held = m < all && entry(m, o, rows);
+                if (m0) __syncthreads();
+                const int at = tx_place(held, cnt, &n);
+                if (held) {
+                    ent[at] = o;
+                    step[at] = rows;
+                }
+                __syncthreads();
+                if (in) acc = tx_sum(acc, E + k * R.elems + ci, ent, n, step, wi);
+            }
         }
     }
     if (!in) return;

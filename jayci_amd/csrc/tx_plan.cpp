@@ -294,9 +294,13 @@ struct Builder {
     }
 
     // one piece of a round: external parts [w0, w0 + nw) and column tiles [t0, t0 + nt) of
-    // first-spin group f, for some of its tasks
-    void piece(int o, int f, const std::vector<int> &tasks, int w0, int nw, int t0, int nt, TxRound &R)
+    // first-spin group f, for some of its tasks; nj > 0: strings JL [j0, j0 + nj) of the only task
+    void piece(int o, int f, const std::vector<int> &tasks, int w0, int nw, int t0, int nt, TxRound &R,
+               int j0 = 0, int nj = 0)
     {
+        P->split[0] += w0 > 0;
+        P->split[1] += t0 > 0;
+        P->split[2] += j0 > 0;
         const SpaceDesc &O = *dd[o];
         const SpinDesc &L = O.s[0];
         std::vector<ll> eb;
@@ -309,10 +313,12 @@ struct Builder {
             it.nw = nw;
             it.p0 = t0;
             it.pn = nt;
+            it.j0 = j0;
+            it.nj = nj ? nj : t.na;
             it.rg = (t.La + TX_ROWS - 1) / TX_ROWS;
             it.ebase = R.elems;
             eb.push_back(R.elems);
-            R.elems += (ll)t.na * nw * t.La * nt * 16;
+            R.elems += (ll)it.nj * nw * t.La * nt * 16;
             // long rows of tiles in several items: the launch's last work-groups end sooner
             const int most = std::max(2, TX_PASSES / t.nch), parts = (nt + most - 1) / most;
             for (int k = 0; k < parts; k++) {
@@ -337,9 +343,12 @@ struct Builder {
                 s.La = t.La;
                 s.r0 = -1;
                 s.ebase = eb[i];
+                s.j0 = j0;
+                s.nj = nj ? nj : t.na;
                 for (int k = 0; k < t.nsec; k++) if (t.sg[k] == l) s.r0 = t.sr0[k];
                 s.diag = t.diag && t.l1 == l;
                 if (s.r0 < 0 && !s.diag) continue;
+                if (s.nj < t.na) u.part = 1;
                 P->src.push_back(s);
                 u.nsrc++;
             }
@@ -367,6 +376,13 @@ struct Builder {
         }
     }
 
+    void count(const TxRound &R)
+    {
+        P->elems = std::max(P->elems, R.elems);
+        P->total += R.elems;
+        P->grid = std::max(P->grid, std::max(std::max(R.items, R.small), R.blocks));
+    }
+
     void rounds()
     {
         TxRound R;
@@ -391,10 +407,10 @@ struct Builder {
                 for (int i = 0; i < R.ni; i++) {
                     TxItem &a = first[i];
                     a.item0 = R.items;
-                    R.items += (ll)P->task[a.task].na * a.nw * a.rg;
+                    R.items += (ll)a.nj * a.nw * a.rg;
                 }
                 P->ab.push_back(R);
-                P->elems = std::max(P->elems, R.elems);
+                count(R);
             }
             open();
         };
@@ -406,7 +422,7 @@ struct Builder {
                 const int nt = t.nIp / 16;
                 // elements of one external part for all tasks; where one alone exceeds the
                 // buffer the tasks go one by one (their sums add up in the result), a single
-                // one past the buffer by column tiles
+                // one past the buffer by column tiles, and a column tile past it by strings JL
                 ll all = 0;
                 for (int ti : by[o][f]) all += (ll)P->task[ti].na * P->task[ti].La * 16 * nt;
                 std::vector<std::vector<int>> sets;
@@ -426,18 +442,29 @@ struct Builder {
                             piece(o, f, set, w, n, 0, nt, R);
                             w += n;
                         }
-                    } else {
+                    } else if (tile <= budget) {
                         for (int w = 0; w < t.nsv; w++)
                             for (int c = 0; c < nt;) {
                                 const ll room = (budget - R.elems) / tile;
-                                if (room <= 0 && R.elems) {
+                                if (room <= 0) {
                                     close();
                                     continue;
                                 }
-                                const int n = (int)std::min<ll>(std::max(1LL, room), nt - c);
+                                const int n = (int)std::min<ll>(room, nt - c);
                                 piece(o, f, set, w, 1, c, n, R);
                                 c += n;
                             }
+                    } else {
+                        const TxTask &a = P->task[set[0]];
+                        const ll most = std::max(1LL, budget / ((ll)a.La * 16)), parts = (a.na + most - 1) / most;
+                        for (int w = 0; w < t.nsv; w++)
+                            for (int c = 0; c < nt; c++)
+                                for (ll k = 0; k < parts; k++) {
+                                    const int j0 = (int)(a.na * k / parts), j1 = (int)(a.na * (k + 1) / parts);
+                                    close();
+                                    piece(o, f, set, w, 1, c, 1, R, j0, j1 - j0);
+                                }
+                        close();
                     }
                     // two pieces of one round may not add to the same results
                     if (sets.size() > 1) close();
@@ -484,18 +511,27 @@ struct Builder {
         }
     }
 
-    void pair_piece(int o, int f, int c0, int nc, TxRound &R)
+    // N - 2 electron strings [k0, k0 + nk) of a task
+    struct Part { int task, k0, nk; };
+
+    // one piece of a round: columns [c0, c0 + nc) of column group f for some strings of its tasks;
+    // add: a piece before has written the results
+    void pair_piece(int o, int f, int c0, int nc, const std::vector<Part> &parts, bool add, TxRound &R)
     {
         static const int ts[TX_NTYPE][2] = {{0, 0}, {0, 1}, {0, 2}, {1, 1}, {1, 2}, {2, 2}};
         const SpaceDesc &O = *dd[o];
         const SpinDesc &L = O.s[0];
         const int ncp = (int)up(nc, 16);
         std::vector<ll> eb;
-        for (int ti : pby[o][f]) {
-            const TxPairTask &t = P->ptask[ti];
+        P->split[3] += c0 > 0;
+        for (const Part &p : parts) {
+            const TxPairTask &t = P->ptask[p.task];
             TxPairItem it;
             memset(&it, 0, sizeof(it));
-            it.task = ti;
+            it.task = p.task;
+            it.k0 = p.k0;
+            it.nk = p.nk;
+            P->split[4] += p.k0 > 0;
             it.c0 = c0;
             it.nc = nc;
             it.ncp = ncp;
@@ -504,10 +540,10 @@ struct Builder {
             it.cb = t.R <= 16 ? 16 : t.R <= 32 ? 8 : t.R <= TX_RMAX ? 4 : 1;
             it.ct = (nc + 64 * it.cb - 1) / (64 * it.cb);
             it.item0 = R.items;
-            R.items += (ll)t.n * it.rg * it.ct;
+            R.items += (ll)p.nk * it.rg * it.ct;
             it.ebase = R.elems;
             eb.push_back(R.elems);
-            R.elems += (ll)t.n * t.R * ncp;
+            R.elems += (ll)p.nk * t.R * ncp;
             P->pitem.push_back(it);
             R.ni++;
         }
@@ -529,7 +565,9 @@ struct Builder {
             u.yb = O.boff[blk];
             u.blk0 = R.blocks;
             R.blocks += (ll)u.na * u.cblk;
+            u.add = add;
             const int e[3] = {L.gd[l], L.ga[l], L.gv[l]};
+            int first = 0;
             for (int k = 0; k < TX_NTYPE; k++) {
                 const int s0 = ts[k][0], s1 = ts[k][1];
                 const int n = s0 == s1 ? e[s0] * (e[s0] - 1) / 2 : e[s0] * e[s1];
@@ -537,10 +575,14 @@ struct Builder {
                 int o3[3] = {e[0], e[1], e[2]};
                 o3[s0]--;
                 o3[s1]--;
-                for (size_t i = 0; i < pby[o][f].size(); i++) {
-                    const TxPairTask &t = P->ptask[pby[o][f][i]];
+                for (size_t i = 0; i < parts.size(); i++) {
+                    const TxPairTask &t = P->ptask[parts[i].task];
                     const TxPairGroup &g = P->pg[o][t.g2];
                     if (g.d != o3[0] || g.a != o3[1] || g.v != o3[2]) continue;
+                    u.g0[u.nsec] = first;
+                    u.k0[u.nsec] = parts[i].k0;
+                    u.nk[u.nsec] = parts[i].nk;
+                    if (parts[i].nk < t.n) u.part = 1;
                     u.np[u.nsec] = n;
                     u.R[u.nsec] = t.R;
                     u.eb[u.nsec] = eb[i];
@@ -548,6 +590,11 @@ struct Builder {
                         if (t.so[s] == g.off[k] && t.sc[s] == g.cnt[k]) u.r0[u.nsec] = t.sr[s];
                     u.nsec++;
                 }
+                first += n;
+            }
+            if (add && !u.nsec) {
+                R.blocks -= (ll)u.na * u.cblk;
+                continue;
             }
             P->pout.push_back(u);
             R.no++;
@@ -565,7 +612,7 @@ struct Builder {
         auto close = [&]() {
             if (R.ni) {
                 // strings of few pairs first, in a launch of their own where they fill one
-                auto groups = [&](const TxPairItem &it) { return (ll)P->ptask[it.task].n * it.rg * it.ct; };
+                auto groups = [&](const TxPairItem &it) { return (ll)it.nk * it.rg * it.ct; };
                 auto few = [&](const TxPairItem &it) { return P->ptask[it.task].R <= TX_RSMALL; };
                 const auto first = P->pitem.begin() + R.i0, end = P->pitem.end();
                 ll small = 0;
@@ -583,7 +630,7 @@ struct Builder {
                     }
                 }
                 P->ss.push_back(R);
-                P->elems = std::max(P->elems, R.elems);
+                count(R);
             }
             open();
         };
@@ -594,20 +641,53 @@ struct Builder {
                 ll col = 0;                      // elements of 16 columns
                 for (int ti : pby[o][f]) col += (ll)P->ptask[ti].n * P->ptask[ti].R * 16;
                 const int nb = P->ptask[pby[o][f][0]].nb;
-                for (int c = 0; c < nb;) {
-                    const ll room = (budget - R.elems) / col * 16;
-                    // whole 64-column blocks, the rest of the group if it fits, at least one
-                    // block in an empty round
-                    ll n = room >= nb - c ? nb - c : room / 64 * 64;
-                    if (n <= 0) {
-                        if (R.elems) {
+                if (col * std::min(4, (nb + 15) / 16) <= budget) {
+                    std::vector<Part> all;
+                    for (int ti : pby[o][f]) all.push_back(Part{ti, 0, P->ptask[ti].n});
+                    for (int c = 0; c < nb;) {
+                        // whole 64-column blocks, or the rest of the group if it fits
+                        const ll room = (budget - R.elems) / col * 16;
+                        const ll n = room >= nb - c ? nb - c : room / 64 * 64;
+                        if (n <= 0) {
                             close();
                             continue;
                         }
-                        n = std::min<ll>(64, nb - c);
+                        pair_piece(o, f, c, (int)n, all, false, R);
+                        c += (int)n;
                     }
-                    pair_piece(o, f, c, (int)n, R);
-                    c += (int)n;
+                    continue;
+                }
+                // 64 columns of all tasks past the buffer: a range of their strings at a time, the
+                // sums of each added to those before
+                for (int c = 0; c < nb; c += 64) {
+                    const int nc = std::min(64, nb - c);
+                    std::vector<Part> parts;
+                    ll used = 0;
+                    bool add = false;
+                    auto flush = [&]() {
+                        close();
+                        pair_piece(o, f, c, nc, parts, add, R);
+                        close();
+                        parts.clear();
+                        used = 0;
+                        add = true;
+                    };
+                    for (int ti : pby[o][f]) {
+                        const TxPairTask &t = P->ptask[ti];
+                        const ll row = (ll)t.R * up(nc, 16);
+                        for (int k = 0; k < t.n;) {
+                            const ll room = (budget - used) / row;
+                            if (room <= 0 && used) {
+                                flush();
+                                continue;
+                            }
+                            const int n = (int)std::min<ll>(std::max(1LL, room), t.n - k);
+                            parts.push_back(Part{ti, k, n});
+                            used += n * row;
+                            k += n;
+                        }
+                    }
+                    flush();
                 }
             }
         close();
@@ -618,8 +698,9 @@ struct Builder {
 int tx_plan(const SpaceDesc &D, const SpaceDesc &T, ll budget, TxPlan *P)
 {
     if (D.s[0].nelec < 2 || D.s[1].nelec < 2 || D.norbs < 2) return 1;
-    P->elems = 0;
+    P->elems = P->total = P->grid = 0;
     P->ldt = P->rmax = 0;
+    memset(P->split, 0, sizeof(P->split));
     for (int s = 0; s < 2; s++) {
         if (plan_lists(D, D.s[s], P->lists[s], &P->nlst[s])) return 1;
         if (plan_pairs(D, D.s[s], P->pg[s], &P->nkl[s])) return 1;
@@ -643,5 +724,6 @@ int tx_plan(const SpaceDesc &D, const SpaceDesc &T, ll budget, TxPlan *P)
         B->pair_rounds();
     }
     delete B;
+    if (P->grid > TX_GRID) rc = 1;
     return rc;
 }

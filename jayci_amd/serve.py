@@ -26,7 +26,7 @@ from concurrent.futures import ThreadPoolExecutor
 import numpy as np
 
 from . import (Batch, Context, Hamiltonian, Space, DIRECT_TABLES, GUESS_DIAG, PREC_FP64,
-               RESTART_GDK, SYNTH_ENUC, synth_integrals)
+               RESTART_GDK, SYNTH_ENUC, contraction_plan, synth_integrals)
 
 
 def instance_spec(rng):
@@ -70,16 +70,47 @@ def ndets_of(spec):
     return None
 
 
-def lane_vector_bytes(N, krymax, kb):
+def _round_elems(n):
+    return -(-n // (16 << 20)) * (16 << 20)
+
+
+def sigma_elems(spec, N):
+    """Elements per vector of the sigma's intermediate for a space (the plan's largest round,
+    rounded up to 16M), 0 where the table kernels run; without a space's description the bound
+    that every plan keeps."""
+    if "norbs" not in spec:
+        return _round_elems(max(256 << 20, N))
+    p = contraction_plan(*(spec[k] for k in ("na", "nb", "norbs", "ndocc", "nactv", "xlvl", "rule")))
+    return _round_elems(p["elems"]) if p else 0
+
+
+def sigma_buffer_bytes(N, k, elems):
+    """Device bytes of the contraction form's buffers for k vectors at a time: inputs and results
+    in both orientations (FP64) and the intermediate."""
+    return k * (32 * N + 8 * elems)
+
+
+def lane_vector_bytes(N, krymax, kb, elems=None, at_once=None):
     """Device bytes of a lane solve over N determinants: basis and sigma vectors (2 krymax),
-    new directions and the determinant-major sigma input (2 kb), the sigma's reordered inputs
-    and results in both orientations (4 kb, FP64), its intermediate (kb times at most 2 GiB; 60
-    elements per determinant where all of it is less), the diagonal, and the lists of singles
-    and pairs (bounded by 24 bytes per determinant)."""
-    return N * (8 * (2 * krymax + 6 * kb) + 8 + 24) + kb * min(2 << 30, 480 * N)
+    new directions and the determinant-major sigma input (2 kb), the diagonal, and the sigma's
+    own: buffers for `at_once` vectors (default kb; fewer go in passes) with `elems` elements of
+    intermediate each (sigma_elems; default its bound), the block that spaces of up to 16M
+    determinants keep for at least one, and the lists of singles and pairs (24 bytes per
+    determinant), or, for the table kernels (elems 0), the transposed input in FP64,
+    its FP32 copy and the excitation tables (120 bytes per determinant for excitation level 2:
+    104 at 16e/60o)."""
+    vectors = N * (8 * (2 * krymax + 2 * kb) + 8)
+    if elems == 0:
+        return vectors + N * (12 * kb + 120)
+    if elems is None:
+        elems = sigma_elems({}, N)
+    kept = max(64 << 20, sigma_buffer_bytes(N, 1, elems)) if N <= 16 << 20 else 0
+    return (vectors + 24 * N + kept
+            + sigma_buffer_bytes(N, kb if at_once is None else at_once, elems))
 
 
-def lane_solve_params(spec, N, restol=1e-6, etol=1e-9, buftol=1e-3, budget=None, kfac=4):
+def lane_solve_params(spec, N, restol=1e-6, etol=1e-9, buftol=1e-3, budget=None, kfac=4,
+                      at_once=None):
     """Davidson settings of a lane request (a space far larger than the batched ones): one
     buffer pair for a single root, none above; a subspace of kfac times the tracked pairs
     (at least 8), or the largest that keeps lane_vector_bytes within `budget`, but not below
@@ -90,7 +121,9 @@ def lane_solve_params(spec, N, restol=1e-6, etol=1e-9, buftol=1e-3, budget=None,
     nbuf = 1 if nr == 1 else 0
     nt = nr + nbuf
     kmax, kmin = max(kfac * nt, 8), max(2 * nt, 6)
-    while budget is not None and kmax > kmin and lane_vector_bytes(N, kmax, nt) > budget:
+    elems = sigma_elems(spec, N)
+    while (budget is not None and kmax > kmin
+           and lane_vector_bytes(N, kmax, nt, elems, at_once) > budget):
         kmax -= 1
     return dict(nroots=nr, restol=restol, krymin=min(nt + 1, N), krymax=min(kmax, N),
                 refdim=min(64, N), guess=GUESS_DIAG, totfrze=SYNTH_ENUC, nbuffer=nbuf,
@@ -100,7 +133,7 @@ def lane_solve_params(spec, N, restol=1e-6, etol=1e-9, buftol=1e-3, budget=None,
 def lane_bytes(spec, N, restol=1e-6, budget=None):
     """Device bytes a lane request holds with lane_solve_params(..., budget)."""
     p = lane_solve_params(spec, N, restol, budget=budget)
-    return lane_vector_bytes(N, p["krymax"], p["nroots"] + p["nbuffer"])
+    return lane_vector_bytes(N, p["krymax"], p["nroots"] + p["nbuffer"], sigma_elems(spec, N))
 
 
 def solve_params(spec, N, restol=1e-6, nbuffer=1, etol=1e-9, kfac=8, buftol=1e-3,
@@ -186,10 +219,14 @@ class Server:
                         s["xlvl"], s["rule"])
         r.ham = Hamiltonian(r.space, m1, m2, DIRECT_TABLES)
         r.t_admit = time.perf_counter() - self.t0
+        p = lane_solve_params(s, r.space.ndets, self.restol, budget=self.budget)
+        elems = sigma_elems(s, r.space.ndets)
+        if elems:
+            # no more than admission has counted
+            r.ham.contraction(nbytes=sigma_buffer_bytes(r.space.ndets, p["nroots"] + p["nbuffer"],
+                                                        elems))
         ev, _, st = r.ham.solve(precision=self.precision, mixed_switch=self.mixed_switch,
-                                vectors=False, check=False,
-                                **lane_solve_params(s, r.space.ndets, self.restol,
-                                                    budget=self.budget))
+                                vectors=False, check=False, **p)
         self.lctx.sync()
         r.t_done = time.perf_counter() - self.t0
         r.energies = ev
