@@ -619,11 +619,12 @@ static void free_doubles(jci_ham *h)
 #define TX_ELEMS (256LL << 20)
 static long long tx_bound(const SpaceDesc &D) { return std::max(TX_ELEMS, D.ndets); }
 
+#define TX_ALIGN ((size_t)2 << 20)
 // one block for nvec vectors: the intermediate, the inputs in both orders, the results in both
 static size_t tx_pieces(const jci_ham *h, int prec, int nvec, size_t at[3])
 {
     const size_t N = (size_t)h->sp->h.ndets, sz = prec == 64 ? sizeof(double) : sizeof(float);
-    auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+    auto up = [](size_t n) { return (n + TX_ALIGN - 1) / TX_ALIGN * TX_ALIGN; };
     at[0] = 0;
     at[1] = up(sz * nvec * (size_t)h->tx->elems);
     at[2] = at[1] + up(sz * 2 * nvec * N);

@@ -140,7 +140,6 @@ struct TxOut {
     int na, ls0, nI, nIp, nsv;
     int w0, nw, t0, nt;
     int src0, nsrc;
-    int part;                        // 1: a source holds some of its strings only
     int nb;                          // strings of the first-spin group
     long long yb;                    // block offset
     long long blk0;                  // first work-group of the launch
@@ -181,12 +180,12 @@ struct TxPairItem {
 struct TxPairOut {
     int o, p, f, na, ls0, nb;
     int c0, nc, ncp, cblk;
-    int add, part;                   // 1: adds to the result; 1: not every N - 2 string is there
     long long yb, blk0;
     int nsec, np[TX_NTYPE], r0[TX_NTYPE], R[TX_NTYPE];   // pairs of I per type, rows of E
-    int g0[TX_NTYPE];                // first pair of the type in the string's list
-    int k0[TX_NTYPE], nk[TX_NTYPE];  // N - 2 strings that the round holds
     long long eb[TX_NTYPE];
+    // rounds in part: 1 adds to the result; first pair of the type in the string's list, N - 2
+    // strings that the round holds
+    int add, g0[TX_NTYPE], k0[TX_NTYPE], nk[TX_NTYPE];
 };
 
 // one spin's lists (device)
@@ -231,6 +230,7 @@ struct TxDev {
 // one launch pair (E, gather) of either part
 struct TxRound {
     int i0, ni, o0, no;              // items and outputs in their tables
+    int part;                        // 1: some strings of a source only, or results to add to
     int nsmall;                      // same spin: first items, strings of up to TX_RSMALL pairs
     long long small;                 // their work-groups
     long long items, blocks;         // waves (opposite spin) or work-groups (same spin); gather

@@ -384,9 +384,9 @@ template <> __device__ __forceinline__ const float *tx_w<float>(const TxSpin &s)
 // keep their whole W block in LDS for several column blocks, without barriers in between; the
 // others stage W one 16-deep step ahead.  In a step lane group g takes the pairs
 // 4 g .. 4 g + 3, so that its four W entries of a row are one or two 16-byte reads.  The pair
-// list is padded to whole steps by the zero row of W and by zeros in place of the vector's rows
-// (an infinite element would make NaN of the padding).  Offsets are 32 bits while the vector is
-// below 4 GB (BIG: 64).  16e/28o FP64 writes 31 GB in 17.6 ms (one
+// list is padded to whole steps by the zero row of W and the last pair's row of the vector (an
+// infinite element there makes NaN of the padding, in results it is connected to anyway).  Offsets
+// are 32 bits while the vector is below 4 GB (BIG: 64).  16e/28o FP64 writes 31 GB in 17.6 ms (one
 // 64-column block per work-group: 23.1 ms).
 // RT: row tiles of a work-group, 4, or 2 for strings of up to 32 pairs, whose work-groups are the
 // most and the shortest: with half the registers and a quarter of the LDS seven fit on a CU
@@ -416,17 +416,12 @@ __global__ __launch_bounds__(256, RT == 2 ? 6 : 4) void k_tx_ess(TxDev A, TxRoun
     O *__restrict__ off = (O *)tx_smem;
     int *__restrict__ pr = (int *)(off + Rp);
     for (int r = tid; r < Rp; r += 256) {
-        int p = np;
-        O o = (O)t.sx[0];
-        if (r < Rr) {
-            int s = 0;
-            while (s + 1 < t.nsec && t.sr[s + 1] <= r) s++;
-            const int2 en = S.kl[t.lbase + K2 * t.Rfull + t.so[s] + (r - t.sr[s])];
-            o = (O)(t.sx[s] + (long long)en.x * t.nb);
-            p = en.y;
-        }
-        off[r] = o;
-        pr[r] = p;
+        const int q = std::min(r, Rr - 1);
+        int s = 0;
+        while (s + 1 < t.nsec && t.sr[s + 1] <= q) s++;
+        const int2 en = S.kl[t.lbase + K2 * t.Rfull + t.so[s] + (q - t.sr[s])];
+        off[r] = (O)(t.sx[s] + (long long)en.x * t.nb);
+        pr[r] = r < Rr ? en.y : np;
     }
     __syncthreads();
     const T *__restrict__ W = tx_w<T>(S);
@@ -462,15 +457,6 @@ __global__ __launch_bounds__(256, RT == 2 ? 6 : 4) void k_tx_ess(TxDev A, TxRoun
             rb[j] = BIG ? x[(long long)o + xc] : tx_at(x, (uint32_t)o + xc);
         }
     };
-    // the vector's operands of step k0
-    auto take = [&](int k0, T *b) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) b[j] = rb[j];
-        if (k0 + 16 > Rr) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) if (k0 + kk * 4 + j >= Rr) b[j] = (T)0;
-        }
-    };
     auto store = [&](int c) __attribute__((always_inline)) {
         if (c >= ncp) return;
 #pragma unroll
@@ -497,7 +483,8 @@ __global__ __launch_bounds__(256, RT == 2 ? 6 : 4) void k_tx_ess(TxDev A, TxRoun
             load_x(0, xc);
             for (int k0 = 0; k0 < Rp; k0 += 16) {
                 T b[4];
-                take(k0, b);
+#pragma unroll
+                for (int j = 0; j < 4; j++) b[j] = rb[j];
                 if (k0 + 16 < Rp) load_x(k0 + 16, xc);
 #pragma unroll
                 for (int i = 0; i < RT; i++)
@@ -524,7 +511,8 @@ __global__ __launch_bounds__(256, RT == 2 ? 6 : 4) void k_tx_ess(TxDev A, TxRoun
     int buf = 0;
     for (int k0 = 0; k0 < Rp; k0 += 16) {
         T b[4];
-        take(k0, b);
+#pragma unroll
+        for (int j = 0; j < 4; j++) b[j] = rb[j];
         const bool more = k0 + 16 < Rp;
         if (more) {
             load_w(k0 + 16);
@@ -597,12 +585,12 @@ __device__ __forceinline__ int tx_place(bool keep, int *cnt, int *n)
 }
 
 // the same-spin sums: y(I, c) = sum over the pairs of I, one E row each (coalesced); the first
-// writer of the result.  The rows' offsets are set up in LDS once for the string's columns.  Where
-// a round holds some of the N - 2 electron strings only, the entries of the others are left out and
-// the sums of its successors are added.
+// writer of the result.  The rows' offsets are set up in LDS once for the string's columns.  PART:
+// the round holds some of the N - 2 electron strings only, the entries of the others are left out
+// and the sums of its successors are added.
 #define TX_ENT 512
 #define TX_SRC 64            // one wave's scan
-template <typename T>
+template <typename T, bool PART>
 __global__ __launch_bounds__(256) void k_tx_gss(TxDev A, TxRound R, long long N,
                                                 const T *__restrict__ E, double *__restrict__ y0,
                                                 double *__restrict__ y1)
@@ -622,15 +610,15 @@ __global__ __launch_bounds__(256) void k_tx_gss(TxDev A, TxRound R, long long N,
     T acc = (T)0;
     // offset of entry r (complemented: less), false where its N - 2 string is not in the round
     auto entry = [&](int r, long long &o) __attribute__((always_inline)) {
-        int s = 0;
-        while (r >= t.np[s]) r -= t.np[s++];
-        const int2 e = g[t.g0[s] + r];
-        const int K = e.x - t.k0[s];
+        int s = 0, m = r;
+        while (m >= t.np[s]) m -= t.np[s++];
+        const int2 e = g[PART ? t.g0[s] + m : r];
+        const int K = PART ? e.x - t.k0[s] : e.x;
         o = t.eb[s] + ((long long)K * t.R[s] + t.r0[s] + (e.y & 0x7FFFFFFF)) * t.ncp;
         if (e.y < 0) o = ~o;
-        return (unsigned)K < (unsigned)t.nk[s];
+        return !PART || (unsigned)K < (unsigned)t.nk[s];
     };
-    if (!t.part) {
+    if (!PART) {
         for (int m0 = 0; m0 < np; m0 += TX_ENT) {
             const int n = std::min(TX_ENT, np - m0);
             if (m0) __syncthreads();
@@ -658,7 +646,7 @@ __global__ __launch_bounds__(256) void k_tx_gss(TxDev A, TxRound R, long long N,
     if (c >= t.nc) return;
     const long long n = t.yb + (long long)il * t.nb + t.c0 + c;
     double *y = (t.o ? y1 : y0) + (k * N + n);
-    *y = t.add ? *y + (double)acc : (double)acc;
+    *y = PART && t.add ? *y + (double)acc : (double)acc;
 }
 
 // ---- opposite-spin part ------------------------------------------------------------------------
@@ -970,9 +958,9 @@ __global__ __launch_bounds__(256, TxV<T>::WPE) void k_tx_eab(
 // 256 columns of one string per work-group.  The rows' offsets, over all sources, are set up in
 // LDS first: the sum is then one stream of loads, eight in flight per lane, at the copy rate for
 // large spaces, and small ones (chains of list loads before) take 16.2 -> 9.1 us at 4a4b/10o and
-// 0.22 -> 0.19 ms at 7a6b/17o.  Where a round holds some of a source's strings JL only, the entries
+// 0.22 -> 0.19 ms at 7a6b/17o.  PART: the round holds some of a source's strings JL only, the entries
 // of the others are left out.
-template <typename T>
+template <typename T, bool PART>
 __global__ __launch_bounds__(256) void k_tx_gab(TxDev A, TxRound R, long long N,
                                                 const T *__restrict__ E, double *__restrict__ y0,
                                                 double *__restrict__ y1)
@@ -1030,12 +1018,12 @@ __global__ __launch_bounds__(256) void k_tx_gab(TxDev A, TxRound R, long long N,
                 row = q.r0 + S.rk[e];
                 neg = en.y & (1 << 12);
             }
-            J -= q.j0;
+            if (PART) J -= q.j0;
             o = q.ebase + J * t.nw * rows + row * ntc;
             if (neg) o = ~o;
-            return (unsigned long long)J < (unsigned long long)q.nj;
+            return !PART || (unsigned long long)J < (unsigned long long)q.nj;
         };
-        if (!t.part) {
+        if (!PART) {
             for (int m0 = 0; m0 < all; m0 += TX_ENT) {
                 const int n = std::min(TX_ENT, all - m0);
                 if (m0) __syncthreads();
@@ -1092,8 +1080,12 @@ static int tx_run(int nvec, const TxDev &D, const TxPlan &P, const TxVec &V, T *
             else hipLaunchKernelGGL((k_tx_ess<T, false, 4>), g, dim3(256), rp * 8, st, D, R, i0, ni, V.N, x0, x1, E);
             TX_CHECK();
         }
-        hipLaunchKernelGGL(k_tx_gss<T>, dim3((unsigned)R.blocks, nvec), dim3(256), 0, st, D, R, V.N, E,
-                           V.y0, V.y1);
+        if (R.part)
+            hipLaunchKernelGGL((k_tx_gss<T, true>), dim3((unsigned)R.blocks, nvec), dim3(256), 0, st, D, R,
+                               V.N, E, V.y0, V.y1);
+        else
+            hipLaunchKernelGGL((k_tx_gss<T, false>), dim3((unsigned)R.blocks, nvec), dim3(256), 0, st, D, R,
+                               V.N, E, V.y0, V.y1);
         TX_CHECK();
     }
     const int ldt = P.ldt + TxV<T>::PAD;
@@ -1105,8 +1097,12 @@ static int tx_run(int nvec, const TxDev &D, const TxPlan &P, const TxVec &V, T *
                            dim3(256), (unsigned)(64 * ldt * sizeof(T)), st, D, R, nvec, kper, V.N, x0,
                            x1, E, ldt);
         TX_CHECK();
-        hipLaunchKernelGGL(k_tx_gab<T>, dim3((unsigned)R.blocks, nvec), dim3(256), 0, st, D, R, V.N, E,
-                           V.y0, V.y1);
+        if (R.part)
+            hipLaunchKernelGGL((k_tx_gab<T, true>), dim3((unsigned)R.blocks, nvec), dim3(256), 0, st, D, R,
+                               V.N, E, V.y0, V.y1);
+        else
+            hipLaunchKernelGGL((k_tx_gab<T, false>), dim3((unsigned)R.blocks, nvec), dim3(256), 0, st, D, R,
+                               V.N, E, V.y0, V.y1);
         TX_CHECK();
     }
     return 0;

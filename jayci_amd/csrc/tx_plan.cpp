@@ -348,7 +348,7 @@ struct Builder {
                 for (int k = 0; k < t.nsec; k++) if (t.sg[k] == l) s.r0 = t.sr0[k];
                 s.diag = t.diag && t.l1 == l;
                 if (s.r0 < 0 && !s.diag) continue;
-                if (s.nj < t.na) u.part = 1;
+                if (s.nj < t.na) R.part = 1;
                 P->src.push_back(s);
                 u.nsrc++;
             }
@@ -523,6 +523,8 @@ struct Builder {
         const SpinDesc &L = O.s[0];
         const int ncp = (int)up(nc, 16);
         std::vector<ll> eb;
+        // (the gather takes a string's pairs as they come only where all tasks are there)
+        if (add || parts.size() != pby[o][f].size()) R.part = 1;
         P->split[3] += c0 > 0;
         for (const Part &p : parts) {
             const TxPairTask &t = P->ptask[p.task];
@@ -532,6 +534,7 @@ struct Builder {
             it.k0 = p.k0;
             it.nk = p.nk;
             P->split[4] += p.k0 > 0;
+            if (p.nk < t.n) R.part = 1;
             it.c0 = c0;
             it.nc = nc;
             it.ncp = ncp;
@@ -582,7 +585,6 @@ struct Builder {
                     u.g0[u.nsec] = first;
                     u.k0[u.nsec] = parts[i].k0;
                     u.nk[u.nsec] = parts[i].nk;
-                    if (parts[i].nk < t.n) u.part = 1;
                     u.np[u.nsec] = n;
                     u.R[u.nsec] = t.R;
                     u.eb[u.nsec] = eb[i];
