@@ -54,6 +54,22 @@
 // a SIMD.  More rows per scattered tile at two waves: 16e/28o FP64 93 -> 97 ms; 48 at three in
 // FP32, two vectors 16e/20o: 22.0 -> 22.7 ms
 #define TX_ROWS 32
+// Spaces that keep the table kernels: those with few internal orbitals and many excitations, whose
+// column tiles of 16 internal parts are mostly padding and whose blocks are few and large, which
+// the tables suit.  Estimated times, FP64, one vector: an element of the intermediate 16 ps
+// (opposite spin) and 7 ps (same spin); the tables 1.1 ps per opposite-spin connection and 0.25 us
+// per connection of the best connected determinant, one after another.  Estimated and measured
+// speed of the contraction form relative to the tables (FP64, one vector / three): 2a2b in 60
+// orbitals (2 active, 4 excitations) 0.53, 0.23 / 0.24 (186 against 44 ms); 4a4b/20 (2, 6) 0.32,
+// 0.31 / 0.29 (37.8 against 11.9); 5a5b/18 (4, 6) 0.81, 0.81 / 0.86 (31.9 against 25.9); 3a3b/20 (2,
+// 4) 0.96, 1.01 / 0.72 (0.96 both); on the other side 4a4b/24 (4, 4) 1.17, 1.59 / 1.36 (6.7 against
+// 10.6), 7a7b/14 (2 doubly occupied + 10, 2) 1.40, 2.49 / 1.58 (5.9 against 14.7), 16e/20o 1.89,
+// 2.93 / 2.07 (18 against 53).  Of 87 spaces none on the tables' side was more than 1.1 times
+// faster in the contraction form (FP64), none on the other more than 1.15 times slower.
+#define TX_COST_AB 16e-12
+#define TX_COST_SS 7e-12
+#define TX_COST_ENTRY 1.1e-12
+#define TX_COST_CHAIN 0.25e-6
 // work-groups of a launch: 256 threads each, and a grid holds fewer than 2^32 threads
 #define TX_GRID ((1LL << 24) - 1024)
 #define TX_PAD 0x7FF00000u   // list entry of a padded row or column (no position, string 0)
@@ -388,6 +404,7 @@ struct TxPlan {
     std::vector<int> q;
     std::vector<TxRound> ab, ss;           // rounds of the two parts
     long long elems, total;                // largest E of a round, sum over the rounds
+    long long sum[2];                      // of the opposite-spin and the same-spin rounds
     long long grid;                        // most work-groups of a launch
     int split[5];                          // pieces that start past the first external part, column
                                            // tile, JL (opposite spin), column, N - 2 string (same spin)
@@ -397,7 +414,8 @@ struct TxPlan {
 };
 // budget: bound on a round's E (what one string of a task needs for one column tile, or one N - 2
 // electron string for 64 columns, where that is more).
-// 0: built; 1: the space is outside what the lists can index (the caller keeps the tables)
+// 0: built; 1: the space is outside what the lists can index, or the tables are faster on it (the
+// caller keeps them)
 int tx_plan(const SpaceDesc &D, const SpaceDesc &T, long long budget, TxPlan *P);
 
 // ---- kernels (sigma_tx.hip) ----

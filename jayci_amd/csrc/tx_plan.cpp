@@ -376,8 +376,9 @@ struct Builder {
         }
     }
 
-    void count(const TxRound &R)
+    void count(const TxRound &R, int part)
     {
+        P->sum[part] += R.elems;
         P->elems = std::max(P->elems, R.elems);
         P->total += R.elems;
         P->grid = std::max(P->grid, std::max(std::max(R.items, R.small), R.blocks));
@@ -410,7 +411,7 @@ struct Builder {
                     R.items += (ll)a.nj * a.nw * a.rg;
                 }
                 P->ab.push_back(R);
-                count(R);
+                count(R, 0);
             }
             open();
         };
@@ -632,7 +633,7 @@ struct Builder {
                     }
                 }
                 P->ss.push_back(R);
-                count(R);
+                count(R, 1);
             }
             open();
         };
@@ -702,6 +703,7 @@ int tx_plan(const SpaceDesc &D, const SpaceDesc &T, ll budget, TxPlan *P)
     if (D.s[0].nelec < 2 || D.s[1].nelec < 2 || D.norbs < 2) return 1;
     P->elems = P->total = P->grid = 0;
     P->ldt = P->rmax = 0;
+    P->sum[0] = P->sum[1] = 0;
     memset(P->split, 0, sizeof(P->split));
     for (int s = 0; s < 2; s++) {
         if (plan_lists(D, D.s[s], P->lists[s], &P->nlst[s])) return 1;
@@ -727,5 +729,17 @@ int tx_plan(const SpaceDesc &D, const SpaceDesc &T, ll budget, TxPlan *P)
     }
     delete B;
     if (P->grid > TX_GRID) rc = 1;
+    // the table kernels' estimate: opposite-spin connections, and those of one determinant
+    double entries = 0.0, chain = 0.0;
+    for (int b = 0; b < D.nblk; b++) {
+        double each = 0.0;
+        for (int c = 0; c < D.nblk; c++)
+            each += (double)std::max(0LL, singles(D, D.s[0], D.bp[b], D.bp[c])) *
+                    (double)std::max(0LL, singles(D, D.s[1], D.bq[b], D.bq[c]));
+        entries += each * (double)D.s[0].gn[D.bp[b]] * (double)D.s[1].gn[D.bq[b]];
+        chain = std::max(chain, each);
+    }
+    if (TX_COST_AB * P->sum[0] + TX_COST_SS * P->sum[1] > TX_COST_ENTRY * entries + TX_COST_CHAIN * chain)
+        rc = 1;
     return rc;
 }

@@ -65,3 +65,19 @@ def test_lane_counts_the_planned_buffers(J):
         assert need <= serve.lane_vector_bytes(N, p["krymax"], nt, e, at_once) <= 300e9
     # one block: the table kernels' transposed input and tables
     assert serve.sigma_elems(dict(d, ndocc=0, nactv=60, xlvl=0), 10 ** 6) == 0
+
+
+@pytest.mark.parametrize("spec,taken", [
+    # few internal orbitals, many excitations: the table kernels are faster
+    ((2, 2, 60, 0, 2, 4, 0), False), ((2, 2, 50, 1, 0, 4, 0), False), ((3, 3, 34, 0, 2, 6, 0), False),
+    ((4, 4, 20, 0, 2, 6, 0), False), ((4, 4, 16, 0, 4, 8, 0), False), ((4, 4, 30, 2, 1, 4, 0), False),
+    ((5, 5, 18, 0, 4, 6, 0), False), ((3, 3, 26, 0, 2, 4, 0), False),
+    # few internal orbitals, two excitations or few connections; and truncated CAS spaces
+    ((2, 2, 60, 0, 2, 2, 0), True), ((8, 8, 60, 8, 0, 2, 1), True), ((4, 4, 24, 0, 4, 4, 0), True),
+    ((3, 3, 16, 0, 2, 4, 0), True), ((2, 2, 6, 1, 2, 2, 1), True), ((4, 4, 10, 2, 4, 2, 1), True),
+    ((7, 7, 14, 2, 10, 2, 1), True), ((6, 6, 16, 0, 12, 2, 0), True), ((8, 8, 60, 4, 8, 2, 1), True),
+    # one electron of a spin; one block
+    ((3, 1, 8, 1, 3, 2, 0), False), ((3, 3, 8, 0, 8, 0, 1), False),
+])
+def test_form_chosen(J, spec, taken):
+    assert (J.contraction_plan(*spec) is not None) == taken
