@@ -765,6 +765,20 @@ static int tx_tables(jci_ham *h)
     return 0;
 }
 
+// the contraction form's memory; the FAST methods run the table kernels then
+static void drop_tx(jci_ham *h)
+{
+    hipStreamSynchronize(h->sp->ctx->stream);
+    for (int i = 0; i < h->tx_nmem; i++) hipFree(h->tx_mem[i]);
+    h->tx_nmem = 0;
+    hipFree(h->d_txtab);
+    h->d_txtab = nullptr;
+    tx_drop(&h->d_txkeep, &h->txkeep_bytes);
+    tx_drop(&h->d_txmore, &h->txmore_bytes);
+    delete h->tx;
+    h->tx = nullptr;
+}
+
 // lists and tables of the contraction form; leaves h->tx null where it does not apply
 static int build_tx(jci_ham *h)
 {
@@ -810,8 +824,13 @@ static int build_tx(jci_ham *h)
         RCHECK(tx_alloc(h, sizeof(float) * nrow * d.ms, (void **)&x.m32));
         TxList *dl = nullptr;
         TxPairGroup *dp = nullptr;
-        JCI_CHECK(hipMallocAsync((void **)&dl, sizeof(TxList) * P->lists[sp].size(), c->stream));
-        JCI_CHECK(hipMallocAsync((void **)&dp, sizeof(TxPairGroup) * P->pg[sp].size(), c->stream));
+        if (hipMallocAsync((void **)&dl, sizeof(TxList) * P->lists[sp].size(), c->stream) != hipSuccess ||
+            hipMallocAsync((void **)&dp, sizeof(TxPairGroup) * P->pg[sp].size(), c->stream) != hipSuccess) {
+            (void)hipGetLastError();
+            if (dl) hipFreeAsync(dl, c->stream);
+            jci_set_error("contraction lists: out of device memory");
+            return -3;
+        }
         JCI_CHECK(hipMemcpyAsync(dl, P->lists[sp].data(), sizeof(TxList) * P->lists[sp].size(),
                                  hipMemcpyHostToDevice, c->stream));
         JCI_CHECK(hipMemcpyAsync(dp, P->pg[sp].data(), sizeof(TxPairGroup) * P->pg[sp].size(),
@@ -886,26 +905,52 @@ static int build_fast(jci_ham *h, int W)
     h->fast_xg = 64;
     const int widths[3] = {64, 128, 256};
     for (int wi = 0; wi < 3; wi++) h->fast[wi].W = widths[wi];
-    if (multi) RCHECK(build_tx(h));
+    if (multi) {
+        // without memory for the contraction form the table kernels serve the space
+        const int rc = build_tx(h);
+        if (rc) drop_tx(h);
+        if (rc && rc != -3) return rc;
+    }
     h->have_fast = 1;
     if (!h->tx) RCHECK(ensure_tables(h));
     return multi ? 0 : build_gf(h);
 }
 
+static void free_tables(jci_ham *h)
+{
+    hipStreamSynchronize(h->sp->ctx->stream);
+    free_doubles(h);
+    auto drop = [](auto **p) {
+        hipFree(*p);
+        *p = nullptr;
+    };
+    for (int i = 0; i < 3; i++) drop(&h->d_tile_off[i]);
+    for (int i = 0; i < 3; i++) drop(&h->d_tileT_off[i]);
+    for (int i = 0; i < 4; i++) drop(&h->d_cls_off[i]);
+    for (int i = 0; i < 16; i++) drop(&h->d_ooff[i]);
+    drop(&h->d_descT);
+    drop(&h->d_tt_off);
+    drop(&h->d_xT);
+    h->xT_bytes = 0;
+    h->have_tables = 0;
+}
+
+static int make_tables(jci_ham *h);
+
 static int ensure_tables(jci_ham *h)
 {
     if (h->have_tables) return 0;
+    const int rc = make_tables(h);
+    if (rc) free_tables(h);   // whatever was built: a later call starts anew
+    return rc;
+}
+
+static int make_tables(jci_ham *h)
+{
     jci_space *s = h->sp;
     jci_ctx *c = s->ctx;
     const SpaceDesc &D = s->h;
-    if (!h->d_off2[0]) {
-        const int rc = build_exc(h, 2);
-        if (rc) {
-            hipStreamSynchronize(c->stream);
-            free_doubles(h);
-            return rc;
-        }
-    }
+    if (!h->d_off2[0]) RCHECK(build_exc(h, 2));
     const int mp = D.norbs * (D.norbs + 1) / 2;
     const int widths[3] = {64, 128, 256};
     for (int wi = 0; wi < 3; wi++) {
@@ -933,7 +978,6 @@ static int ensure_tables(jci_ham *h)
         a.m1 = mp;
         a.m1int = (D.ndocc + D.nactv) * (D.ndocc + D.nactv + 1) / 2;
         a.W = Wd;
-        a.A = 0;
         a.ldy = 0;
         a.xg = 0;
         a.tout = 0;
@@ -1059,10 +1103,8 @@ JCI_API void jci_ham_destroy(jci_ham *h)
     if (!h) return;
     hipSetDevice(h->sp->ctx->device);
     hipStreamSynchronize(h->sp->ctx->stream);
-    for (int i = 0; i < h->tx_nmem; i++) hipFree(h->tx_mem[i]);
-    hipFree(h->d_txtab); hipFree(h->d_txkeep); hipFree(h->d_txmore);
-    delete h->tx;
-    free_doubles(h);
+    drop_tx(h);
+    free_tables(h);
     hipFree(h->d_m1); hipFree(h->d_m2); hipFree(h->d_hd);
     hipFree(h->d_rowptr); hipFree(h->d_col); hipFree(h->d_val64); hipFree(h->d_val32);
     hipFree(h->d_xf);
@@ -1071,13 +1113,6 @@ JCI_API void jci_ham_destroy(jci_ham *h)
         hipFree(h->d_off1[sp]); hipFree(h->d_e1[sp]); hipFree(h->d_goff1[sp]); hipFree(h->d_v1[sp]);
     }
     hipFree(h->d_m2sq);
-    for (int wi = 0; wi < 3; wi++) hipFree(h->d_tile_off[wi]);
-    for (int wi = 0; wi < 3; wi++) hipFree(h->d_tileT_off[wi]);
-    for (int ci = 0; ci < 4; ci++) hipFree(h->d_cls_off[ci]);
-    for (int i = 0; i < 16; i++) hipFree(h->d_ooff[i]);
-    hipFree(h->d_descT);
-    hipFree(h->d_tt_off);
-    hipFree(h->d_xT);
     if (h->d_gfH64[1] != h->d_gfH64[0]) { hipFree(h->d_gfH64[1]); hipFree(h->d_gfH32[1]); }
     hipFree(h->d_gfH64[0]); hipFree(h->d_gfH32[0]);
     hipFree(h->d_gfM64); hipFree(h->d_gfM32); hipFree(h->d_gfla); hipFree(h->d_gflb);
