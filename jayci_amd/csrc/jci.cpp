@@ -1727,22 +1727,19 @@ static int use_tables(jci_ham *h)
 JCI_API int jci_ham_fast_tiles(jci_ham *h, int *width, int *chunk)
 {
     if (!h->have_fast) { jci_set_error("ham: no excitation tables"); return -1; }
-    if ((width && *width >= 0) || (chunk && *chunk >= 0)) RCHECK(use_tables(h));
-    if (width && *width >= 0) {
-        int wi = *width == 64 ? 0 : *width == 128 ? 1 : *width == 256 ? 2 : *width == 0 ? 3 : -1;
-        if (wi < 0) {
-            jci_set_error("ham: tile width %d not available (64, 128, 256, or 0: per block)", *width);
-            return -1;
-        }
-        h->fast_w = wi;
+    const bool set_w = width && *width >= 0, set_a = chunk && *chunk >= 0;
+    const int wi = !set_w ? h->fast_w : *width == 64 ? 0 : *width == 128 ? 1 : *width == 256 ? 2 : *width == 0 ? 3 : -1;
+    if (wi < 0) {
+        jci_set_error("ham: tile width %d not available (64, 128, 256, or 0: per block)", *width);
+        return -1;
     }
-    if (chunk && *chunk >= 0) {
-        if (*chunk != 0 && *chunk != 1 && *chunk != 2 && *chunk != 4 && *chunk != 8) {
-            jci_set_error("ham: alpha chunk %d not available (0, 1, 2, 4, 8)", *chunk);
-            return -1;
-        }
-        for (int w2 = 0; w2 < 3; w2++) h->fast[w2].A = *chunk;
+    if (set_a && *chunk != 0 && *chunk != 1 && *chunk != 2 && *chunk != 4 && *chunk != 8) {
+        jci_set_error("ham: alpha chunk %d not available (0, 1, 2, 4, 8)", *chunk);
+        return -1;
     }
+    if (set_w || set_a) RCHECK(use_tables(h));
+    h->fast_w = wi;
+    if (set_a) for (int w2 = 0; w2 < 3; w2++) h->fast[w2].A = *chunk;
     if (width) *width = h->fast_w == 3 ? 0 : h->fast[h->fast_w].W;
     if (chunk) *chunk = h->fast[h->fast_w == 3 ? 0 : h->fast_w].A;
     return 0;
@@ -1764,11 +1761,9 @@ JCI_API int jci_ham_fast_split(jci_ham *h, int *split)
 JCI_API int jci_ham_fast_xcd(jci_ham *h, int *group, int *chunk_major)
 {
     if (!h->have_fast) { jci_set_error("ham: no excitation tables"); return -1; }
+    if (group && *group > 4096) { jci_set_error("ham: XCD run of %d tiles too long", *group); return -1; }
     if ((group && *group >= 0) || (chunk_major && *chunk_major >= 0)) RCHECK(use_tables(h));
-    if (group && *group >= 0) {
-        if (*group > 4096) { jci_set_error("ham: XCD run of %d tiles too long", *group); return -1; }
-        h->fast_xg = *group;
-    }
+    if (group && *group >= 0) h->fast_xg = *group;
     if (chunk_major && *chunk_major >= 0) h->fast_cm = *chunk_major ? 1 : 0;
     if (group) *group = h->fast_xg;
     if (chunk_major) *chunk_major = h->fast_cm;
