@@ -368,7 +368,8 @@ int jci_ham_fast_xcd(jci_ham *h, int *group, int *chunk_major);
  * determinants where they are more; plans anew and moves the buffers, so not while a captured
  * graph uses them); *bytes > 0: bound on the block that
  * calls of several vectors grow (beyond it, or where device memory ends, they go in passes).
- * Other values keep.  Returned: the form in use, the elements of the largest round, the bytes
+ * Other values keep.  Returned: the form in use (FAST64's; the
+ * autotuner chooses one for each precision), the elements of the largest round, the bytes
  * of the buffers held, and the numbers of opposite-spin and same-spin rounds (0 without the form;
  * any pointer may be NULL) */
 int jci_ham_contraction(jci_ham *h, int *use, long long *elems, long long *bytes, int rounds[2]);

@@ -304,7 +304,7 @@ struct jci_ham {
     // methods where it applies; a table-kernel shape chosen by the caller turns it off
     TxPlan *tx;
     TxDev txd;
-    int tx_off;
+    int tx_off[2];              // FP64, FP32
     void *tx_mem[24];           // device arrays behind txd
     int tx_nmem;
     long long *d_ttx, nttx;     // 16 x 16 transpose tiles per block
@@ -1392,7 +1392,7 @@ static int fast_run(jci_ham *h, int method, int nvec, const double *x, double *y
     const long long N = h->sp->h.ndets;
     if (!h->have_fast) { jci_set_error("sigma: no excitation tables (JCI_DIRECT_TABLES)"); return -1; }
     const int prec = method == JCI_SIGMA_FAST64 ? 64 : 32;
-    if (h->tx && !h->tx_off) {
+    if (h->tx && !h->tx_off[prec == 32]) {
         const long long ys = ldy ? 1 : nvec, yk = ldy ? ldy : 1;
         if (!s) return tx_sigma(h, prec, nvec, x, nvec, 1, y, ys, yk, 1);
         // allocation-free: the staging of the table kernels bounds the sizes taken, the vectors
@@ -1625,6 +1625,64 @@ JCI_API int jci_bench_sigma(jci_ham *h, int method, int nvec, int reps, double *
     return rc;
 }
 
+// best tile width x alpha chunk x passes of the table kernels (FP64) and their time
+static int tune_tables(jci_ham *h, int nvec, int reps, double *best_ms)
+{
+    *best_ms = 1e300;
+    int best_w = h->fast_w, best_a = 0, best_split = h->fast_split;
+    const int chunks[4] = {0, 1, 2, 4};
+    for (int sp = 0; sp < 3; sp++)
+        for (int wi = 0; wi < 4; wi++)
+            for (int ai = 0; ai < 4; ai++) {
+                if (h->fast_split != sp) {
+                    h->fast_split = sp;
+                    RCHECK(set_orient(h));
+                }
+                h->fast_w = wi;
+                for (int w2 = 0; w2 < 3; w2++) h->fast[w2].A = chunks[ai];
+                double ms = 0;
+                RCHECK(jci_bench_sigma(h, JCI_SIGMA_FAST64, nvec, reps, &ms));
+                if (ms < *best_ms) {
+                    *best_ms = ms; best_w = wi; best_a = chunks[ai]; best_split = sp;
+                }
+            }
+    h->fast_w = best_w;
+    if (h->fast_split != best_split) {
+        h->fast_split = best_split;
+        RCHECK(set_orient(h));
+    }
+    for (int w2 = 0; w2 < 3; w2++) h->fast[w2].A = best_a;
+    return 0;
+}
+
+// the FAST methods' forms, each precision's by its own times.  Tables built for this alone go
+// again where neither takes them; without memory for them the contraction form stays.
+static int tune_fast(jci_ham *h, int nvec, int reps, double *t)
+{
+    const int had = h->have_tables;
+    double form[2] = {1e300, 1e300}, tab[2];
+    if (h->tx) {
+        h->tx_off[0] = h->tx_off[1] = 0;
+        RCHECK(jci_bench_sigma(h, JCI_SIGMA_FAST64, nvec, reps, &form[0]));
+        RCHECK(jci_bench_sigma(h, JCI_SIGMA_FAST32, nvec, reps, &form[1]));
+        const int rc = ensure_tables(h);
+        if (rc && rc != -3) return rc;
+        if (rc) {
+            t[JCI_SIGMA_FAST64] = form[0];
+            t[JCI_SIGMA_FAST32] = form[1];
+            return 0;
+        }
+        h->tx_off[0] = h->tx_off[1] = 1;
+    }
+    RCHECK(tune_tables(h, nvec, reps, &tab[0]));
+    RCHECK(jci_bench_sigma(h, JCI_SIGMA_FAST32, nvec, reps, &tab[1]));
+    for (int i = 0; i < 2; i++) h->tx_off[i] = form[i] > tab[i];
+    if (!had && !h->tx_off[0] && !h->tx_off[1]) free_tables(h);
+    t[JCI_SIGMA_FAST64] = std::min(form[0], tab[0]);
+    t[JCI_SIGMA_FAST32] = std::min(form[1], tab[1]);
+    return 0;
+}
+
 // Times every available sigma variant (pair list, matrix-free with tile widths 64/128/256,
 // one-thread-per-row) for nvec vectors and makes the fastest FP64 and FP32 ones the
 // defaults of JCI_SIGMA_AUTO.  times[] (may be NULL) receives ms per launch indexed by
@@ -1633,43 +1691,15 @@ JCI_API int jci_ham_autotune(jci_ham *h, int nvec, int reps, int *best64, int *b
                              double *times)
 {
     double t[JCI_SIGMA_GEMM32 + 1] = {0};
-    double best_w_ms = 1e300;
-    int best_w = h->fast_w;
     if (h->have_fast) {
-        double tx_ms = 1e300;
-        if (h->tx) {
-            h->tx_off = 0;
-            RCHECK(jci_bench_sigma(h, JCI_SIGMA_FAST64, nvec, reps, &tx_ms));
+        // a failure leaves the forms as they were
+        const int off[2] = {h->tx_off[0], h->tx_off[1]};
+        const int rc = tune_fast(h, nvec, reps, t);
+        if (rc) {
+            h->tx_off[0] = off[0];
+            h->tx_off[1] = off[1];
+            return rc;
         }
-        RCHECK(ensure_tables(h));
-        h->tx_off = 1;
-        // beta tile width x alpha chunk of the table kernel
-        int best_a = 0, best_split = h->fast_split;
-        const int chunks[4] = {0, 1, 2, 4};
-        for (int sp = 0; sp < 3; sp++)
-            for (int wi = 0; wi < 4; wi++)
-                for (int ai = 0; ai < 4; ai++) {
-                    if (h->fast_split != sp) {
-                        h->fast_split = sp;
-                        RCHECK(set_orient(h));
-                    }
-                    h->fast_w = wi;
-                    for (int w2 = 0; w2 < 3; w2++) h->fast[w2].A = chunks[ai];
-                    double ms = 0;
-                    RCHECK(jci_bench_sigma(h, JCI_SIGMA_FAST64, nvec, reps, &ms));
-                    if (ms < best_w_ms) {
-                        best_w_ms = ms; best_w = wi; best_a = chunks[ai]; best_split = sp;
-                    }
-                }
-        h->fast_w = best_w;
-        if (h->fast_split != best_split) {
-            h->fast_split = best_split;
-            RCHECK(set_orient(h));
-        }
-        for (int w2 = 0; w2 < 3; w2++) h->fast[w2].A = best_a;
-        if (tx_ms <= best_w_ms) h->tx_off = 0;
-        t[JCI_SIGMA_FAST64] = std::min(tx_ms, best_w_ms);
-        RCHECK(jci_bench_sigma(h, JCI_SIGMA_FAST32, nvec, reps, &t[JCI_SIGMA_FAST32]));
     }
     if (h->have_fci) {
         RCHECK(jci_bench_sigma(h, JCI_SIGMA_FCI64, nvec, reps, &t[JCI_SIGMA_FCI64]));
@@ -1720,7 +1750,7 @@ static int use_tables(jci_ham *h)
 {
     JCI_CHECK(hipSetDevice(h->sp->ctx->device));
     RCHECK(ensure_tables(h));
-    h->tx_off = 1;
+    h->tx_off[0] = h->tx_off[1] = 1;
     return 0;
 }
 
@@ -1822,8 +1852,8 @@ JCI_API int jci_ham_contraction(jci_ham *h, int *use, long long *elems, long lon
         if (h->txmore_bytes > h->tx_cap) tx_drop(&h->d_txmore, &h->txmore_bytes);
     }
     if (want == 0) RCHECK(use_tables(h));
-    if (want == 1) h->tx_off = 0;
-    if (use) *use = h->tx && !h->tx_off;
+    if (want == 1) h->tx_off[0] = h->tx_off[1] = 0;
+    if (use) *use = h->tx && !h->tx_off[0] ? 1 : 0;
     if (elems) *elems = h->tx ? h->tx->elems : 0;
     if (bytes) *bytes = (long long)(h->txkeep_bytes + h->txmore_bytes);
     if (rounds) {
@@ -2496,7 +2526,7 @@ static int ham_sigma_cols(void *self, int method, int k, const double *V, long l
     jci_ham *h = (jci_ham *)self;
     method = resolve_method(h, method, 0);
     if (method == JCI_SIGMA_FAST64 || method == JCI_SIGMA_FAST32) {
-        if (h->have_fast && h->tx && !h->tx_off)
+        if (h->have_fast && h->tx && !h->tx_off[method == JCI_SIGMA_FAST32])
             return tx_sigma(h, method == JCI_SIGMA_FAST64 ? 64 : 32, k, V, 1, ldv, S, 1, lds, 1);
         // the table sigma reads determinant-major input and writes the columns directly
         RCHECK(jk_pack(k, h->sp->h.ndets, V, ldv, stage, h->sp->ctx->stream));
