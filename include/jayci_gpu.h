@@ -153,6 +153,8 @@ typedef struct jci_ham jci_ham;
 #define JCI_PAIRS_FP32 2    /* ... and/or with FP32 values */
 #define JCI_PAIRS_UPPER 4   /* store only j > i (symmetric sigma with atomics) */
 #define JCI_DIRECT_TABLES 8 /* per-string excitation tables for the matrix-free sigma */
+#define JCI_TABLE_KERNELS 16 /* with it: truncated spaces get the table kernels' doubles tables at
+                                creation and no contraction form (for instances of a batch) */
 
 #define JCI_SIGMA_AUTO 0
 #define JCI_SIGMA_PAIRS64 1
@@ -253,7 +255,8 @@ int jci_sigma(jci_ham *h, int method, int nvec, const double *x, double *y);
  * 128 MiB / (8 La) determinants in FP64).  All calls on one GPU share the array, so calls
  * that overlap on one GPU race; results equal jci_sigma_dev's bit for bit.  (Truncated spaces
  * that this size admits hold buffers of their own for this from creation on; no other call moves
- * or frees them but jci_ham_contraction with another *elems and jci_ham_destroy.) */
+ * or frees them once this one has used them but jci_ham_contraction with another *elems and
+ * jci_ham_destroy.) */
 int jci_sigma_dev_noalloc(jci_ham *h, int method, int nvec, const double *x_dev, double *y_dev);
 long long jci_sigma_noalloc_capacity(void);
 
@@ -362,7 +365,7 @@ int jci_ham_fast_split(jci_ham *h, int *split);
  * keeps; the values in use are returned */
 int jci_ham_fast_xcd(jci_ham *h, int *group, int *chunk_major);
 /* the two forms of the FAST methods on truncated spaces.  *use 1: products over the strings'
- * replacements (the default where the space has that form), 0: the table kernels, as the three
+ * replacements (the default where the space has that form; built where it was left out), 0: the table kernels, as the three
  * shapes above choose them; *elems > 0: that form in rounds of at most that many elements of its
  * intermediate per vector, or of one string's where that is more (default 256M, or the
  * determinants where they are more; plans anew and moves the buffers, so not while a captured
@@ -411,6 +414,10 @@ int jci_batch_set_tiles(jci_batch *b, int bn64, int bn32);
 int jci_batch_tune_tiles(jci_batch *b, jci_ham *h, int nvec, int reps, int *bn64, int *bn32);
 /* device bytes a slot of ndets determinants takes (basis, sigma and staging vectors) */
 long long jci_batch_bytes(long long ndets, int krymax);
+/* A truncated space's instance runs the table kernels in a batch: where the Hamiltonian was not
+ * created with JCI_TABLE_KERNELS their tables are built here, and its own FAST methods run them
+ * from then on, the contraction form's memory given back (jci_ham_contraction with *use 1 brings
+ * the form back; it stays where jci_sigma_dev_noalloc has used its buffers) */
 int jci_batch_add(jci_batch *b, jci_ham *h, const jci_solve_params *p, int *slot);
 /* the initial block of h's next jci_batch_add with parameters p, computed now (on h's
  * context, from any host thread that uses no other call on that context meanwhile), so that

@@ -16,7 +16,7 @@ LIB_PATH = os.path.join(HERE, "libjayci_gpu.so")
 HEADER = os.path.join(os.path.dirname(HERE), "include", "jayci_gpu.h")
 
 RULE_SERIAL, RULE_MRCISD = 0, 1
-PAIRS_FP64, PAIRS_FP32, PAIRS_UPPER, DIRECT_TABLES = 1, 2, 4, 8
+PAIRS_FP64, PAIRS_FP32, PAIRS_UPPER, DIRECT_TABLES, TABLE_KERNELS = 1, 2, 4, 8, 16
 (SIGMA_AUTO, SIGMA_PAIRS64, SIGMA_PAIRS32, SIGMA_PAIRS_SYM64, SIGMA_DIRECT64, SIGMA_DIRECT32,
  SIGMA_FAST64, SIGMA_FAST32, SIGMA_FCI64, SIGMA_FCI32, SIGMA_GEMM64, SIGMA_GEMM32) = range(12)
 NMETHODS = 12

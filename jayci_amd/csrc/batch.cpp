@@ -359,9 +359,8 @@ JCI_API int jci_batch_add(jci_batch *b, jci_ham *h, const jci_solve_params *p, i
     for (int i = 0; i < b->cap; i++) if (!b->in[i].used) { k = i; break; }
     if (k < 0) { jci_set_error("batch: no free slot"); return -1; }
     FastArgs fa;
-    RCHECK(jci_ham_fastargs(h, &fa));
+    RCHECK(jci_ham_fastargs(h, b->m1max, &fa));
     if (fa.W != b->W) { jci_set_error("batch: tile width of the Hamiltonian differs"); return -1; }
-    if (fa.m1 > b->m1max) { jci_set_error("batch: more orbitals than the batch was created for"); return -1; }
     BInst &s = b->in[k];
     s = BInst();
     s.h = h;

@@ -55,7 +55,8 @@ int jb_sigma(int prec, int W, int K, const BHeader *h, const BSigma *dS, int m1m
              hipStream_t st);
 
 // access to a Hamiltonian's matrix-free arguments (jci.cpp)
-int jci_ham_fastargs(jci_ham *h, FastArgs *out);
+// (m1max: orbital pairs the batch has room for)
+int jci_ham_fastargs(jci_ham *h, int m1max, FastArgs *out);
 const double *jci_ham_hd(jci_ham *h);
 long long jci_ham_ndets(jci_ham *h);
 jci_ctx *jci_ham_ctx(jci_ham *h);

@@ -305,6 +305,7 @@ struct jci_ham {
     TxPlan *tx;
     TxDev txd;
     int tx_off[2];              // FP64, FP32
+    int tx_pinned;              // the allocation-free entry point has used the kept block
     void *tx_mem[24];           // device arrays behind txd
     int tx_nmem;
     long long *d_ttx, nttx;     // 16 x 16 transpose tiles per block
@@ -887,7 +888,7 @@ static int tx_sigma(jci_ham *h, int prec, int nvec, const double *x, long long x
 // form build the doubles tables and the maps only when a table kernel is asked for.
 static int ensure_tables(jci_ham *h);
 
-static int build_fast(jci_ham *h, int W)
+static int build_fast(jci_ham *h, int W, int tables)
 {
     jci_space *s = h->sp;
     jci_ctx *c = s->ctx;
@@ -905,7 +906,7 @@ static int build_fast(jci_ham *h, int W)
     h->fast_xg = 64;
     const int widths[3] = {64, 128, 256};
     for (int wi = 0; wi < 3; wi++) h->fast[wi].W = widths[wi];
-    if (multi) {
+    if (multi && !tables) {
         // without memory for the contraction form the table kernels serve the space
         const int rc = build_tx(h);
         if (rc) drop_tx(h);
@@ -1090,7 +1091,7 @@ JCI_API int jci_ham_create(jci_space *s, const double *m1, const double *m2, int
         if (rc) { jci_ham_destroy(h); return rc; }
     }
     if (flags & JCI_DIRECT_TABLES) {
-        int rc = build_fast(h, 256);
+        int rc = build_fast(h, 256, flags & JCI_TABLE_KERNELS);
         if (rc) { jci_ham_destroy(h); return rc; }
     }
     JCI_CHECK(hipStreamSynchronize(c->stream));
@@ -1402,6 +1403,7 @@ static int fast_run(jci_ham *h, int method, int nvec, const double *x, double *y
         if (prec == 32) RCHECK(ensure_xf(h, N * nvec, s, &xf));
         RCHECK(jci_scratch_carve(s, (size_t)N * nvec * (prec == 64 ? sizeof(double) : sizeof(float)),
                                  &xT, "the transposed input"));
+        h->tx_pinned = 1;
         return tx_sigma(h, prec, nvec, x, nvec, 1, y, ys, yk, 0);
     }
     RCHECK(ensure_tables(h));
@@ -1825,12 +1827,17 @@ JCI_API int jci_ham_contraction(jci_ham *h, int *use, long long *elems, long lon
 {
     if (!h->have_fast) { jci_set_error("ham: no excitation tables"); return -1; }
     const int want = use ? *use : -1;
-    if (want > 1 || (want == 1 && !h->tx)) {
-        jci_set_error("ham: the space has no contraction form, or use %d not 0 or 1", want);
-        return -1;
+    if (want > 1) { jci_set_error("ham: use %d not 0 or 1", want); return -1; }
+    JCI_CHECK(hipSetDevice(h->sp->ctx->device));
+    if (want == 1 && !h->tx) {
+        const int rc = h->sp->h.nblk > 1 ? build_tx(h) : 0;
+        if (rc) {
+            drop_tx(h);
+            return rc;
+        }
+        if (!h->tx) { jci_set_error("ham: the space has no contraction form"); return -1; }
     }
     if (h->tx && elems && *elems > 0 && *elems != h->tx_elems) {
-        JCI_CHECK(hipSetDevice(h->sp->ctx->device));
         SpaceDesc T;
         jci_transpose_desc(h->sp->h, &T);
         TxPlan *P = new TxPlan();
@@ -2602,10 +2609,16 @@ int jci_ham_solve_op(jci_ham *h, const double *d_pre, SolveOp *op)
 }
 
 // ---- accessors for the batched engine ---------------------------------------------------------
-int jci_ham_fastargs(jci_ham *h, FastArgs *out)
+int jci_ham_fastargs(jci_ham *h, int m1max, FastArgs *out)
 {
     if (!h->have_fast) { jci_set_error("batch: the Hamiltonian has no excitation tables"); return -1; }
+    const int n = h->sp->h.norbs;
+    if (n * (n + 1) / 2 > m1max) { jci_set_error("batch: more orbitals than the batch was created for"); return -1; }
+    JCI_CHECK(hipSetDevice(h->sp->ctx->device));
     RCHECK(ensure_tables(h));
+    // the batch runs the table kernels: the contraction form's memory goes, unless a graph may
+    // hold its buffers
+    if (h->tx && !h->tx_pinned) drop_tx(h);
     *out = h->fast[2];            // the batched sigma uses 256-string beta tiles
     return 0;
 }

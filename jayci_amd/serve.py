@@ -26,7 +26,7 @@ from concurrent.futures import ThreadPoolExecutor
 import numpy as np
 
 from . import (Batch, Context, Hamiltonian, Space, DIRECT_TABLES, GUESS_DIAG, PREC_FP64,
-               RESTART_GDK, SYNTH_ENUC, contraction_plan, synth_integrals)
+               RESTART_GDK, SYNTH_ENUC, TABLE_KERNELS, contraction_plan, synth_integrals)
 
 
 def instance_spec(rng):
@@ -240,7 +240,8 @@ class Server:
         m1, m2 = synth_integrals(s["norbs"], r.seed)
         r.space = Space(self.bctx, s["na"], s["nb"], s["norbs"], s["ndocc"], s["nactv"],
                         s["xlvl"], s["rule"])
-        r.ham = Hamiltonian(r.space, m1, m2, DIRECT_TABLES)
+        # (the batch's kernels only, built here rather than at admission)
+        r.ham = Hamiltonian(r.space, m1, m2, DIRECT_TABLES | TABLE_KERNELS)
         r.params = self._params(r)
         r.ham.prepare_guess(r.params)
 
