@@ -16,7 +16,7 @@ typedef double DvTwo __attribute__((ext_vector_type(2), aligned(8)));
 // Columns past the last repeat it (their products are not written).
 //
 // Bound by the reads of A and B (m <= 64 columns: at most 16 products per element read).  Gram
-// products of a three-root solve of 6a6b in 14 orbitals: 150 launches of 9.2 -> 1.9 ms in all
+// products of a two-root solve (one buffer pair) of 6a6b in 14 orbitals: 150 launches of 9.2 -> 1.9 ms in all
 // (32-row tiles through LDS, one work-group per 2048 rows, before); of a batch of 12 full-CI
 // solves in 8 to 12 orbitals: 8.4 -> 5.6 ms.
 template <int MT, int WT>

@@ -41,3 +41,18 @@ template <> struct Mf<float> {
     static __device__ __forceinline__ int row(int l, int v) { return 4 * (l / 16) + v; }
     static constexpr int LROW = 4, VROW = 1;
 };
+
+__device__ __forceinline__ void wave_sync()
+{
+    // LDS accesses of one wave execute in order; this keeps the compiler from moving them
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// a value that all lanes share, in scalar registers (divisions leave theirs in vector registers)
+__device__ __forceinline__ int wave_uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ long long wave_uni(long long v)
+{
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)v);
+    return (long long)(int)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | lo;
+}

@@ -413,20 +413,6 @@ template <> struct GeL<float> {
         return __int_as_float(__float_as_int(v) ^ (int)(e & 0x80000000u));
     }
 };
-__device__ __forceinline__ void gf_wave_sync()
-{
-    // LDS accesses of one wave execute in order; this keeps the compiler from moving them
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-// a value that all lanes share, in scalar registers (divisions leave theirs in vector registers)
-__device__ __forceinline__ int gf_uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ long long gf_uni(long long v)
-{
-    const unsigned lo = __builtin_amdgcn_readfirstlane((int)v);
-    return (long long)(int)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | lo;
-}
 
 // element i past a uniform pointer, by a 32-bit offset per lane
 template <typename T>
@@ -484,7 +470,7 @@ __device__ __forceinline__ void gE_span(const GfTask &t, long long r, int Ja, in
     T *Dt = (T *)gf_smem + dofs;                   // two tiles of 16 columns
     const T *xs = (const T *)gf_smem + xo;         // staged row (ST; else gathered from memory)
     const GemmFci &g = t.g;
-    const int La = gf_uni(g.La), nb = gf_uni((int)g.nb);
+    const int La = wave_uni(g.La), nb = wave_uni((int)g.nb);
     T a[RT][KS];
 #pragma unroll
     for (int i = 0; i < RT; i++) {
@@ -508,9 +494,9 @@ __device__ __forceinline__ void gE_span(const GfTask &t, long long r, int Ja, in
             for (int q = 0; q < VK; q++) ar[s * VK + q] = v[q];
         }
     }
-    const auto lb = gptr((const uint32_t *)gf_uni((long long)g.lb));
-    const auto xr = gptr((const T *)gf_uni((long long)xg));
-    const auto E = gptr_w((T *)gf_uni((long long)t.E)) + r * La * nb;
+    const auto lb = gptr((const uint32_t *)wave_uni((long long)g.lb));
+    const auto xr = gptr((const T *)wave_uni((long long)xg));
+    const auto E = gptr_w((T *)wave_uni((long long)t.E)) + r * La * nb;
     // rows of a lane: LROW * part + VROW * v, in the last row tile up to the last one
     const uint32_t eofs = (uint32_t)(Mf<T>::LROW * part * nb);
     uint32_t elast[4];
@@ -564,7 +550,7 @@ __device__ __forceinline__ void gE_span(const GfTask &t, long long r, int Ja, in
     for (int i = 0; i < NL / 4; i++) fetch(std::min(tile0 + 1, tile1 - 1), i);
 #pragma unroll
     for (int j = 0; j < NL; j++) get(j);
-    gf_wave_sync();
+    wave_sync();
 #pragma unroll
     for (int j = 0; j < NL; j++) put(Dt + col * LDC, j);
 #pragma unroll
@@ -572,7 +558,7 @@ __device__ __forceinline__ void gE_span(const GfTask &t, long long r, int Ja, in
     cres = (uint32_t)std::min(tile0 * 16 + col, nb - 1);
     int cur = 0;
     for (int tile = tile0; tile < tile1; tile++) {
-        gf_wave_sync();
+        wave_sync();
         const T *b0 = Dt + cur + col * LDC + part * KS;
         T *Dn = Dt + (16 * LDC - cur);
 #pragma unroll
@@ -689,12 +675,12 @@ __device__ __forceinline__ void gf_opposite(const GfHeader *__restrict__ H,
         }
         const long long w1 = u + ((end - u) * (w + 1) >> 2);
         for (long long q = u + ((end - u) * w >> 2); q < w1;) {
-            const long long r = gf_uni((q - base) / per);
-            const int k = gf_uni((int)(r / g.na)), Ja = gf_uni((int)(r - k * g.na));
+            const long long r = wave_uni((q - base) / per);
+            const int k = wave_uni((int)(r / g.na)), Ja = wave_uni((int)(r - k * g.na));
             const int un = (int)(q - base - r * per), m = (int)std::min<long long>(w1 - q, per - un);
-            const int xo = gf_uni(room > 0 ? 4 * dw + (int)(r - r0) * (int)g.nb : -1);
+            const int xo = wave_uni(room > 0 ? 4 * dw + (int)(r - r0) * (int)g.nb : -1);
             const T *xg = xin<T>(t, k) + Ja * g.nb;
-            const int t0 = gf_uni(un * S), t1 = gf_uni(std::min(nct, (un + m) * S)), dofs = gf_uni(w * dw);
+            const int t0 = wave_uni(un * S), t1 = wave_uni(std::min(nct, (un + m) * S)), dofs = wave_uni(w * dw);
             gE_shape<T>(t, r, Ja, ex, t0, t1, xo, xg, dofs);
             q += m;
         }

@@ -717,21 +717,6 @@ __device__ __forceinline__ void tx_mma(typename Mf<T>::acc *acc, const T (*a)[KS
     }
 }
 
-__device__ __forceinline__ void tx_wave_sync()
-{
-    // LDS accesses of one wave execute in order; this keeps the compiler from moving them
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-// a value that all lanes share, in scalar registers
-__device__ __forceinline__ int tx_uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ long long tx_uni(long long v)
-{
-    const unsigned lo = __builtin_amdgcn_readfirstlane((int)v);
-    return (long long)(int)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | lo;
-}
-
 // what one wave works on: one JL, one external part w, row tiles from r0, vectors k0 .. k1 - 1
 struct TxUnit {
     int ja, w, r0, nrt, dr;          // dr: row of the diagonal pairs relative to r0 (or outside)
@@ -755,7 +740,7 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
     asm volatile("" : "+s"(u.w));
     asm volatile("" : "+s"(u.r0));
     const int col = l & 15, part = l >> 4;
-    const int La = tx_uni(t.La), nIp = tx_uni(t.nIp);
+    const int La = wave_uni(t.La), nIp = wave_uni(t.nIp);
 
     // integral fragments: row r0 + 16 i + col, steps part * KS .. part * KS + KS - 1
     T a[RT][KS];
@@ -800,7 +785,7 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
                         for (int h = 0; h < (KC > 64 ? 2 : 1); h++)
                             if (l + 64 * h < KC) Dt[(g + j) * LDC + l + 64 * h] = v[j][h];
                 }
-                tx_wave_sync();
+                wave_sync();
                 if (u.dr >> 4 == i && u.dr >= 0) {
                     // the external electrons of JL add to its diagonal row
                     for (uint64_t z = A.nint >= 64 ? 0 : SL.mask[J] >> A.nint << A.nint; z; z &= z - 1) {
@@ -810,7 +795,7 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
                         for (int h = 0; h < (KC > 64 ? 2 : 1); h++)
                             if (l + 64 * h < KC) Dt[(u.dr & 15) * LDC + l + 64 * h] += tx_at(Mr, Q[h]);
                     }
-                    tx_wave_sync();
+                    wave_sync();
                 }
             }
 #pragma unroll
@@ -822,15 +807,15 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
                     for (int ii = 0; ii < RT; ii++)
                         if (ii == i) a[ii][s + q] = TxV<T>::at(v, q);
             }
-            tx_wave_sync();
+            wave_sync();
         }
     }
 
     // list of external part w; a lane reads row `part` of four, column `col` of a tile
-    const uint32_t *__restrict__ lst = A.s[1 - t.o].lst + tx_uni(t.lbase + (long long)u.w * t.lrows * nIp);
+    const uint32_t *__restrict__ lst = A.s[1 - t.o].lst + wave_uni(t.lbase + (long long)u.w * t.lrows * nIp);
     const uint32_t lofs = (uint32_t)(part * nIp + col);
     // vector base, list row and chunk steps of slot j in lane j (chunks hold at most 64 slots)
-    const int nsl = tx_uni(ch.nslot);
+    const int nsl = wave_uni(ch.nslot);
     int vxl, vxh, vlo, vki;
     {
         const TxSlot &q = A.slot[ch.slot0 + std::min(l, nsl - 1)];
@@ -842,8 +827,8 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
     }
     T *Dc = Dt + col * LDC;
     const uint32_t jm = (1u << TX_JBITS) - 1;
-    const int tile0 = tx_uni(it.t0), tile1 = tile0 + tx_uni(it.nt);
-    const int p0 = tx_uni(it.p0), ntc = tx_uni(it.pn) * 16;
+    const int tile0 = wave_uni(it.t0), tile1 = tile0 + wave_uni(it.nt);
+    const int p0 = wave_uni(it.p0), ntc = wave_uni(it.pn) * 16;
     // a lane's rows are LROW * part + VROW v + 16 i from r0: one offset per lane, the rest scalar
     const uint32_t eofs = (uint32_t)(Mf<T>::LROW * part * ntc + col);
     const int rleft = La - u.r0 - Mf<T>::LROW * part;
@@ -888,7 +873,7 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
             }
         for (int tile = tile0; tile < tile1; tile++) {
             for (int z = l; z < LDC * (int)sizeof(T); z += 64) ((V *)Dt)[z] = zv;
-            tx_wave_sync();
+            wave_sync();
 #pragma unroll
             for (int g = 0; g < NP; g++)
                 if (4 * g < nsl) puts(4 * g, le + 4 * g, xv + 4 * g);
@@ -899,7 +884,7 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
                 values(j, e, v);
                 puts(j, e, v);
             }
-            tx_wave_sync();
+            wave_sync();
             // entries and vector elements of the next tile, behind the products below
 #pragma unroll
             for (int g = 0; g < NP; g++)
@@ -924,7 +909,7 @@ __device__ __forceinline__ void tx_eab(const TxDev &A, const TxItem &it, const T
             const T *b0 = Dc + part * KS;
             if (u.nrt == 1) tx_mma<T, 1, KS>(acc, a, b0);
             else if (u.nrt == 2) tx_mma<T, RT, KS>(acc, a, b0);
-            tx_wave_sync();
+            wave_sync();
 #pragma unroll
             for (int i = 0; i < RT; i++)
 #pragma unroll
