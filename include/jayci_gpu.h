@@ -163,9 +163,9 @@ typedef struct jci_ham jci_ham;
 #define JCI_SIGMA_DIRECT64 4
 #define JCI_SIGMA_DIRECT32 5
 #define JCI_SIGMA_FAST64 6  /* matrix-free, FP64: spaces of several blocks by dense products
-                               over their strings' replacements on MFMA, the others (and
-                               after jci_ham_fast_tiles / _split / _xcd set a shape) from
-                               excitation tables */
+                               over their strings' replacements on MFMA where that is the
+                               faster form, the others (and after jci_ham_fast_tiles / _split
+                               / _xcd set a shape) from excitation tables */
 #define JCI_SIGMA_FAST32 7  /* ... FP32 products and sums */
 #define JCI_SIGMA_FCI64 8   /* matrix-free, single-block (FCI) spaces, n <= 16, FP64 */
 #define JCI_SIGMA_FCI32 9   /* ... FP32 accumulation */

@@ -708,6 +708,7 @@ int tx_plan(const SpaceDesc &D, const SpaceDesc &T, ll budget, TxPlan *P)
     for (int s = 0; s < 2; s++) {
         if (plan_lists(D, D.s[s], P->lists[s], &P->nlst[s])) return 1;
         if (plan_pairs(D, D.s[s], P->pg[s], &P->nkl[s])) return 1;
+        if (P->nlst[s] / 256 >= TX_GRID) return 1;   // one thread an entry fills them
         ll n = 0;
         for (int g = 0; g < D.s[s].ngrp; g++) {
             P->iI0[s][g] = (int)n;
