@@ -1855,8 +1855,12 @@ JCI_API int jci_ham_contraction(jci_ham *h, int *use, long long *elems, long lon
         h->tx = P;
         h->tx_elems = *elems;
         tx_drop(&h->d_txmore, &h->txmore_bytes);
-        RCHECK(tx_tables(h));
-        RCHECK(tx_keep(h));
+        int rc = tx_tables(h);
+        if (!rc) rc = tx_keep(h);
+        if (rc) {
+            drop_tx(h);
+            return rc;
+        }
     }
     if (bytes && *bytes > 0) {
         h->tx_cap = (size_t)*bytes;
